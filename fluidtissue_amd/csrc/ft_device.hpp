@@ -1,6 +1,6 @@
 // ft_device.hpp -- device-side building blocks shared by the reinit kernels:
-// bit tests, wave64/block scans, Morton codes, box bounds and the
-// point/triangle distance functions.
+// bit tests, wave64/block scans, Morton codes and the point/triangle
+// distance functions.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -52,6 +52,25 @@ __device__ __forceinline__ uint32_t shfl_up_any(uint32_t v, int d, int width = k
 __device__ __forceinline__ uint64_t shfl_up_any(uint64_t v, int d, int width = kWave)
 {
     return shfl_up_u64(v, d, width);
+}
+
+// Five 32-bit counters scanned together (the index's levels): a = primitives
+// and level-1 nodes, b = level 2 and level 3, c = level 4; low halves first.
+struct Lv {
+    uint64_t a, b, c;
+    Lv() = default;
+    __device__ explicit Lv(int v) : a((uint64_t)v), b((uint64_t)v), c((uint64_t)v) {}
+    __device__ Lv& operator+=(const Lv& o) { a += o.a; b += o.b; c += o.c; return *this; }
+    __device__ Lv operator+(const Lv& o) const { Lv r = *this; r += o; return r; }
+    __device__ Lv operator-(const Lv& o) const { Lv r = *this; r.a -= o.a; r.b -= o.b; r.c -= o.c; return r; }
+};
+__device__ __forceinline__ Lv shfl_up_any(const Lv& v, int d, int width = kWave)
+{
+    Lv r;
+    r.a = shfl_up_u64(v.a, d, width);
+    r.b = shfl_up_u64(v.b, d, width);
+    r.c = shfl_up_u64(v.c, d, width);
+    return r;
 }
 
 template <class T>
@@ -111,6 +130,8 @@ struct Grid {
     float inv_b;          // 1 / bin edge
     int dim[3];
     float h;              // the field's node spacing
+    float org[3], inv_s;  // scaled coordinates of the index's boxes: (p - org) inv_s
+    int root_lv;          // level of the field's tree root
 };
 
 __device__ __forceinline__ uint32_t grid_code(const Grid& g, float x, float y, float z)
@@ -139,50 +160,12 @@ __device__ __forceinline__ int field_of(const int64_t* off, int nf, int64_t x)
     return lo;
 }
 
-// Squared distance from x to an axis-aligned box (0 inside).
-__device__ __forceinline__ float box_dist2(float x, float y, float z, const float* lo,
-                                           const float* hi)
-{
-    const float dx = fmaxf(fmaxf(lo[0] - x, x - hi[0]), 0.0f);
-    const float dy = fmaxf(fmaxf(lo[1] - y, y - hi[1]), 0.0f);
-    const float dz = fmaxf(fmaxf(lo[2] - z, z - hi[2]), 0.0f);
-    return __fmaf_rn(dz, dz, __fmaf_rn(dy, dy, dx * dx));
-}
-
-// ---- bounding volumes --------------------------------------------------------
-// An axis-aligned box plus a cylinder (centre c, unit axis n, radius rho,
-// half-thickness tau) that both contain every primitive below a tree node.
-// A patch of a smooth surface lies in a thin cylinder around its normal, so
-// for a node far away the cylinder bound is close to the true distance where
-// the box bound is loose by about the patch size.  tau < 0: no cylinder.
-struct __align__(16) Bound {
-    float lo[3], hi[3];
-    float c[3], n[3];
-    float rho, tau;
-    float pad[2];
-};
-
 // Square root for lower bounds only: the hardware v_sqrt_f32 (within 1 ulp),
 // not the correctly rounded sequence the build flags give sqrtf.  Every bound
 // that uses it subtracts a relative slack of 2^-20 or more afterwards, which
 // covers the 2^-23 relative error; a flushed tiny input gives 0, still a
 // lower bound.
 __device__ __forceinline__ float sqrt_lb(float x) { return __builtin_amdgcn_sqrtf(x); }
-
-__device__ __forceinline__ float cyl_dist2(float x, float y, float z, const Bound& b)
-{
-    if (b.tau < 0.0f) return 0.0f;
-    const float dx = x - b.c[0], dy = y - b.c[1], dz = z - b.c[2];
-    const float hn = __fmaf_rn(dz, b.n[2], __fmaf_rn(dy, b.n[1], dx * b.n[0]));
-    const float cx = __fmaf_rn(b.n[1], dz, -b.n[2] * dy);
-    const float cy = __fmaf_rn(b.n[2], dx, -b.n[0] * dz);
-    const float cz = __fmaf_rn(b.n[0], dy, -b.n[1] * dx);
-    const float lat = sqrt_lb(__fmaf_rn(cz, cz, __fmaf_rn(cy, cy, cx * cx)));
-    const float slack = 0x1.0p-20f * (fabsf(hn) + lat);     // rounding of hn and lat
-    const float a = fmaxf(fabsf(hn) - b.tau - slack, 0.0f);
-    const float r = fmaxf(lat - b.rho - slack, 0.0f);
-    return __fmaf_rn(r, r, a * a);
-}
 
 // ---- FP64 vector helpers (index build, FP64 settle) -------------------------
 __device__ inline double dot3d(const double* u, const double* v)
@@ -253,82 +236,44 @@ __device__ inline double tri_dist2_f64(const float* x, const float* a, const flo
 }
 
 // ---- FP32 point-triangle distance -------------------------------------------
-// Triangle record (80 B), an orthonormal frame at vertex a, built in FP64 when
-// the index is built, with u along ab (the longest edge) and n the unit
-// normal; in it the triangle is (0,0), (B,0), (Cx,Cy), Cy >= 0:
-//   F0 = (a, +-R)  F1 = (u, B)  F2 = (v, n.x)  F3 = (n.y, n.z, Cx, Cy)
-//   F4 = (1/B, 1/|ac|^2, 1/|bc|^2, Cx - B)
-// (inverse lengths are 0 for zero-length edges; R is the radius, rounded up,
-// of the disk about the midpoint of ab that holds the triangle; its sign is
-// negative for collinear vertices, which have no interior and whose distance
-// is that of the edge segments).  The culling test reads F0-F3 only, one
-// contiguous run of scalar loads.  The point is
-// projected once (X, Y, Z); the in-plane distance is 0 inside the triangle,
-// else the nearest clamped edge projection; d^2 = d2D^2 + Z^2.  With ab the
-// longest edge the 2D problem stays well conditioned however thin the
-// triangle is, so no case needs FP64 at query time.
+// Triangle record (80 B): an orthonormal frame at vertex a, built in FP64
+// when the index is built, with u along ab (the longest edge), the unit normal
+// n and v = n x u; in it the triangle is (0,0), (B,0), (Cx,Cy), Cy >= 0:
+//   a = (a, Cx - B)  u = (u, B)  v = (v, Cx)  n = (n, Cy)
+//   i = (1/B, 1/|ac|^2, 1/|bc|^2, id)
+// (inverse lengths are 0 for zero-length edges; id as bits, the top one set
+// for collinear vertices, which have no interior and whose distance is that
+// of the edge segments).  The point is projected once (X, Y, Z); the in-plane
+// distance is 0 inside the triangle, else the nearest clamped edge
+// projection; d^2 = d2D^2 + Z^2.  With ab the longest edge the 2D problem
+// stays well conditioned however thin the triangle is, so no case needs FP64
+// at query time.
 struct TriRec {
-    float4 F0, F1, F2, F3, F4;
+    float4 a, u, v, n, i;
 };
+__device__ __forceinline__ int32_t tri_id(const TriRec& r) { return __float_as_int(r.i.w) & INT32_MAX; }
 
-// Projection of the point into the triangle's frame.
-struct TriProj {
-    float X, Y, Z;
-};
-__device__ __forceinline__ TriProj tri_project(float x, float y, float z, const TriRec& r)
+__device__ __forceinline__ float tri_dist2(float x, float y, float z, const TriRec& r)
 {
-    const float wx = x - r.F0.x, wy = y - r.F0.y, wz = z - r.F0.z;
-    TriProj p;
-    p.X = __fmaf_rn(wz, r.F1.z, __fmaf_rn(wy, r.F1.y, wx * r.F1.x));
-    p.Y = __fmaf_rn(wz, r.F2.z, __fmaf_rn(wy, r.F2.y, wx * r.F2.x));
-    p.Z = __fmaf_rn(wz, r.F3.y, __fmaf_rn(wy, r.F3.x, wx * r.F2.w));
-    return p;
-}
-
-// Squared distance to the rectangle [0, B] x [0, Cy] of the triangle's frame,
-// which holds it: ab is the longest edge, so C projects inside [0, B], and
-// Cy >= 0 (0 for collinear vertices, a segment).  Tighter than a disk about
-// the triangle for thin triangles, and with no square root.  As computed it
-// may exceed the exact value by its rounding, within a relative 2^-18: the
-// caller compares it with a bound raised by that much (rect_bound).
-__device__ __forceinline__ float tri_rect_d2(const TriProj& p, const TriRec& r)
-{
-    const float dx = fmaxf(fmaxf(-p.X, p.X - r.F1.w), 0.0f);
-    const float dy = fmaxf(fmaxf(-p.Y, p.Y - r.F3.w), 0.0f);
-    return __fmaf_rn(dx, dx, __fmaf_rn(dy, dy, p.Z * p.Z));
-}
-
-// The bound to compare tri_rect_d2 with: b (1 + 2^-17), which after rounding
-// is still at least b / (1 - 2^-18), so that d2 (1 - 2^-18) <= b implies
-// d2 <= rect_bound(b).  Computed once per change of b, not per triangle.
-__device__ __forceinline__ float rect_bound(float b) { return b * (1.0f + 0x1.0p-17f); }
-
-// Larger of two non-negative floats (squared distances): ordered as their
-// bit patterns, so one integer max gives fmaxf's value without the NaN
-// canonicalisation fmaxf costs.
-__device__ __forceinline__ float max_nonneg(float a, float b)
-{
-    return __int_as_float(max(__float_as_int(a), __float_as_int(b)));
-}
-
-__device__ __forceinline__ float tri_dist2_from(const TriProj& p, const TriRec& r)
-{
-    const float X = p.X, Y = p.Y, Z = p.Z;
-    const float B = r.F1.w, Cx = r.F3.z, Cy = r.F3.w, dCx = r.F4.w;
+    const float wx = x - r.a.x, wy = y - r.a.y, wz = z - r.a.z;
+    const float X = __fmaf_rn(wz, r.u.z, __fmaf_rn(wy, r.u.y, wx * r.u.x));
+    const float Y = __fmaf_rn(wz, r.v.z, __fmaf_rn(wy, r.v.y, wx * r.v.x));
+    const float Z = __fmaf_rn(wz, r.n.z, __fmaf_rn(wy, r.n.y, wx * r.n.x));
+    const float B = r.u.w, Cx = r.v.w, Cy = r.n.w, dCx = r.a.w;
     const float xb = X - B;
     const bool inside = (int)(Y >= 0.0f) & (int)(__fmaf_rn(Cy, X, -Cx * Y) >= 0.0f) &
-                        (int)(__fmaf_rn(dCx, Y, -Cy * xb) >= 0.0f) & (int)(r.F0.w > 0.0f);
+                        (int)(__fmaf_rn(dCx, Y, -Cy * xb) >= 0.0f) & (int)(__float_as_int(r.i.w) >= 0);
     // edge ab
-    float t = fminf(fmaxf(X * r.F4.x, 0.0f), 1.0f);
+    float t = fminf(fmaxf(X * r.i.x, 0.0f), 1.0f);
     float ex = __fmaf_rn(-t, B, X);
     float d = __fmaf_rn(Y, Y, ex * ex);
     // edge ac
-    t = fminf(fmaxf(__fmaf_rn(Y, Cy, X * Cx) * r.F4.y, 0.0f), 1.0f);
+    t = fminf(fmaxf(__fmaf_rn(Y, Cy, X * Cx) * r.i.y, 0.0f), 1.0f);
     ex = __fmaf_rn(-t, Cx, X);
     float ey = __fmaf_rn(-t, Cy, Y);
     d = fminf(d, __fmaf_rn(ey, ey, ex * ex));
     // edge bc
-    t = fminf(fmaxf(__fmaf_rn(Y, Cy, xb * dCx) * r.F4.z, 0.0f), 1.0f);
+    t = fminf(fmaxf(__fmaf_rn(Y, Cy, xb * dCx) * r.i.z, 0.0f), 1.0f);
     ex = __fmaf_rn(-t, dCx, xb);
     ey = __fmaf_rn(-t, Cy, Y);
     d = fminf(d, __fmaf_rn(ey, ey, ex * ex));

@@ -18,9 +18,9 @@
 //                     rule, normal lengths                   (LevelSet.cpp:330-347, 393-399)
 //   9 p2t / area      per-point triangle lists (CSR, ascending) and the
 //                     ordered area sums                      (LevelSet.cpp:349-356)
-//  10 index           uniform-bin counting sort of the primitives (points or
-//                     triangles), leaves = non-empty bins in Morton order,
-//                     binary radix tree over the leaves
+//  10 index           primitives (points or triangles) sorted by uniform bin,
+//                     leaves = non-empty bins in Morton order, 64-ary tree of
+//                     oriented boxes over the leaves
 //  11 schedule        64-node tiles deep inside the surface listed first
 //                     (k_tile_deep, scan, k_tile_list; full domain only)
 //  12 k_query         per node (Morton-sorted order): exact nearest primitive
@@ -52,13 +52,11 @@
 
 using ftd::Grid;
 using ftd::TriRec;
-using ftd::Bound;
 
 namespace {
 
 constexpr int kBS = 256;                 // threads per block of the streaming kernels
 constexpr int kScanTile = 2048;          // elements per scan block (256 x 8)
-constexpr int kStack = 24;               // traversal stack depth (tree depth <= 24)
 constexpr int kMaxBinsLog2PerAxis = 8;   // <= 256 bins per axis, 2^24 Morton cells
 
 #define FT_HIP(call)                                                                   \
@@ -81,17 +79,15 @@ inline unsigned grid1d(int64_t n, int bs = kBS) { return (unsigned)((n + bs - 1)
 //   S_BLK    (crossing tets << 32) | triangles
 //   S_EDGES  crossing points (low 32 bits)
 //   S_ERR    ~0, or (code << 40) | first failing tet
-//   S_BINS   (leaves << 32) | primitives
+//   S_BINS   leaves of the index (low 32 bits)
 //   S_DEEP   query tiles scheduled first (low 32 bits), of which the very deep
 //            ones, split over several waves (high 32 bits)
-//   S_OVF    traversal stack/budget overflow of the query
 //   S_CAP    a stage total exceeded the capacity its buffers were sized for
 //   S_Q      the query's work-queue counters (9 x u32: deep tiles, then one
 //            per XCD), zeroed per launch
-//   S_MARGIN the bins schedule: largest distance from a triangle's centroid to
-//            its vertices (float bits, low 32)
-enum Slot { S_BLK = 0, S_EDGES = 1, S_ERR = 2, S_P2T = 3, S_BINS = 4, S_DEEP = 5, S_OVF = 6, S_CAP = 7,
-            S_Q = 8, S_MARGIN = 13, S_N = 14 };
+//   S_LV     3 slots: primitives and tree nodes per level (ftd::Lv)
+enum Slot { S_BLK = 0, S_EDGES = 1, S_ERR = 2, S_P2T = 3, S_BINS = 4, S_DEEP = 5, S_CAP = 6,
+            S_Q = 7, S_LV = 12, S_N = 15 };
 
 // Stage totals of the running reinit as the kernels see them.  Kernels after
 // a scan read the total from the device, so a launch sized for a capacity
@@ -99,7 +95,7 @@ enum Slot { S_BLK = 0, S_EDGES = 1, S_ERR = 2, S_P2T = 3, S_BINS = 4, S_DEEP = 5
 __device__ __forceinline__ int64_t cnt_xtets(const uint64_t* sc) { return (int64_t)(sc[S_BLK] >> 32); }
 __device__ __forceinline__ int64_t cnt_tris(const uint64_t* sc) { return (int64_t)(sc[S_BLK] & 0xffffffffull); }
 __device__ __forceinline__ int64_t cnt_points(const uint64_t* sc) { return (int64_t)(sc[S_EDGES] & 0xffffffffull); }
-__device__ __forceinline__ int64_t cnt_leaves(const uint64_t* sc) { return (int64_t)(sc[S_BINS] >> 32); }
+__device__ __forceinline__ int64_t cnt_leaves(const uint64_t* sc) { return (int64_t)(sc[S_BINS] & 0xffffffffull); }
 // Set once a stage failed (t2e or degenerate tet) or outgrew its buffers:
 // every later kernel of the reinit then does nothing and phi stays as it was.
 __device__ __forceinline__ bool halted(const uint64_t* sc)
@@ -178,9 +174,6 @@ struct LoadSame {
 struct LoadPopc {  // u64 bitmap word -> popcount
     __device__ uint32_t operator()(uint64_t v) const { return (uint32_t)__popcll(v); }
 };
-struct LoadNonEmpty {  // bin count -> (non-empty << 32) | count
-    __device__ uint64_t operator()(uint32_t c) const { return ((uint64_t)(c > 0) << 32) | c; }
-};
 struct LoadTileClass {  // tile class 0 / 1 deep / 2 very deep -> (very deep << 32) | deep
     __device__ uint64_t operator()(uint32_t c) const { return ((uint64_t)(c == 2) << 32) | (uint64_t)(c >= 1); }
 };
@@ -205,7 +198,7 @@ template <class TO>
 __global__ __launch_bounds__(1024) void k_scan_top(TO* bsum, int64_t nb, TO* total)
 {
     __shared__ TO lds[1024 / 64 + 1];
-    TO carry = 0;
+    TO carry = TO(0);
     for (int64_t c = 0; c < nb; c += 1024) {
         const int64_t i = c + threadIdx.x;
         const TO v = i < nb ? bsum[i] : TO(0);
@@ -691,18 +684,71 @@ __global__ __launch_bounds__(kBS) void k_point_area(const uint32_t* off, uint64_
 }
 
 // ============================================================================
-// Spatial index: uniform bins by counting sort, binary radix tree on bins
+// Spatial index: uniform bins as a bitmap, 64-ary tree of oriented boxes
 // ============================================================================
-// Leaves per block of the local refit pass: a node whose leaf range stays
-// inside one block is fitted by that block's workgroup; the rest ("top"
-// nodes) by the single-workgroup pass after it.
-constexpr int kRefitBlock = 256;
+// The bins of a field are numbered along the Morton curve, one bit each.  A
+// 64-bit word of the bitmap is then a 4 x 4 x 4 block of bins, and words of
+// words are the larger blocks: the tree has one node per non-empty block and
+// its children (at most 64) are consecutive in the Morton order of the
+// non-empty bins.  Leaves (non-empty bins) and nodes of all levels share one
+// numbering, level by level (LevelOff), so first[g], first[g + 1] is a
+// node's range of children, or a leaf's range of primitives.
+//
+// Nothing here grows with the bins but the bitmap and its prefix (12 bytes
+// per 64 bins): at 256^3, 2^24 bins, clearing, scanning and compacting
+// one counter per bin took 0.30 ms of a reinit; the bitmap's take 0.03 ms.
+constexpr int kNodeBlocks = 2048;            // workgroups of a node level (waves take nodes in turn)
+constexpr int kLevels = 5;                   // leaves and 4 levels of nodes (2^24 bins per field)
 
-struct __align__(16) BNode {  // child bounds, children, parent
-    Bound l, r;
-    int32_t left, right, parent;
-    int32_t top;                 // 1: the leaf range spans refit blocks
+struct LevelOff {
+    uint32_t off[kLevels];                   // first index of each level
 };
+
+// Bounding volume of a primitive, a leaf or a node as the search reads it: a
+// box with unit axes x, y, z and half extents e, in the field's scaled
+// coordinates p' = (p - org) inv_s.  Row k = (axis, offset) applied to (p', 1)
+// is p's coordinate along axis k from the box centre, so four boxes are 16
+// rows (the fourth of each, its extents, is a spare one) of a 16 x 16 matrix
+// product and 16 nodes its columns.
+//
+// A row is kept as eight halves (axis, offset) + (axis, offset): each value
+// is the sum of its nearest half and the half of what is left, 22 bits, and
+// the node's coordinates are split the same way.  The 16 terms of a row's
+// product are then exact in the f16 matrix instruction's FP32 sum, which
+// leaves 2^-22.8 of a scaled unit at most (measured over random boxes and
+// nodes; 2^-23.9 for the FP32 instruction); the search allows 2^-20.  The FP32
+// instruction 16x16x4 holds the vector unit for its 32 cycles (4 of them and
+// 32 fma: 290 cycles per wave on a full SIMD, 136 and 138 each alone); the f16
+// 16x16x16 runs beside it (153 cycles with the same 32 fma).
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+struct __align__(16) Row {
+    v4h hi, lo;
+};
+struct __align__(16) Item {
+    Row x, y, z;
+    float4 e;                                // half extents (scaled), 0
+};
+__device__ __forceinline__ Row make_row(float x, float y, float z, float w)
+{
+    Row r;
+    r.hi = v4h{(_Float16)x, (_Float16)y, (_Float16)z, (_Float16)w};
+    r.lo = v4h{(_Float16)(x - (float)r.hi[0]), (_Float16)(y - (float)r.hi[1]), (_Float16)(z - (float)r.hi[2]),
+               (_Float16)(w - (float)r.hi[3])};
+    return r;
+}
+__device__ __forceinline__ float4 row_values(const Row& r)
+{
+    return make_float4((float)r.hi[0] + (float)r.lo[0], (float)r.hi[1] + (float)r.lo[1],
+                       (float)r.hi[2] + (float)r.lo[2], (float)r.hi[3] + (float)r.lo[3]);
+}
+// The item that admits every point.
+__device__ __forceinline__ Item open_item()
+{
+    Item it;
+    it.x = it.y = it.z = make_row(0.0f, 0.0f, 0.0f, 0.0f);
+    it.e = make_float4(1e30f, 1e30f, 1e30f, 0.0f);
+    return it;
+}
 
 __device__ __forceinline__ void tri_vertices(const int4* tris, const float* ifp, int32_t f,
                                              float* a, float* b, float* c)
@@ -716,16 +762,18 @@ __device__ __forceinline__ void tri_vertices(const int4* tris, const float* ifp,
     }
 }
 
-// Index geometry of one reinit: per-field grids and counter offsets, the
-// field of a crossing point through its edge (edge_off), and the key layout
-// (field << code_bits) | Morton code.
+// Index geometry of one reinit: per-field grids and bin offsets (multiples
+// of 64), the field of a crossing point through its edge (edge_off).
 struct IndexGeom {
     const int64_t* edge_off;         // nf + 1
     const int64_t* cnt_off;          // nf + 1
     const Grid* grids;               // nf
     int nf;
-    int code_bits;
 };
+__device__ __forceinline__ int bin_field(const IndexGeom& ig, uint32_t c)
+{
+    return ig.nf > 1 ? ftd::field_of(ig.cnt_off, ig.nf, (int64_t)c) : 0;
+}
 
 // mode 0: points (ifp), mode 1: triangles (centroid).
 __device__ __forceinline__ int64_t cnt_prims(int mode, const uint64_t* sc)
@@ -733,9 +781,11 @@ __device__ __forceinline__ int64_t cnt_prims(int mode, const uint64_t* sc)
     return mode == 0 ? cnt_points(sc) : cnt_tris(sc);
 }
 
+// Bin of each primitive, marked in the bitmap (a word already holding the bit
+// needs no atomic: most primitives share their bin).
 __global__ __launch_bounds__(kBS) void k_prim_bin(int mode, const uint64_t* sc, const float* ifp,
                                                   const int4* tris, const int32_t* ifp2e,
-                                                  IndexGeom ig, uint32_t* code, uint32_t* count)
+                                                  IndexGeom ig, uint32_t* code, unsigned long long* bits)
 {
     if (halted(sc)) return;
     const int64_t j = (int64_t)blockIdx.x * kBS + threadIdx.x;
@@ -754,59 +804,166 @@ __global__ __launch_bounds__(kBS) void k_prim_bin(int mode, const uint64_t* sc, 
     const int f = ifp2e ? ftd::field_of(ig.edge_off, ig.nf, ifp2e[v0]) : 0;
     const uint32_t cc = (uint32_t)ig.cnt_off[f] + ftd::grid_code(ig.grids[f], c[0], c[1], c[2]);
     code[j] = cc;
-    atomicAdd(&count[cc], 1u);
+    const unsigned long long m = 1ull << (cc & 63);
+    if (!(__hip_atomic_load(&bits[cc >> 6], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & m))
+        atomicOr(&bits[cc >> 6], m);
 }
 
-__global__ __launch_bounds__(kBS) void k_leaves(const uint32_t* count, const uint64_t* prefix,
-                                                int64_t G, IndexGeom ig, uint32_t* leaf_key,
-                                                uint32_t* leaf_start, uint32_t* leaf_cnt)
-{
-    const int64_t c = (int64_t)blockIdx.x * kBS + threadIdx.x;
-    if (c >= G) return;
-    const uint32_t n = count[c];
-    if (!n) return;
-    const uint64_t p = prefix[c];
-    const uint32_t l = (uint32_t)(p >> 32);
-    const int f = ftd::field_of(ig.cnt_off, ig.nf, c);
-    leaf_key[l] = ((uint32_t)f << ig.code_bits) | (uint32_t)(c - ig.cnt_off[f]);
-    leaf_start[l] = (uint32_t)p;
-    leaf_cnt[l] = n;
-}
-
-// Leaf range [leaf_off[f], leaf_off[f+1]) of each field and its tree root:
-// none (INT_MIN) without leaves, the leaf itself when alone; fields with two
-// or more leaves get the internal node covering exactly their range from
-// k_karras.
-__global__ void k_field_roots(int nf, const int64_t* cnt_off, const uint64_t* prefix,
-                              const uint64_t* total, int64_t G, int32_t* leaf_off, int32_t* roots)
-{
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f > nf) return;
-    const uint32_t L = (uint32_t)(*total >> 32);
-    const int64_t c = cnt_off[f];
-    const uint32_t lf = c < G ? (uint32_t)(prefix[c] >> 32) : L;
-    leaf_off[f] = (int32_t)lf;
-    if (f == nf) return;
-    const int64_t c1 = cnt_off[f + 1];
-    const uint32_t ll = c1 < G ? (uint32_t)(prefix[c1] >> 32) : L;
-    roots[f] = (ll == lf) ? INT32_MIN : (ll == lf + 1 ? ~(int32_t)lf : -1);
-}
-
-// Scatter primitives into bin order and write their search records.
-__global__ __launch_bounds__(kBS) void k_prim_scatter(int mode, const uint64_t* sc, const float* ifp,
-                                                      const int4* tris, const uint32_t* code,
-                                                      uint32_t* count, const uint64_t* prefix,
-                                                      float4* prec, TriRec* trec,
-                                                      int32_t* pidx)
+// Leaf of each primitive (the rank of its bin's bit) and its place among the
+// leaf's primitives; code becomes the leaf.
+__global__ __launch_bounds__(kBS) void k_prim_rank(int mode, const uint64_t* sc, const uint64_t* bits,
+                                                   const uint32_t* wprefix, uint32_t* code, uint32_t* place,
+                                                   uint32_t* leaf_cnt, uint32_t* leaf_bin)
 {
     if (halted(sc)) return;
     const int64_t j = (int64_t)blockIdx.x * kBS + threadIdx.x;
     if (j >= cnt_prims(mode, sc)) return;
     const uint32_t c = code[j];
-    const uint32_t slot = (uint32_t)prefix[c] + atomicSub(&count[c], 1u) - 1u;
+    const uint64_t below = bits[c >> 6] & ((1ull << (c & 63)) - 1ull);
+    const uint32_t l = wprefix[c >> 6] + (uint32_t)__popcll(below);
+    code[j] = l;
+    place[j] = atomicAdd(&leaf_cnt[l], 1u);
+    leaf_bin[l] = c;                             // the same value from each of its primitives
+}
+
+// What leaf l adds to the level scan: its primitives, and 1 for each level
+// at which it opens a new node (its bin's code differs from the previous
+// leaf's above that level's bits, or the field does).
+__device__ __forceinline__ ftd::Lv leaf_elem(int64_t l, int64_t L, const uint32_t* leaf_cnt,
+                                             const uint32_t* leaf_bin, const IndexGeom& ig, uint32_t* opens,
+                                             int* field)
+{
+    *opens = 0u;
+    *field = 0;
+    if (l >= L) return ftd::Lv(0);
+    const uint32_t c = leaf_bin[l];
+    const int f = bin_field(ig, c);
+    const uint32_t f0 = (uint32_t)ig.cnt_off[f];
+    const uint32_t p = l > 0 ? leaf_bin[l - 1] : 0u;
+    uint32_t o = 31u;                            // bit 4: the field's first leaf
+    if (l > 0 && p >= f0) {
+        const uint32_t x = (p - f0) ^ (c - f0);
+        o = ((x >> 6) ? 1u : 0u) | ((x >> 12) ? 2u : 0u) | ((x >> 18) ? 4u : 0u) | ((x >> 24) ? 8u : 0u);
+    }
+    *opens = o;
+    *field = f;
+    ftd::Lv v;
+    v.a = (uint64_t)leaf_cnt[l] | ((uint64_t)(o & 1u) << 32);
+    v.b = (uint64_t)((o >> 1) & 1u) | ((uint64_t)((o >> 2) & 1u) << 32);
+    v.c = (uint64_t)((o >> 3) & 1u);
+    return v;
+}
+
+__global__ __launch_bounds__(kBS) void k_level_reduce(const uint64_t* sc, const uint32_t* leaf_cnt,
+                                                      const uint32_t* leaf_bin, IndexGeom ig, ftd::Lv* bsum)
+{
+    __shared__ ftd::Lv lds[kBS / 64 + 1];
+    const int64_t L = halted(sc) ? 0 : cnt_leaves(sc);
+    const int64_t base = (int64_t)blockIdx.x * kScanTile;
+    ftd::Lv s(0);
+    if (base < L)
+        for (int k = 0; k < kScanTile / kBS; k++) {
+            uint32_t o;
+            int f;
+            s += leaf_elem(base + (int64_t)k * kBS + threadIdx.x, L, leaf_cnt, leaf_bin, ig, &o, &f);
+        }
+    ftd::Lv tot;
+    ftd::block_excl_scan<ftd::Lv, kBS>(s, lds, &tot);
+    if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
+}
+
+// first[] of the leaves and of the nodes of every level, and the fields'
+// roots: the node of the level that covers the whole field (Grid::root_lv).
+__global__ __launch_bounds__(kBS) void k_level_down(const uint64_t* sc, const uint32_t* leaf_cnt,
+                                                    const uint32_t* leaf_bin, IndexGeom ig, const ftd::Lv* bsum,
+                                                    LevelOff lo, uint32_t* first, uint32_t* roots)
+{
+    __shared__ ftd::Lv lds[kBS / 64 + 1];
+    constexpr int IPT = kScanTile / kBS;
+    const int64_t L = halted(sc) ? 0 : cnt_leaves(sc);
+    if ((int64_t)blockIdx.x * kScanTile >= L) return;            // whole block
+    const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * IPT;
+    ftd::Lv s(0);
+    for (int k = 0; k < IPT; k++) {
+        uint32_t o;
+        int f;
+        s += leaf_elem(base + k, L, leaf_cnt, leaf_bin, ig, &o, &f);
+    }
+    ftd::Lv tot;
+    ftd::Lv ex = ftd::block_excl_scan<ftd::Lv, kBS>(s, lds, &tot) + bsum[blockIdx.x];
+    for (int k = 0; k < IPT; k++) {
+        const int64_t l = base + k;
+        if (l >= L) break;
+        uint32_t o;
+        int f;
+        const ftd::Lv v = leaf_elem(l, L, leaf_cnt, leaf_bin, ig, &o, &f);
+        // this leaf's node at each level, were it to open one
+        uint32_t g[kLevels] = {(uint32_t)l, lo.off[1] + (uint32_t)(ex.a >> 32), lo.off[2] + (uint32_t)ex.b,
+                               lo.off[3] + (uint32_t)(ex.b >> 32), lo.off[4] + (uint32_t)ex.c};
+        first[l] = (uint32_t)ex.a;
+#pragma unroll
+        for (int q = 1; q < kLevels; q++)
+            if ((o >> (q - 1)) & 1u) first[g[q]] = g[q - 1];
+        if (o & 16u) {
+            const int r = ig.grids[f].root_lv;
+            roots[f] = r == 1 ? g[1] : r == 2 ? g[2] : r == 3 ? g[3] : g[4];
+        }
+        ex += v;
+        if (l == L - 1) {                        // the ends of the last node of each level
+            first[L] = (uint32_t)ex.a;
+            first[lo.off[1] + (uint32_t)(ex.a >> 32)] = (uint32_t)L;
+            first[lo.off[2] + (uint32_t)ex.b] = lo.off[1] + (uint32_t)(ex.a >> 32);
+            first[lo.off[3] + (uint32_t)(ex.b >> 32)] = lo.off[2] + (uint32_t)ex.b;
+            first[lo.off[4] + (uint32_t)ex.c] = lo.off[3] + (uint32_t)(ex.b >> 32);
+        }
+    }
+}
+
+// The item of a box given by its axes, its centre m and half extents h in the
+// mesh's coordinates.  The extents are rounded up by the error of a row's
+// product (the search's own allowance covers centres within one scaled unit
+// of the origin; farther ones, primitives outside the field's box, carry
+// theirs here).  A box that is not finite admits every point.
+__device__ __forceinline__ Item make_item(const Grid& g, const float ax[3][3], const double m[3], const float h[3])
+{
+    const double s = (double)g.inv_s;
+    double mm[3], far2 = 0.0;
+    for (int k = 0; k < 3; k++) {
+        mm[k] = (m[k] - (double)g.org[k]) * s;
+        far2 += mm[k] * mm[k];
+    }
+    Row r[3];
+    float e[3];
+    bool ok = far2 < 1e8;                              // offsets within the halves' range
+    const float slack = 0x1.0p-22f + (far2 > 1.0 ? 0x1.0p-19f * sqrtf((float)far2) : 0.0f);
+    for (int k = 0; k < 3; k++) {
+        const double w = -((double)ax[k][0] * mm[0] + (double)ax[k][1] * mm[1] + (double)ax[k][2] * mm[2]);
+        r[k] = make_row(ax[k][0], ax[k][1], ax[k][2], (float)w);
+        e[k] = h[k] * g.inv_s * (1.0f + 0x1.0p-20f) + slack;
+        ok = ok && fabsf(ax[k][0]) <= 2.0f && fabsf(ax[k][1]) <= 2.0f && fabsf(ax[k][2]) <= 2.0f && e[k] <= 1e15f;
+    }
+    if (!ok) return open_item();
+    Item it;
+    it.x = r[0]; it.y = r[1]; it.z = r[2];
+    it.e = make_float4(e[0], e[1], e[2], 0.0f);
+    return it;
+}
+
+// Scatter primitives into leaf order and write their search records.
+__global__ __launch_bounds__(kBS) void k_prim_scatter(int mode, const uint64_t* sc, const float* ifp,
+                                                      const int4* tris, const uint32_t* code,
+                                                      const uint32_t* place, const uint32_t* first,
+                                                      const uint32_t* leaf_bin, IndexGeom ig,
+                                                      float4* prec, Item* titem, TriRec* trec, int32_t* pidx)
+{
+    if (halted(sc)) return;
+    const int64_t j = (int64_t)blockIdx.x * kBS + threadIdx.x;
+    if (j >= cnt_prims(mode, sc)) return;
+    const uint32_t l = code[j];
+    const uint32_t slot = first[l] + place[j];
     pidx[slot] = (int32_t)j;
     if (mode == 0) {
-        prec[slot] = make_float4(ifp[3 * j], ifp[3 * j + 1], ifp[3 * j + 2], 0.0f);
+        prec[slot] = make_float4(ifp[3 * j], ifp[3 * j + 1], ifp[3 * j + 2], __int_as_float((int32_t)j));
         return;
     }
     float v3[3][3];
@@ -819,9 +976,9 @@ __global__ __launch_bounds__(kBS) void k_prim_scatter(int mode, const uint64_t* 
     for (int q = 0; q < 3; q++) {
         const float* p0 = v3[q];
         const float* p1 = v3[(q + 1) % 3];
-        double l = 0.0;
-        for (int k = 0; k < 3; k++) { const double dd = (double)p1[k] - p0[k]; l += dd * dd; }
-        len[q] = l;
+        double s = 0.0;
+        for (int k = 0; k < 3; k++) { const double dd = (double)p1[k] - p0[k]; s += dd * dd; }
+        len[q] = s;
     }
     const int r0 = (len[0] >= len[1] && len[0] >= len[2]) ? 0 : (len[1] >= len[2] ? 1 : 2);
     const float* a = v3[r0];
@@ -854,16 +1011,27 @@ __global__ __launch_bounds__(kBS) void k_prim_scatter(int mode, const uint64_t* 
     const double dCx = Cx - L0;
     const double lac = Cx * Cx + Cy * Cy, lbc = dCx * dCx + Cy * Cy;
     TriRec r;
-    // disk about the midpoint of ab holding the triangle (ab is the longest
-    // edge), radius rounded up; its sign carries the interior flag
-    const double Rm = fmax(0.5 * L0, sqrt((Cx - 0.5 * L0) * (Cx - 0.5 * L0) + Cy * Cy)) * (1.0 + 1e-6);
-    r.F0 = make_float4(a[0], a[1], a[2], interior ? (float)Rm : -(float)Rm);
-    r.F1 = make_float4((float)u[0], (float)u[1], (float)u[2], (float)L0);
-    r.F2 = make_float4((float)v[0], (float)v[1], (float)v[2], (float)nu[0]);
-    r.F3 = make_float4((float)nu[1], (float)nu[2], (float)Cx, (float)Cy);
-    r.F4 = make_float4(L0 > 0.0 ? (float)(1.0 / L0) : 0.0f, lac > 0.0 ? (float)(1.0 / lac) : 0.0f,
-                       lbc > 0.0 ? (float)(1.0 / lbc) : 0.0f, (float)dCx);
+    r.a = make_float4(a[0], a[1], a[2], (float)dCx);
+    r.u = make_float4((float)u[0], (float)u[1], (float)u[2], (float)L0);
+    r.v = make_float4((float)v[0], (float)v[1], (float)v[2], (float)Cx);
+    r.n = make_float4((float)nu[0], (float)nu[1], (float)nu[2], (float)Cy);
+    r.i = make_float4(L0 > 0.0 ? (float)(1.0 / L0) : 0.0f, lac > 0.0 ? (float)(1.0 / lac) : 0.0f,
+                      lbc > 0.0 ? (float)(1.0 / lbc) : 0.0f,
+                      __int_as_float((int32_t)j | (interior ? 0 : INT32_MIN)));
     trec[slot] = r;
+    // The rectangle [0, L0] x [0, Cy] of the frame holds the triangle: ab is
+    // the longest edge, so C projects inside [0, L0], and Cy >= 0.
+    const Grid& g = ig.grids[bin_field(ig, leaf_bin[l])];
+    const double s = (double)g.inv_s;
+    double m[3];
+    for (int k = 0; k < 3; k++) m[k] = ((double)a[k] - (double)g.org[k] + 0.5 * (L0 * u[k] + Cy * v[k])) * s;
+    Item it;
+    it.x = make_row((float)u[0], (float)u[1], (float)u[2], (float)-ftd::dot3d(u, m));
+    it.y = make_row((float)v[0], (float)v[1], (float)v[2], (float)-ftd::dot3d(v, m));
+    it.z = make_row((float)nu[0], (float)nu[1], (float)nu[2], (float)-ftd::dot3d(nu, m));
+    it.e = make_float4((float)(0.5 * L0 * s) * (1.0f + 0x1.0p-20f), (float)(0.5 * Cy * s) * (1.0f + 0x1.0p-20f), 0.0f,
+                       0.0f);
+    titem[slot] = it;
 }
 
 // Unit eigenvector of the smallest eigenvalue of the symmetric 3x3 matrix C
@@ -902,332 +1070,230 @@ __device__ inline bool smallest_eigvec(const double c[6], double n[3])
     return true;
 }
 
-// The vertices a leaf's bound must hold: the triangles' three vertices, or
-// the crossing points themselves.
+// Orthonormal axes with the unit vector n last.
+__device__ __forceinline__ void frame_about(const double n[3], float ax[3][3])
+{
+    const double a[3] = {fabs(n[0]), fabs(n[1]), fabs(n[2])};
+    const int k0 = a[0] <= a[1] && a[0] <= a[2] ? 0 : (a[1] <= a[2] ? 1 : 2);
+    const double t[3] = {k0 == 0 ? 1.0 : 0.0, k0 == 1 ? 1.0 : 0.0, k0 == 2 ? 1.0 : 0.0};
+    double u[3], v[3];
+    ftd::cross3d(n, t, u);
+    const double iu = 1.0 / sqrt(ftd::dot3d(u, u));
+    for (int k = 0; k < 3; k++) u[k] *= iu;
+    ftd::cross3d(n, u, v);
+    for (int k = 0; k < 3; k++) {
+        ax[0][k] = (float)u[k];
+        ax[1][k] = (float)v[k];
+        ax[2][k] = (float)n[k];
+    }
+}
+
+// Half the surface of a box of half extents h: the smaller of two boxes about
+// the same primitives is kept.
+__device__ __forceinline__ float box_cost(const float h[3]) { return h[0] * h[1] + h[1] * h[2] + h[0] * h[2]; }
+
+template <int W>
+__device__ __forceinline__ float group_min(float v)
+{
+#pragma unroll
+    for (int o = W / 2; o >= 1; o >>= 1) v = fminf(v, __shfl_xor(v, o));
+    return v;
+}
+template <int W>
+__device__ __forceinline__ float group_max(float v)
+{
+#pragma unroll
+    for (int o = W / 2; o >= 1; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
+    return v;
+}
+template <int W>
+__device__ __forceinline__ double group_sum(double v)
+{
+#pragma unroll
+    for (int o = W / 2; o >= 1; o >>= 1) v += __shfl_xor(v, o);
+    return v;
+}
+
+// Leaf boxes, kLeafLanes lanes per leaf: the smaller of the axis-aligned box
+// of the vertices and one about an axis, for triangles the area-weighted mean
+// normal, for crossing points the normal of their least-squares plane (three
+// or more points that are not collinear).  A patch of a smooth surface is
+// thin along that axis, so for a node far away the box's distance is close to
+// the patch's.  naxis: that axis times its weight (area, or points), for the
+// nodes above.  NaN vertices bound nothing (their distances never win).
+constexpr int kLeafLanes = 16;
 template <int MODE>
-struct LeafVerts {
-    static constexpr int kPerPrim = MODE == 0 ? 1 : 3;
-    const int32_t* pidx;
-    const float* ifp;
-    const int4* tris;
-    // the vertices of primitive s into v[0..kPerPrim)
-    __device__ void get(uint32_t s, float v[3][3]) const
-    {
+__global__ __launch_bounds__(kBS) void k_leaf_items(const uint64_t* sc, const uint32_t* first,
+                                                    const uint32_t* leaf_bin, IndexGeom ig, const int32_t* pidx,
+                                                    const float* ifp, const int4* tris, Item* items, float4* naxis)
+{
+    if (halted(sc)) return;
+    const int64_t l = ((int64_t)blockIdx.x * kBS + threadIdx.x) / kLeafLanes;
+    if (l >= cnt_leaves(sc)) return;                   // whole group
+    constexpr int NV = MODE == 0 ? 1 : 3;
+    const uint32_t sub = threadIdx.x % kLeafLanes, b = first[l], e = first[l + 1];
+    auto verts = [&](uint32_t s, float v[3][3]) {
         const int32_t j = pidx[s];
         if (MODE == 0) {
             for (int k = 0; k < 3; k++) v[0][k] = ifp[3 * (int64_t)j + k];
         } else {
             tri_vertices(tris, ifp, j, v[0], v[1], v[2]);
         }
-    }
-};
-
-// Leaf bounds: box of the vertices and a cylinder about an axis: for
-// triangles the area-weighted mean normal, for crossing points the normal of
-// their least-squares plane (three or more points that are not collinear).
-template <int MODE>
-__global__ __launch_bounds__(kBS) void k_leaf_bounds(const uint64_t* sc, const uint32_t* leaf_start,
-                                                     const uint32_t* leaf_cnt, const int32_t* pidx,
-                                                     const float* ifp, const int4* tris, Bound* leaf_b)
-{
-    if (halted(sc)) return;
-    const int64_t l = (int64_t)blockIdx.x * kBS + threadIdx.x;
-    if (l >= cnt_leaves(sc)) return;
-    using LV = LeafVerts<MODE>;
-    const LV lv{pidx, ifp, tris};
+    };
     float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-    double ns[3] = {0.0, 0.0, 0.0}, m[3] = {0.0, 0.0, 0.0};
-    const uint32_t b = leaf_start[l], e = b + leaf_cnt[l];
-    for (uint32_t s = b; s < e; s++) {
+    double ns[3] = {0.0, 0.0, 0.0};                    // triangles: area vector; points: sum
+    for (uint32_t s = b + sub; s < e; s += kLeafLanes) {
         float v[3][3];
-        lv.get(s, v);
-        for (int q = 0; q < LV::kPerPrim; q++) {
+        verts(s, v);
+        for (int q = 0; q < NV; q++)
             for (int k = 0; k < 3; k++) {
                 lo[k] = fminf(lo[k], v[q][k]);
                 hi[k] = fmaxf(hi[k], v[q][k]);
-                if (MODE == 0) m[k] += v[q][k];
             }
-        }
         if (MODE == 1) {
             double e0[3], e1[3], nn[3];
             for (int k = 0; k < 3; k++) { e0[k] = (double)v[1][k] - v[0][k]; e1[k] = (double)v[2][k] - v[0][k]; }
             ftd::cross3d(e0, e1, nn);
             for (int k = 0; k < 3; k++) ns[k] += nn[k];
+        } else {
+            for (int k = 0; k < 3; k++) ns[k] += v[0][k];
         }
     }
-    Bound B;
-    for (int k = 0; k < 3; k++) { B.lo[k] = lo[k]; B.hi[k] = hi[k]; B.c[k] = 0.5f * (lo[k] + hi[k]); }
-    B.pad[0] = B.pad[1] = 0.0f;
-    double n[3];
-    bool axis = false;
+    float c[3], hb[3];
+    for (int k = 0; k < 3; k++) {
+        lo[k] = group_min<kLeafLanes>(lo[k]);
+        hi[k] = group_max<kLeafLanes>(hi[k]);
+        ns[k] = group_sum<kLeafLanes>(ns[k]);
+        c[k] = 0.5f * (lo[k] + hi[k]);
+        hb[k] = fmaxf(hi[k] - c[k], c[k] - lo[k]);
+    }
+    double n[3] = {0.0, 0.0, 0.0}, wt = 0.0;
     if (MODE == 1) {
-        const double nl = sqrt(ftd::dot3d(ns, ns));
-        if (nl > 0.0) {
-            for (int k = 0; k < 3; k++) n[k] = ns[k] / nl;
-            axis = true;
-        }
+        wt = sqrt(ftd::dot3d(ns, ns));
+        if (wt > 0.0) for (int k = 0; k < 3; k++) n[k] = ns[k] / wt;
+        else wt = 0.0;
     } else if (e - b >= 3) {
         double cov[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         const double cnt = (double)(e - b);
-        for (int k = 0; k < 3; k++) m[k] /= cnt;
-        for (uint32_t s = b; s < e; s++) {
+        for (uint32_t s = b + sub; s < e; s += kLeafLanes) {
             float v[3][3];
-            lv.get(s, v);
-            const double d0 = v[0][0] - m[0], d1 = v[0][1] - m[1], d2 = v[0][2] - m[2];
+            verts(s, v);
+            const double d0 = v[0][0] - ns[0] / cnt, d1 = v[0][1] - ns[1] / cnt, d2 = v[0][2] - ns[2] / cnt;
             cov[0] += d0 * d0; cov[1] += d1 * d1; cov[2] += d2 * d2;
             cov[3] += d0 * d1; cov[4] += d0 * d2; cov[5] += d1 * d2;
         }
-        axis = smallest_eigvec(cov, n);
+        for (int k = 0; k < 6; k++) cov[k] = group_sum<kLeafLanes>(cov[k]);
+        if (smallest_eigvec(cov, n)) wt = cnt;
     }
-    if (!axis) {
-        B.n[0] = 0.0f; B.n[1] = 0.0f; B.n[2] = 1.0f;
-        B.rho = 0.0f; B.tau = -1.0f;                 // box only
-    } else {
-        for (int k = 0; k < 3; k++) { B.n[k] = (float)n[k]; n[k] = B.n[k]; }
-        // One pass over the vertices, relative to the box centre c: their
-        // extent [hlo, hhi] along n and their largest distance rho0 from the
-        // axis through c.  The slab is then centred on that extent, not on the
-        // box centre: a surface patch can pass well off its box's centre, and
-        // a slab centred off the patch is thicker by that offset.  Moving the
-        // centre along n leaves the axis distances as they are, up to the
-        // float rounding of the moved centre, which is added to rho.
-        double hlo = INFINITY, hhi = -INFINITY, rho0 = 0.0;
-        for (uint32_t s = b; s < e; s++) {
+    float ax[3][3] = {{1.0f, 0.0f, 0.0f}, {0.0f, 1.0f, 0.0f}, {0.0f, 0.0f, 1.0f}};
+    float h[3] = {hb[0], hb[1], hb[2]};
+    double m[3] = {c[0], c[1], c[2]};
+    if (wt > 0.0) {
+        float fx[3][3];
+        frame_about(n, fx);
+        float l3[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, h3[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
+        for (uint32_t s = b + sub; s < e; s += kLeafLanes) {
             float v[3][3];
-            lv.get(s, v);
-            for (int q = 0; q < LV::kPerPrim; q++) {
-                double d[3], cr[3];
-                for (int k = 0; k < 3; k++) d[k] = (double)v[q][k] - B.c[k];
-                const double hv = ftd::dot3d(n, d);
-                hlo = fmin(hlo, hv);
-                hhi = fmax(hhi, hv);
-                ftd::cross3d(n, d, cr);
-                rho0 = fmax(rho0, ftd::dot3d(cr, cr));
+            verts(s, v);
+            for (int q = 0; q < NV; q++) {
+                const float d0 = v[q][0] - c[0], d1 = v[q][1] - c[1], d2 = v[q][2] - c[2];
+                for (int k = 0; k < 3; k++) {
+                    const float t = __fmaf_rn(fx[k][2], d2, __fmaf_rn(fx[k][1], d1, fx[k][0] * d0));
+                    l3[k] = fminf(l3[k], t);
+                    h3[k] = fmaxf(h3[k], t);
+                }
             }
         }
-        const double mid = 0.5 * (hlo + hhi);
-        double sh[3], cr[3];
+        float ho[3], mid[3];
         for (int k = 0; k < 3; k++) {
-            const float ck = (float)(B.c[k] + mid * n[k]);
-            sh[k] = (double)ck - B.c[k];              // the centre's actual move
-            B.c[k] = ck;
+            l3[k] = group_min<kLeafLanes>(l3[k]);
+            h3[k] = group_max<kLeafLanes>(h3[k]);
+            mid[k] = 0.5f * (l3[k] + h3[k]);
+            // the rounding of the projections: their terms are below 2 |hb|
+            ho[k] = fmaxf(h3[k] - mid[k], mid[k] - l3[k]) + 0x1.0p-21f * (hb[0] + hb[1] + hb[2]);
         }
-        const double m = ftd::dot3d(n, sh);
-        ftd::cross3d(n, sh, cr);
-        const double tau = fmax(hhi - m, m - hlo);
-        const double rho = sqrt(rho0) + sqrt(ftd::dot3d(cr, cr));
-        B.tau = (float)(tau * (1.0 + 1e-6));
-        B.rho = (float)(rho * (1.0 + 1e-6));
-    }
-    leaf_b[l] = B;
-}
-
-// Binary radix tree over L >= 2 sorted, distinct keys (T. Karras, "Maximizing
-// parallelism in the construction of BVHs, octrees, and k-d trees", HPG 2012).
-// Children >= 0 are internal nodes, ~l is leaf l.
-__device__ __forceinline__ int kdelta(const uint32_t* keys, int L, int i, int j)
-{
-    if (j < 0 || j >= L) return -1;
-    return __clz(keys[i] ^ keys[j]);
-}
-
-__global__ __launch_bounds__(kBS) void k_karras(const uint32_t* keys, const uint64_t* sc, BNode* nodes,
-                                                int32_t* leaf_parent, int code_bits,
-                                                const int32_t* leaf_off, int32_t* roots)
-{
-    if (halted(sc)) return;
-    const int L = (int)cnt_leaves(sc);
-    const int i = blockIdx.x * kBS + threadIdx.x;
-    if (i >= L - 1) return;
-    const int d = (kdelta(keys, L, i, i + 1) - kdelta(keys, L, i, i - 1)) >= 0 ? 1 : -1;
-    const int dmin = kdelta(keys, L, i, i - d);
-    int lmax = 2;
-    while (kdelta(keys, L, i, i + lmax * d) > dmin) lmax <<= 1;
-    int l = 0;
-    for (int t = lmax >> 1; t >= 1; t >>= 1)
-        if (kdelta(keys, L, i, i + (l + t) * d) > dmin) l += t;
-    const int j = i + l * d;
-    const int dnode = kdelta(keys, L, i, j);
-    int s = 0, div = 2, t;
-    do {
-        t = (l + div - 1) / div;
-        if (kdelta(keys, L, i, i + (s + t) * d) > dnode) s += t;
-        div <<= 1;
-    } while (t > 1);
-    const int gamma = i + s * d + (d < 0 ? d : 0);
-    const int left = (min(i, j) == gamma) ? ~gamma : gamma;
-    const int right = (max(i, j) == gamma + 1) ? ~(gamma + 1) : gamma + 1;
-    nodes[i].left = left;
-    nodes[i].right = right;
-    if (left >= 0) nodes[left].parent = i; else leaf_parent[~left] = i;
-    if (right >= 0) nodes[right].parent = i; else leaf_parent[~right] = i;
-    if (i == 0) nodes[0].parent = -1;
-    // the node whose range is exactly one field's leaves is that field's root
-    const int lo = min(i, j), hi = max(i, j);
-    nodes[i].top = (lo / kRefitBlock) != (hi / kRefitBlock);
-    const int f = (int)(keys[lo] >> code_bits);
-    if (leaf_off[f] == lo && leaf_off[f + 1] == hi + 1) roots[f] = i;
-}
-
-// Parent bound of two children: box union and a cylinder that contains both
-// child cylinders.  For a child cylinder (c_i, n_i, rho_i, tau_i) seen from
-// the parent axis n at centre c, with cos = |n.n_i| and sin = |n x n_i|:
-//   thickness  |n.(c_i-c)| + tau_i cos + rho_i sin
-//   radius     |n x (c_i-c)| + rho_i + tau_i sin
-// In FP32 with hardware square roots (the merge is on the refit's critical
-// path, one per tree level): every term is a sum of non-negative parts with a
-// relative error under 1e-6, the axis is unit to 3e-7, and the results are
-// rounded up by 2^-12 relative plus 2^-18 of the box extent, so the cylinder
-// still contains both children.
-__device__ inline Bound merge_bounds(const Bound& A, const Bound& Bb)
-{
-    Bound P;
-    float ext = 0.0f;
-    for (int k = 0; k < 3; k++) {
-        P.lo[k] = fminf(A.lo[k], Bb.lo[k]);
-        P.hi[k] = fmaxf(A.hi[k], Bb.hi[k]);
-        P.c[k] = 0.5f * (P.lo[k] + P.hi[k]);
-        ext = fmaxf(ext, P.hi[k] - P.lo[k]);
-    }
-    P.pad[0] = P.pad[1] = 0.0f;
-    if (A.tau < 0.0f || Bb.tau < 0.0f) {
-        P.n[0] = 0.0f; P.n[1] = 0.0f; P.n[2] = 1.0f;
-        P.rho = 0.0f; P.tau = -1.0f;
-        return P;
-    }
-    const float wa = A.rho * A.rho + 1e-30f, wb = Bb.rho * Bb.rho + 1e-30f;
-    float n[3];
-    for (int k = 0; k < 3; k++) n[k] = wa * A.n[k] + wb * Bb.n[k];
-    const float nn = n[0] * n[0] + n[1] * n[1] + n[2] * n[2];
-    if (nn > 1e-20f * (wa + wb) * (wa + wb) && nn > 1e-30f) {
-        const float inv = __builtin_amdgcn_rsqf(nn);
-        for (int k = 0; k < 3; k++) n[k] *= inv;
-    } else {
-        for (int k = 0; k < 3; k++) n[k] = A.n[k];
-    }
-    // The centre may be any point (thickness and radius below are taken
-    // about the rounded one); it is moved along n to centre the slab on the
-    // children's extents along n.
-    const Bound* ch[2] = {&A, &Bb};
-    float cs[2], sn[2], hlo = INFINITY, hhi = -INFINITY;
-    for (int i = 0; i < 2; i++) {
-        const Bound& C = *ch[i];
-        cs[i] = fminf(1.0f, fabsf(n[0] * C.n[0] + n[1] * C.n[1] + n[2] * C.n[2]));
-        const float sx = n[1] * C.n[2] - n[2] * C.n[1], sy = n[2] * C.n[0] - n[0] * C.n[2],
-                    sz = n[0] * C.n[1] - n[1] * C.n[0];
-        sn[i] = __builtin_amdgcn_sqrtf(sx * sx + sy * sy + sz * sz);
-        const float hc = n[0] * (C.c[0] - P.c[0]) + n[1] * (C.c[1] - P.c[1]) + n[2] * (C.c[2] - P.c[2]);
-        const float ec = C.tau * cs[i] + C.rho * sn[i];
-        hlo = fminf(hlo, hc - ec);
-        hhi = fmaxf(hhi, hc + ec);
-    }
-    const float mid = 0.5f * (hlo + hhi);
-    for (int k = 0; k < 3; k++) P.c[k] += mid * n[k];
-    float tau = 0.0f, rho = 0.0f;
-    for (int i = 0; i < 2; i++) {
-        const Bound& C = *ch[i];
-        const float dc[3] = {C.c[0] - P.c[0], C.c[1] - P.c[1], C.c[2] - P.c[2]};
-        const float ax = fabsf(n[0] * dc[0] + n[1] * dc[1] + n[2] * dc[2]);
-        const float rx = n[1] * dc[2] - n[2] * dc[1], ry = n[2] * dc[0] - n[0] * dc[2],
-                    rz = n[0] * dc[1] - n[1] * dc[0];
-        const float rad = __builtin_amdgcn_sqrtf(rx * rx + ry * ry + rz * rz);
-        tau = fmaxf(tau, ax + C.tau * cs[i] + C.rho * sn[i]);
-        rho = fmaxf(rho, rad + C.rho + C.tau * sn[i]);
-    }
-    for (int k = 0; k < 3; k++) P.n[k] = n[k];
-    P.tau = tau * (1.0f + 0x1.0p-12f) + 0x1.0p-18f * ext;
-    P.rho = rho * (1.0f + 0x1.0p-12f) + 0x1.0p-18f * ext;
-    return P;
-}
-
-// Bottom-up fitting: the second child to arrive at a node merges both.
-// A cylinder whose volume is not below alpha times its box's prunes little
-// beyond the box test and costs more: such a bound is kept as a box only.
-__device__ __forceinline__ void drop_loose_cylinder(Bound& b, float alpha)
-{
-    if (alpha <= 0.0f || b.tau < 0.0f) return;
-    const float vb = (b.hi[0] - b.lo[0]) * (b.hi[1] - b.lo[1]) * (b.hi[2] - b.lo[2]);
-    const float vc = 3.14159265f * b.rho * b.rho * 2.0f * b.tau;
-    if (vc >= alpha * vb) { b.rho = 0.0f; b.tau = -1.0f; }
-}
-
-// Bottom-up fitting in two passes, with no device-wide fence: with one L2 per
-// XCD, an agent-scope release or acquire writes back or invalidates that L2,
-// and a fence per tree level made the one-pass form the index's slowest
-// kernel.  Karras node i spans leaves [min(i,j), max(i,j)] with i one end, so
-// a node inside refit block b has its index in that block.
-//
-// Pass 1, one workgroup per block of kRefitBlock leaves: a thread per leaf
-// climbs while the parent is inside the block.  Arrivals are counted in LDS;
-// the second child to arrive merges both (workgroup-scope fences order the
-// bound stores, which the workgroup's waves see through their CU).  At a top
-// node it stores its bound and counts the arrival in flags[p]; the second
-// arrival there appends p to the ready list (both children done).
-__global__ __launch_bounds__(kRefitBlock) void k_refit_local(const uint64_t* sc, const int32_t* leaf_parent,
-                                                             const Bound* leaf_b, BNode* nodes,
-                                                             unsigned* flags, unsigned* ready,
-                                                             float alpha)
-{
-    __shared__ unsigned arrived[kRefitBlock];
-    if (halted(sc)) return;
-    const int L = (int)cnt_leaves(sc);
-    const int b0 = blockIdx.x * kRefitBlock;
-    if (L < 2 || b0 >= L) return;                 // uniform over the block
-    arrived[threadIdx.x] = 0u;
-    __syncthreads();
-    const int l = b0 + threadIdx.x;
-    if (l >= L) return;
-    Bound cur_b = leaf_b[l];
-    int cur = ~l;
-    int p = leaf_parent[l];
-    for (int depth = 0; p >= 0 && depth < 64; depth++) {   // depth <= 32 for 32-bit keys
-        BNode* nd = &nodes[p];
-        const bool is_left = (nd->left == cur);
-        if (is_left) nd->l = cur_b; else nd->r = cur_b;
-        if (nd->top) {
-            if (atomicAdd(&flags[p], 1u) == 1u) ready[1 + atomicAdd(&ready[0], 1u)] = (unsigned)p;
-            return;
+        if (box_cost(ho) < box_cost(hb)) {
+            for (int k = 0; k < 3; k++) {
+                h[k] = ho[k];
+                for (int q = 0; q < 3; q++) {
+                    ax[k][q] = fx[k][q];
+                    m[q] += (double)mid[k] * fx[k][q];
+                }
+            }
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        if (atomicAdd(&arrived[p - b0], 1u) == 0u) return;   // sibling not done yet
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-        const Bound sib = is_left ? nd->r : nd->l;
-        cur_b = is_left ? merge_bounds(cur_b, sib) : merge_bounds(sib, cur_b);
-        drop_loose_cylinder(cur_b, alpha);
-        cur = p;
-        p = nd->parent;
+    }
+    if (sub == 0) {
+        items[l] = make_item(ig.grids[bin_field(ig, leaf_bin[l])], ax, m, h);
+        naxis[l] = make_float4((float)(n[0] * wt), (float)(n[1] * wt), (float)(n[2] * wt), 0.0f);
     }
 }
 
-// Pass 2, one workgroup: from each ready top node up.  flags[p] already counts
-// the children that pass 1 finished; the thread whose arrival completes a node
-// carries on with it.  All threads share one workgroup (one CU), so the
-// bound stores need only workgroup-scope fences; pass 1's stores are visible
-// across the kernel boundary.
-constexpr int kRefitTopThreads = 1024;
-__global__ __launch_bounds__(kRefitTopThreads) void k_refit_top(const uint64_t* sc, BNode* nodes,
-                                                                unsigned* flags, const unsigned* ready,
-                                                                float alpha)
+// Node boxes of one level, one wave per node with a child per lane: the
+// smaller of two boxes that hold the children's, axis-aligned and about the
+// weighted mean of their axes (signs aligned: two opposite sheets share
+// theirs).  Everything in scaled coordinates.  Levels are fitted one after
+// the other; nodes past the level's count leave at once.
+__device__ __forceinline__ int64_t cnt_level(const uint64_t* lv, int level)
+{
+    const uint64_t v = level == 1 ? lv[0] >> 32 : level == 2 ? lv[1] : level == 3 ? lv[1] >> 32 : lv[2];
+    return (int64_t)(v & 0xffffffffull);
+}
+
+__global__ __launch_bounds__(kBS) void k_node_items(const uint64_t* sc, int level, uint32_t off,
+                                                    const uint32_t* first, Item* items, float4* naxis)
 {
     if (halted(sc)) return;
-    const unsigned nr = ready[0];
-    for (unsigned k = threadIdx.x; k < nr; k += kRefitTopThreads) {
-        int cur = (int)ready[1 + k];
-        Bound cur_b = merge_bounds(nodes[cur].l, nodes[cur].r);
-        drop_loose_cylinder(cur_b, alpha);
-        int p = nodes[cur].parent;
-        for (int depth = 0; p >= 0 && depth < 64; depth++) {
-            BNode* nd = &nodes[p];
-            const bool is_left = (nd->left == cur);
-            if (is_left) nd->l = cur_b; else nd->r = cur_b;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-            if (atomicAdd(&flags[p], 1u) == 0u) break;   // the other child is still on its way
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-            const Bound sib = is_left ? nd->r : nd->l;
-            cur_b = is_left ? merge_bounds(cur_b, sib) : merge_bounds(sib, cur_b);
-            drop_loose_cylinder(cur_b, alpha);
-            cur = p;
-            p = nd->parent;
+    const int64_t n_nodes = cnt_leaves(sc) > 0 ? cnt_level(sc + S_LV, level) : 0;
+    const int lane = ftd::lane_id();
+    for (int64_t i = ((int64_t)blockIdx.x * kBS + threadIdx.x) >> 6; i < n_nodes; i += (int64_t)gridDim.x * (kBS / 64)) {
+        const uint32_t g = off + (uint32_t)i, c0 = first[g], cnt = first[g + 1] - c0;
+        const bool on = (uint32_t)lane < cnt;
+        const Item it = items[c0 + (on ? lane : 0)];
+        const float4 na = naxis[c0 + (on ? lane : 0)];
+        const float4 r[3] = {row_values(it.x), row_values(it.y), row_values(it.z)};
+        const float he[3] = {it.e.x, it.e.y, it.e.z};
+        const bool open = __ballot(on && !(it.e.x <= 1e15f)) != 0ull;    // a child that admits every point
+        float m[3];                                     // child centre: minus the rows' offsets along the axes
+        for (int q = 0; q < 3; q++) {
+            const float a0 = q == 0 ? r[0].x : q == 1 ? r[0].y : r[0].z, a1 = q == 0 ? r[1].x : q == 1 ? r[1].y : r[1].z,
+                        a2 = q == 0 ? r[2].x : q == 1 ? r[2].y : r[2].z;
+            m[q] = -__fmaf_rn(r[2].w, a2, __fmaf_rn(r[1].w, a1, r[0].w * a0));
+        }
+        const float r0x = __shfl(na.x, 0), r0y = __shfl(na.y, 0), r0z = __shfl(na.z, 0);
+        const double sg = on ? (na.x * r0x + na.y * r0y + na.z * r0z < 0.0f ? -1.0 : 1.0) : 0.0;
+        double ns[3] = {sg * na.x, sg * na.y, sg * na.z};
+        for (int k = 0; k < 3; k++) ns[k] = group_sum<64>(ns[k]);
+        const double wt = sqrt(ftd::dot3d(ns, ns));
+        float fx[2][3][3] = {{{1.0f, 0.0f, 0.0f}, {0.0f, 1.0f, 0.0f}, {0.0f, 0.0f, 1.0f}}, {}};
+        const bool axis = wt > 0.0;
+        if (axis) {
+            const double n[3] = {ns[0] / wt, ns[1] / wt, ns[2] / wt};
+            frame_about(n, fx[1]);
+        }
+        float mid[2][3], h[2][3], far = 0.0f;
+        for (int k = 0; k < 3; k++) far = fmaxf(far, group_max<64>(on ? fabsf(m[k]) : 0.0f));
+        for (int t = 0; t < (axis ? 2 : 1); t++)
+            for (int k = 0; k < 3; k++) {
+                const float* a = fx[t][k];
+                const float c = __fmaf_rn(a[2], m[2], __fmaf_rn(a[1], m[1], a[0] * m[0]));
+                float rad = 0.0f;
+                for (int q = 0; q < 3; q++)
+                    rad += he[q] * fabsf(__fmaf_rn(a[2], r[q].z, __fmaf_rn(a[1], r[q].y, a[0] * r[q].x)));
+                const float lo = group_min<64>(on ? c - rad : FLT_MAX), hi = group_max<64>(on ? c + rad : -FLT_MAX);
+                mid[t][k] = 0.5f * (lo + hi);
+                // centres, radii and projections are good to a few 2^-24 of the
+                // farthest child centre's distance from the origin
+                h[t][k] = fmaxf(hi - mid[t][k], mid[t][k] - lo) * (1.0f + 0x1.0p-20f) + 0x1.0p-19f * (far + 0.25f);
+            }
+        if (lane == 0) {
+            const int t = axis && box_cost(h[1]) < box_cost(h[0]) ? 1 : 0;
+            Item p;
+            p.x = make_row(fx[t][0][0], fx[t][0][1], fx[t][0][2], -mid[t][0]);
+            p.y = make_row(fx[t][1][0], fx[t][1][1], fx[t][1][2], -mid[t][1]);
+            p.z = make_row(fx[t][2][0], fx[t][2][1], fx[t][2][2], -mid[t][2]);
+            p.e = make_float4(h[t][0], h[t][1], h[t][2], 0.0f);
+            items[g] = open || !(h[t][0] <= 1e15f && h[t][1] <= 1e15f && h[t][2] <= 1e15f) ? open_item() : p;
+            naxis[g] = axis ? make_float4((float)ns[0], (float)ns[1], (float)ns[2], 0.0f) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         }
     }
 }
@@ -1244,15 +1310,14 @@ struct QueryArgs {
     const int32_t* tile_field;       // 64-slot tile -> field
     const int32_t* tile_list;        // launch order of the tiles, deep ones first (null: slot order)
     const uint64_t* n_deep;          // deep tiles at the head of tile_list (low 32 bits)
-    const int32_t* roots;            // field -> tree root (>= 0 node, < 0 ~leaf, INT_MIN none)
-    const float4* prec;              // point records (mode 0)
-    const TriRec* trec;              // triangle records (mode 1)
-    const int32_t* pidx;             // sorted slot -> primitive id
-    const uint32_t* leaf_start;
-    const uint32_t* leaf_cnt;
-    const Bound* leaf_b;
-    const BNode* nodes;
-    int L;                           // leaves
+    const Grid* grids;               // per field: scaled coordinates
+    const uint32_t* roots;           // field -> tree root (~0: no primitives)
+    const uint32_t* first;           // children of each node, primitives of each leaf (LevelOff numbering)
+    const Item* items;               // boxes of the same
+    uint32_t leaf_end;               // indices below are leaves
+    const float4* prec;              // point records (mode 0): coordinates, id
+    const Item* titem;               // triangles' frames and rectangles (mode 1)
+    const TriRec* trec;              // their other constants
     float band;                      // > 0: narrow band
     const float* ifp;
     const int4* tris;
@@ -1264,10 +1329,9 @@ struct QueryArgs {
     int epi;
     double w_phi, w_ifn;
     unsigned long long* n_clamped;   // per field
-    unsigned* overflow;
     unsigned long long* stats;       // nullable: per distance bucket
     float h_est;                     // node spacing (statistics only)
-    int probe;                       // greedy first candidate
+    int probe;                       // a first candidate from the search for the tile's centre
     const uint64_t* sc;              // stage totals and halt flags
     unsigned xcd_chunk;              // tiles per XCD chunk (0: dispatch order)
     uint32_t* queue;                 // work-queue schedule: deep counter, then one per XCD (null: static)
@@ -1315,110 +1379,15 @@ __device__ __forceinline__ uint64_t cand_key(float d, int32_t j)
     return ((uint64_t)__float_as_uint(d) << 32) | (uint32_t)j;
 }
 
-template <int MODE>
-struct Searcher {
+// End of a node's search.  Points: the nearest (distance, lowest id).
+// Triangles: the best two by FP32 squared distance, for the FP64 settle.
+struct Found {
     float x, y, z;
-    uint64_t bkey;   // best: mode 0 distance, mode 1 squared distance; primitive (original id)
-    const float4* prec;
-    const TriRec* trec;
-    const int32_t* pidx;
-    const uint32_t* leaf_start;
-    const uint32_t* leaf_cnt;
-    const float* ifp;
-    const int4* tris;
-
+    uint64_t bkey, skey;
     __device__ __forceinline__ float best() const { return __uint_as_float((uint32_t)(bkey >> 32)); }
     __device__ __forceinline__ int32_t bj() const { return (int32_t)(uint32_t)bkey; }
     __device__ __forceinline__ float sec() const { return __uint_as_float((uint32_t)(skey >> 32)); }
     __device__ __forceinline__ int32_t sj() const { return (int32_t)(uint32_t)skey; }
-    __device__ __forceinline__ float best2() const { return MODE == 0 ? best() * best() : best(); }
-    float bnd;       // prune_bound(best2()), refreshed whenever best changes
-    float bnd_r;     // mode 1: rect_bound(bnd), the triangle cull's bound
-    // no candidate yet, distance d (the band, or no limit)
-    __device__ __forceinline__ void init_best(float d)
-    {
-        bkey = cand_key(d, -1);
-        skey = bkey;
-        bnd = prune_bound(best2());
-        bnd_r = ftd::rect_bound(bnd);
-    }
-
-    // Mode 0 keeps the nearest point (ties: lowest id, the reference's strict
-    // < over ascending ids).  Mode 1 keeps the best two triangles by FP32
-    // distance, so that the epilogue can settle near-ties in FP64.  j is the
-    // primitive's original id (wave-uniform).  Written with selects, not
-    // branches: a lane-divergent branch costs exec-mask bookkeeping on every
-    // call, which is most of the work here.
-    // d is finite and non-negative.  A primitive seen again has the same key
-    // as before, so it is neither a new best nor a new second.
-    __device__ __forceinline__ void consider(float d, int32_t j)
-    {
-        // (bitwise & and |: short-circuit operators compile to branches)
-        const uint64_t key = cand_key(d, j);
-        const bool nb = key < bkey;
-        if (MODE == 1) {
-            // the old best becomes second (no candidate yet: it equals the
-            // initial second); else a key between the two is the new second
-            const bool ns = !nb & (key != bkey) & (key < skey);
-            skey = nb ? bkey : (ns ? key : skey);
-        }
-        bkey = nb ? key : bkey;
-        const float nbnd = prune_bound(MODE == 0 ? d * d : d);
-        bnd = nb ? nbnd : bnd;
-        if (MODE == 1) bnd_r = nb ? ftd::rect_bound(nbnd) : bnd_r;
-    }
-
-    uint32_t n_leaves = 0, n_prims = 0, n_pairs = 0;   // statistics (FT_QUERY_STATS)
-    uint64_t skey;   // mode 1: second best squared distance and its triangle
-    int parts = 1, part = 0;   // a split tile's part: only leaves l with l % parts == part are tested
-
-    // One triangle for all lanes: a wave-uniform early out when the bounding
-    // rectangle of its frame rules it out for every lane, else the exact FP32
-    // distance.
-    __device__ __forceinline__ void test_tri(const TriRec& r, int32_t j)
-    {
-        const ftd::TriProj pj = ftd::tri_project(x, y, z, r);
-        if (__ballot(ftd::tri_rect_d2(pj, r) <= bnd_r) == 0ull) return;
-        consider(ftd::tri_dist2_from(pj, r), j);
-    }
-
-    // Leaf test at a wave-uniform leaf: records read through scalar loads.
-    __device__ void test_leaf_uniform(int l, uint64_t admit = ~0ull)
-    {
-        if (parts > 1 && l % parts != part) return;
-        const uint32_t b = ftd::cload(leaf_start, l), e = b + ftd::cload(leaf_cnt, l);
-        n_leaves++;
-        n_prims += e - b;
-        n_pairs += (uint32_t)__popcll(admit) * (e - b);   // lane-triangle pairs whose lane admits the leaf
-        if (MODE == 0) {
-            for (uint32_t s = b; s < e; s++) {
-                const float4 p = ftd::cload(prec, s);
-                const int32_t j = ftd::cload(pidx, s);
-                const float dx = p.x - x, dy = p.y - y, dz = p.z - z;
-                const float s2 = dx * dx + dy * dy + dz * dz;
-                // bnd = best^2 (1 + 2^-16): beyond it sqrtf(s2) > best, which the
-                // strict compare would reject anyway, so the point is skipped
-                // when no lane is within it
-                if (__ballot(s2 <= bnd) == 0ull) continue;
-                const float d = sqrtf(s2);                            // EuclideanDistance.cu:20-28
-                consider(d, j);
-            }
-        } else {
-            // two records per step: their scalar loads are in flight together
-            // (three or four need more scalar registers than full occupancy
-            // leaves: 106 SGPRs, occupancy 7, spills)
-            uint32_t s = b;
-            for (; s + 1 < e; s += 2) {
-                const TriRec r0 = ftd::cload(trec, s);
-                const TriRec r1 = ftd::cload(trec, s + 1);
-                const int32_t j0 = ftd::cload(pidx, s), j1 = ftd::cload(pidx, s + 1);
-                test_tri(r0, j0);
-                test_tri(r1, j1);
-            }
-            if (s < e) test_tri(ftd::cload(trec, s), ftd::cload(pidx, s));
-        }
-    }
-
 };
 
 // Epilogue of one node (EuclideanDistance.cu:54-57, LevelSet.cpp:438-448, 74,
@@ -1458,7 +1427,7 @@ __device__ inline double node_tri_dist2(const QueryArgs& a, float x, float y, fl
 // lower wins, ties to the lower id.  No candidate: +-band in a narrow band,
 // else +-FLT_MAX.
 template <int MODE>
-__device__ __forceinline__ void finish_node(const QueryArgs& a, const Searcher<MODE>& S, int64_t node)
+__device__ __forceinline__ void finish_node(const QueryArgs& a, const Found& S, int64_t node)
 {
     if (MODE == 0) {
         const float d = (a.band > 0.0f && S.bj() < 0) ? a.band : S.best();
@@ -1482,52 +1451,33 @@ __device__ __forceinline__ void finish_node(const QueryArgs& a, const Searcher<M
     }
 }
 
-template <int MODE>
-__device__ __forceinline__ void record_stats(const QueryArgs& a, const Searcher<MODE>& S,
-                                             int64_t node, uint32_t n_nodes)
-{
-    // buckets: distance < 2h, < 8h, < 32h, beyond; +4 when phi < 0
-    const float dd = MODE == 0 ? S.best() : sqrtf(S.best());
-    const float hh = a.h_est;
-    int bkt = dd < 2 * hh ? 0 : dd < 8 * hh ? 1 : dd < 32 * hh ? 2 : 3;
-    if (a.phi_old[node] < 0.0) bkt += 4;
-    unsigned long long* st = a.stats + 5 * bkt;
-    atomicAdd(&st[0], 1ull);
-    atomicAdd(&st[1], (unsigned long long)n_nodes);
-    atomicAdd(&st[2], (unsigned long long)S.n_leaves);
-    atomicAdd(&st[3], (unsigned long long)S.n_prims);
-    atomicAdd(&st[4], (unsigned long long)S.n_pairs);
-}
-
-// Query schedule.  A tile that lies deep inside the surface costs 10-20x the
-// median tile (near the middle of a closed surface every triangle is nearly
-// equidistant, and the exact search must certify them all); started late,
-// such tiles set the kernel's end.  A tile is deep when one of its nodes has
-// phi_old <= -kDeepTileH h of its field.  Deep tiles are listed first and
-// take the lowest workgroups, which the dispatcher starts first and deals
-// over all XCDs; the rest keep their slot (Morton) order.  Measured at 256^3
-// (64 spheres, full domain): step 15.3 -> 12.6 ms; thresholds of 6-10 h do
-// about the same there, 10 h is best on the 128^3 field, 3 h and 20 h lose.
-constexpr float kDeepTileH = 10.0f;
-
-// The deepest tiles still set the kernel's end when they start first: at
-// 256^3 the tiles at the centres of the largest spheres (phi_old near -29 h)
-// test some 25k triangles each, and one wave's chain of dependent record
-// loads took 9.3-9.6 ms of a 9.6 ms kernel while the other tiles had ended by
-// about 9.0 ms (per-tile timestamps, a probe build).  A tile is very deep when
-// one of its nodes has phi_old <= -kSplitTileH h: it is searched by
+// Query schedule.  A tile deep inside a closed surface is the longest: near
+// the middle every triangle is nearly equidistant, and the exact search must
+// certify them all.  Its time grows with the square of the depth (256^3, 64
+// spheres: 3.3 ms at phi_old = -29 h where the mean tile takes 0.14 ms), so
+// such tiles, started late or in a small field, set the kernel's end.  A tile
+// is deep when one of its nodes has phi_old <= -kDeepTile split_h h of its
+// field: the deep tiles are listed first and take the lowest workgroups, which
+// the dispatcher starts first and deals over all XCDs; the rest keep their
+// slot (Morton) order.  A tile is very deep from -split_h h: it is searched by
 // kSplitParts waves, each with all 64 nodes but testing only the leaves l with
 // l % kSplitParts equal to its part, and k_split_merge combines the parts.
-// Each part repeats the walk of the inner tree nodes, so splitting costs work:
-// at 256^3 (query ms, this field and its mirror image across x = z) 2 parts
-// from 25 h gave 9.05 / 8.98, 4 parts 9.07-9.25 / 9.02, 4 parts from 20 h
-// 9.17 / 9.25, 8 parts 9.36, from 30 h the deepest tiles ran whole again
-// (10.9), and the unsplit query took 9.6-11.2 / 8.9-9.4 depending on the
-// order of the tiles.  Four parts keep more margin for fields deeper than
-// this one.  At most split_tiles_cap tiles per launch are split (the parts'
-// results take kSplitParts x 1 KiB per tile); the rest run whole.  The split
-// only changes which wave tests a leaf: each node's result is the same.
+// Each part repeats the walk above the leaves, so splitting costs work, and
+// the depth from which it pays goes down with the launch's own length: split_h
+// = 25 for 2^18 tiles (256^3 nodes), as the square root of the tiles below
+// that, at least 2.5 (a 32^3 sphere: 127 -> 69 us; at 256^3 15 h in place of
+// 25 h is 1% slower, 8 parts in place of 4 the same).  At most split_tiles_cap
+// tiles per launch are split (the parts' results take kSplitParts x 1 KiB per
+// tile); the rest run whole.  The split only changes which wave tests a leaf:
+// each node's result is the same.
+constexpr float kDeepTile = 0.4f;            // of split_tile_h
 constexpr float kSplitTileH = 25.0f;
+constexpr float kSplitTileMinH = 2.5f;
+inline float split_tile_h(int64_t n_tiles)
+{
+    const float h = kSplitTileH * std::sqrt((float)n_tiles / 262144.0f);
+    return std::min(kSplitTileH, std::max(kSplitTileMinH, h));
+}
 constexpr int kSplitParts = 4;
 constexpr int64_t kSplitCap = 1024;
 
@@ -1540,8 +1490,8 @@ __host__ __device__ inline int64_t split_tiles_cap(int64_t n_tiles)
 // One wave per tile: cls[t] = 2 when some node of tile t is very deep, 1 when
 // deep, else 0.
 __global__ __launch_bounds__(kBS) void k_tile_deep(int64_t n_tiles, const int32_t* perm, const double* phi,
-                                                   const int32_t* tile_field, const Grid* grids,
-                                                   uint32_t* cls, const uint64_t* sc)
+                                                   const int32_t* tile_field, const Grid* grids, float deep_h,
+                                                   float split_h, uint32_t* cls, const uint64_t* sc)
 {
     if (halted(sc)) return;
     const int64_t t = ((int64_t)blockIdx.x * kBS + threadIdx.x) >> 6;
@@ -1549,8 +1499,8 @@ __global__ __launch_bounds__(kBS) void k_tile_deep(int64_t n_tiles, const int32_
     const int32_t node = perm[t * 64 + ftd::lane_id()];
     const float h = grids[tile_field[t]].h;
     const double p = node >= 0 ? phi[node] : 0.0;
-    const uint64_t m1 = __ballot(p <= -(double)(kDeepTileH * h));
-    const uint64_t m2 = __ballot(p <= -(double)(kSplitTileH * h));
+    const uint64_t m1 = __ballot(p <= -(double)(deep_h * h));
+    const uint64_t m2 = __ballot(p <= -(double)(split_h * h));
     if (ftd::lane_id() == 0) cls[t] = m2 ? 2u : (m1 ? 1u : 0u);
 }
 
@@ -1571,104 +1521,565 @@ __global__ __launch_bounds__(kBS) void k_tile_list(int64_t n_tiles, const uint32
     list[at] = (int32_t)t;
 }
 
-// Wave-coherent search: the 64 lanes of a wave hold 64 consecutive slots of
-// one field in Morton order (a compact tile) and walk that field's tree
-// together.  A child is entered when any lane's bound admits it; each lane
-// keeps its own best.  All control flow is wave-uniform (ballots), node and
-// primitive records are read at wave-uniform addresses through scalar loads,
-// the stack is one per wave in LDS.
-// split >= 0: part split % kSplitParts of split tile split / kSplitParts,
-// whose best and second keys go to a.split_out instead of the epilogue.
+// ---- the search of one tile -------------------------------------------------
+// Traversal counts of a tile (FT_QUERY_STATS).
+struct TileStats {
+    uint32_t nodes = 0, boxes = 0, leaves = 0, prims = 0, pairs = 0;
+};
+
 template <int MODE>
-__device__ __forceinline__ void search_tile(const QueryArgs& a, int64_t base, int32_t* stack, int split = -1)
+__device__ __forceinline__ void record_stats(const QueryArgs& a, const Found& S, int64_t node, const TileStats& t)
 {
-    const int64_t slot = base + (threadIdx.x & 63);
-    const int32_t node = a.perm[slot];                 // -1: padding lane
-    const float px = a.sx[slot], py = a.sy[slot], pz = a.sz[slot];
-    const int field = __builtin_amdgcn_readfirstlane(a.tile_field[base >> 6]);
-    const int32_t root = __builtin_amdgcn_readfirstlane(ftd::cload(a.roots, field));
-    Searcher<MODE> S;
-    S.x = px; S.y = py; S.z = pz;
-    if (MODE == 0) S.init_best(a.band > 0.0f ? a.band : FLT_MAX);
-    else S.init_best(a.band > 0.0f ? a.band * a.band : INFINITY);
-    S.prec = a.prec; S.trec = a.trec; S.pidx = a.pidx;
-    S.leaf_start = a.leaf_start; S.leaf_cnt = a.leaf_cnt;
-    S.ifp = a.ifp; S.tris = a.tris;
-    if (split >= 0) {
-        S.parts = kSplitParts;
-        S.part = __builtin_amdgcn_readfirstlane(split % kSplitParts);
-    }
-    uint32_t n_nodes = 0;
-    if (root != INT32_MIN && root < 0) {
-        S.test_leaf_uniform(~root);
-    } else if (root >= 0) {
-        if (a.probe) {
-            // Greedy descent for the tile's middle slot to a leaf near it: a
-            // first exact candidate for every lane.  The child whose bound
-            // centre is nearer is taken (cheaper than the bounds and, in a
-            // model of the traversal, a seed after which less is tested).
-            const float cx = __shfl(px, 32), cy = __shfl(py, 32), cz = __shfl(pz, 32);
-            int cur = root;
-            for (int depth = 0; depth < kStack + 1 && cur >= 0; depth++) {
-                const BNode nd = ftd::cload(a.nodes, cur);
-                const float lx = cx - nd.l.c[0], ly = cy - nd.l.c[1], lz = cz - nd.l.c[2];
-                const float rx = cx - nd.r.c[0], ry = cy - nd.r.c[1], rz = cz - nd.r.c[2];
-                const float ll = __fmaf_rn(lz, lz, __fmaf_rn(ly, ly, lx * lx));
-                const float lr = __fmaf_rn(rz, rz, __fmaf_rn(ry, ry, rx * rx));
-                cur = __builtin_amdgcn_readfirstlane(ll <= lr ? nd.left : nd.right);
-            }
-            if (cur < 0) S.test_leaf_uniform(~cur);
-        }
-        int sp = 0;
-        int cur = root;
-        int budget = 2 * a.L + 8;
-        while (--budget > 0) {
-            const BNode nd = ftd::cload(a.nodes, cur);    // scalar loads: cur is uniform
-            const int left = nd.left, right = nd.right;
-            const float bnd = S.bnd;
-            // box bound first; the cylinder only where some lane's box admits it
-            float ll = ftd::box_dist2(px, py, pz, nd.l.lo, nd.l.hi);
-            float lr = ftd::box_dist2(px, py, pz, nd.r.lo, nd.r.hi);
-            if (__ballot(ll <= bnd)) ll = ftd::max_nonneg(ll, ftd::cyl_dist2(px, py, pz, nd.l));
-            if (__ballot(lr <= bnd)) lr = ftd::max_nonneg(lr, ftd::cyl_dist2(px, py, pz, nd.r));
-            n_nodes++;
-            const uint64_t mL = __ballot(ll <= bnd), mR = __ballot(lr <= bnd);
-            const uint64_t any = mL | mR;
-            const bool left_first = 2 * __popcll(__ballot(ll <= lr) & any) >= __popcll(any);
-            const int c0 = left_first ? left : right, c1 = left_first ? right : left;
-            const uint64_t m0 = left_first ? mL : mR, m1 = left_first ? mR : mL;
-            int next = -1;
-            if (m0) {
-                if (c0 < 0) S.test_leaf_uniform(~c0, m0);
-                else next = c0;
-            }
-            if (m1) {
-                if (c1 < 0) S.test_leaf_uniform(~c1, m1);
-                else if (next < 0) next = c1;
-                else if (sp < kStack) stack[sp++] = c1;
-                else atomicOr(a.overflow, 1u);
-            }
-            if (next < 0) {
-                if (sp == 0) break;
-                next = stack[--sp];
-            }
-            cur = __builtin_amdgcn_readfirstlane(next);
-        }
-        if (budget <= 0) atomicOr(a.overflow, 2u);
-    }
-    if (split >= 0) {                                  // full domain: nothing is clamped
-        a.split_out[(int64_t)split * 64 + (threadIdx.x & 63)] = make_ulonglong2(S.bkey, S.skey);
-        return;
-    }
-    const bool clamped = node >= 0 && a.band > 0.0f && S.bj() < 0;
-    const uint64_t cm = __ballot(clamped);
-    if ((threadIdx.x & 63) == 0 && cm) atomicAdd(&a.n_clamped[field], (unsigned long long)__popcll(cm));
-    if (node < 0) return;
-    if (a.stats) record_stats<MODE>(a, S, node, n_nodes);
-    finish_node<MODE>(a, S, node);
+    // buckets: distance < 2h, < 8h, < 32h, beyond; +4 when phi < 0
+    const float dd = MODE == 0 ? S.best() : sqrtf(S.best());
+    const float hh = a.h_est;
+    int bkt = dd < 2 * hh ? 0 : dd < 8 * hh ? 1 : dd < 32 * hh ? 2 : 3;
+    if (a.phi_old[node] < 0.0) bkt += 4;
+    unsigned long long* st = a.stats + 6 * bkt;
+    atomicAdd(&st[0], 1ull);
+    atomicAdd(&st[1], (unsigned long long)t.nodes);
+    atomicAdd(&st[2], (unsigned long long)t.boxes);
+    atomicAdd(&st[3], (unsigned long long)t.leaves);
+    atomicAdd(&st[4], (unsigned long long)t.prims);
+    atomicAdd(&st[5], (unsigned long long)t.pairs);
 }
 
-// Query schedule of a launch: deep tiles first (kDeepTileH), the rest in
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+// Squared length with the parts' negative values as 0 and each part at most
+// 1 (scaled coordinates: the clamp is the subtraction's own output modifier,
+// one instruction; a part cut to 1 only lowers the bound).
+__device__ __forceinline__ float sat(float v) { return __builtin_amdgcn_fmed3f(v, 0.0f, 1.0f); }
+__device__ __forceinline__ float box_d2(float x, float y, float z, const float4& e)
+{
+    const float dx = sat(fabsf(x) - e.x), dy = sat(fabsf(y) - e.y), dz = sat(fabsf(z) - e.z);
+    return __fmaf_rn(dx, dx, __fmaf_rn(dy, dy, dz * dz));
+}
+// The same to a triangle's rectangle (no extent along its normal).
+__device__ __forceinline__ float rect_d2(float x, float y, float z, const float2& e)
+{
+    const float dx = sat(fabsf(x) - e.x), dy = sat(fabsf(y) - e.y);
+    return __fmaf_rn(dx, dx, __fmaf_rn(dy, dy, z * z));
+}
+
+// Least of the wave's keys (the lanes of a wave run together; every lane
+// holds one): row shifts, then broadcasts over the rows, the total in lane 63.
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v)
+{
+#define FT_DPP_MIN(ctrl) \
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp((int)0xffffffffu, (int)v, ctrl, 0xf, 0xf, false))
+    FT_DPP_MIN(0x111);                        // row_shr 1, 2, 4, 8
+    FT_DPP_MIN(0x112);
+    FT_DPP_MIN(0x114);
+    FT_DPP_MIN(0x118);
+    FT_DPP_MIN(0x142);                        // row_bcast 15, 31
+    FT_DPP_MIN(0x143);
+#undef FT_DPP_MIN
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// LDS of one wave.  The nodes' keys, coordinates and pruning bounds are kept
+// here and not in registers, because the search works on (node, primitive)
+// pairs, whose node is any lane's.
+constexpr int kQueue = 64 + 256;              // pairs: less than a wave's, then one group's
+template <int MODE>
+struct __align__(16) WaveLds {
+    unsigned long long best[64];
+    unsigned long long sec[MODE == 1 ? 64 : 1];
+    float px[64], py[64], pz[64];
+    uint2 queue[kQueue];                      // (primitive slot, node's lane); the seed search's lists before
+    float thr[MODE == 0 ? 128 : 64];
+    uint32_t range[kLevels - 1][66];          // per level of the walk: the children's ranges (first[])
+    uint4 stack[kLevels - 1];                 // lists of the levels above: first child, mask
+};
+
+// Orders the wave's LDS stores before its loads (a wave runs its lanes
+// together: a wave-scope fence waits for its own LDS accesses).
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Search of the tile of 64 nodes held by a wave, one node per lane.
+//
+// Pruning is separated from the exact distances:
+//  - four boxes (the children of a node, or the rectangles of a leaf's
+//    triangles) are taken against the 64 nodes by four 16 x 16 x 4 matrix
+//    instructions: the coordinates of 16 nodes along the 12 box axes at once.
+//    In the product lane l holds box l / 16 and node l % 16 of the 16, its
+//    three coordinates in three registers, so the distance to the box is 6 or
+//    7 instructions for 64 (node, box) pairs and a compare against the node's
+//    bound.  Crossing points take 16 per instruction: |q|^2 - 2 p.q about the
+//    tile's centre against the bound less |p|^2.
+//  - the pairs that pass go to a queue in LDS, and every 64 of them are
+//    evaluated together, one pair per lane, whichever nodes and primitives
+//    they are: a primitive that concerns 9 nodes costs 9 lanes and not 64.
+//    Their keys go to the nodes' best (and second) by LDS minimum.
+//  - nothing is sorted: a first search for the tile's centre alone (children
+//    on the lanes, nearest first) finds a primitive near every node's nearest
+//    before the walk, and with bounds that good the order of the walk is
+//    worth 4% (in a model of the traversal at 256^3; without that first
+//    search the walk takes twice the boxes and triangles).
+// Every cut is a lower bound compared with the node's best so far raised by
+// its rounding: scaled coordinates are good to 2^-20 along each axis, so the
+// bound is (sqrt(best) + 2^-19)^2; results are the exact search's.
+//
+// What bounds it: vector issue (79% of its rate at 256^3: 11.1k vector
+// instructions per tile, 205k matrix ones in all).  256^3, 64 spheres, full
+// domain: 6.1 ms, against 9.1-9.5 ms for a wave-wide walk of a binary tree that
+// tested every box and triangle on all 64 lanes (19.9k instructions per tile);
+// crossing points 3.2 against 3.9 ms.
+template <int MODE, bool STATS>
+struct TileSearch {
+    const QueryArgs& a;
+    WaveLds<MODE>& lds;
+    const int lane;
+    uint32_t qn = 0;                          // queued pairs
+    float thr[4];                             // scaled bounds of nodes 16 cb + lane % 16
+    v4h B[4];                                 // matrix operand of those nodes: coordinates and 1, split (see Item)
+    float inv_s;
+    float cen[3], pp = 0.0f;                  // tile centre; points: |p - cen|^2 of the lane's node, lowered
+    float rel[MODE == 0 ? 4 : 1];             // points: operand about the centre
+    TileStats st;
+
+    __device__ __forceinline__ TileSearch(const QueryArgs& q, WaveLds<MODE>& l, int ln) : a(q), lds(l), lane(ln) {}
+
+    // The lane as a value the compiler takes for new: what is derived from it
+    // is formed again here rather than kept (or spilled) across the search.
+    __device__ __forceinline__ int fresh_lane() const
+    {
+        int l = lane;
+        asm volatile("" : "+v"(l));
+        return l;
+    }
+
+    __device__ __forceinline__ float node_best(int i) const
+    {
+        return __uint_as_float((uint32_t)(lds.best[i] >> 32));
+    }
+
+    // The nodes' bounds from their keys.
+    __device__ __forceinline__ void refresh()
+    {
+        wave_lds_sync();
+        const float b = node_best(lane);
+        const float bnd = prune_bound(MODE == 0 ? b * b : b);
+        const float s = __fmaf_rn(ftd::sqrt_lb(bnd) * inv_s, 1.0f + 0x1.0p-20f, 0x1.0p-19f);
+        lds.thr[lane] = s * s;
+        if (MODE == 0) lds.thr[64 + lane] = __fmaf_rn(bnd, 1.0f + 0x1.0p-18f, -pp);
+        wave_lds_sync();
+#pragma unroll
+        for (int cb = 0; cb < 4; cb++) thr[cb] = lds.thr[16 * cb + (lane & 15)];
+    }
+
+    // The exact FP32 distance of the queue's last n (<= 64) pairs.
+    __device__ __forceinline__ void flush(uint32_t n)
+    {
+        wave_lds_sync();
+        const bool on = (uint32_t)lane < n;
+        const uint2 p = lds.queue[qn - n + (on ? lane : 0)];
+        qn -= n;
+        if (STATS) st.pairs += n;
+        const float x = lds.px[p.y], y = lds.py[p.y], z = lds.pz[p.y];
+        if (MODE == 0) {
+            const float4 r = a.prec[p.x];
+            const float dx = r.x - x, dy = r.y - y, dz = r.z - z;
+            const float d = sqrtf(dx * dx + dy * dy + dz * dz);        // EuclideanDistance.cu:20-28
+            if (on) atomicMin(&lds.best[p.y], (unsigned long long)cand_key(d, __float_as_int(r.w)));
+        } else {
+            const TriRec r = a.trec[p.x];
+            const uint64_t key = cand_key(ftd::tri_dist2(x, y, z, r), ftd::tri_id(r));
+            if (on) {
+                // a key that is beaten, or beats one, leaves the loser to the second
+                const uint64_t old = atomicMin(&lds.best[p.y], (unsigned long long)key);
+                if (old != key) atomicMin(&lds.sec[p.y], (unsigned long long)(old > key ? old : key));
+            }
+        }
+        refresh();
+    }
+
+    // Queues the (slot, node) pairs of the lanes in m.
+    __device__ __forceinline__ void enqueue(uint64_t m, uint32_t slot, uint32_t node)
+    {
+        const uint32_t at = qn + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+        if (__builtin_amdgcn_inverse_ballot_w64(m)) lds.queue[at] = make_uint2(slot, node);
+        qn += (uint32_t)__popcll(m);
+    }
+
+    // Boxes it[0..3] of the n (1..4, more count as 4) left against the nodes:
+    // passing (box, node) pairs per 16 nodes.
+    __device__ __forceinline__ static float item_d2(const v4f& p, const float4& e) { return box_d2(p[0], p[1], p[2], e); }
+    __device__ __forceinline__ static float item_d2(const v4f& p, const float2& e) { return rect_d2(p[0], p[1], p[2], e); }
+    template <class E>
+    __device__ __forceinline__ void cull4(v4h av, const E& e, uint32_t n, uint64_t m[4]) const
+    {
+        const uint64_t live = n >= 4 ? ~0ull : (1ull << (16 * n)) - 1ull;
+        v4f d[4];
+#pragma unroll
+        for (int cb = 0; cb < 4; cb++) d[cb] = __builtin_amdgcn_mfma_f32_16x16x16f16(av, B[cb], v4f{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+        for (int cb = 0; cb < 4; cb++) m[cb] = __ballot(item_d2(d[cb], e) <= thr[cb]) & live;
+    }
+    // This lane's element of the matrix operand of items it[0..3], and the
+    // extents of item lane / 16.  (Up to three items past the last are read.)
+    template <class E>
+    __device__ __forceinline__ static void load4(const Item* it, int lane, v4h& av, E& e)
+    {
+        const v4h* f = reinterpret_cast<const v4h*>(it);       // 8 per item: a row's hi and lo in turn
+        av = f[(uint32_t)(((lane & 15) >> 2) * 8 + (lane & 3) * 2 + (lane >> 5))];
+        e = *reinterpret_cast<const E*>(f + (uint32_t)((lane >> 4) * 8 + 6));
+    }
+
+    // Which of the children [c0, c0 + cnt), cnt <= 64, some node admits; their
+    // ranges go to lds.range[d].
+    __device__ __forceinline__ uint64_t admitted(uint32_t c0, uint32_t cnt, int d)
+    {
+        const int lane = fresh_lane();
+        v4h av;
+        float4 e;
+        load4(a.items + c0, lane, av, e);
+        const uint32_t f = a.first[c0 + lane], fe = a.first[c0 + cnt];   // (past the children: unused)
+        if (STATS) {
+            st.nodes++;
+            st.boxes += cnt;
+        }
+        uint32_t keep = 0;                             // lane k: child k's nodes (any of the 4 sets of 16)
+        for (uint32_t i = 0; i < cnt; i += 4) {
+            v4h av1 = av;
+            float4 e1 = e;
+            if (i + 4 < cnt) load4(a.items + c0 + i + 4, lane, av1, e1);
+            uint64_t m[4];
+            cull4(av, e, cnt - i, m);
+            const uint64_t u = (m[0] | m[1]) | (m[2] | m[3]);
+            const uint32_t mine = (uint32_t)(u >> (16 * (lane & 3))) & 0xffffu;
+            keep = (uint32_t)lane >> 2 == i >> 2 ? mine : keep;
+            av = av1;
+            e = e1;
+        }
+        lds.range[d][lane] = f;
+        lds.range[d][cnt] = fe;                        // (after the lanes' own: a wave's LDS writes keep their order)
+        wave_lds_sync();
+        return __ballot(keep != 0u);
+    }
+
+    // Range of element b of list d.
+    __device__ __forceinline__ void range_of(int d, uint32_t b, uint32_t& s0, uint32_t& s1) const
+    {
+        s0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds.range[d][b]);
+        s1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds.range[d][b + 1]);
+    }
+
+    // The next leaf of a list: element b of mask, taken out of it; of a split
+    // tile's leaves only those of its part.  False when there is none.
+    __device__ __forceinline__ bool next_leaf(uint64_t& mask, int d, uint32_t& s0, uint32_t& s1)
+    {
+        if (!mask) return false;
+        const uint32_t b = (uint32_t)(__ffsll((unsigned long long)mask) - 1);
+        mask &= mask - 1;
+        range_of(d, b, s0, s1);
+        if (STATS) {
+            st.leaves++;
+            st.prims += s1 - s0;
+        }
+        return true;
+    }
+
+    // The primitives of the leaves of mask (list d), the next group's loads in
+    // flight while one is taken, across leaves.
+    __device__ __forceinline__ void leaves(uint64_t mask, int d)
+    {
+        const int lane = fresh_lane();
+        uint32_t s, s1;
+        if (!next_leaf(mask, d, s, s1)) return;
+        if (MODE == 1) {
+            v4h av;
+            float2 e;
+            load4(a.titem + s, lane, av, e);
+            for (;;) {
+                uint32_t ns = s + 4, ns1 = s1;
+                const bool more = ns < s1 || next_leaf(mask, d, ns, ns1);
+                v4h av1 = av;
+                float2 e1 = e;
+                if (more) load4(a.titem + ns, lane, av1, e1);
+                uint64_t m[4];
+                cull4(av, e, s1 - s, m);
+                if ((m[0] | m[1]) | (m[2] | m[3])) {
+#pragma unroll
+                    for (int cb = 0; cb < 4; cb++)
+                        if (m[cb]) enqueue(m[cb], s + (uint32_t)(lane >> 4), (uint32_t)(16 * cb + (lane & 15)));
+                    while (qn >= 64) flush(64);
+                }
+                if (!more) return;
+                av = av1;
+                e = e1;
+                s = ns;
+                s1 = ns1;
+            }
+        } else {
+            const int k = lane >> 4;
+            const uint32_t i = (uint32_t)(lane & 15);
+            float4 r = a.prec[s + (i < s1 - s ? i : 0u)];
+            for (;;) {
+                uint32_t ns = s + 16, ns1 = s1;
+                const bool more = ns < s1 || next_leaf(mask, d, ns, ns1);
+                const float qx = r.x - cen[0], qy = r.y - cen[1], qz = r.z - cen[2];
+                if (more) r = a.prec[ns + (i < ns1 - ns ? i : 0u)];
+                const float qq = __fmaf_rn(qz, qz, __fmaf_rn(qy, qy, qx * qx)) * (1.0f - 0x1.0p-18f);
+                const float q3 = k == 0 ? qx : k == 1 ? qy : qz;
+                const float av = k == 3 ? qq : -2.0f * q3;
+                v4f p[4];
+#pragma unroll
+                for (int cb = 0; cb < 4; cb++)
+                    p[cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, rel[cb], v4f{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                const uint32_t left = s1 - s;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {              // points 4 (lane / 16) + q of the 16
+                    const uint32_t pi = (uint32_t)(4 * k + q);
+                    const uint64_t live = __ballot(pi < left);
+                    uint64_t m[4];
+#pragma unroll
+                    for (int cb = 0; cb < 4; cb++)
+                        m[cb] = __ballot(p[cb][q] <= lds.thr[64 + 16 * cb + (int)i]) & live;
+                    if ((m[0] | m[1]) | (m[2] | m[3])) {
+#pragma unroll
+                        for (int cb = 0; cb < 4; cb++)
+                            if (m[cb]) enqueue(m[cb], s + pi, 16 * cb + i);
+                        while (qn >= 64) flush(64);
+                    }
+                }
+                if (!more) return;
+                s = ns;
+                s1 = ns1;
+            }
+        }
+    }
+
+    // Squared distance, scaled, of a scaled point to an item's box, from the
+    // rows' upper halves alone (2^-12 of a unit: a seed need not be exact).
+    __device__ __forceinline__ static float box_of(const Item& it, float x, float y, float z)
+    {
+        auto at = [&](const Row& r) {
+            return __fmaf_rn((float)r.hi[0], x, __fmaf_rn((float)r.hi[1], y, __fmaf_rn((float)r.hi[2], z, (float)r.hi[3])));
+        };
+        return box_d2(at(it.x), at(it.y), at(it.z), it.e);
+    }
+
+    // The node just above the leaves with the leaf box nearest to the point
+    // (x, y, z) (scaled), and a primitive of that leaf near it: the children of
+    // a node one per lane, nearest first, boxes beyond the nearest leaf so far
+    // left out, as are those beyond `best` (squared, scaled).  At most
+    // kSeedSteps steps (the centre of a sphere would visit all of it): any
+    // primitive will do.
+    static constexpr int kSeedSteps = 48;
+    __device__ __forceinline__ void seed(uint32_t root, float x, float y, float z, float best, uint32_t& slot, uint32_t& node)
+    {
+        // per level, 64 each: the children's bounds, and their ranges
+        float* lists = reinterpret_cast<float*>(lds.queue);
+        uint32_t* begins = reinterpret_cast<uint32_t*>(lds.queue) + 64 * (kLevels - 2);
+        uint32_t f0, fb, fe, cur = root, s0 = 0, s1 = 0;
+        float lb;
+        int d = 0;
+        auto enter = [&](uint32_t c0, uint32_t c1) {   // the children [c0, c1)
+            f0 = c0;
+            fb = a.first[c0 + lane];
+            fe = a.first[c0 + lane + 1];
+            lb = (uint32_t)lane < c1 - c0 ? box_of(a.items[c0 + lane], x, y, z) : INFINITY;
+        };
+        enter(ftd::cload(a.first, root), ftd::cload(a.first, root + 1));
+        for (int step = 0; step < kSeedSteps; step++) {
+            const uint32_t key = wave_min_u32((__float_as_uint(lb) & ~63u) | (uint32_t)lane);
+            const uint32_t sel = key & 63u;
+            const bool nearer = __uint_as_float(key & ~63u) < best;
+            const uint32_t g0 = (uint32_t)__builtin_amdgcn_readlane((int)fb, sel), g1 = (uint32_t)__builtin_amdgcn_readlane((int)fe, sel);
+            const bool above = f0 >= a.leaf_end;       // the children are nodes
+            if (nearer && above) {
+                if ((uint32_t)lane == sel) lb = INFINITY;
+                lists[64 * d + lane] = lb;
+                begins[128 * d + lane] = fb;
+                begins[128 * d + 64 + lane] = fe;
+                if (lane == 0) lds.stack[d].x = f0;
+                d++;
+                cur = f0 + sel;
+                enter(g0, g1);
+                continue;
+            }
+            if (nearer) {
+                best = __uint_as_float(key & ~63u);
+                s0 = g0;
+                s1 = g1;
+                node = cur;
+            }
+            if (d == 0) break;
+            d--;
+            wave_lds_sync();
+            lb = lists[64 * d + lane];
+            fb = begins[128 * d + lane];
+            fe = begins[128 * d + 64 + lane];
+            f0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds.stack[d].x);
+        }
+        wave_lds_sync();
+        if (s0 == s1) return;
+        float t = INFINITY;
+        if (s0 + lane < s1) {
+            if (MODE == 1) {
+                t = box_of(a.titem[s0 + lane], x, y, z);
+            } else {
+                const float4 r = a.prec[s0 + lane];
+                const float dx = (r.x - cen[0]) * inv_s, dy = (r.y - cen[1]) * inv_s, dz = (r.z - cen[2]) * inv_s;
+                t = __fmaf_rn(dx, dx, __fmaf_rn(dy, dy, dz * dz));
+            }
+        }
+        slot = s0 + (wave_min_u32((__float_as_uint(t) & ~63u) | (uint32_t)lane) & 63u);
+    }
+
+    // The leaves of node g; part of parts: only leaves l % parts == part.
+    __device__ __forceinline__ uint64_t of_part(uint64_t mask, uint32_t c0, int parts, int part) const
+    {
+        if (parts == 1) return mask;
+        return __ballot(((mask >> lane) & 1ull) && (int)((c0 + (uint32_t)lane) % (uint32_t)parts) == part);
+    }
+
+    // Walks the tree at root: first the node `start` above the leaves (~0:
+    // none), whose primitives bring most nodes near their final bound, then
+    // the rest.
+    __device__ __forceinline__ void walk(uint32_t root, uint32_t start, int parts, int part)
+    {
+        bool first = start != ~0u && start != root;
+        const uint32_t skip = first ? start : ~0u;
+        uint32_t c0 = ftd::cload(a.first, first ? start : root), c1 = ftd::cload(a.first, (first ? start : root) + 1);
+        int sp = 0;                                    // list sp: the children of a node
+        for (;;) {
+            uint32_t f0 = c0;                          // the list's first child, and those still to visit
+            uint64_t mask = admitted(c0, c1 - c0, sp);
+            if (f0 < a.leaf_end) {
+                leaves(of_part(mask, f0, parts, part), sp);
+                mask = 0;
+            }
+            if (first) {
+                first = false;
+                c0 = ftd::cload(a.first, root);
+                c1 = ftd::cload(a.first, root + 1);
+                continue;
+            }
+            uint32_t b;
+            do {
+                while (!mask) {                        // back to a list with something left
+                    if (sp == 0) {
+                        if (qn) flush(qn);
+                        return;
+                    }
+                    sp--;
+                    const uint4 t = lds.stack[sp];
+                    f0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)t.x);
+                    mask = (uint32_t)__builtin_amdgcn_readfirstlane((int)t.y) |
+                           ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)t.z) << 32);
+                }
+                b = (uint32_t)(__ffsll((unsigned long long)mask) - 1);
+                mask &= mask - 1;
+            } while (f0 + b == skip);
+            range_of(sp, b, c0, c1);
+            if (lane == 0) lds.stack[sp] = make_uint4(f0, (uint32_t)mask, (uint32_t)(mask >> 32), 0u);
+            sp++;                                      // at most kLevels - 2: a leaf is no list
+        }
+    }
+};
+
+// A wave's tile: 64 consecutive slots of one field in Morton order.
+// split >= 0: part split % kSplitParts of split tile split / kSplitParts,
+// whose best and second keys go to a.split_out instead of the epilogue.
+template <int MODE, bool STATS>
+__device__ __forceinline__ void search_tile(const QueryArgs& a, int64_t base, WaveLds<MODE>& lds, int split = -1)
+{
+    // opaque to the compiler, which would else hoist everything that depends on
+    // the lane alone out of the work queue's loop, and spill it
+    int lane = ftd::lane_id();
+    asm volatile("" : "+v"(lane));
+    TileSearch<MODE, STATS> S(a, lds, lane);
+    const int64_t slot = base + lane;
+    const int32_t node = a.perm[slot];                 // -1: padding lane
+    Found F;
+    F.x = a.sx[slot]; F.y = a.sy[slot]; F.z = a.sz[slot];
+    const int field = __builtin_amdgcn_readfirstlane(a.tile_field[base >> 6]);
+    const uint32_t root = (uint32_t)__builtin_amdgcn_readfirstlane((int)ftd::cload(a.roots, field));
+    const uint64_t none = MODE == 0 ? cand_key(a.band > 0.0f ? a.band : FLT_MAX, -1)
+                                    : cand_key(a.band > 0.0f ? a.band * a.band : INFINITY, -1);
+    F.bkey = F.skey = none;
+    if (root != ~0u) {                                 // the field has primitives
+        const Grid* g = a.grids + field;
+        const float ox = ftd::cload(&g->org[0], 0), oy = ftd::cload(&g->org[1], 0), oz = ftd::cload(&g->org[2], 0);
+        S.inv_s = ftd::cload(&g->inv_s, 0);
+        wave_lds_sync();                               // the wave's last tile is done with its LDS
+        lds.px[lane] = F.x;
+        lds.py[lane] = F.y;
+        lds.pz[lane] = F.z;
+        lds.best[lane] = none;
+        if (MODE == 1) lds.sec[lane] = none;
+        // the middle of the tile's first and last node
+        auto middle = [](float v) {
+            return 0.5f * (__int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0)) +
+                           __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63)));
+        };
+        S.cen[0] = middle(F.x);
+        S.cen[1] = middle(F.y);
+        S.cen[2] = middle(F.z);
+        wave_lds_sync();
+        const int k = lane >> 4;
+#pragma unroll
+        for (int cb = 0; cb < 4; cb++) {
+            const int j = 16 * cb + (lane & 15);
+            if (MODE == 0)
+                S.rel[cb] = k == 0 ? lds.px[j] - S.cen[0] : k == 1 ? lds.py[j] - S.cen[1] : k == 2 ? lds.pz[j] - S.cen[2] : 1.0f;
+            // rows k = 0, 2 take the coordinates' upper halves (and 1), 1 and 3 the lower
+            const Row r = make_row((lds.px[j] - ox) * S.inv_s, (lds.py[j] - oy) * S.inv_s, (lds.pz[j] - oz) * S.inv_s, 1.0f);
+            S.B[cb] = (k & 1) ? r.lo : r.hi;
+        }
+        if (MODE == 0) {
+            const float dx = F.x - S.cen[0], dy = F.y - S.cen[1], dz = F.z - S.cen[2];
+            S.pp = __fmaf_rn(dz, dz, __fmaf_rn(dy, dy, dx * dx)) * (1.0f - 0x1.0p-18f);
+        }
+        uint32_t start = ~0u;
+        if (a.probe) {
+            uint32_t s = ~0u;
+            // in a narrow band: none beyond the band and the tile's half diagonal
+            const float hx = F.x - S.cen[0], hy = F.y - S.cen[1], hz = F.z - S.cen[2];
+            const float half = sqrtf(middle(hx * hx + hy * hy + hz * hz));
+            const float lim = (a.band + half) * S.inv_s;
+            S.seed(root, (S.cen[0] - ox) * S.inv_s, (S.cen[1] - oy) * S.inv_s, (S.cen[2] - oz) * S.inv_s,
+                   a.band > 0.0f ? lim * lim : INFINITY, s, start);
+            if (s != ~0u) {                            // every node to it
+                uint64_t key;
+                if (MODE == 0) {
+                    const float4 r = ftd::cload(a.prec, s);
+                    const float dx = r.x - F.x, dy = r.y - F.y, dz = r.z - F.z;
+                    key = cand_key(sqrtf(dx * dx + dy * dy + dz * dz), __float_as_int(r.w));
+                } else {
+                    const TriRec r = ftd::cload(a.trec, s);
+                    key = cand_key(ftd::tri_dist2(F.x, F.y, F.z, r), ftd::tri_id(r));
+                }
+                if (key < none) lds.best[lane] = key;
+            }
+        }
+        S.refresh();
+        S.walk(root, start, split >= 0 ? kSplitParts : 1, split >= 0 ? __builtin_amdgcn_readfirstlane(split % kSplitParts) : 0);
+        wave_lds_sync();
+        F.bkey = lds.best[lane];
+        if (MODE == 1) F.skey = lds.sec[lane];
+    }
+    if (split >= 0) {                                  // full domain: nothing is clamped
+        a.split_out[(int64_t)split * 64 + lane] = make_ulonglong2(F.bkey, F.skey);
+        return;
+    }
+    const bool clamped = node >= 0 && a.band > 0.0f && F.bj() < 0;
+    const uint64_t cm = __ballot(clamped);
+    if (lane == 0 && cm) atomicAdd(&a.n_clamped[field], (unsigned long long)__popcll(cm));
+    if (node < 0) return;
+    if (STATS) record_stats<MODE>(a, F, node, S.st);
+    finish_node<MODE>(a, F, node);
+}
+
+// Query schedule of a launch: deep tiles first (k_tile_deep), the rest in
 // XCD-chunked Morton order (xcd_block).  Static: one tile per wave, the
 // deep tiles on the first workgroups (which the dispatcher deals over all
 // XCDs; a very deep tile on kSplitParts of them, a.split_out), the others
@@ -1678,29 +2089,32 @@ __device__ __forceinline__ void search_tile(const QueryArgs& a, int64_t base, in
 // XCD b % 8), each XCD's share being its chunks of the static order; a wave
 // whose XCD has none left takes from the other XCDs' counters in turn.
 // Every wave leaves once all nine counters are past their ends.
-// Launch bound: WPS waves per SIMD (8: at most 64 VGPRs).  Unbounded, the
-// FP64 settle of the epilogue takes 84 VGPRs and the occupancy drops to 5
-// (measured 25% slower at 256^3); bounded at 8, it spills a few registers
-// that are touched once per node.
-template <int MODE, int BS, int WPS>
+// Launch bound: WPS waves per SIMD.  Six (80 VGPRs, 52 B of spills around
+// the FP64 settle) beat five (no spills) and seven at 256^3: triangles 6.79 /
+// 6.10 / 6.33 ms at 5 / 6 / 7, points 3.57 / 3.20 / 3.31; the wave's LDS allows
+// seven.  One wave per workgroup: with four, a workgroup's place is held by its
+// slowest wave (256^3: 8.8 ms).
+template <int MODE, int BS, int WPS, bool STATS = false>
 __global__ __launch_bounds__(BS, WPS) void k_query_wave(QueryArgs a)
 {
-    __shared__ int32_t wstack[BS / 64][kStack];
+    __shared__ WaveLds<MODE> wlds[BS / 64];
     if (halted(a.sc)) return;                         // an earlier stage failed: phi untouched
     const int w = threadIdx.x >> 6;
-    if (a.queue) {
-        // with no tile list (narrow band): the tiles in slot order, none deep
-        const int64_t n_tiles = a.n_slots / 64;
-        const uint32_t K = a.tile_list ? (uint32_t)ftd::cload(a.n_deep, 0) : 0u;
-        const uint32_t nn = (uint32_t)(n_tiles - K);
-        const uint32_t chunk = a.xcd_chunk;
-        const unsigned xcd = blockIdx.x % kXcds;
-        unsigned src = 0;                              // 0: deep counter; 1..8: XCD counters
-        for (;;) {
+    const int64_t n_tiles = a.n_slots / 64;
+    const uint64_t nd = a.tile_list ? ftd::cload(a.n_deep, 0) : 0ull;
+    const uint32_t K = (uint32_t)nd;                  // deep tiles (none in a narrow band: slot order)
+    unsigned src = 0;                                 // work queue: 0 the deep counter, 1..8 the XCDs'
+    for (;;) {
+        int64_t r;                                    // place in the launch order
+        int split = -1;
+        if (a.queue) {
+            const uint32_t nn = (uint32_t)(n_tiles - K);
+            const uint32_t chunk = a.xcd_chunk;
+            const unsigned xcd = blockIdx.x % kXcds;
             uint32_t got = 0;
             if (ftd::lane_id() == 0) got = atomicAdd(&a.queue[src == 0 ? 0 : 1 + (xcd + src - 1) % kXcds], 1u);
-            got = (uint32_t)__shfl(got, 0);
-            int64_t r = -1;
+            got = (uint32_t)__builtin_amdgcn_readfirstlane((int)got);
+            r = -1;
             if (src == 0) {
                 if (got < K) r = got;
             } else {
@@ -1710,53 +2124,48 @@ __global__ __launch_bounds__(BS, WPS) void k_query_wave(QueryArgs a)
                 const uint64_t t = (uint64_t)(got / chunk) * kXcds * chunk + (uint64_t)x * chunk + got % chunk;
                 if (t < nn) r = (int64_t)K + (int64_t)t;
             }
-            if (r >= 0) {
-                search_tile<MODE>(a, (a.tile_list ? (int64_t)a.tile_list[r] : r) * 64, wstack[w]);
+            if (r < 0) {
+                if (++src > kXcds) return;            // every counter exhausted
                 continue;
             }
-            if (++src > kXcds) break;                  // every counter exhausted
-        }
-        return;
-    }
-    int64_t base;
-    if (a.tile_list) {
-        // deep tiles on the first Kb workgroups (Kb a multiple of the 8 XCDs):
-        // first kSplitParts waves for each split tile, then one per other deep
-        // tile; the rest on the workgroups after them in XCD-chunked order
-        constexpr unsigned wpb = BS / 64;
-        const int64_t n_tiles = a.n_slots / 64;
-        const uint64_t nd = ftd::cload(a.n_deep, 0);
-        const unsigned K = (unsigned)nd;
-        // (explicit compares: min() of two 64-bit integers resolves to a
-        // floating-point overload here and rounds them)
-        const uint64_t cap = (uint64_t)split_tiles_cap(n_tiles);
-        const unsigned K2 = a.split_out ? (unsigned)((nd >> 32) < cap ? (nd >> 32) : cap) : 0u;
-        const unsigned D = K2 * kSplitParts + (K - K2);          // deep waves
-        const unsigned Kb = ((D + wpb - 1) / wpb + 7u) & ~7u;
-        const unsigned b = blockIdx.x;
-        int64_t r;
-        if (b < Kb) {
-            const unsigned rr = b * wpb + w;
-            if (rr >= D) return;                       // whole wave: padding of the deep workgroups
-            if (rr < K2 * kSplitParts) {
-                search_tile<MODE>(a, (int64_t)a.tile_list[rr / kSplitParts] * 64, wstack[w], (int)rr);
-                return;
+        } else if (a.tile_list) {
+            // deep tiles on the first Kb workgroups (Kb a multiple of the 8 XCDs):
+            // first kSplitParts waves for each split tile, then one per other deep
+            // tile; the rest on the workgroups after them in XCD-chunked order
+            constexpr unsigned wpb = BS / 64;
+            // (explicit compares: min() of two 64-bit integers resolves to a
+            // floating-point overload here and rounds them)
+            const uint64_t cap = (uint64_t)split_tiles_cap(n_tiles);
+            const unsigned K2 = a.split_out ? (unsigned)((nd >> 32) < cap ? (nd >> 32) : cap) : 0u;
+            const unsigned D = K2 * kSplitParts + (K - K2);          // deep waves
+            const unsigned Kb = ((D + wpb - 1) / wpb + 7u) & ~7u;
+            const unsigned b = blockIdx.x;
+            if (b < Kb) {
+                const unsigned rr = b * wpb + w;
+                if (rr >= D) return;                   // whole wave: padding of the deep workgroups
+                if (rr < K2 * kSplitParts) {
+                    split = (int)rr;
+                    r = rr / kSplitParts;
+                } else {
+                    r = (int64_t)K2 + (rr - K2 * kSplitParts);
+                }
+            } else {
+                const int64_t nn = n_tiles - K;
+                const unsigned nbn = (unsigned)((nn + wpb - 1) / wpb);
+                if (b - Kb >= nbn) return;             // whole wave: past the last tile
+                r = (int64_t)xcd_block(b - Kb, nbn, a.xcd_chunk) * wpb + w;
+                if (r >= nn) return;
+                r += K;
             }
-            r = (int64_t)K2 + (rr - K2 * kSplitParts);
         } else {
-            const int64_t nn = n_tiles - K;
-            const unsigned nbn = (unsigned)((nn + wpb - 1) / wpb);
-            if (b - Kb >= nbn) return;                 // whole wave: past the last tile
-            r = (int64_t)xcd_block(b - Kb, nbn, a.xcd_chunk) * wpb + w;
-            if (r >= nn) return;
-            r += K;
+            r = (int64_t)xcd_block(blockIdx.x, gridDim.x, a.xcd_chunk) * (BS / 64) + w;
+            if (r >= n_tiles) return;                  // whole wave out of range
         }
-        base = (int64_t)a.tile_list[r] * 64;
-    } else {
-        base = (int64_t)xcd_block(blockIdx.x, gridDim.x, a.xcd_chunk) * BS + (threadIdx.x & ~63);
-        if (base >= a.n_slots) return;                // whole wave out of range
+        // the wave's tile as uniform values
+        const int64_t tile = __builtin_amdgcn_readfirstlane(a.tile_list ? a.tile_list[r] : (int)r);
+        search_tile<MODE, STATS>(a, tile * 64, wlds[w], __builtin_amdgcn_readfirstlane(split));
+        if (!a.queue) return;
     }
-    search_tile<MODE>(a, base, wstack[w]);
 }
 
 // The parts of each split tile combined, one wave per tile: per lane the
@@ -1788,225 +2197,11 @@ __global__ __launch_bounds__(kBS) void k_split_merge(QueryArgs a)
         best = nb;
     }
     if (node < 0) return;
-    Searcher<MODE> S;
-    S.x = a.sx[slot]; S.y = a.sy[slot]; S.z = a.sz[slot];
-    S.bkey = best;
-    S.skey = second;
-    S.ifp = a.ifp; S.tris = a.tris;
-    finish_node<MODE>(a, S, node);
-}
-
-// ----------------------------------------------------------------------------
-// Narrow band without the tree (schedule FT_SCHED_BINS, triangles): each wave
-// takes its tile's box, widened by the band and by the largest distance from
-// a triangle's centroid to its vertices (the primitives are binned by
-// centroid), and walks the index bins in that box in their Morton order.  The
-// triangles of each non-empty bin are staged in LDS, 64 at a time, by the
-// wave's lanes, and every lane then tests each staged triangle (the frame
-// rectangle cull against its own bound, then the exact distance).  Each lane
-// keeps its own best two, as the tree walk does, so no cross-lane reduction
-// is needed.  Every triangle within the band of a lane has its centroid in
-// the widened box, and the lane's first bound is the band: the results are
-// the tree walk's, bit for bit.
-// ----------------------------------------------------------------------------
-struct BinQuery {
-    int64_t G;                       // bins over all fields (cnt_off[f] + code)
-    const uint64_t* prefix;          // (bins with triangles before << 32) | triangles before
-                                     // (the index's scan; the scatter consumed the counts)
-    const Grid* grids;               // per field
-    const int64_t* cnt_off;          // per field: its first bin
-};
-
-// Largest distance from a triangle's centroid (as k_prim_bin computes it) to
-// its vertices, as float bits (non-negative: integer max orders them).  A
-// grid-stride loop and one atomic per workgroup (one per wave contended).
-constexpr int kMarginBlocks = 512;
-__global__ __launch_bounds__(kBS) void k_tri_margin(const uint64_t* sc, const float* ifp, const int4* tris,
-                                                    uint32_t* out)
-{
-    __shared__ float part[kBS / 64];
-    if (halted(sc)) return;
-    const int64_t F = cnt_tris(sc);
-    float r = 0.0f;
-    for (int64_t j = (int64_t)blockIdx.x * kBS + threadIdx.x; j < F; j += (int64_t)gridDim.x * kBS) {
-        float a[3], b[3], d[3], c[3];
-        tri_vertices(tris, ifp, (int32_t)j, a, b, d);
-        for (int k = 0; k < 3; k++) c[k] = (a[k] + b[k] + d[k]) * (1.0f / 3.0f);
-        float m = 0.0f;
-        const float* v[3] = {a, b, d};
-        for (int q = 0; q < 3; q++) {
-            const float dx = v[q][0] - c[0], dy = v[q][1] - c[1], dz = v[q][2] - c[2];
-            m = fmaxf(m, sqrtf(dx * dx + dy * dy + dz * dz));
-        }
-        r = fmaxf(r, m);
-    }
-    for (int o = 32; o >= 1; o >>= 1) r = fmaxf(r, __shfl_xor(r, o));
-    if (ftd::lane_id() == 0) part[threadIdx.x >> 6] = r;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float m = part[0];
-        for (int k = 1; k < kBS / 64; k++) m = fmaxf(m, part[k]);
-        if (m > 0.0f) atomicMax(out, __float_as_uint(m));
-    }
-}
-
-// Orders the wave's LDS stores before its loads (a wave runs its lanes
-// together: a wave-scope fence waits for its own LDS accesses).
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-constexpr int kBinStage = 64;        // triangles staged per pass (one per lane)
-
-template <int BS>
-__global__ __launch_bounds__(BS, 8) void k_query_bins(QueryArgs a, BinQuery bq)
-{
-    __shared__ TriRec srec[BS / 64][kBinStage];
-    __shared__ int32_t sid[BS / 64][kBinStage];
-    if (halted(a.sc)) return;
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int64_t base = (int64_t)xcd_block(blockIdx.x, gridDim.x, a.xcd_chunk) * BS + (threadIdx.x & ~63);
-    if (base >= a.n_slots) return;                    // whole wave out of range
-    const int64_t slot = base + lane;
-    const int32_t node = a.perm[slot];
-    const float px = a.sx[slot], py = a.sy[slot], pz = a.sz[slot];
-    const int field = __builtin_amdgcn_readfirstlane(a.tile_field[base >> 6]);
-    Searcher<1> S;
-    S.x = px; S.y = py; S.z = pz;
-    S.init_best(a.band * a.band);
-    S.ifp = a.ifp; S.tris = a.tris;
-    // the tile's box over its real nodes, widened
-    float lo[3] = {node >= 0 ? px : INFINITY, node >= 0 ? py : INFINITY, node >= 0 ? pz : INFINITY};
-    float hi[3] = {node >= 0 ? px : -INFINITY, node >= 0 ? py : -INFINITY, node >= 0 ? pz : -INFINITY};
-    for (int o = 32; o >= 1; o >>= 1)
-        for (int k = 0; k < 3; k++) {
-            lo[k] = fminf(lo[k], __shfl_xor(lo[k], o));
-            hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], o));
-        }
-    const Grid g = bq.grids[field];
-    const float wide = a.band + __uint_as_float((uint32_t)ftd::cload(a.sc, S_MARGIN));
-    int b0[3], n[3];
-    for (int k = 0; k < 3; k++) {
-        // one more bin each side: the centroid's bin and this range round alike
-        // only up to the last ulp
-        // (clamped to the grid before the conversion: a wide band overflows int)
-        const float dmax = (float)g.dim[k];
-        const float f0 = fminf((lo[k] - wide - g.lo[k]) * g.inv_b, dmax);
-        const float f1 = fminf((hi[k] + wide - g.lo[k]) * g.inv_b, dmax);
-        const int i0 = f0 >= 1.0f ? (int)f0 - 1 : 0;
-        int i1 = f1 >= 0.0f ? (int)f1 + 1 : 0;
-        i1 = i1 < g.dim[k] - 1 ? i1 : g.dim[k] - 1;
-        b0[k] = __builtin_amdgcn_readfirstlane(i0 < g.dim[k] ? i0 : g.dim[k] - 1);
-        n[k] = __builtin_amdgcn_readfirstlane(i1 >= b0[k] ? i1 - b0[k] + 1 : 0);
-    }
-    // The widened range is walked in blocks of 4 x 4 x 4 bins, 64 consecutive
-    // Morton codes, whose triangle count is a difference of two prefix entries:
-    // a tile far from the surface finds every block empty in one pass.
-    const uint32_t off = (uint32_t)bq.cnt_off[field], fend = (uint32_t)bq.cnt_off[field + 1];
-    const uint32_t total = (uint32_t)cnt_tris(a.sc);
-    auto before = [&](uint32_t x) -> uint32_t { return (int64_t)x < bq.G ? (uint32_t)bq.prefix[x] : total; };
-    int B0[3], nB[3];
-    for (int k = 0; k < 3; k++) {
-        B0[k] = b0[k] >> 2;
-        nB[k] = n[k] > 0 ? ((b0[k] + n[k] - 1) >> 2) - B0[k] + 1 : 0;
-    }
-    const int64_t nblk = (int64_t)nB[0] * nB[1] * nB[2];
-    // this lane's place in a block (Morton bits: z0 y0 x0 z1 y1 x1)
-    const int lz = (lane & 1) | ((lane >> 2) & 2), ly = ((lane >> 1) & 1) | ((lane >> 3) & 2),
-              lx = ((lane >> 2) & 1) | ((lane >> 4) & 2);
-    for (int64_t q0 = 0; q0 < nblk; q0 += 64) {
-        const int64_t q = q0 + lane;
-        uint32_t first = 0, bc = 0;
-        int bxq = 0, byq = 0, bzq = 0;
-        if (q < nblk) {
-            bzq = B0[2] + (int)(q % nB[2]);
-            byq = B0[1] + (int)((q / nB[2]) % nB[1]);
-            bxq = B0[0] + (int)(q / ((int64_t)nB[2] * nB[1]));
-            first = off + (ftd::morton3((uint32_t)bxq, (uint32_t)byq, (uint32_t)bzq) << 6);
-            const uint32_t last = first + 64 < fend ? first + 64 : fend;
-            bc = first < fend ? before(last) - before(first) : 0u;
-        }
-        // non-empty blocks nearest the tile first (the nodes' bounds then
-        // tighten early and reject more of the later bins): distance from the
-        // tile's box to the block's, only to order them
-        float bd = INFINITY;
-        if (bc > 0) {
-            const float e = 4.0f / g.inv_b;
-            const int bq3[3] = {bxq, byq, bzq};
-            float d2 = 0.0f;
-            for (int k = 0; k < 3; k++) {
-                const float l0 = g.lo[k] + (float)bq3[k] * e;
-                const float gap = fmaxf(fmaxf(l0 - hi[k], lo[k] - (l0 + e)), 0.0f);
-                d2 = __fmaf_rn(gap, gap, d2);
-            }
-            bd = fminf(d2, FLT_MAX);                  // finite for every block in `blocks`
-        }
-        uint64_t blocks = __ballot(bc > 0);
-        // each pass takes out one block (a lane in `blocks` has the least key:
-        // finite, against infinity for the others), so at most 64 passes
-        for (int pass = 0; pass < 64 && blocks; pass++) {
-            // the lane holding the nearest remaining block
-            float mv = bd;
-            int ml = lane;
-            for (int o = 32; o >= 1; o >>= 1) {
-                const float ov = __shfl_xor(mv, o);
-                const int ol = __shfl_xor(ml, o);
-                if (ov < mv || (ov == mv && ol < ml)) { mv = ov; ml = ol; }
-            }
-            const int sb = __builtin_amdgcn_readfirstlane(ml);
-            blocks &= ~(1ull << sb);
-            if (lane == sb) bd = INFINITY;
-            const uint32_t c = (uint32_t)__shfl((int)first, sb) + (uint32_t)lane;
-            const int bx = 4 * __shfl(bxq, sb) + lx, by = 4 * __shfl(byq, sb) + ly, bz = 4 * __shfl(bzq, sb) + lz;
-            uint32_t cnt = 0;
-            if (bx >= b0[0] && bx < b0[0] + n[0] && by >= b0[1] && by < b0[1] + n[1] && bz >= b0[2] &&
-                bz < b0[2] + n[2]) {
-                const uint64_t pc = bq.prefix[c];
-                cnt = before(c + 1) - (uint32_t)pc;
-                if (cnt) {
-                    // the bin's leaf box against the tile's box: beyond the band
-                    // of every node, skipped (the box gap is a lower bound on
-                    // each node's distance to the leaf)
-                    const Bound& lb = a.leaf_b[(uint32_t)(pc >> 32)];
-                    float d2 = 0.0f;
-                    for (int k = 0; k < 3; k++) {
-                        const float gap = fmaxf(fmaxf(lb.lo[k] - hi[k], lo[k] - lb.hi[k]), 0.0f);
-                        d2 = __fmaf_rn(gap, gap, d2);
-                    }
-                    if (d2 > prune_bound(a.band * a.band)) cnt = 0;
-                }
-            }
-            uint64_t has = __ballot(cnt > 0);
-            while (has) {
-                const int src = __ffsll((unsigned long long)has) - 1;
-                has &= has - 1;
-                const uint32_t cc = (uint32_t)__shfl((int)c, src), nt = (uint32_t)__shfl((int)cnt, src);
-                const uint64_t pcc = bq.prefix[cc];
-                const uint32_t start = (uint32_t)pcc;
-                // each node against the bin's leaf box, with its bound so far
-                const Bound& lb = a.leaf_b[(uint32_t)(pcc >> 32)];
-                if (__ballot(ftd::box_dist2(px, py, pz, lb.lo, lb.hi) <= S.bnd) == 0ull) continue;
-                for (uint32_t s0 = 0; s0 < nt; s0 += kBinStage) {
-                    const uint32_t k = nt - s0 < (uint32_t)kBinStage ? nt - s0 : (uint32_t)kBinStage;
-                    if ((uint32_t)lane < k) {
-                        srec[w][lane] = a.trec[start + s0 + lane];
-                        sid[w][lane] = a.pidx[start + s0 + lane];
-                    }
-                    wave_lds_sync();
-                    for (uint32_t t = 0; t < k; t++) S.test_tri(srec[w][t], sid[w][t]);
-                    wave_lds_sync();                   // before the next pass overwrites them
-                }
-            }
-        }
-    }
-    const bool clamped = node >= 0 && S.bj() < 0;
-    const uint64_t cm = __ballot(clamped);
-    if (lane == 0 && cm) atomicAdd(&a.n_clamped[field], (unsigned long long)__popcll(cm));
-    if (node < 0) return;
-    finish_node<1>(a, S, node);
+    Found F;
+    F.x = a.sx[slot]; F.y = a.sy[slot]; F.z = a.sz[slot];
+    F.bkey = best;
+    F.skey = second;
+    finish_node<MODE>(a, F, node);
 }
 
 // ============================================================================
@@ -3313,13 +3508,15 @@ struct ft_ctx {
     uint64_t n2t_layout = ~0ull;
     bool have_normals = false;
     // index
-    DevBuf bin_count, bin_prefix, pcode, prec, trec, pidx, leaf_key, leaf_start, leaf_cnt;
-    DevBuf leaf_b, leaf_parent, bnodes, bflags, stats;
-    DevBuf d_grids, d_cnt_off, leaf_off, roots;
+    DevBuf bin_count, bin_prefix;    // the node sort's bins (mesh set-up)
+    DevBuf bbits, bprefix, pcode, place, prec, titem, trec, pidx;
+    DevBuf leaf_cnt, leaf_bin, nfirst, nitem, naxis, stats;
+    DevBuf d_grids, d_cnt_off, roots;
     uint64_t idx_layout = ~0ull;     // layout and bin scale the grids were made for
     float idx_bin_scale = 0.0f;
-    int64_t idx_G = 0;               // bins over all fields
-    int idx_code_bits = 0;
+    int64_t idx_G = 0;               // bins over all fields (a multiple of 64)
+    int64_t idx_words[5] = {0, 0, 0, 0, 0};   // blocks of 64^k bins over all fields
+    int idx_top = 1;                 // highest level that holds a field's root
     GraphState graph;
     // capacities for the next eager call on the same fields and mode
     Caps spec_caps;
@@ -3354,14 +3551,13 @@ std::vector<DevBuf*> all_buffers(ft_ctx* h)
 {
     return {&h->xyz, &h->tets, &h->edges, &h->t2e, &h->perm, &h->sx, &h->sy, &h->sz,
             &h->tile_field, &h->tile_sched, &h->gather_tab, &h->field_tab, &h->d_node_off, &h->d_tet_off, &h->d_edge_off, &h->d_slot_off,
-            &h->fcounts, &h->fclamp, &h->d_grids, &h->d_cnt_off, &h->leaf_off, &h->roots,
+            &h->fcounts, &h->fclamp, &h->d_grids, &h->d_cnt_off, &h->roots,
             &h->phi_tmp, &h->phi_ifn_tmp, &h->sbits, &h->retain, &h->tbits, &h->blk,
             &h->xtet, &h->xtri_off, &h->xedges, &h->ebits, &h->eprefix, &h->ifp,
             &h->ifp2e, &h->tris, &h->tri_norm, &h->if_elems, &h->p2t_off,
             &h->p2t_cursor, &h->p2t, &h->ifp_area, &h->nearest, &h->bin_count,
-            &h->bin_prefix, &h->pcode, &h->prec, &h->trec, &h->pidx, &h->leaf_key,
-            &h->leaf_start, &h->leaf_cnt, &h->leaf_b, &h->leaf_parent,
-            &h->bnodes, &h->bflags, &h->stats, &h->scan_bsum, &h->scan_side, &h->deep_part, &h->scalars,
+            &h->bin_prefix, &h->bbits, &h->bprefix, &h->pcode, &h->place, &h->prec, &h->titem, &h->trec,
+            &h->pidx, &h->leaf_cnt, &h->leaf_bin, &h->nfirst, &h->nitem, &h->naxis, &h->stats, &h->scan_bsum, &h->scan_side, &h->deep_part, &h->scalars,
             &h->n2t_off, &h->n2t_ids, &h->grad_t, &h->normals, &h->phi_ifn_int,
             &h->gsplit, &h->kmesh, &h->k_if, &h->st_cnt, &h->st_off, &h->st_ids, &h->st_f,
             &h->fem_len, &h->fem_w, &h->fem_soff, &h->fem_cols, &h->fem_m, &h->fem_l, &h->fem_flag, &h->fem_map,
@@ -3470,6 +3666,14 @@ Grid make_grid(const FieldHost& f, float edge, int max_lg, int* lg_out)
     }
     g.inv_b = 1.0f / b;
     g.h = f.h;
+    // scaled coordinates: about the box's middle, in units of a power of two
+    // of at least twice its longest side (scaling rounds nothing; the field
+    // and what lies within half a side of it stay within one unit)
+    int ex = 0;
+    (void)std::frexp(std::min(std::max(ext_max, 1e-30f), 1e30f), &ex);   // ext_max < 2^ex
+    for (int k = 0; k < 3; k++) g.org[k] = f.lo[k] + 0.5f * (f.hi[k] - f.lo[k]);
+    g.inv_s = std::ldexp(1.0f, -(ex + 1));
+    g.root_lv = std::max(1, (lg + 1) / 2);
     *lg_out = lg;
     return g;
 }
@@ -3780,7 +3984,7 @@ int sort_nodes(ft_ctx* c)
 // with more room (phi is only written by the last kernel, so nothing is lost).
 // Default bin edge, in node spacings, per distance mode (0 points, 1
 // triangles).  A bin's primitives form one leaf.  Points are cheap to test and
-// their least-squares-plane cylinder tightens with more points, so their
+// their least-squares-plane box tightens with more points, so their
 // optimum is larger: measured on 32^3..256^3 fields, points 2.0-2.5, triangles
 // 1.25.
 constexpr float kDefaultBinScale[2] = {2.0f, 1.25f};
@@ -3793,16 +3997,19 @@ int index_setup(ft_ctx* c, hipStream_t s, float bin_scale, int mode)
     if (c->idx_layout == c->layout_gen && c->idx_bin_scale == bs) return FT_OK;
     const int nf = c->nf;
     const int fb = field_bits(nf);
-    // keys (field << code_bits) | code stay below 2^30
+    // bins of all fields together stay near 2^30
     const int max_lg = std::min(kMaxBinsLog2PerAxis, (30 - fb) / 3);
     std::vector<Grid> grids(nf);
     std::vector<int64_t> cnt_off(nf + 1, 0);
-    int lg_max = 0;
+    int64_t words[kLevels] = {0, 0, 0, 0, 0};
+    int top = 1;
     for (int k = 0; k < nf; k++) {
         int lg = 0;
         grids[k] = make_grid(c->fh[k], bs * c->fh[k].h, max_lg, &lg);
-        lg_max = std::max(lg_max, lg);
-        cnt_off[k + 1] = cnt_off[k] + ((int64_t)1 << (3 * lg));
+        top = std::max(top, grids[k].root_lv);
+        const int64_t bins = (int64_t)1 << (3 * lg);
+        cnt_off[k + 1] = cnt_off[k] + std::max<int64_t>(64, bins);   // whole bitmap words
+        for (int q = 1; q < kLevels; q++) words[q] += std::max<int64_t>(1, bins >> (6 * q));
     }
     const int64_t G = cnt_off[nf];
     if (G > ((int64_t)1 << 32))
@@ -3814,7 +4021,8 @@ int index_setup(ft_ctx* c, hipStream_t s, float bin_scale, int mode)
                           hipMemcpyHostToDevice, s));
     FT_HIP(hipStreamSynchronize(s));
     c->idx_G = G;
-    c->idx_code_bits = 3 * lg_max;
+    for (int q = 0; q < kLevels; q++) c->idx_words[q] = q ? words[q] : G;
+    c->idx_top = top;
     c->idx_layout = c->layout_gen;
     c->idx_bin_scale = bs;
     return FT_OK;
@@ -3822,11 +4030,27 @@ int index_setup(ft_ctx* c, hipStream_t s, float bin_scale, int mode)
 
 inline int64_t at_least1(int64_t v) { return std::max<int64_t>(1, v); }
 
-// Cylinder kept only while its volume is below its box's (measured at 256^3:
-// 0 -> 21.2 ms, 0.5 -> 20.9, 1 -> 20.8, 2 -> 21.1, 4 -> 21.2 ms query).
-constexpr float kCylAlpha = 1.0f;
-float cyl_alpha() { return kCylAlpha; }
 inline int64_t scan_blocks(int64_t n) { return std::max<int64_t>(1, (n + kScanTile - 1) / kScanTile); }
+
+// Numbering of the index's leaves and nodes for at most n primitives: each
+// level's capacity, and one more entry for the end of its last range.
+struct LevelPlan {
+    LevelOff lo;
+    int64_t cap[kLevels];
+    int64_t total;
+};
+LevelPlan level_plan(const ft_ctx* c, int64_t n)
+{
+    LevelPlan p{};
+    int64_t at = 0;
+    for (int k = 0; k < kLevels; k++) {
+        p.cap[k] = std::min(n, c->idx_words[k]);
+        p.lo.off[k] = (uint32_t)at;
+        at += p.cap[k] + 1;
+    }
+    p.total = at;
+    return p;
+}
 
 // Device buffers of the stages of one reinit.  Stage 0: sized by the mesh;
 // 1: by crossing tets and triangles; 2: by crossing points; 3: the index over
@@ -3846,8 +4070,7 @@ int ensure_stage(ft_ctx* c, int stage, const Caps& cp, int mode, bool want_neare
         FT_TRY(ensure(c->eprefix, 4 * at_least1(nw_edges)));
         FT_TRY(ensure(c->fcounts, sizeof(int64_t) * 3 * nf));
         FT_TRY(ensure(c->fclamp, sizeof(uint64_t) * nf));
-        FT_TRY(ensure(c->roots, sizeof(int32_t) * nf));
-        FT_TRY(ensure(c->leaf_off, sizeof(int32_t) * (nf + 1)));
+        FT_TRY(ensure(c->roots, sizeof(uint32_t) * nf));
         if (want_nearest) FT_TRY(ensure(c->nearest, sizeof(int32_t) * at_least1(N)));
         if (want_normals) {
             FT_TRY(ensure(c->normals, 12 * at_least1(N)));
@@ -3872,25 +4095,35 @@ int ensure_stage(ft_ctx* c, int stage, const Caps& cp, int mode, bool want_neare
         FT_TRY(ensure(c->scan_side, sizeof(uint64_t) * std::max(scan_blocks(cp.P), scan_blocks(c->n_slots / 64))));
     } else {
         const int64_t n = mode == 0 ? cp.P : cp.F;
-        const int64_t G = c->idx_G;
-        const int64_t L = std::min(G, n);
-        FT_TRY(ensure(c->bin_count, sizeof(uint32_t) * at_least1(G)));
-        FT_TRY(ensure(c->bin_prefix, sizeof(uint64_t) * at_least1(G)));
+        const int64_t W = c->idx_G / 64;
+        const LevelPlan lp = level_plan(c, n);
+        if (lp.total > (int64_t)UINT32_MAX)
+            return ft::set_error(FT_ERR_ARG, "index: too many leaves (%lld)", (long long)lp.total);
+        // the limit of ft_reinit_device_noalloc on the index's bins (about
+        // 128^3 nodes) is part of its contract: 12 bytes a bin
+        if (t_arena && t_arena->used + 12 * (size_t)c->idx_G > t_arena->size)
+            return ft::set_error(FT_ERR_BUDGET, "%lld index bins are more than the %zu-byte scratch of "
+                                 "ft_reinit_device_noalloc takes; use ft_reinit_device", (long long)c->idx_G,
+                                 t_arena->size);
+        FT_TRY(ensure(c->bbits, 8 * at_least1(W)));
+        FT_TRY(ensure(c->bprefix, 4 * at_least1(W)));
         FT_TRY(ensure(c->pcode, sizeof(uint32_t) * at_least1(n)));
+        FT_TRY(ensure(c->place, sizeof(uint32_t) * at_least1(n)));
         FT_TRY(ensure(c->pidx, sizeof(int32_t) * at_least1(n)));
-        if (mode == 0) FT_TRY(ensure(c->prec, sizeof(float4) * at_least1(n)));
-        else FT_TRY(ensure(c->trec, sizeof(TriRec) * at_least1(n)));
-        FT_TRY(ensure(c->leaf_key, sizeof(uint32_t) * at_least1(L)));
-        FT_TRY(ensure(c->leaf_start, sizeof(uint32_t) * at_least1(L)));
-        FT_TRY(ensure(c->leaf_cnt, sizeof(uint32_t) * at_least1(L)));
-        FT_TRY(ensure(c->leaf_b, sizeof(Bound) * at_least1(L)));
-        FT_TRY(ensure(c->leaf_parent, sizeof(int32_t) * at_least1(L)));
-        FT_TRY(ensure(c->bnodes, sizeof(BNode) * at_least1(L - 1)));
-        // arrival counters (L - 1), then the ready count and list (1 + L - 1)
-        FT_TRY(ensure(c->bflags, sizeof(unsigned) * at_least1(2 * L)));
+        if (mode == 0) {
+            FT_TRY(ensure(c->prec, sizeof(float4) * at_least1(n)));
+        } else {
+            FT_TRY(ensure(c->titem, sizeof(Item) * (n + 4)));        // the search reads items by fours
+            FT_TRY(ensure(c->trec, sizeof(TriRec) * at_least1(n)));
+        }
+        FT_TRY(ensure(c->leaf_cnt, sizeof(uint32_t) * at_least1(lp.cap[0])));
+        FT_TRY(ensure(c->leaf_bin, sizeof(uint32_t) * at_least1(lp.cap[0])));
+        FT_TRY(ensure(c->nfirst, sizeof(uint32_t) * (lp.total + 64)));   // (read a wave at a time)
+        FT_TRY(ensure(c->nitem, sizeof(Item) * (lp.total + 4)));
+        FT_TRY(ensure(c->naxis, sizeof(float4) * lp.total));
         // scan scratch of the largest scan of a reinit
-        const int64_t nb = std::max({scan_blocks(nblk), scan_blocks(nw_edges), scan_blocks(cp.P),
-                                     scan_blocks(G)});
+        const int64_t nb = std::max({scan_blocks(nblk), scan_blocks(nw_edges), scan_blocks(cp.P), scan_blocks(W),
+                                     3 * scan_blocks(lp.cap[0])});
         FT_TRY(ensure(c->scan_bsum, sizeof(uint64_t) * nb));
         FT_TRY(ensure(c->deep_part, sizeof(ulonglong2) * 64 * kSplitParts * at_least1(split_tiles_cap(c->n_slots / 64))));
     }
@@ -3956,9 +4189,8 @@ struct SearchSpec {
     bool want_normals = false;       // Assembler::grad_nodes of phi_ifn after the epilogue
     bool int_ifn = false;            // phi_ifn into the handle's buffer (normals need it)
     int query_block = 0;
-    int waves_per_simd = 8;          // launch bound of the query (triangles: 5..8)
+    int waves_per_simd = 6;          // launch bound of the query (triangles: 5..8)
     bool work_queue = false;         // persistent query over tile counters
-    bool bins = false;               // narrow band: bins staged in LDS instead of the tree walk
 };
 
 // Copies of the resident meshes ms into the handle's concatenated arrays,
@@ -4103,7 +4335,6 @@ int enqueue_marching(ft_ctx* c, hipStream_t s, double* phi, int mode, bool want_
     FT_TRY(fill<uint64_t>(s, c->ebits.as<uint64_t>(), nw_edges, 0ull));
     FT_TRY(fill<uint64_t>(s, sc + S_ERR, 1, ~0ull));
     FT_TRY(fill<uint64_t>(s, sc + S_CAP, 1, 0ull));
-    FT_TRY(fill<uint64_t>(s, sc + S_OVF, 1, 0ull));
     FT_TRY(fill<uint64_t>(s, sc + S_EDGES, 1, 0ull));   // the edge scan writes the low 32 bits
     if (T > 0)
         hipLaunchKernelGGL(k_classify, dim3((unsigned)((nblk + kClassifyGroups - 1) / kClassifyGroups)),
@@ -4185,21 +4416,26 @@ int enqueue_marching(ft_ctx* c, hipStream_t s, double* phi, int mode, bool want_
 }
 
 // The query kernel for (mode, threads per workgroup, waves per SIMD); points
-// mode has the 8-wave bound only (its epilogue has no FP64 settle to spill).
+// mode has its best bound only.
 template <int MODE, int BS>
 int launch_query_bs(int wps, dim3 g, dim3 b, hipStream_t s, const QueryArgs& q)
 {
-    switch (MODE == 0 ? 8 : wps) {
-    case 5: hipLaunchKernelGGL((k_query_wave<MODE, BS, 5>), g, b, 0, s, q); break;
-    case 6: hipLaunchKernelGGL((k_query_wave<MODE, BS, 6>), g, b, 0, s, q); break;
-    case 7: hipLaunchKernelGGL((k_query_wave<MODE, BS, 7>), g, b, 0, s, q); break;
-    default: hipLaunchKernelGGL((k_query_wave<MODE, BS, 8>), g, b, 0, s, q); break;
+    switch (MODE == 0 ? 6 : wps) {
+    case 5: hipLaunchKernelGGL((k_query_wave<MODE, BS, MODE == 0 ? 6 : 5>), g, b, 0, s, q); break;
+    case 7: hipLaunchKernelGGL((k_query_wave<MODE, BS, MODE == 0 ? 6 : 7>), g, b, 0, s, q); break;
+    case 8: hipLaunchKernelGGL((k_query_wave<MODE, BS, MODE == 0 ? 6 : 8>), g, b, 0, s, q); break;
+    default: hipLaunchKernelGGL((k_query_wave<MODE, BS, 6>), g, b, 0, s, q); break;
     }
     return check_launch();
 }
 
 int launch_query(int mode, int qb, int wps, dim3 g, dim3 b, hipStream_t s, const QueryArgs& q)
 {
+    if (q.stats) {                                    // counting build (qb is 64)
+        if (mode == 0) hipLaunchKernelGGL((k_query_wave<0, 64, 5, true>), g, b, 0, s, q);
+        else hipLaunchKernelGGL((k_query_wave<1, 64, 5, true>), g, b, 0, s, q);
+        return check_launch();
+    }
     if (mode == 0) {
         if (qb == 64) return launch_query_bs<0, 64>(wps, g, b, s, q);
         if (qb == 128) return launch_query_bs<0, 128>(wps, g, b, s, q);
@@ -4240,50 +4476,46 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
         uint64_t* ex = reinterpret_cast<uint64_t*>(cls + 2 * n_tiles);
         hipLaunchKernelGGL(k_tile_deep, dim3(grid1d(64 * n_tiles)), dim3(kBS), 0, ss, n_tiles,
                            c->perm.as<int32_t>(), sp.phi_old, c->tile_field.as<int32_t>(),
-                           c->d_grids.as<Grid>(), cls, sc);
+                           c->d_grids.as<Grid>(), kDeepTile * split_tile_h(n_tiles), split_tile_h(n_tiles), cls, sc);
         FT_TRY(scan<uint32_t, uint64_t>(c, ss, cls, ex, n_tiles, sc + S_DEEP, LoadTileClass{}, &c->scan_side));
         hipLaunchKernelGGL(k_tile_list, dim3(grid1d(n_tiles)), dim3(kBS), 0, ss, n_tiles, cls, ex, sc,
                            tile_list);
     }
-    const int64_t G = c->idx_G;
-    const int64_t L_cap = std::min(G, n_cap);
-    IndexGeom ig{c->d_edge_off.as<int64_t>(), c->d_cnt_off.as<int64_t>(), c->d_grids.as<Grid>(), nf,
-                 c->idx_code_bits};
-    uint32_t* bcnt = c->bin_count.as<uint32_t>();
-    uint64_t* pre = c->bin_prefix.as<uint64_t>();
-    FT_TRY(fill<uint32_t>(s, bcnt, G, 0u));
-    if (n_cap > 0)
-        hipLaunchKernelGGL(k_prim_bin, dim3(grid1d(n_cap)), dim3(kBS), 0, s, mode, sc, ifp, tris,
-                           nf > 1 ? c->ifp2e.as<int32_t>() : nullptr, ig, c->pcode.as<uint32_t>(), bcnt);
-    FT_TRY(scan<uint32_t, uint64_t>(c, s, bcnt, pre, G, sc + S_BINS, LoadNonEmpty{}));
-    hipLaunchKernelGGL(k_field_roots, dim3((nf + 1 + 63) / 64), dim3(64), 0, s, nf,
-                       c->d_cnt_off.as<int64_t>(), pre, sc + S_BINS, G,
-                       c->leaf_off.as<int32_t>(), c->roots.as<int32_t>());
+    const int64_t W = c->idx_G / 64;
+    const LevelPlan lp = level_plan(c, n_cap);
+    const IndexGeom ig{c->d_edge_off.as<int64_t>(), c->d_cnt_off.as<int64_t>(), c->d_grids.as<Grid>(), nf};
+    uint64_t* bits = c->bbits.as<uint64_t>();
+    uint32_t* lcnt = c->leaf_cnt.as<uint32_t>();
+    uint32_t* lbin = c->leaf_bin.as<uint32_t>();
+    uint32_t* first = c->nfirst.as<uint32_t>();
+    uint32_t* code = c->pcode.as<uint32_t>();
+    FT_TRY(fill<uint64_t>(s, bits, W, 0ull));
+    FT_TRY(fill<uint32_t>(s, lcnt, lp.cap[0], 0u));
+    FT_TRY(fill<uint32_t>(s, c->roots.as<uint32_t>(), nf, ~0u));
+    FT_TRY(fill<uint64_t>(s, sc + S_BINS, 1, 0ull));      // the bitmap scan writes the low 32 bits
     if (n_cap > 0) {
-        hipLaunchKernelGGL(k_leaves, dim3(grid1d(G)), dim3(kBS), 0, s, bcnt, pre, G, ig,
-                           c->leaf_key.as<uint32_t>(), c->leaf_start.as<uint32_t>(),
-                           c->leaf_cnt.as<uint32_t>());
-        hipLaunchKernelGGL(k_prim_scatter, dim3(grid1d(n_cap)), dim3(kBS), 0, s, mode, sc, ifp, tris,
-                           c->pcode.as<uint32_t>(), bcnt, pre, c->prec.as<float4>(),
+        hipLaunchKernelGGL(k_prim_bin, dim3(grid1d(n_cap)), dim3(kBS), 0, s, mode, sc, ifp, tris,
+                           nf > 1 ? c->ifp2e.as<int32_t>() : nullptr, ig, code, (unsigned long long*)bits);
+        FT_TRY(scan<uint64_t, uint32_t>(c, s, bits, c->bprefix.as<uint32_t>(), W,
+                                        reinterpret_cast<uint32_t*>(sc + S_BINS), LoadPopc{}));
+        hipLaunchKernelGGL(k_prim_rank, dim3(grid1d(n_cap)), dim3(kBS), 0, s, mode, sc, bits,
+                           c->bprefix.as<uint32_t>(), code, c->place.as<uint32_t>(), lcnt, lbin);
+        const int64_t nb = scan_blocks(lp.cap[0]);
+        ftd::Lv* bs = c->scan_bsum.as<ftd::Lv>();
+        hipLaunchKernelGGL(k_level_reduce, dim3((unsigned)nb), dim3(kBS), 0, s, sc, lcnt, lbin, ig, bs);
+        hipLaunchKernelGGL(k_scan_top<ftd::Lv>, dim3(1), dim3(1024), 0, s, bs, nb,
+                           reinterpret_cast<ftd::Lv*>(sc + S_LV));
+        hipLaunchKernelGGL(k_level_down, dim3((unsigned)nb), dim3(kBS), 0, s, sc, lcnt, lbin, ig, bs, lp.lo, first,
+                           c->roots.as<uint32_t>());
+        hipLaunchKernelGGL(k_prim_scatter, dim3(grid1d(n_cap)), dim3(kBS), 0, s, mode, sc, ifp, tris, code,
+                           c->place.as<uint32_t>(), first, lbin, ig, c->prec.as<float4>(), c->titem.as<Item>(),
                            c->trec.as<TriRec>(), c->pidx.as<int32_t>());
-        hipLaunchKernelGGL(mode == 0 ? k_leaf_bounds<0> : k_leaf_bounds<1>, dim3(grid1d(L_cap)), dim3(kBS), 0, s, sc,
-                           c->leaf_start.as<uint32_t>(), c->leaf_cnt.as<uint32_t>(),
-                           c->pidx.as<int32_t>(), ifp, tris, c->leaf_b.as<Bound>());
-    }
-    if (L_cap > 1) {
-        // arrival counters and the ready count
-        FT_TRY(fill<unsigned>(s, c->bflags.as<unsigned>(), L_cap, 0u));
-        hipLaunchKernelGGL(k_karras, dim3(grid1d(L_cap - 1)), dim3(kBS), 0, s,
-                           c->leaf_key.as<uint32_t>(), sc, c->bnodes.as<BNode>(),
-                           c->leaf_parent.as<int32_t>(), c->idx_code_bits,
-                           c->leaf_off.as<int32_t>(), c->roots.as<int32_t>());
-        unsigned* ready = c->bflags.as<unsigned>() + (L_cap - 1);
-        hipLaunchKernelGGL(k_refit_local, dim3((unsigned)((L_cap + kRefitBlock - 1) / kRefitBlock)),
-                           dim3(kRefitBlock), 0, s, sc, c->leaf_parent.as<int32_t>(),
-                           c->leaf_b.as<Bound>(), c->bnodes.as<BNode>(), c->bflags.as<unsigned>(),
-                           ready, cyl_alpha());
-        hipLaunchKernelGGL(k_refit_top, dim3(1), dim3(kRefitTopThreads), 0, s, sc,
-                           c->bnodes.as<BNode>(), c->bflags.as<unsigned>(), ready, cyl_alpha());
+        hipLaunchKernelGGL(mode == 0 ? k_leaf_items<0> : k_leaf_items<1>, dim3(grid1d(kLeafLanes * lp.cap[0])),
+                           dim3(kBS), 0, s, sc, first, lbin, ig, c->pidx.as<int32_t>(), ifp, tris,
+                           c->nitem.as<Item>(), c->naxis.as<float4>());
+        for (int k = 1; k < c->idx_top; k++)               // a root's own box is never tested
+            hipLaunchKernelGGL(k_node_items, dim3((unsigned)std::min<int64_t>(grid1d(64 * lp.cap[k]), kNodeBlocks)),
+                               dim3(kBS), 0, s, sc, k, lp.lo.off[k], first, c->nitem.as<Item>(), c->naxis.as<float4>());
     }
     FT_TRY(check_launch());
 
@@ -4294,15 +4526,14 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
     q.sx = c->sx.as<float>(); q.sy = c->sy.as<float>(); q.sz = c->sz.as<float>();
     q.perm = c->perm.as<int32_t>();
     q.tile_field = c->tile_field.as<int32_t>();
-    q.roots = c->roots.as<int32_t>();
+    q.grids = c->d_grids.as<Grid>();
+    q.roots = c->roots.as<uint32_t>();
+    q.first = first;
+    q.items = c->nitem.as<Item>();
+    q.leaf_end = lp.lo.off[1];
     q.prec = c->prec.as<float4>();
+    q.titem = c->titem.as<Item>();
     q.trec = c->trec.as<TriRec>();
-    q.pidx = c->pidx.as<int32_t>();
-    q.leaf_start = c->leaf_start.as<uint32_t>();
-    q.leaf_cnt = c->leaf_cnt.as<uint32_t>();
-    q.leaf_b = c->leaf_b.as<Bound>();
-    q.nodes = c->bnodes.as<BNode>();
-    q.L = (int)L_cap;
     q.band = sp.band;
     q.ifp = ifp;
     q.tris = tris;
@@ -4318,16 +4549,14 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
     static const bool want_stats = getenv("FT_QUERY_STATS") != nullptr;
     q.h_est = c->h_est;
     if (want_stats && eager) {
-        FT_TRY(ensure(c->stats, 8 * 40));
-        FT_TRY(fill<uint64_t>(s, c->stats.as<uint64_t>(), 40, 0ull));
+        FT_TRY(ensure(c->stats, 8 * 48));
+        FT_TRY(fill<uint64_t>(s, c->stats.as<uint64_t>(), 48, 0ull));
         q.stats = c->stats.as<unsigned long long>();
     }
-    q.overflow = (unsigned*)(sc + S_OVF);
-    // The greedy probe seeds each full-domain search with a candidate (256^3:
-    // query 11.3 -> 10.4 ms).  In a narrow band the band itself bounds the
-    // search and most tiles end clamped, for which the probe is wasted work
-    // (128^3 star, 6h band: 0.696 -> 0.675 ms without it).
-    q.probe = sp.band <= 0.0f && !(getenv("FT_PROBE") && !strcmp(getenv("FT_PROBE"), "0"));
+    // the first search for each tile's centre; in a narrow band too (128^3
+    // star, 6 h: surface tiles test half the leaves and a third of the pairs,
+    // query 0.597 -> 0.511 ms)
+    q.probe = !(getenv("FT_PROBE") && !strcmp(getenv("FT_PROBE"), "0"));
     q.sc = sc;
     q.xcd_chunk = kXcdChunk;
     if (timed) (void)hipEventRecord(c->ev[2], s);
@@ -4337,22 +4566,9 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
         q.n_deep = sc + S_DEEP;
     }
     if (c->n_slots > 0) {
-        const int qb = sp.query_block == 64 || sp.query_block == 128 ? sp.query_block : 256;
+        const int qb = q.stats || sp.query_block == 0 ? 64 : sp.query_block;
         q.xcd_chunk = qb == 64 ? kXcdChunk64 : kXcdChunk;
-        const int wps = mode == 0 ? 8 : sp.waves_per_simd;
-        if (sp.bins) {
-            // narrow band from the bins, staged in LDS (no tree walk)
-            FT_TRY(fill<uint64_t>(s, sc + S_MARGIN, 1, 0ull));
-            if (n_cap > 0)
-                hipLaunchKernelGGL(k_tri_margin, dim3((unsigned)std::min<int64_t>(grid1d(n_cap), kMarginBlocks)),
-                                   dim3(kBS), 0, s, sc, ifp, tris, reinterpret_cast<uint32_t*>(sc + S_MARGIN));
-            const BinQuery bq{G, c->bin_prefix.as<uint64_t>(), c->d_grids.as<Grid>(), c->d_cnt_off.as<int64_t>()};
-            const dim3 gb(grid1d(c->n_slots, qb)), bb(qb);
-            if (qb == 64) hipLaunchKernelGGL(k_query_bins<64>, gb, bb, 0, s, q, bq);
-            else if (qb == 128) hipLaunchKernelGGL(k_query_bins<128>, gb, bb, 0, s, q, bq);
-            else hipLaunchKernelGGL(k_query_bins<256>, gb, bb, 0, s, q, bq);
-            FT_TRY(check_launch());
-        } else {
+        const int wps = mode == 0 ? 6 : sp.waves_per_simd;
         // with a tile list: up to 7 padding workgroups after the deep ones,
         // one more for the split of the remainder, and the extra waves of
         // the split tiles (static schedule)
@@ -4374,7 +4590,6 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
             if (mode == 0) hipLaunchKernelGGL(k_split_merge<0>, gm, dim3(kBS), 0, s, q);
             else hipLaunchKernelGGL(k_split_merge<1>, gm, dim3(kBS), 0, s, q);
             FT_TRY(check_launch());
-        }
         }
     }
     if (timed) (void)hipEventRecord(c->ev[3], s);
@@ -4414,9 +4629,6 @@ int collect(ft_ctx* c, hipStream_t s, bool want_nearest, ft_counts* cnt)
     if (hs[S_CAP]) return FT_ERR_BUDGET;
     FT_TRY(stage_error(hs[S_ERR], cnt));
     c->have_interface = true;
-    if (hs[S_OVF])
-        return ft::set_error(FT_ERR_HIP, "search: traversal exceeded its bounds (%llu)",
-                             (unsigned long long)hs[S_OVF]);
     c->field_counts.assign(nf, ft_counts{});
     for (int k = 0; k < nf; k++) {
         ft_counts& f = c->field_counts[k];
@@ -4437,24 +4649,23 @@ int collect(ft_ctx* c, hipStream_t s, bool want_nearest, ft_counts* cnt)
 
 void print_query_stats(ft_ctx* c, int mode)
 {
-    uint64_t st[40];
+    uint64_t st[48];
     if (hipMemcpy(st, c->stats.p, sizeof st, hipMemcpyDeviceToHost) != hipSuccess) return;
     static const char* names[8] = {"out <2h", "out 2-8h", "out 8-32h", "out >32h",
                                    "in <2h", "in 2-8h", "in 8-32h", "in >32h"};
-    double tn = 0, tl = 0, tp = 0, tq = 0;
+    static const char* what = "nodes %.1f boxes %.1f leaves %.1f primitives %.1f pairs %.1f\n";
+    double t[6] = {0, 0, 0, 0, 0, 0};
+    for (int b = 0; b < 8; b++)
+        for (int q = 0; q < 6; q++) t[q] += (double)st[6 * b + q];
+    // the counts are the tile's, added once per node
+    fprintf(stderr, "[ftreinit] query mode %d: N=%lld, per tile: ", mode, (long long)c->N);
+    fprintf(stderr, what, t[1] / t[0], t[2] / t[0], t[3] / t[0], t[4] / t[0], t[5] / t[0]);
     for (int b = 0; b < 8; b++) {
-        tn += st[5 * b + 1]; tl += st[5 * b + 2]; tp += st[5 * b + 3]; tq += st[5 * b + 4];
-    }
-    fprintf(stderr, "[ftreinit] query mode %d: N=%lld per node: tree nodes %.1f, leaves %.1f, "
-            "primitives %.1f, lanes admitting a tested leaf %.1f%%\n", mode, (long long)c->N,
-            tn / c->N, tl / c->N, tp / c->N, tp > 0 ? 100.0 * tq / (64.0 * tp) : 0.0);
-    for (int b = 0; b < 8; b++) {
-        const double nn = (double)st[5 * b];
-        if (nn > 0)
-            fprintf(stderr, "[ftreinit]   %-9s %5.1f%% of nodes: tree %.1f leaves %.1f prims %.1f "
-                    "admitting lanes %.1f%%\n", names[b], 100.0 * nn / c->N, st[5 * b + 1] / nn,
-                    st[5 * b + 2] / nn, st[5 * b + 3] / nn,
-                    st[5 * b + 3] > 0 ? 100.0 * st[5 * b + 4] / (64.0 * st[5 * b + 3]) : 0.0);
+        const double nn = (double)st[6 * b];
+        if (!(nn > 0)) continue;
+        fprintf(stderr, "[ftreinit]   %-9s %5.1f%% of nodes: ", names[b], 100.0 * nn / c->N);
+        fprintf(stderr, what, st[6 * b + 1] / nn, st[6 * b + 2] / nn, st[6 * b + 3] / nn, st[6 * b + 4] / nn,
+                st[6 * b + 5] / nn);
     }
 }
 
@@ -4474,9 +4685,8 @@ SearchSpec reinit_search_spec(double* phi, double* phi_ifn, const ft_opts* o)
     sp.want_normals = o->want_normals != 0;
     sp.int_ifn = sp.want_normals && !phi_ifn;
     sp.query_block = o->query_block;
-    sp.waves_per_simd = o->waves_per_simd > 0 ? o->waves_per_simd : 8;
+    sp.waves_per_simd = o->waves_per_simd > 0 ? o->waves_per_simd : 6;
     sp.work_queue = o->schedule == FT_SCHED_QUEUE;
-    sp.bins = o->schedule == FT_SCHED_BINS;
     return sp;
 }
 
@@ -4726,9 +4936,9 @@ std::vector<DevBuf*> call_buffers(ft_ctx* h)
             &h->xtri_off, &h->xedges, &h->ebits, &h->eprefix, &h->ifp, &h->ifp2e, &h->tris,
             &h->tri_norm, &h->if_elems, &h->p2t_off, &h->p2t_cursor, &h->p2t, &h->ifp_area,
             &h->nearest, &h->fcounts, &h->fclamp, &h->normals, &h->grad_t, &h->phi_ifn_int,
-            &h->bin_count, &h->bin_prefix, &h->pcode, &h->prec, &h->trec, &h->pidx, &h->leaf_key,
-            &h->leaf_start, &h->leaf_cnt, &h->leaf_b, &h->leaf_parent, &h->bnodes, &h->bflags,
-            &h->stats, &h->d_grids, &h->d_cnt_off, &h->leaf_off, &h->roots, &h->scan_bsum,
+            &h->bbits, &h->bprefix, &h->pcode, &h->place, &h->prec, &h->titem, &h->trec, &h->pidx,
+            &h->leaf_cnt, &h->leaf_bin, &h->nfirst, &h->nitem, &h->naxis,
+            &h->stats, &h->d_grids, &h->d_cnt_off, &h->roots, &h->scan_bsum,
             &h->scan_side, &h->deep_part};
 }
 
@@ -4751,7 +4961,9 @@ int reinit_noalloc(ft_ctx* c, double* d_phi, double* d_phi_ifn, const ft_opts* o
     const uint64_t idx_layout = c->idx_layout;
     const float idx_bs = c->idx_bin_scale;
     const int64_t idx_G = c->idx_G;
-    const int idx_bits = c->idx_code_bits;
+    int64_t idx_words[kLevels];
+    std::copy(c->idx_words, c->idx_words + kLevels, idx_words);
+    const int idx_top = c->idx_top;
     c->idx_layout = ~0ull;                           // grids are uploaded into the scratch
     Arena arena;
     arena.base = static_cast<char*>(base);
@@ -4766,7 +4978,8 @@ int reinit_noalloc(ft_ctx* c, double* d_phi, double* d_phi_ifn, const ft_opts* o
     c->idx_layout = idx_layout;
     c->idx_bin_scale = idx_bs;
     c->idx_G = idx_G;
-    c->idx_code_bits = idx_bits;
+    std::copy(idx_words, idx_words + kLevels, c->idx_words);
+    c->idx_top = idx_top;
     c->have_interface = c->have_nearest = c->have_normals = false;
     // Every buffer a reinit sizes must be in call_buffers; one that is not
     // would keep pointing into the shared scratch after the call.  Such a
@@ -5653,7 +5866,6 @@ int ft_reset_phi_points(ft_handle h, const float* ifp, int64_t n_ifp, double* ph
     FT_TRY(fill<uint64_t>(s, sc + S_EDGES, 1, (uint64_t)n_ifp));
     FT_TRY(fill<uint64_t>(s, sc + S_ERR, 1, ~0ull));
     FT_TRY(fill<uint64_t>(s, sc + S_CAP, 1, 0ull));
-    FT_TRY(fill<uint64_t>(s, sc + S_OVF, 1, 0ull));
     SideJoin join{h, s};
     FT_TRY(enqueue_search(h, s, sp, cp, true, false));
     ft_counts cnt{};

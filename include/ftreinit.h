@@ -76,20 +76,19 @@ typedef struct ft_opts {
                             the mode's default (points 2.0, triangles 1.25)     */
     int32_t want_nearest;/* 1: keep the per-node nearest primitive index       */
     int32_t query_block; /* threads per block of the distance query: 64, 128,
-                            256 (waves per workgroup 1, 2, 4); 0 = default     */
+                            256 (waves per workgroup 1, 2, 4); 0 = 64          */
     int32_t want_normals;/* 1: also the level-set normals of phi_ifn, as
                             LevelSet::resetPhi_ ends (LevelSet.cpp:451-453,
                             Assembler::grad_nodes, Assembler.cpp:11-71)        */
     int32_t waves_per_simd; /* launch bound of the triangle-mode query: 5..8
                             waves per SIMD (register budget against
-                            occupancy); 0 = 8                                  */
+                            occupancy); 0 = 6                                  */
     int32_t schedule;    /* FT_SCHED_STATIC: one tile per wave, deep tiles on
                             the first workgroups; FT_SCHED_QUEUE: persistent
                             waves taking tiles from per-XCD counters;
-                            FT_SCHED_BINS (narrow band, triangles only): no
-                            tree walk, each tile tests the triangles of the
-                            index bins within the band, staged in LDS; the
-                            same results as the tree walk                    */
+                            FT_SCHED_BINS (narrow band, triangles only): as
+                            FT_SCHED_STATIC (a search of the band's bins
+                            without the tree was slower than the tree walk) */
     int32_t reserved[2];
 } ft_opts;
 

@@ -290,13 +290,6 @@ __global__ __launch_bounds__(kBS) void k_scan_down(const TI* in, TO* out, int64_
 // Fields: a handle holds one or more independent fields (a plain reinit has
 // one).  Field k owns nodes [node_off[k], node_off[k+1]) and likewise tets and
 // edges; its index bins and query tiles never mix with another field's.
-struct FieldGeom {
-    const int64_t* node_off;         // nf + 1
-    const int64_t* cnt_off;          // unused by the slot padding
-    const Grid* grids;               // unused by the slot padding
-    int nf;
-};
-
 // Node sort of one field (nodes node_base.. of xyz, local index i).
 __global__ __launch_bounds__(kBS) void k_node_bin(const float* xyz, int64_t n, Grid g,
                                                   uint32_t* code, uint32_t* count)
@@ -308,40 +301,61 @@ __global__ __launch_bounds__(kBS) void k_node_bin(const float* xyz, int64_t n, G
     atomicAdd(&count[c], 1u);
 }
 
-// Sorted position p of local node i goes to query slot slot_base + p.
+// Query tiles (64 slots) of each block of cpb consecutive bins.
+__global__ __launch_bounds__(kBS) void k_block_tiles(const uint32_t* offset, int64_t n, int64_t n_bins, int cpb,
+                                                     uint32_t* tiles)
+{
+    const int64_t b = (int64_t)blockIdx.x * kBS + threadIdx.x;
+    if (b * cpb >= n_bins) return;
+    const uint32_t e = (b + 1) * cpb < n_bins ? offset[(b + 1) * cpb] : (uint32_t)n;
+    tiles[b] = (e - offset[b * cpb] + 63u) / 64u;
+}
+
+// Local node i to its query slot: its place in the sorted order, or, with
+// cpb > 0, in its block's tiles (block_tile: the tiles before each block).
+// cap: the field's slots; a node past them is left out and flagged.
 __global__ __launch_bounds__(kBS) void k_node_scatter(const float* xyz, int64_t n, int64_t node_base,
                                                       const uint32_t* code, uint32_t* count,
-                                                      const uint32_t* offset, int32_t* perm,
+                                                      const uint32_t* offset, int cpb, const uint32_t* block_tile,
+                                                      int64_t cap, unsigned long long* misfit, int32_t* perm,
                                                       float* sx, float* sy, float* sz)
 {
     const int64_t i = (int64_t)blockIdx.x * kBS + threadIdx.x;
     if (i >= n) return;
     const uint32_t c = code[i];
-    const int64_t slot = (int64_t)offset[c] + atomicSub(&count[c], 1u) - 1u;
+    int64_t slot = (int64_t)offset[c] + atomicSub(&count[c], 1u) - 1u;
+    if (cpb) {
+        const uint32_t b = c / (uint32_t)cpb;
+        slot += 64 * (int64_t)block_tile[b] - (int64_t)offset[b * (uint32_t)cpb];
+    }
+    if (slot >= cap) {
+        *misfit = 1ull;
+        return;
+    }
     perm[slot] = (int32_t)(node_base + i);
     sx[slot] = xyz[3 * i];
     sy[slot] = xyz[3 * i + 1];
     sz[slot] = xyz[3 * i + 2];
 }
 
-// Pad slots of each field's last wave: perm -1, coordinates of the field's
-// first slot (lanes that only shadow a real node); tile -> field table.
-__global__ __launch_bounds__(kBS) void k_pad_slots(int64_t n_slots, FieldGeom fg,
-                                                   const int64_t* slot_off, int32_t* perm,
-                                                   float* sx, float* sy, float* sz,
-                                                   int32_t* tile_field)
+// Padding slots (perm -1): coordinates of their tile's first slot, a node
+// (lanes that only shadow it); tile -> field table.
+__global__ __launch_bounds__(kBS) void k_pad_slots(int64_t n_slots, int nf, const int64_t* slot_off, const int32_t* perm,
+                                                   float* sx, float* sy, float* sz, int32_t* tile_field,
+                                                   unsigned long long* misfit)
 {
     const int64_t s = (int64_t)blockIdx.x * kBS + threadIdx.x;
     if (s >= n_slots) return;
-    const int k = ftd::field_of(slot_off, fg.nf, s);
-    if ((s & 63) == 0) tile_field[s >> 6] = k;
-    const int64_t nk = fg.node_off[k + 1] - fg.node_off[k];
-    if (s - slot_off[k] < nk) return;
-    const int64_t f0 = slot_off[k];
-    perm[s] = -1;
-    sx[s] = sx[f0];
-    sy[s] = sy[f0];
-    sz[s] = sz[f0];
+    const int64_t t0 = s & ~(int64_t)63;
+    if (s == t0) tile_field[s >> 6] = ftd::field_of(slot_off, nf, s);
+    if (perm[s] >= 0) return;
+    if (perm[t0] < 0) {                                // a tile without nodes: fewer blocks than expected
+        *misfit = 1ull;
+        return;
+    }
+    sx[s] = sx[t0];
+    sy[s] = sy[t0];
+    sz[s] = sz[t0];
 }
 
 // ============================================================================
@@ -3817,12 +3831,10 @@ int set_fields(ft_ctx* c, int nf, const int64_t* node_off, const int64_t* tet_of
     c->tet_off.assign(tet_off, tet_off + nf + 1);
     c->edge_off.assign(edge_off, edge_off + nf + 1);
     c->slot_off.assign(nf + 1, 0);
-    for (int k = 0; k < nf; k++)
-        c->slot_off[k + 1] = c->slot_off[k] + ((node_off[k + 1] - node_off[k] + 63) / 64) * 64;
     c->N = node_off[nf];
     c->T = tet_off[nf];
     c->E = edge_off[nf];
-    c->n_slots = c->slot_off[nf];
+    c->n_slots = 0;                  // set with the node sort (set_slots)
     c->fh.assign(nf, FieldHost{});
     c->field_counts.assign(nf, ft_counts{});
     const size_t ob = sizeof(int64_t) * (nf + 1);
@@ -3833,7 +3845,24 @@ int set_fields(ft_ctx* c, int nf, const int64_t* node_off, const int64_t* tet_of
     FT_HIP(hipMemcpyAsync(c->d_node_off.p, c->node_off.data(), ob, hipMemcpyHostToDevice, c->stream));
     FT_HIP(hipMemcpyAsync(c->d_tet_off.p, c->tet_off.data(), ob, hipMemcpyHostToDevice, c->stream));
     FT_HIP(hipMemcpyAsync(c->d_edge_off.p, c->edge_off.data(), ob, hipMemcpyHostToDevice, c->stream));
-    FT_HIP(hipMemcpyAsync(c->d_slot_off.p, c->slot_off.data(), ob, hipMemcpyHostToDevice, c->stream));
+    FT_HIP(hipStreamSynchronize(c->stream));
+    return FT_OK;
+}
+
+// Query slots of each field (multiples of 64).
+int set_slots(ft_ctx* c, const std::vector<int64_t>& slots)
+{
+    for (int k = 0; k < c->nf; k++) c->slot_off[k + 1] = c->slot_off[k] + slots[k];
+    c->n_slots = c->slot_off[c->nf];
+    const size_t n = (size_t)std::max<int64_t>(1, c->n_slots);
+    FT_TRY(ensure(c->perm, sizeof(int32_t) * n));
+    FT_TRY(ensure(c->sx, sizeof(float) * n));
+    FT_TRY(ensure(c->sy, sizeof(float) * n));
+    FT_TRY(ensure(c->sz, sizeof(float) * n));
+    FT_TRY(ensure(c->tile_field, sizeof(int32_t) * std::max<size_t>(1, n / 64)));
+    FT_TRY(ensure(c->tile_sched, 4 * sizeof(int32_t) * std::max<size_t>(1, n / 64)));
+    FT_HIP(hipMemcpyAsync(c->d_slot_off.p, c->slot_off.data(), sizeof(int64_t) * (c->nf + 1), hipMemcpyHostToDevice,
+                          c->stream));
     FT_HIP(hipStreamSynchronize(c->stream));
     return FT_OK;
 }
@@ -3870,14 +3899,20 @@ void boxes_from_host(ft_ctx* c, const float* xyz)
 // ny - 1, nz - 1 spacings s along the box's edges, as a box mesher's (or
 // the Kuhn generator's) grid, jittered by less than s / 2 -- the bins are
 // kf s wide and start s / 2 before the box: every bin then holds the
-// kf^3 nodes of one block, and 64 consecutive slots in Morton order are an
-// aligned 4 x 4 x 4 block of nodes (kf = 1 or 2).  Bins of the estimated
-// spacing from the box corner cut those blocks where jittered nodes cross a
-// bin edge; at 256^3 aligned blocks made the query 4.6% faster.  Any other
-// field keeps the grid of about one node per bin.  The order only affects
-// speed: each node's result is the same in any slot.
-Grid node_sort_grid(const FieldHost& f, int64_t n, int max_lg, int* lg_out)
+// kf^3 nodes of one block (kf = 1 or 2), and *cpb consecutive bins along the
+// Morton curve an aligned 4 x 4 x 4 block of nodes, which gets a tile of its
+// own: *tiles in all.  Packed without gaps, a grid whose sides are no
+// multiples of 4 has its blocks cut by the tiles, and a tile that holds the
+// end of one octant and the start of the next spans half the field (127^3:
+// the last 2% of the tiles took as long as the rest).  Grids whose
+// blocks would be emptier than kBlockFill keep the packed order (*cpb = 0),
+// as does any other field, on a grid of about one node per bin.  The order
+// only affects speed: each node's result is the same in any slot.
+constexpr double kBlockFill = 0.6;
+Grid node_sort_grid(const FieldHost& f, int64_t n, int max_lg, int* lg_out, int* cpb, int64_t* tiles)
 {
+    *cpb = 0;
+    *tiles = (n + 63) / 64;
     const Grid fallback = make_grid(f, f.h, max_lg, lg_out);
     double ext[3], ext_max = 0.0;
     for (int k = 0; k < 3; k++) {
@@ -3927,50 +3962,78 @@ Grid node_sort_grid(const FieldHost& f, int64_t n, int max_lg, int* lg_out)
     g.inv_b = (float)(1.0 / ((double)kf * s));
     g.h = f.h;
     *lg_out = lg;
+    int64_t blocks = 1;
+    for (int k = 0; k < 3; k++) blocks *= (nk[k] + 3) / 4;
+    const int block_bins = kf == 1 ? 64 : 8;
+    if ((double)n >= kBlockFill * 64.0 * (double)blocks && ((int64_t)1 << (3 * lg)) >= block_bins) {
+        *cpb = block_bins;
+        *tiles = blocks;
+    }
     return g;
 }
 
 // Morton order of each field's nodes into the query slots (device xyz):
-// one counting sort per field on node_sort_grid.
-int sort_nodes(ft_ctx* c)
+// one counting sort per field on node_sort_grid.  blocks: a tile per block of
+// a structured grid; a field that only looked like one (a block of more than
+// 64 nodes, or an empty one) sends the whole handle back to the packed order.
+int sort_nodes(ft_ctx* c, bool blocks = true)
 {
     const int nf = c->nf;
-    FT_TRY(ensure(c->perm, sizeof(int32_t) * std::max<int64_t>(1, c->n_slots)));
-    FT_TRY(ensure(c->sx, sizeof(float) * std::max<int64_t>(1, c->n_slots)));
-    FT_TRY(ensure(c->sy, sizeof(float) * std::max<int64_t>(1, c->n_slots)));
-    FT_TRY(ensure(c->sz, sizeof(float) * std::max<int64_t>(1, c->n_slots)));
-    FT_TRY(ensure(c->tile_field, sizeof(int32_t) * std::max<int64_t>(1, c->n_slots / 64)));
-    FT_TRY(ensure(c->tile_sched, 4 * sizeof(int32_t) * std::max<int64_t>(1, c->n_slots / 64)));
+    std::vector<Grid> grids(nf);
+    std::vector<int> lgs(nf, 0), cpb(nf, 0);
+    std::vector<int64_t> slots(nf, 0);
+    for (int k = 0; k < nf; k++) {
+        const int64_t n = c->node_off[k + 1] - c->node_off[k];
+        int64_t tiles = 0;
+        if (n > 0) grids[k] = node_sort_grid(c->fh[k], n, kMaxBinsLog2PerAxis, &lgs[k], &cpb[k], &tiles);
+        if (!blocks && cpb[k]) {
+            cpb[k] = 0;
+            tiles = (n + 63) / 64;
+        }
+        slots[k] = 64 * tiles;
+    }
+    FT_TRY(set_slots(c, slots));
     if (c->N == 0) return FT_OK;
     hipStream_t s = c->stream;
+    unsigned long long* misfit = c->scalars.as<unsigned long long>() + S_P2T;
+    FT_TRY(fill<unsigned long long>(s, misfit, 1, 0ull));
+    FT_TRY(fill<int32_t>(s, c->perm.as<int32_t>(), c->n_slots, -1));
     for (int k = 0; k < nf; k++) {
         const int64_t n = c->node_off[k + 1] - c->node_off[k];
         if (n == 0) continue;
-        int lg = 0;
-        const Grid g = node_sort_grid(c->fh[k], n, kMaxBinsLog2PerAxis, &lg);
-        const int64_t G = (int64_t)1 << (3 * lg);
+        const Grid& g = grids[k];
+        const int64_t G = (int64_t)1 << (3 * lgs[k]);
         FT_TRY(ensure(c->bin_count, sizeof(uint32_t) * G));
         FT_TRY(ensure(c->bin_prefix, sizeof(uint64_t) * G));
         FT_TRY(ensure(c->pcode, sizeof(uint32_t) * n));
         uint32_t* cnt = c->bin_count.as<uint32_t>();
-        uint32_t* off = reinterpret_cast<uint32_t*>(c->bin_prefix.p);
+        uint32_t* off = c->bin_prefix.as<uint32_t>();
+        uint32_t* btile = off + G;                     // per block (at most G of them)
+        uint32_t* total = reinterpret_cast<uint32_t*>(c->scalars.as<uint64_t>() + S_BINS);
         const float* xk = c->xyz.as<float>() + 3 * c->node_off[k];
         const int64_t sb = c->slot_off[k];
         FT_TRY(fill<uint32_t>(s, cnt, G, 0u));
         hipLaunchKernelGGL(k_node_bin, dim3(grid1d(n)), dim3(kBS), 0, s, xk, n, g, c->pcode.as<uint32_t>(), cnt);
-        FT_TRY(scan<uint32_t, uint32_t>(c, s, cnt, off, G,
-                                        reinterpret_cast<uint32_t*>(c->scalars.as<uint64_t>() + S_BINS),
-                                        LoadSame{}));
+        FT_TRY(scan<uint32_t, uint32_t>(c, s, cnt, off, G, total, LoadSame{}));
+        if (cpb[k]) {
+            const int64_t nb = G / cpb[k];
+            hipLaunchKernelGGL(k_block_tiles, dim3(grid1d(nb)), dim3(kBS), 0, s, off, n, G, cpb[k], btile);
+            FT_TRY(scan<uint32_t, uint32_t>(c, s, btile, btile, nb, total, LoadSame{}));
+        }
         hipLaunchKernelGGL(k_node_scatter, dim3(grid1d(n)), dim3(kBS), 0, s, xk, n, c->node_off[k],
-                           c->pcode.as<uint32_t>(), cnt, off, c->perm.as<int32_t>() + sb,
-                           c->sx.as<float>() + sb, c->sy.as<float>() + sb, c->sz.as<float>() + sb);
+                           c->pcode.as<uint32_t>(), cnt, off, cpb[k], btile, slots[k], misfit,
+                           c->perm.as<int32_t>() + sb, c->sx.as<float>() + sb, c->sy.as<float>() + sb,
+                           c->sz.as<float>() + sb);
     }
-    FieldGeom fg{c->d_node_off.as<int64_t>(), nullptr, nullptr, nf};
-    hipLaunchKernelGGL(k_pad_slots, dim3(grid1d(c->n_slots)), dim3(kBS), 0, s, c->n_slots, fg,
+    hipLaunchKernelGGL(k_pad_slots, dim3(grid1d(c->n_slots)), dim3(kBS), 0, s, c->n_slots, nf,
                        c->d_slot_off.as<int64_t>(), c->perm.as<int32_t>(), c->sx.as<float>(),
-                       c->sy.as<float>(), c->sz.as<float>(), c->tile_field.as<int32_t>());
+                       c->sy.as<float>(), c->sz.as<float>(), c->tile_field.as<int32_t>(), misfit);
     FT_TRY(check_launch());
-    FT_HIP(hipStreamSynchronize(s));
+    FT_TRY(read_scalars(c, s, S_N));
+    if (c->h_scalars[S_P2T]) {
+        if (!blocks) return ft::set_error(FT_ERR_INTERNAL, "node sort: more nodes than slots");
+        return sort_nodes(c, false);
+    }
     return FT_OK;
 }
 
@@ -5404,12 +5467,9 @@ int ft_set_batch_meshes(ft_handle h, int32_t n_fields, const int32_t* mesh_ids)
     FT_TRY(set_fields(h, n_fields, no.data(), to.data(), eo.data()));
     hipStream_t s = h->stream;
     FT_TRY(ensure(h->xyz, 12 * no[n_fields]));
-    FT_TRY(ensure(h->perm, 4 * std::max<int64_t>(1, h->n_slots)));
-    FT_TRY(ensure(h->sx, 4 * std::max<int64_t>(1, h->n_slots)));
-    FT_TRY(ensure(h->sy, 4 * std::max<int64_t>(1, h->n_slots)));
-    FT_TRY(ensure(h->sz, 4 * std::max<int64_t>(1, h->n_slots)));
-    FT_TRY(ensure(h->tile_field, 4 * std::max<int64_t>(1, h->n_slots / 64)));
-    FT_TRY(ensure(h->tile_sched, 16 * std::max<int64_t>(1, h->n_slots / 64)));
+    std::vector<int64_t> slots(n_fields);
+    for (int k = 0; k < n_fields; k++) slots[k] = ms[k]->n_slots;
+    FT_TRY(set_slots(h, slots));
     // per-field connectivity pointers: tets, t2e, edges of each mesh
     std::vector<const void*> tab(3 * (size_t)n_fields);
     for (int k = 0; k < n_fields; k++) {

@@ -28,7 +28,7 @@ def _check_triangles(m, h, ifn, near, nodes, itf):
 
 
 @pytest.mark.parametrize("n,bin_scale", [(9, 1e6), (9, 4.0), (9, 2.0), (9, 1.6), (17, 1.0), (18, 1.0), (33, 0.5),
-                                         (72, 1.0), (21, 20.0), ((5, 40, 3), 1.0)])
+                                         (72, 1.0), (21, 20.0), ((5, 40, 3), 1.0), ((300, 12, 10), 2.0)])
 @pytest.mark.parametrize("field", ["sphere_wave", "ellipsoids"])
 def test_tree_shapes_match_the_oracle(n, bin_scale, field):
     dims = (n, n, n) if np.isscalar(n) else n
@@ -36,8 +36,8 @@ def test_tree_shapes_match_the_oracle(n, bin_scale, field):
     m = fa.kuhn_mesh(dims, spacing=h, jitter=0.2, seed=2)
     phi = fa.phi_field(field, m.xyz, seed=4)
     ifp, ifp2e = oracle.find_interface_nodes(m.edges, m.xyz, phi)
-    if len(ifp) == 0:                              # the field misses this thin slab: cut it by a plane
-        phi = m.xyz[:, 1].astype(np.float64) - 0.37
+    if len(ifp) == 0:                              # the field misses this thin slab: cut its long side by a plane
+        phi = m.xyz[:, int(np.argmax(dims))].astype(np.float64) - 0.37
         ifp, ifp2e = oracle.find_interface_nodes(m.edges, m.xyz, phi)
     tris, _, _ = oracle.reconstruct_interface(m.tets, m.t2e, m.edges, m.xyz, phi, ifp, ifp2e)
     nodes = np.random.default_rng(1).permutation(m.n_nodes)[:4000]
@@ -90,6 +90,25 @@ def test_non_finite_points_do_not_hide_the_others():
     ref = ref[0] if isinstance(ref, tuple) else ref
     with fa.EuclideanDistance(0) as d:
         d.init(m.xyz)
+        got = phi.copy()
+        d.reset_phi(ifp, len(ifp), got)
+    assert np.array_equal(got.view(np.uint64), ref.view(np.uint64))
+
+
+@pytest.mark.parametrize("n", [16, 24])
+def test_scattered_nodes_that_count_and_bound_like_a_grid(n):
+    """n^3 nodes over the unit cube, its corners among them, but not a grid:
+    blocks of 4 x 4 x 4 spacings hold any number of nodes."""
+    rng = np.random.default_rng(n)
+    xyz = rng.random((n ** 3, 3)).astype(np.float32)
+    xyz[:8] = [[i, j, k] for i in (0, 1) for j in (0, 1) for k in (0, 1)]
+    xyz[8:200] = xyz[8]                                   # more than a tile in one place
+    ifp = rng.random((400, 3)).astype(np.float32)
+    phi = rng.standard_normal(n ** 3)
+    ref = oracle.reset_phi_points(xyz, ifp, phi.copy())
+    ref = ref[0] if isinstance(ref, tuple) else ref
+    with fa.EuclideanDistance(0) as d:
+        d.init(xyz)
         got = phi.copy()
         d.reset_phi(ifp, len(ifp), got)
     assert np.array_equal(got.view(np.uint64), ref.view(np.uint64))

@@ -2356,7 +2356,7 @@ __global__ __launch_bounds__(kBS) void k_n2t_sort(const uint64_t* off, int64_t N
 // g = ((u0 c0 + u1 c1) + u2 c2) + u3 c3, cast to float.  A singular tet (det
 // 0, which the reference only reports) gets a zero gradient.
 __global__ __launch_bounds__(kBS) void k_tet_grad(const int4* tets, int64_t T, const float* xyz,
-                                                  const double* u, float* grad_t, const uint64_t* sc)
+                                                  const double* u, float4* grad_t, const uint64_t* sc)
 {
     const int64_t t = (int64_t)blockIdx.x * kBS + threadIdx.x;
     if (t >= T || halted(sc)) return;
@@ -2385,72 +2385,87 @@ __global__ __launch_bounds__(kBS) void k_tet_grad(const int4* tets, int64_t T, c
             g[r] = (float)(((u0 * c0 + u1 * b0) + u2 * b1) + u3 * b2);
         }
     }
-    grad_t[3 * t] = g[0];
-    grad_t[3 * t + 1] = g[1];
-    grad_t[3 * t + 2] = g[2];
+    grad_t[t] = make_float4(g[0], g[1], g[2], 0.0f);
+}
+
+// The block of nodes of this workgroup: each of the chip's eight dies, which
+// get workgroups in turn, has one range of the node numbers to itself, so that
+// the gradients that neighbouring nodes share are fetched once into its L2.
+__device__ __forceinline__ int64_t die_block()
+{
+    const uint32_t per = (gridDim.x + 7) / 8;
+    const uint32_t full = gridDim.x % 8 == 0 ? 8 : gridDim.x % 8, die = blockIdx.x % 8;
+    return (int64_t)die * per - (die > full ? die - full : 0) + blockIdx.x / 8;
+}
+
+// Sum of a node's tet gradients in list order.  The loads bound it (nodes of a
+// wave share tets only by chance of the numbering), so they are few and in
+// flight together: a gradient is one 16-byte load (padded to four floats), the
+// list entries come four to a load, and kNodeGather tets are taken at a time.
+// Three 4-byte loads a gradient and one an entry took 0.53 ms at
+// 160 x 144 x 131; this 0.385 ms, and 0.305 ms with die_block() above, where
+// reading the lists and the gradients once at a large copy's rate takes 0.14.
+// The list array holds kNodeGather more entries than there are.
+constexpr int kNodeGather = 8;
+__device__ __forceinline__ void sum_gradients(const int32_t* ids, uint64_t b, uint64_t e, const float4* grad_t, float n[3])
+{
+    n[0] = n[1] = n[2] = 0.0f;
+    for (uint64_t j0 = b; j0 < e; j0 += kNodeGather) {
+        int32_t t[kNodeGather];
+        memcpy(t, ids + j0, sizeof t);
+        float4 g[kNodeGather];
+#pragma unroll
+        for (int u = 0; u < kNodeGather; u++) {
+            g[u] = grad_t[j0 + u < e ? t[u] : t[0]];
+        }
+#pragma unroll
+        for (int u = 0; u < kNodeGather; u++)
+            if (j0 + u < e) {
+                n[0] += g[u].x;
+                n[1] += g[u].y;
+                n[2] += g[u].z;
+            }
+    }
 }
 
 // Assembler::grad_nodes: per node, the float mean of its tets' gradients,
 // summed in increasing tet id.
-constexpr int kNodeGather = 8;
-
 __global__ __launch_bounds__(kBS) void k_node_normals(const uint64_t* off, const int32_t* ids,
-                                                      const float* grad_t, int64_t N, float* out,
+                                                      const float4* grad_t, int64_t N, float* out,
                                                       const uint64_t* sc)
 {
-    const int64_t i = (int64_t)blockIdx.x * kBS + threadIdx.x;
+    const int64_t i = die_block() * kBS + threadIdx.x;
     if (i >= N || halted(sc)) return;
     const uint64_t b = off[i], e = off[i + 1];
-    float n0 = 0.0f, n1 = 0.0f, n2 = 0.0f;
-    // in list order; the list entries, then their gradients, kNodeGather at a
-    // time (loads in flight together instead of one dependent pair per tet)
-    for (uint64_t j0 = b; j0 < e; j0 += kNodeGather) {
-        int64_t t[kNodeGather];
-#pragma unroll
-        for (int u = 0; u < kNodeGather; u++) t[u] = j0 + u < e ? (int64_t)ids[j0 + u] : -1;
-        float g[kNodeGather][3];
-#pragma unroll
-        for (int u = 0; u < kNodeGather; u++)
-            for (int c = 0; c < 3; c++) g[u][c] = t[u] >= 0 ? grad_t[3 * t[u] + c] : 0.0f;
-#pragma unroll
-        for (int u = 0; u < kNodeGather; u++)
-            if (j0 + u < e) {
-                n0 += g[u][0];
-                n1 += g[u][1];
-                n2 += g[u][2];
-            }
-    }
+    float n[3];
+    sum_gradients(ids, b, e, grad_t, n);
     const float cnt = (float)(e - b);
-    out[3 * i] = n0 / cnt;
-    out[3 * i + 1] = n1 / cnt;
-    out[3 * i + 2] = n2 / cnt;
+    out[3 * i] = n[0] / cnt;
+    out[3 * i + 1] = n[1] / cnt;
+    out[3 * i + 2] = n[2] / cnt;
 }
 
 // ---- interface curvature (LevelSet::getInterfaceCurvature, LevelSet.cpp:215-253)
-// g / |g| per node in float (|g| = sqrt(x^2 + (y^2 + z^2))), kept as three
-// double fields (g_x, g_y, g_z, :224-230).
-__global__ __launch_bounds__(kBS) void k_unit_split(const float* g, int64_t N, double* gx, double* gy,
-                                                    double* gz)
+// g / |g| per node in float (|g| = sqrt(x^2 + (y^2 + z^2)), g_x, g_y, g_z of
+// :224-230).  The fields are doubles that hold float values: they are kept as
+// floats, four to a node, and widened where they are used.
+__global__ __launch_bounds__(kBS) void k_unit_split(const float* g, int64_t N, float4* unit)
 {
     const int64_t i = (int64_t)blockIdx.x * kBS + threadIdx.x;
     if (i >= N) return;
     const float x = g[3 * i], y = g[3 * i + 1], z = g[3 * i + 2];
     const float nrm = sqrtf(x * x + (y * y + z * z));
-    gx[i] = (double)(x / nrm);
-    gy[i] = (double)(y / nrm);
-    gz[i] = (double)(z / nrm);
+    unit[i] = make_float4(x / nrm, y / nrm, z / nrm, 0.0f);
 }
 
-// One component of grad_nodes (the float mean over the node's tets of that
-// component) added into k: k = mean on the first call, k += mean after, so
-// k = gg_x.x + gg_y.y + gg_z.z in that order (:237-238).
 // The curvature's gradients (LevelSet.cpp:233-235, the entries :238 uses):
 // for c = x, y, z the c-th entry of
 // the P1 gradient of g_c, in k_tet_grad's frame and operation order, with one
-// frame per tet for the three fields instead of one pass per field.
+// frame per tet for the three fields instead of one pass per field.  Gathers
+// bound it: one 16-byte load per corner for the three fields (three 8-byte
+// loads of separate fields took 0.24 ms at 160 x 144 x 131, now 0.15).
 __global__ __launch_bounds__(kBS) void k_tet_grad_diag(const int4* tets, int64_t T, const float* xyz,
-                                                       const double* gx, const double* gy, const double* gz,
-                                                       float* out, const uint64_t* sc)
+                                                       const float4* unit, float4* out, const uint64_t* sc)
 {
     const int64_t t = (int64_t)blockIdx.x * kBS + threadIdx.x;
     if (t >= T || halted(sc)) return;
@@ -2472,46 +2487,35 @@ __global__ __launch_bounds__(kBS) void k_tet_grad_diag(const int4* tets, int64_t
     float g[3] = {0.0f, 0.0f, 0.0f};
     if (det != 0.0) {
         const double inv = 1.0 / det;
-        const double* uf[3] = {gx, gy, gz};
+        float uf[4][3];
+        for (int j = 0; j < 4; j++) {
+            const float4 f = unit[qi[j]];
+            uf[j][0] = f.x;
+            uf[j][1] = f.y;
+            uf[j][2] = f.z;
+        }
         for (int r = 0; r < 3; r++) {
-            const double u0 = uf[r][qi[0]], u1 = uf[r][qi[1]], u2 = uf[r][qi[2]], u3 = uf[r][qi[3]];
+            const double u0 = uf[0][r], u1 = uf[1][r], u2 = uf[2][r], u3 = uf[3][r];
             const double b0 = C[r][0] * inv, b1 = C[r][1] * inv, b2 = C[r][2] * inv;
             const double c0 = (b0 * -1.0 + b1 * -1.0) + b2 * -1.0;
             g[r] = (float)(((u0 * c0 + u1 * b0) + u2 * b1) + u3 * b2);
         }
     }
-    out[3 * t] = g[0];
-    out[3 * t + 1] = g[1];
-    out[3 * t + 2] = g[2];
+    out[t] = make_float4(g[0], g[1], g[2], 0.0f);
 }
 
 // Node curvature (LevelSet.cpp:237-239): per component the float mean over the node's
 // tets in increasing id (grad_nodes), then the sum x + y + z in that order.
-__global__ __launch_bounds__(kBS) void k_node_div(const uint64_t* off, const int32_t* ids, const float* gd,
+__global__ __launch_bounds__(kBS) void k_node_div(const uint64_t* off, const int32_t* ids, const float4* gd,
                                                   int64_t N, float* k)
 {
-    const int64_t i = (int64_t)blockIdx.x * kBS + threadIdx.x;
+    const int64_t i = die_block() * kBS + threadIdx.x;
     if (i >= N) return;
     const uint64_t b = off[i], e = off[i + 1];
-    float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f;
-    for (uint64_t j0 = b; j0 < e; j0 += kNodeGather) {      // in list order, as k_node_normals
-        int64_t t[kNodeGather];
-#pragma unroll
-        for (int u = 0; u < kNodeGather; u++) t[u] = j0 + u < e ? (int64_t)ids[j0 + u] : -1;
-        float g[kNodeGather][3];
-#pragma unroll
-        for (int u = 0; u < kNodeGather; u++)
-            for (int c = 0; c < 3; c++) g[u][c] = t[u] >= 0 ? gd[3 * t[u] + c] : 0.0f;
-#pragma unroll
-        for (int u = 0; u < kNodeGather; u++)
-            if (j0 + u < e) {
-                s0 += g[u][0];
-                s1 += g[u][1];
-                s2 += g[u][2];
-            }
-    }
+    float s[3];
+    sum_gradients(ids, b, e, gd, s);
     const float cnt = (float)(e - b);
-    const float m0 = s0 / cnt, m1 = s1 / cnt, m2 = s2 / cnt;
+    const float m0 = s[0] / cnt, m1 = s[1] / cnt, m2 = s[2] / cnt;
     k[i] = (m0 + m1) + m2;
 }
 
@@ -4137,7 +4141,7 @@ int ensure_stage(ft_ctx* c, int stage, const Caps& cp, int mode, bool want_neare
         if (want_nearest) FT_TRY(ensure(c->nearest, sizeof(int32_t) * at_least1(N)));
         if (want_normals) {
             FT_TRY(ensure(c->normals, 12 * at_least1(N)));
-            FT_TRY(ensure(c->grad_t, 12 * at_least1(T)));
+            FT_TRY(ensure(c->grad_t, 16 * at_least1(T)));
             FT_TRY(ensure(c->phi_ifn_int, 8 * at_least1(N)));
         }
     } else if (stage == 1) {
@@ -4220,7 +4224,7 @@ int build_node_tets(ft_ctx* c, hipStream_t s)
     if (c->n2t_layout == c->layout_gen) return FT_OK;
     const int64_t N = c->N, T = c->T;
     FT_TRY(ensure(c->n2t_off, sizeof(uint64_t) * (N + 1)));
-    FT_TRY(ensure(c->n2t_ids, sizeof(int32_t) * at_least1(4 * T)));
+    FT_TRY(ensure(c->n2t_ids, sizeof(int32_t) * (4 * T + kNodeGather)));
     FT_TRY(ensure(c->pcode, sizeof(uint32_t) * at_least1(N)));          // counters
     uint32_t* cnt = c->pcode.as<uint32_t>();
     uint64_t* off = c->n2t_off.as<uint64_t>();
@@ -4661,9 +4665,9 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
             return ft::set_error(FT_ERR_STATE, "node -> tets lists not built for this field layout");
         if (c->T > 0)
             hipLaunchKernelGGL(k_tet_grad, dim3(grid1d(c->T)), dim3(kBS), 0, s, c->tets.as<int4>(), c->T,
-                               c->xyz.as<float>(), q.phi_ifn, c->grad_t.as<float>(), sc);
+                               c->xyz.as<float>(), q.phi_ifn, c->grad_t.as<float4>(), sc);
         hipLaunchKernelGGL(k_node_normals, dim3(grid1d(c->N)), dim3(kBS), 0, s, c->n2t_off.as<uint64_t>(),
-                           c->n2t_ids.as<int32_t>(), c->grad_t.as<float>(), c->N, c->normals.as<float>(), sc);
+                           c->n2t_ids.as<int32_t>(), c->grad_t.as<float4>(), c->N, c->normals.as<float>(), sc);
         FT_TRY(check_launch());
     }
     if (timed) (void)hipEventRecord(c->ev[4], s);
@@ -5559,19 +5563,18 @@ int enqueue_curvature(ft_ctx* h, hipStream_t s)
     if (!h->have_normals || !h->have_interface || !h->last_phi)
         return ft::set_error(FT_ERR_STATE, "curvature needs a reinit with want_normals first");
     const int64_t N = h->N, T = h->T, P = h->last.n_ifp;
-    FT_TRY(ensure(h->gsplit, 24 * at_least1(N)));
+    FT_TRY(ensure(h->gsplit, 16 * at_least1(N)));
     FT_TRY(ensure(h->kmesh, 4 * at_least1(N)));
     FT_TRY(ensure(h->k_if, 4 * at_least1(P)));
     if (N > 0) {
-        double* g = h->gsplit.as<double>();
+        float4* unit = h->gsplit.as<float4>();
         const uint64_t* sc = h->scalars.as<uint64_t>();
-        hipLaunchKernelGGL(k_unit_split, dim3(grid1d(N)), dim3(kBS), 0, s, h->normals.as<float>(), N, g,
-                           g + N, g + 2 * N);
+        hipLaunchKernelGGL(k_unit_split, dim3(grid1d(N)), dim3(kBS), 0, s, h->normals.as<float>(), N, unit);
         if (T > 0)
             hipLaunchKernelGGL(k_tet_grad_diag, dim3(grid1d(T)), dim3(kBS), 0, s, h->tets.as<int4>(), T,
-                               h->xyz.as<float>(), g, g + N, g + 2 * N, h->grad_t.as<float>(), sc);
+                               h->xyz.as<float>(), unit, h->grad_t.as<float4>(), sc);
         hipLaunchKernelGGL(k_node_div, dim3(grid1d(N)), dim3(kBS), 0, s, h->n2t_off.as<uint64_t>(),
-                           h->n2t_ids.as<int32_t>(), h->grad_t.as<float>(), N, h->kmesh.as<float>());
+                           h->n2t_ids.as<int32_t>(), h->grad_t.as<float4>(), N, h->kmesh.as<float>());
         if (P > 0)
             hipLaunchKernelGGL(k_curv_points, dim3(grid1d(P)), dim3(kBS), 0, s, h->ifp2e.as<int32_t>(), P,
                                h->edges.as<int2>(), h->last_phi, h->kmesh.as<float>(), h->k_if.as<float>());

@@ -2611,9 +2611,14 @@ __global__ __launch_bounds__(kBS) void k_st_apply(const uint64_t* off, const int
 constexpr int kFemSlice = 64;          // rows per ELL slice (one wave)
 constexpr int kFemMaxCols = 48;        // columns per row (the node and its tet neighbours)
 
+// The four basis functions at the four quadrature points: phi_j is hi at its
+// own point, lo0 (j = 0) or lo (j = 1, 2, 3) at the other three.  The points in
+// the reference's order are those of j = 1, 2, 3, 0.
 struct FemQuad {
-    double phi[16];                    // phi_j at quadrature point q: [4 j + q]
+    double hi, lo0, lo;
     double w;                          // weight (0.25 / 6)
+    __host__ __device__ static constexpr int point(int j) { return (j + 3) & 3; }
+    __host__ __device__ double phi(int j, int q) const { return q == point(j) ? hi : j == 0 ? lo0 : lo; }
 };
 
 struct FemEll {
@@ -2849,47 +2854,76 @@ __global__ __launch_bounds__(kFemSlice) void k_fem_diags(int64_t N, FemEll e, in
 // for the advection form, its velocity), so that a tet's nodes are read
 // there through its column map (fmap: the row slot of each of its four
 // nodes) instead of through the tet list.  Then in each round lane L
-// computes the four contributions of tet kFemLanes r + L into LDS, and the
-// row's first lane adds that round's tets into the row accumulator in tet
-// order, so every entry is summed exactly as the reference's std::map does.
+// computes the four contributions of tet kFemLanes r + L, and then
+// the row's lanes add that round's tets into the row accumulator in tet order,
+// lane L the node L of each, so every entry is summed exactly as the
+// reference's std::map does.
 // A workgroup is one wave of kFemRowsPerWave rows.
 constexpr int kFemLanes = 4;
 constexpr int kFemRowsPerWave = 64 / kFemLanes;
-constexpr int kFemQb = 4 * kFemLanes + 1;            // round buffer per row, padded against bank conflicts
-constexpr int kFemQm = kFemLanes + 1;                // round column maps per row, padded likewise
+constexpr int kFemCols = 4;                          // columns per lane whose loads are in flight together
+static_assert(kFemLanes == 4, "a row's lanes are a quad (quad_lane, quad_transpose)");
+
+// x of the quad's lane t, in all four.
+template <int T>
+__device__ __forceinline__ uint32_t quad_lane(uint32_t x)
+{
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x55 * T, 0xf, 0xf, true);
+}
+
+template <int CTRL>
+__device__ __forceinline__ double quad_swap(double x)
+{
+    const int2 v = __builtin_bit_cast(int2, x);
+    return __builtin_bit_cast(double, make_int2(__builtin_amdgcn_mov_dpp(v.x, CTRL, 0xf, 0xf, true),
+                                                __builtin_amdgcn_mov_dpp(v.y, CTRL, 0xf, 0xf, true)));
+}
+
+// Of a pair that the lanes with and without `up` hold: the one keeps a and
+// gets the other's, the other keeps b.
+template <int CTRL>
+__device__ __forceinline__ void quad_exchange(double& a, double& b, bool up)
+{
+    const double got = quad_swap<CTRL>(up ? a : b);
+    a = up ? got : a;
+    b = up ? b : got;
+}
+
+// s[j] of lane t becomes s[t] of lane j (t, j: lanes of a quad).
+__device__ __forceinline__ void quad_transpose(double (&s)[4], int lane)
+{
+    quad_exchange<0xB1>(s[0], s[1], lane & 1);        // quad_perm [1, 0, 3, 2]
+    quad_exchange<0xB1>(s[2], s[3], lane & 1);
+    quad_exchange<0x4E>(s[0], s[2], lane & 2);        // quad_perm [2, 3, 0, 1]
+    quad_exchange<0x4E>(s[1], s[3], lane & 2);
+}
 
 // LDS per wave, in this order: kFemRowsPerWave accumulators of `stride`
-// doubles; the round buffers (kFemQb doubles per row); for the advection
-// form the column velocities (3 doubles per column slot); the column
-// coordinates (3 floats per slot); the round maps (kFemQm words per row);
-// the row's own slot (one word per row).  The velocity region is free after
-// the rounds: k_fem_cn reuses it.
+// doubles; for the advection form the column velocities (3 doubles per column
+// slot); the column coordinates (3 floats per slot); the row's own slot (one
+// word per row).  The velocity region is free after the rounds: k_fem_cn
+// reuses it.
 __host__ __device__ inline size_t fem_lds_bytes(int stride, int form)
 {
     const size_t R = kFemRowsPerWave, S = (size_t)stride;
-    return 8 * R * (S + kFemQb) + (form == 1 ? 24 * R * S : 0) + 12 * R * S + 4 * R * kFemQm + 4 * R;
+    return 8 * R * S + (form == 1 ? 24 * R * S : 0) + 12 * R * S + 4 * R;
 }
 
 template <int FORM>
 struct FemLds {
     double* acc;       // the row's accumulator
-    double* qb;        // the row's round buffer
     double* vel;       // the row's column velocities (FORM 1)
     float* xyz;        // the row's column coordinates
-    uint32_t* qm;      // the row's round maps
     int* own;          // the row's own slot
     __device__ FemLds(double* lds, int stride, int rl)
     {
         const size_t R = kFemRowsPerWave, S = (size_t)stride;
         acc = lds + rl * S;
-        qb = lds + R * S + rl * kFemQb;
-        double* v0 = lds + R * (S + kFemQb);
+        double* v0 = lds + R * S;
         vel = v0 + rl * 3 * S;
         float* x0 = reinterpret_cast<float*>(v0 + (FORM == 1 ? 3 * R * S : 0));
         xyz = x0 + rl * 3 * S;
-        uint32_t* m0 = reinterpret_cast<uint32_t*>(x0 + 3 * R * S);
-        qm = m0 + rl * kFemQm;
-        own = reinterpret_cast<int*>(m0 + R * kFemQm) + rl;
+        own = reinterpret_cast<int*>(x0 + 3 * R * S) + rl;
     }
 };
 
@@ -2911,13 +2945,25 @@ __device__ void fem_rows(const uint64_t* __restrict__ n2t_off, const uint32_t* _
         a0 = n2t_off[i];
         na = (int)(n2t_off[i + 1] - a0);
         len = e.len[i];
-        for (int k = lane; k < len; k += kFemLanes) {
-            const int32_t c = e.cols[ell_at(e, i, k)];
-            for (int d = 0; d < 3; d++) L.xyz[3 * k + d] = xyz[3 * (int64_t)c + d];
-            if (FORM == 1)
-                for (int d = 0; d < 3; d++) L.vel[3 * k + d] = vel[3 * (int64_t)c + d];
-            if (c == (int32_t)i) *L.own = k;
-            acc[k] = 0.0;
+        for (int k0 = lane; k0 < len; k0 += kFemCols * kFemLanes) {
+            int32_t c[kFemCols];
+            float cx[kFemCols][3];
+            double cv[kFemCols][3];
+            for (int u = 0; u < kFemCols; u++) c[u] = e.cols[ell_at(e, i, min(k0 + kFemLanes * u, len - 1))];
+            for (int u = 0; u < kFemCols; u++)
+                for (int d = 0; d < 3; d++) {
+                    cx[u][d] = xyz[3 * (int64_t)c[u] + d];
+                    cv[u][d] = FORM == 1 ? vel[3 * (int64_t)c[u] + d] : 0.0;
+                }
+            for (int u = 0; u < kFemCols; u++) {
+                const int k = k0 + kFemLanes * u;
+                if (k >= len) break;
+                for (int d = 0; d < 3; d++) L.xyz[3 * k + d] = cx[u][d];
+                if (FORM == 1)
+                    for (int d = 0; d < 3; d++) L.vel[3 * k + d] = cv[u][d];
+                if (c[u] == (int32_t)i) *L.own = k;
+                acc[k] = 0.0;
+            }
         }
     }
     int na_max = na;                                   // rounds are uniform over the wave
@@ -2929,8 +2975,8 @@ __device__ void fem_rows(const uint64_t* __restrict__ n2t_off, const uint32_t* _
         const int a = r0 + lane;
         const uint32_t mp = mn;
         if (a + kFemLanes < na) mn = fmap[a0 + a + kFemLanes];
+        double add[4] = {0.0, 0.0, 0.0, 0.0};
         if (a < na) {
-            L.qm[lane] = mp;
             int sl[4];
             double x[4][3];
             for (int j = 0; j < 4; j++) {
@@ -2938,30 +2984,37 @@ __device__ void fem_rows(const uint64_t* __restrict__ n2t_off, const uint32_t* _
                 for (int d = 0; d < 3; d++) x[j][d] = (double)L.xyz[3 * sl[j] + d];
             }
             double G[4][3], detB;
-            if (!fem_frame(x, G, detB)) {
-                for (int j = 0; j < 4; j++) L.qb[4 * lane + j] = 0.0;   // no contribution
-            } else {
+            if (fem_frame(x, G, detB)) {               // else no contribution
                 const int li = sl[0] == own ? 0 : sl[1] == own ? 1 : sl[2] == own ? 2 : 3;
                 // quadrature points in the order 0, 2, 1, 3: s02 = f0 w + f2 w and
                 // s13 = f1 w + f3 w per basis function, then (s02 + s13) |det B|
                 const double w = qd.w;
+                double V[4][3];                        // the velocity at the points, summed in node order
+                if (FORM == 1)
+                    for (int d = 0; d < 3; d++) {
+                        // a node's velocity has two products over the four points (hi, lo); a
+                        // sum starts with its first product (the reference's 0.0 + that only
+                        // turns -0 into +0, which no sum of the row can tell: it starts at +0)
+                        double lo[4], hi[4];
+                        for (int j = 0; j < 4; j++) {
+                            const double vj = L.vel[3 * sl[j] + d];
+                            lo[j] = vj * (j == 0 ? qd.lo0 : qd.lo);
+                            hi[j] = vj * qd.hi;
+                        }
+                        const double l01 = lo[0] + lo[1];
+                        V[0][d] = ((lo[0] + hi[1]) + lo[2]) + lo[3];
+                        V[1][d] = (l01 + hi[2]) + lo[3];
+                        V[2][d] = (l01 + lo[2]) + hi[3];
+                        V[3][d] = ((hi[0] + lo[1]) + lo[2]) + lo[3];
+                    }
                 double s02[4], s13[4];
                 for (int qq = 0; qq < 4; qq++) {
                     const int q4 = qq == 1 ? 2 : qq == 2 ? 1 : qq;
-                    const double v = qd.phi[4 * li + q4];
-                    double V0 = 0.0, V1 = 0.0, V2 = 0.0;
-                    if (FORM == 1) {
-                        for (int j = 0; j < 4; j++) {
-                            const double* vj = L.vel + 3 * sl[j];
-                            const double pj = qd.phi[4 * j + q4];
-                            V0 = V0 + vj[0] * pj;
-                            V1 = V1 + vj[1] * pj;
-                            V2 = V2 + vj[2] * pj;
-                        }
-                    }
+                    const double v = q4 == FemQuad::point(li) ? qd.hi : li == 0 ? qd.lo0 : qd.lo;
                     for (int j = 0; j < 4; j++) {
-                        const double f = FORM == 0 ? qd.phi[4 * j + q4] * v
-                                                   : (V0 * (G[j][0] * v) + V1 * (G[j][1] * v)) + V2 * (G[j][2] * v);
+                        const double f = FORM == 0
+                            ? qd.phi(j, q4) * v
+                            : (V[q4][0] * (G[j][0] * v) + V[q4][1] * (G[j][1] * v)) + V[q4][2] * (G[j][2] * v);
                         const double pw = f * w;
                         if (qq == 0) s02[j] = pw;
                         else if (qq == 1) s02[j] = s02[j] + pw;
@@ -2969,26 +3022,18 @@ __device__ void fem_rows(const uint64_t* __restrict__ n2t_off, const uint32_t* _
                         else s13[j] = s13[j] + pw;
                     }
                 }
-                for (int j = 0; j < 4; j++) L.qb[4 * lane + j] = (s02[j] + s13[j]) * detB;
+                for (int j = 0; j < 4; j++) add[j] = (s02[j] + s13[j]) * detB;
             }
         }
-        __syncthreads();
-        if (lane == 0) {
-            // a tet's four nodes are four distinct columns: its four adds are
-            // independent, so they are issued together; tets stay in order
-            const int nt = min(kFemLanes, na - r0);
-            for (int t = 0; t < nt; t++) {
-                const uint32_t pos = L.qm[t];
-                int c[4];
-                double s4[4];
-                for (int j = 0; j < 4; j++) {
-                    c[j] = (int)((pos >> (8 * j)) & 0xffu);
-                    s4[j] = acc[c[j]] + L.qb[4 * t + j];
-                }
-                for (int j = 0; j < 4; j++) acc[c[j]] = s4[j];
-            }
+        // a tet's four nodes are four distinct columns: each of the row's lanes
+        // adds one of them; tets stay in order (the lanes are of one wave, whose
+        // LDS operations are done in order)
+        quad_transpose(add, lane);
+        const uint32_t pos[4] = {quad_lane<0>(mp), quad_lane<1>(mp), quad_lane<2>(mp), quad_lane<3>(mp)};
+        for (int t = 0; t < 4; t++) {
+            if (r0 + t < na) acc[(pos[t] >> (8 * lane)) & 0xffu] += add[t];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
-        __syncthreads();
     }
 }
 
@@ -3066,7 +3111,14 @@ __device__ __forceinline__ void block_sum2(double a, double b, double* part)
 // DiagonalPreconditioner), b = R phi and r = b - L phi (BiCGSTAB's first
 // residual from the guess phi), each summed in column order; r0 = r, x = phi,
 // p = v = 0.
-// At least 5 waves per SIMD: 94 VGPRs, no spills (measured faster than 118 at 4).
+//
+// FP64 arithmetic bounds it (about 260 operations per row and tet, none of them
+// a matrix product: each row's basis gradients differ), with the latency of LDS
+// and of the columns' gathers behind it; LDS holds it at 3 waves per SIMD.  At
+// 200^3 3.13 ms, after 4.23: 3.84 with the quadrature's shared products and
+// the additions spread over a row's lanes, 3.44 with kFemCols columns' loads in
+// flight (one: 3.84), 3.13 with the contributions exchanged between lanes in
+// registers instead of LDS.  91 VGPRs; asking for 4 waves changes nothing.
 __global__ __launch_bounds__(64, 3) void k_fem_cn(const uint64_t* __restrict__ n2t_off,
                                                const uint32_t* __restrict__ fmap, const float* __restrict__ xyz,
                                                const double* __restrict__ vel, int64_t N, FemQuad qd, FemEll e,
@@ -3083,43 +3135,51 @@ __global__ __launch_bounds__(64, 3) void k_fem_cn(const uint64_t* __restrict__ n
     int len;
     fem_rows<1>(n2t_off, fmap, xyz, vel, N, qd, e, stride, fem_lds, i, A, len);
     // the row's entries split over its lanes: L = M + s A into lvals, the
-    // products R phi_c (in place of A) and L phi_c into LDS; then the first
-    // lane sums both in column order, as a sequential row loop would
+    // products R phi_c (in place of A) and L phi_c into LDS; then two lanes
+    // sum them in column order, as a sequential row loop would
     const int lane = threadIdx.x % kFemLanes;
     double* LP = FemLds<1>(fem_lds, stride, threadIdx.x / kFemLanes).vel;   // free after the rounds
-    double id = 0.0;
-    int found = 0;
-    for (int k = lane; k < len; k += kFemLanes) {
-        const int64_t at = ell_at(e, i, k);
-        const int32_t c = e.cols[at];
-        const double m = mvals[at], sa = s * A[k];
-        const double L = m + sa, R = m - sa;
-        const double pc = phi[c];
-        lvals[at] = L;
-        A[k] = R * pc;
-        LP[k] = L * pc;
-        if (c == (int32_t)i && L != 0.0) {
-            id = 1.0 / L;
-            found = 1;
+    double id = 0.0;                                   // L_ii, in the lane that has it
+    for (int k0 = lane; k0 < len; k0 += kFemCols * kFemLanes) {
+        const int64_t at0 = ell_at(e, i, k0);
+        int32_t c[kFemCols];
+        double m[kFemCols], pc[kFemCols];
+        for (int u = 0; u < kFemCols; u++) {
+            const int64_t at = ell_at(e, i, min(k0 + kFemLanes * u, len - 1));
+            c[u] = e.cols[at];
+            m[u] = mvals[at];
+        }
+        for (int u = 0; u < kFemCols; u++) pc[u] = phi[c[u]];
+        for (int u = 0; u < kFemCols; u++) {
+            const int k = k0 + kFemLanes * u;
+            if (k >= len) break;
+            const double sa = s * A[k];
+            const double L = m[u] + sa, R = m[u] - sa;
+            lvals[at0 + kFemLanes * kFemSlice * u] = L;
+            A[k] = R * pc[u];
+            LP[k] = L * pc[u];
+            if (c[u] == (int32_t)i) id = L;
         }
     }
-    for (int o = 1; o < kFemLanes; o <<= 1) {          // the diagonal's lane to all
+    for (int o = 1; o < kFemLanes; o <<= 1) {          // the diagonal to all
         const double vo = __shfl_xor(id, o);
-        const int fo = __shfl_xor(found, o);
-        if (!found && fo) {
-            id = vo;
-            found = 1;
-        }
+        if (id == 0.0) id = vo;
     }
     __syncthreads();
-    if (i < N && lane == 0) {
-        double bi = 0.0, lx = 0.0;
-        for (int k = 0; k < len; k++) {
-            bi += A[k];
-            lx += LP[k];
+    // lane 0 sums b_i, lane 1 (L phi)_i, kFemLanes terms read at a time
+    const double* S = lane == 0 ? A : LP;
+    double sum = 0.0;
+    if (lane < 2)
+        for (int k0 = 0; k0 < len; k0 += kFemLanes) {
+            double a[kFemLanes];
+            for (int u = 0; u < kFemLanes; u++) a[u] = S[min(k0 + u, len - 1)];
+            for (int u = 0; u < kFemLanes; u++)
+                if (k0 + u < len) sum += a[u];
         }
-        const double ri = bi - lx;
-        invdiag[i] = found ? id : 1.0;
+    const double lx = __shfl_xor(sum, 1);
+    if (i < N && lane == 0) {
+        const double bi = sum, ri = bi - lx;
+        invdiag[i] = id != 0.0 ? 1.0 / id : 1.0;
         b[i] = bi;
         x[i] = phi[i];
         r[i] = ri;
@@ -5709,19 +5769,16 @@ int ft_surface_tension(ft_handle h, float st, int32_t rho, double* fx, double* f
 // ---- Advection (LevelSet::update, LevelSet.cpp:89-141) ---------------------
 // Quadrature(2, P1) (Quadrature.hpp:23-36) at the float shape functions
 // (Tetrahedron.hpp:30-34): the point coordinates go in as float and phi_0 =
-// 1.0 - x - y - z comes back rounded to float.
+// 1.0 - x - y - z comes back rounded to float: at the points (a, b, b),
+// (b, a, b), (b, b, a) the same value, at (b, b, b) the float of a.
 FemQuad fem_quad()
 {
     FemQuad q;
     const double a = (5.0 + 3.0 * std::sqrt(5.0)) / 20.0, b = (5.0 - std::sqrt(5.0)) / 20.0;
-    const double qp[3][4] = {{a, b, b, b}, {b, a, b, b}, {b, b, a, b}};
-    for (int k = 0; k < 4; k++) {
-        const float x = (float)qp[0][k], y = (float)qp[1][k], z = (float)qp[2][k];
-        q.phi[0 * 4 + k] = (double)(float)(((1.0 - (double)x) - (double)y) - (double)z);
-        q.phi[1 * 4 + k] = (double)x;
-        q.phi[2 * 4 + k] = (double)y;
-        q.phi[3 * 4 + k] = (double)z;
-    }
+    const float ha = (float)a, lb = (float)b;
+    q.hi = (double)ha;
+    q.lo = (double)lb;
+    q.lo0 = (double)(float)(((1.0 - (double)ha) - (double)lb) - (double)lb);
     q.w = 0.25 / 6.0;
     return q;
 }

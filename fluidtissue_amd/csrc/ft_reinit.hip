@@ -86,8 +86,9 @@ inline unsigned grid1d(int64_t n, int bs = kBS) { return (unsigned)((n + bs - 1)
 //   S_Q      the query's work-queue counters (9 x u32: deep tiles, then one
 //            per XCD), zeroed per launch
 //   S_LV     3 slots: primitives and tree nodes per level (ftd::Lv)
+//   S_CLAMP  nodes clamped to the band, of a single field
 enum Slot { S_BLK = 0, S_EDGES = 1, S_ERR = 2, S_P2T = 3, S_BINS = 4, S_DEEP = 5, S_CAP = 6,
-            S_Q = 7, S_LV = 12, S_N = 15 };
+            S_Q = 7, S_LV = 12, S_CLAMP = 15, S_N = 16 };
 
 // Stage totals of the running reinit as the kernels see them.  Kernels after
 // a scan read the total from the device, so a launch sized for a capacity
@@ -168,13 +169,49 @@ __global__ __launch_bounds__(kBS) void k_fill(T* p, int64_t n, T v)
     if (i < n) p[i] = v;
 }
 
+// Several ranges of 4-byte words set in one launch (what a stage needs cleared).
+struct WordRanges {
+    static constexpr int kMax = 8;
+    uint32_t* p[kMax];
+    int64_t end[kMax];               // words of the ranges up to and including this one
+    uint32_t v[kMax];
+    int n = 0;
+    void add(void* at, int64_t words, uint32_t value)
+    {
+        if (words <= 0) return;
+        p[n] = static_cast<uint32_t*>(at);
+        end[n] = total() + words;
+        v[n++] = value;
+    }
+    int64_t total() const { return n ? end[n - 1] : 0; }
+};
+__global__ __launch_bounds__(kBS) void k_set_words(WordRanges r)
+{
+    const int64_t i = (int64_t)blockIdx.x * kBS + threadIdx.x;
+    int64_t lo = 0;
+    for (int k = 0; k < r.n; k++) {
+        if (i < r.end[k]) {
+            r.p[k][i - lo] = r.v[k];
+            return;
+        }
+        lo = r.end[k];
+    }
+}
+
+// clear: the scan leaves zeros in its input (cursors of the pass that follows).
 struct LoadSame {
+    static constexpr bool clear = false;
     template <class T> __device__ T operator()(T v) const { return v; }
 };
+struct LoadClear : LoadSame {
+    static constexpr bool clear = true;
+};
 struct LoadPopc {  // u64 bitmap word -> popcount
+    static constexpr bool clear = false;
     __device__ uint32_t operator()(uint64_t v) const { return (uint32_t)__popcll(v); }
 };
 struct LoadTileClass {  // tile class 0 / 1 deep / 2 very deep -> (very deep << 32) | deep
+    static constexpr bool clear = false;
     __device__ uint64_t operator()(uint32_t c) const { return ((uint64_t)(c == 2) << 32) | (uint64_t)(c >= 1); }
 };
 
@@ -236,16 +273,14 @@ __device__ __forceinline__ void store_run16(T* p, const T (&v)[K])
     }
 }
 
-// Each thread scans IPT consecutive elements: read and written as 16-byte
-// accesses when the run is whole and both arrays are 16-byte aligned (the
-// run starts at a multiple of IPT elements, at least 32 bytes).
-template <class TI, class TO, class Ld>
-__global__ __launch_bounds__(kBS) void k_scan_down(const TI* in, TO* out, int64_t n,
-                                                   const TO* bsum, Ld ld)
+// kScanTile / kBS consecutive elements from `base` per thread of a workgroup
+// of BS, scanned from `before`; returns the workgroup's sum.  Read and written
+// as 16-byte accesses when the run is whole and both arrays are 16-byte
+// aligned (the run starts at a multiple of its length, at least 32 bytes).
+template <int BS, class TI, class TO, class Ld>
+__device__ __forceinline__ TO scan_run(const TI* in, TO* out, int64_t n, int64_t base, TO before, TO* lds, Ld ld)
 {
-    __shared__ TO lds[kBS / 64 + 1];
     constexpr int IPT = kScanTile / kBS;
-    const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * IPT;
     const bool vec = base + IPT <= n &&
                      ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
     TO v[IPT];
@@ -265,7 +300,7 @@ __global__ __launch_bounds__(kBS) void k_scan_down(const TI* in, TO* out, int64_
 #pragma unroll
     for (int k = 0; k < IPT; k++) s += v[k];
     TO tot;
-    TO ex = ftd::block_excl_scan<TO, kBS>(s, lds, &tot) + bsum[blockIdx.x];
+    TO ex = ftd::block_excl_scan<TO, BS>(s, lds, &tot) + before;
     if (vec) {
         TO o[IPT];
 #pragma unroll
@@ -282,6 +317,36 @@ __global__ __launch_bounds__(kBS) void k_scan_down(const TI* in, TO* out, int64_
             ex += v[k];
         }
     }
+    if (Ld::clear)
+        for (int k = 0; k < IPT; k++)
+            if (base + k < n) const_cast<TI*>(in)[base + k] = TI(0);
+    return tot;
+}
+
+template <class TI, class TO, class Ld>
+__global__ __launch_bounds__(kBS) void k_scan_down(const TI* in, TO* out, int64_t n,
+                                                   const TO* bsum, Ld ld)
+{
+    __shared__ TO lds[kBS / 64 + 1];
+    scan_run<kBS>(in, out, n, (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * (kScanTile / kBS),
+                  bsum[blockIdx.x], lds, ld);
+}
+
+// A short scan in one launch, by one workgroup, instead of three: small
+// reinits are bound by their launches (32^3 points 305 us with three launches a
+// scan, 256 with one; 47 x 33 x 17 triangles 503 and 466), and up to one step
+// of the workgroup the scan itself is no slower.  With 32768 elements (four
+// steps) a 127^3 reinit loses 25 us of 1320 to the longer scans.
+constexpr int64_t kScanOne = 8192;
+template <class TI, class TO, class Ld>
+__global__ __launch_bounds__(1024) void k_scan_one(const TI* in, TO* out, int64_t n, TO* total, Ld ld)
+{
+    __shared__ TO lds[1024 / 64 + 1];
+    constexpr int IPT = kScanTile / kBS;
+    TO carry = TO(0);
+    for (int64_t at = 0; at < n; at += 1024 * IPT)
+        carry += scan_run<1024>(in, out, n, at + (int64_t)threadIdx.x * IPT, carry, lds, ld);
+    if (threadIdx.x == 0) *total = carry;
 }
 
 // ============================================================================
@@ -361,12 +426,24 @@ __global__ __launch_bounds__(kBS) void k_pad_slots(int64_t n_slots, int nf, cons
 // ============================================================================
 // Marching tets (LevelSet::findInterfaceNodes_ / reconstructInterface_)
 // ============================================================================
-__global__ __launch_bounds__(kBS) void k_node_signs(const double* phi, int64_t n, uint64_t* bits)
+// Opens a reinit: the nodes' signs, and everything that the stages mark or
+// raise cleared.
+__global__ __launch_bounds__(kBS) void k_node_signs(const double* phi, int64_t n, uint64_t* bits, uint64_t* retain,
+                                                    uint64_t* ebits, int64_t nw_edges, uint64_t* sc)
 {
     const int64_t i = (int64_t)blockIdx.x * kBS + threadIdx.x;
+    for (int64_t w = i; w < nw_edges; w += (int64_t)gridDim.x * kBS) ebits[w] = 0ull;
+    if (i == 0) {
+        sc[S_ERR] = ~0ull;
+        sc[S_CAP] = 0ull;
+        sc[S_EDGES] = 0ull;                            // the edge scan writes the low 32 bits
+    }
     const int neg = (i < n) ? ftd::sign_bit(phi[i]) : 0;   // std::signbit (LevelSet.cpp:281,380)
     const uint64_t m = __ballot(neg);
-    if (ftd::lane_id() == 0 && i < n) bits[i >> 6] = m;
+    if (ftd::lane_id() == 0 && i < n) {
+        bits[i >> 6] = m;
+        retain[i >> 6] = 0ull;
+    }
 }
 
 // Crossing iff 1..3 of a tet's nodes are negative (LevelSet.cpp:380-383); 2
@@ -429,13 +506,24 @@ __global__ __launch_bounds__(kBS) void k_classify(MeshView mv, int64_t T,
     }
 }
 
+// Capacities of a reinit whose buffers were sized in advance (graph replay; a
+// negative one is not checked).  The first kernel that writes what a stage total
+// counts compares the two in every thread, writes nothing when the total is
+// larger, and raises S_CAP, which halts every later kernel.
+__device__ __forceinline__ bool outgrown(uint64_t* sc, bool larger, uint64_t bit)
+{
+    if (larger && blockIdx.x == 0 && threadIdx.x == 0) sc[S_CAP] |= bit;
+    return larger;
+}
+
 // One thread per 64-tet word of the crossing bitmap.  Lanes 4k..4k+3 share a
 // k_classify block, whose exclusive offset is blk_prefix[w/4].
 __global__ __launch_bounds__(kBS) void k_compact(const uint64_t* tbits, const uint64_t* t2bits,
                                                  int64_t nwords, const uint64_t* blk_prefix,
-                                                 int32_t* xtet, int32_t* xtri_off, const uint64_t* sc)
+                                                 int32_t* xtet, int32_t* xtri_off, uint64_t* sc,
+                                                 int64_t x_cap, int64_t f_cap)
 {
-    if (halted(sc)) return;
+    if (halted(sc) || outgrown(sc, x_cap >= 0 && (cnt_xtets(sc) > x_cap || cnt_tris(sc) > f_cap), 1ull)) return;
     const int64_t w = (int64_t)blockIdx.x * kBS + threadIdx.x;
     const uint64_t word = w < nwords ? tbits[w] : 0ull;
     const uint64_t two = w < nwords ? t2bits[w] : 0ull;
@@ -459,17 +547,6 @@ __global__ __launch_bounds__(kBS) void k_compact(const uint64_t* tbits, const ui
         bx++;
         bt += 1u + (uint32_t)((two >> b) & 1ull);
     }
-}
-
-// Capacity check of a reinit whose buffers were sized in advance (graph
-// replay): raises S_CAP when a stage total exceeds what was allocated, which
-// halts every later kernel.  One thread.
-__global__ void k_check_caps(uint64_t* sc, int64_t x_cap, int64_t f_cap, int64_t p_cap)
-{
-    uint64_t v = 0;
-    if (x_cap >= 0 && (cnt_xtets(sc) > x_cap || cnt_tris(sc) > f_cap)) v |= 1ull;
-    if (p_cap >= 0 && cnt_points(sc) > p_cap) v |= 2ull;
-    if (v) sc[S_CAP] |= v;
 }
 
 // Error word: (code << 40) | tet, min-reduced so the lowest failing tet wins
@@ -550,9 +627,9 @@ __global__ __launch_bounds__(kBS) void k_points(const uint64_t* ebits, const uin
                                                 int64_t nwords, MeshView mv,
                                                 const float* xyz, const double* phi,
                                                 float* ifp, int32_t* ifp2e,
-                                                unsigned long long* retain, const uint64_t* sc)
+                                                unsigned long long* retain, uint64_t* sc, int64_t p_cap)
 {
-    if (halted(sc)) return;
+    if (halted(sc) || outgrown(sc, p_cap >= 0 && cnt_points(sc) > p_cap, 2ull)) return;
     const int lane = ftd::lane_id();
     const int64_t w = (int64_t)blockIdx.x * kBS + threadIdx.x;
     const int64_t w0 = w - lane;                       // the wave's first word
@@ -888,15 +965,13 @@ __global__ __launch_bounds__(kBS) void k_level_reduce(const uint64_t* sc, const 
 
 // first[] of the leaves and of the nodes of every level, and the fields'
 // roots: the node of the level that covers the whole field (Grid::root_lv).
-__global__ __launch_bounds__(kBS) void k_level_down(const uint64_t* sc, const uint32_t* leaf_cnt,
-                                                    const uint32_t* leaf_bin, IndexGeom ig, const ftd::Lv* bsum,
-                                                    LevelOff lo, uint32_t* first, uint32_t* roots)
+// IPT leaves from `base` per thread of a workgroup of BS, after `before`;
+// returns the workgroup's sum.
+template <int BS, int IPT>
+__device__ __forceinline__ ftd::Lv level_run(int64_t base, int64_t L, const uint32_t* leaf_cnt,
+                                             const uint32_t* leaf_bin, const IndexGeom& ig, ftd::Lv before,
+                                             const LevelOff& lo, uint32_t* first, uint32_t* roots, ftd::Lv* lds)
 {
-    __shared__ ftd::Lv lds[kBS / 64 + 1];
-    constexpr int IPT = kScanTile / kBS;
-    const int64_t L = halted(sc) ? 0 : cnt_leaves(sc);
-    if ((int64_t)blockIdx.x * kScanTile >= L) return;            // whole block
-    const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * IPT;
     ftd::Lv s(0);
     for (int k = 0; k < IPT; k++) {
         uint32_t o;
@@ -904,7 +979,7 @@ __global__ __launch_bounds__(kBS) void k_level_down(const uint64_t* sc, const ui
         s += leaf_elem(base + k, L, leaf_cnt, leaf_bin, ig, &o, &f);
     }
     ftd::Lv tot;
-    ftd::Lv ex = ftd::block_excl_scan<ftd::Lv, kBS>(s, lds, &tot) + bsum[blockIdx.x];
+    ftd::Lv ex = ftd::block_excl_scan<ftd::Lv, BS>(s, lds, &tot) + before;
     for (int k = 0; k < IPT; k++) {
         const int64_t l = base + k;
         if (l >= L) break;
@@ -931,6 +1006,36 @@ __global__ __launch_bounds__(kBS) void k_level_down(const uint64_t* sc, const ui
             first[lo.off[4] + (uint32_t)ex.c] = lo.off[3] + (uint32_t)(ex.b >> 32);
         }
     }
+    return tot;
+}
+
+__global__ __launch_bounds__(kBS) void k_level_down(const uint64_t* sc, const uint32_t* leaf_cnt,
+                                                    const uint32_t* leaf_bin, IndexGeom ig, const ftd::Lv* bsum,
+                                                    LevelOff lo, uint32_t* first, uint32_t* roots)
+{
+    __shared__ ftd::Lv lds[kBS / 64 + 1];
+    constexpr int IPT = kScanTile / kBS;
+    const int64_t L = halted(sc) ? 0 : cnt_leaves(sc);
+    if ((int64_t)blockIdx.x * kScanTile >= L) return;            // whole block
+    level_run<kBS, IPT>((int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * IPT, L, leaf_cnt, leaf_bin, ig,
+                        bsum[blockIdx.x], lo, first, roots, lds);
+}
+
+// All of it for few leaves, in one launch by one workgroup (kScanOne's reason;
+// the leaves are fewer than the bound on them that is compared: a bound of
+// 32768 gives 10 us of 480 over 8192 at 47 x 33 x 17, 8 of 530 at 61^3 points).
+constexpr int64_t kLevelOne = 32768;
+constexpr int kLevelOneRun = 4;                        // leaves per thread and step
+__global__ __launch_bounds__(1024) void k_level_one(uint64_t* sc, const uint32_t* leaf_cnt, const uint32_t* leaf_bin,
+                                                    IndexGeom ig, LevelOff lo, uint32_t* first, uint32_t* roots)
+{
+    __shared__ ftd::Lv lds[1024 / 64 + 1];
+    const int64_t L = halted(sc) ? 0 : cnt_leaves(sc);
+    ftd::Lv carry(0);
+    for (int64_t at = 0; at < L; at += 1024 * kLevelOneRun)
+        carry += level_run<1024, kLevelOneRun>(at + (int64_t)threadIdx.x * kLevelOneRun, L, leaf_cnt, leaf_bin, ig,
+                                               carry, lo, first, roots, lds);
+    if (threadIdx.x == 0) *reinterpret_cast<ftd::Lv*>(sc + S_LV) = carry;
 }
 
 // The item of a box given by its axes, its centre m and half extents h in the
@@ -3762,23 +3867,31 @@ int fill(hipStream_t s, T* p, int64_t n, T v)
     return FT_OK;
 }
 
+int set_words(hipStream_t s, const WordRanges& r)
+{
+    if (r.n == 0) return FT_OK;
+    hipLaunchKernelGGL(k_set_words, dim3(grid1d(r.total())), dim3(kBS), 0, s, r);
+    FT_HIP(hipGetLastError());
+    return FT_OK;
+}
+
 // Exclusive scan of n elements; the total lands in *d_total (device).
 // ws: the block-sum scratch (default: the handle's; each stream needs its own).
 template <class TI, class TO, class Ld>
 int scan(ft_ctx* c, hipStream_t s, const TI* in, TO* out, int64_t n, TO* d_total, Ld ld, DevBuf* ws = nullptr)
 {
+    if (n <= kScanOne) {
+        hipLaunchKernelGGL((k_scan_one<TI, TO, Ld>), dim3(1), dim3(1024), 0, s, in, out, n, d_total, ld);
+        FT_HIP(hipGetLastError());
+        return FT_OK;
+    }
     DevBuf& w = ws ? *ws : c->scan_bsum;
-    const int64_t nb = std::max<int64_t>(1, (n + kScanTile - 1) / kScanTile);
+    const int64_t nb = (n + kScanTile - 1) / kScanTile;
     FT_TRY(ensure(w, sizeof(TO) * (size_t)nb));
     TO* bs = w.as<TO>();
-    if (n > 0) {
-        hipLaunchKernelGGL((k_scan_reduce<TI, TO, Ld>), dim3((unsigned)nb), dim3(kBS), 0, s, in, n, bs, ld);
-    } else {
-        FT_TRY(fill<TO>(s, bs, 1, TO(0)));
-    }
+    hipLaunchKernelGGL((k_scan_reduce<TI, TO, Ld>), dim3((unsigned)nb), dim3(kBS), 0, s, in, n, bs, ld);
     hipLaunchKernelGGL(k_scan_top<TO>, dim3(1), dim3(1024), 0, s, bs, nb, d_total);
-    if (n > 0)
-        hipLaunchKernelGGL((k_scan_down<TI, TO, Ld>), dim3((unsigned)nb), dim3(kBS), 0, s, in, out, n, bs, ld);
+    hipLaunchKernelGGL((k_scan_down<TI, TO, Ld>), dim3((unsigned)nb), dim3(kBS), 0, s, in, out, n, bs, ld);
     FT_HIP(hipGetLastError());
     return FT_OK;
 }
@@ -4348,8 +4461,7 @@ int build_node_tets(ft_ctx* c, hipStream_t s)
     uint64_t* off = c->n2t_off.as<uint64_t>();
     FT_TRY(fill<uint32_t>(s, cnt, N, 0u));
     if (T > 0) hipLaunchKernelGGL(k_n2t_count, dim3(grid1d(T)), dim3(kBS), 0, s, c->tets.as<int4>(), T, cnt);
-    FT_TRY(scan<uint32_t, uint64_t>(c, s, cnt, off, N, off + N, LoadSame{}));
-    FT_TRY(fill<uint32_t>(s, cnt, N, 0u));
+    FT_TRY(scan<uint32_t, uint64_t>(c, s, cnt, off, N, off + N, LoadClear{}));   // cnt: then the fill's cursors
     if (T > 0)
         hipLaunchKernelGGL(k_n2t_fill, dim3(grid1d(T)), dim3(kBS), 0, s, c->tets.as<int4>(), T, off, cnt,
                            c->n2t_ids.as<int32_t>());
@@ -4474,7 +4586,7 @@ MeshView mesh_view(ft_ctx* c)
 // stage totals back after the two counting scans (sizing the buffers exactly,
 // and stopping early on a failed stage).  !eager (graph capture): no host
 // reads and no allocation; the buffers were sized for `cp` beforehand and
-// k_check_caps guards them.  counts_only: stops once the totals are known
+// the kernels guard them (outgrown()).  counts_only: stops once the totals are known
 // (phi is not written).
 // Work enqueued on c->side from now on runs after everything enqueued on s
 // so far.
@@ -4509,18 +4621,14 @@ int enqueue_marching(ft_ctx* c, hipStream_t s, double* phi, int mode, bool want_
 {
     const int64_t N = c->N, T = c->T, E = c->E;
     uint64_t* sc = c->scalars.as<uint64_t>();
-    const int64_t nw_nodes = (N + 63) / 64, nw_tets = (T + 63) / 64, nw_edges = (E + 63) / 64;
+    const int64_t nw_tets = (T + 63) / 64, nw_edges = (E + 63) / 64;
     const int64_t nblk = (T + kBS - 1) / kBS;
     timed = timed && !counts_only;
     FT_TRY(ensure_stage(c, 0, cp, mode, want_nearest, want_normals));
     uint64_t* sbits = c->sbits.as<uint64_t>();
     if (timed) (void)hipEventRecord(c->ev[0], s);
-    hipLaunchKernelGGL(k_node_signs, dim3(grid1d(N)), dim3(kBS), 0, s, phi, N, sbits);
-    FT_TRY(fill<uint64_t>(s, c->retain.as<uint64_t>(), nw_nodes, 0ull));
-    FT_TRY(fill<uint64_t>(s, c->ebits.as<uint64_t>(), nw_edges, 0ull));
-    FT_TRY(fill<uint64_t>(s, sc + S_ERR, 1, ~0ull));
-    FT_TRY(fill<uint64_t>(s, sc + S_CAP, 1, 0ull));
-    FT_TRY(fill<uint64_t>(s, sc + S_EDGES, 1, 0ull));   // the edge scan writes the low 32 bits
+    hipLaunchKernelGGL(k_node_signs, dim3(grid1d(N)), dim3(kBS), 0, s, phi, N, sbits,
+                       c->retain.as<uint64_t>(), c->ebits.as<uint64_t>(), nw_edges, sc);
     if (T > 0)
         hipLaunchKernelGGL(k_classify, dim3((unsigned)((nblk + kClassifyGroups - 1) / kClassifyGroups)),
                            dim3(kBS), 0, s, mesh_view(c), T, sbits, c->tbits.as<uint64_t>(),
@@ -4533,14 +4641,12 @@ int enqueue_marching(ft_ctx* c, hipStream_t s, double* phi, int mode, bool want_
         cp.F = (int64_t)(c->h_scalars[S_BLK] & 0xffffffffull);
         cnt->n_if_elems = cp.X;
         cnt->n_tri = cp.F;
-    } else {
-        hipLaunchKernelGGL(k_check_caps, dim3(1), dim3(1), 0, s, sc, cp.X, cp.F, (int64_t)-1);
     }
     FT_TRY(ensure_stage(c, 1, cp, mode, want_nearest));
     if (nw_tets > 0)
         hipLaunchKernelGGL(k_compact, dim3(grid1d(nw_tets)), dim3(kBS), 0, s, c->tbits.as<uint64_t>(),
                            c->tbits.as<uint64_t>() + nw_tets, nw_tets, c->blk.as<uint64_t>(),
-                           c->xtet.as<int32_t>(), c->xtri_off.as<int32_t>(), sc);
+                           c->xtet.as<int32_t>(), c->xtri_off.as<int32_t>(), sc, eager ? -1 : cp.X, eager ? -1 : cp.F);
     if (cp.X > 0)
         hipLaunchKernelGGL(k_xtet, dim3(grid1d(cp.X)), dim3(kBS), 0, s, c->tbits.as<uint64_t>() + nw_tets,
                            mesh_view(c), sbits, c->xtet.as<int32_t>(), sc,
@@ -4553,15 +4659,13 @@ int enqueue_marching(ft_ctx* c, hipStream_t s, double* phi, int mode, bool want_
         cnt->n_ifp = cp.P;
         FT_TRY(stage_error(c->h_scalars[S_ERR], cnt));
         if (counts_only) return FT_OK;
-    } else {
-        hipLaunchKernelGGL(k_check_caps, dim3(1), dim3(1), 0, s, sc, (int64_t)-1, (int64_t)-1, cp.P);
     }
     FT_TRY(ensure_stage(c, 2, cp, mode, want_nearest));
     if (nw_edges > 0)
         hipLaunchKernelGGL(k_points, dim3(grid1d(nw_edges)), dim3(kBS), 0, s, c->ebits.as<uint64_t>(),
                            c->eprefix.as<uint32_t>(), nw_edges, mesh_view(c), c->xyz.as<float>(),
                            phi, c->ifp.as<float>(), c->ifp2e.as<int32_t>(),
-                           c->retain.as<unsigned long long>(), sc);
+                           c->retain.as<unsigned long long>(), sc, eager ? -1 : cp.P);
     if (cp.X > 0)
         hipLaunchKernelGGL(k_tris, dim3(grid1d(cp.X)), dim3(kBS), 0, s, mesh_view(c), c->xyz.as<float>(),
                            phi, c->xtet.as<int32_t>(), c->xtri_off.as<int32_t>(), c->xedges.as<int4>(),
@@ -4577,9 +4681,9 @@ int enqueue_marching(ft_ctx* c, hipStream_t s, double* phi, int mode, bool want_
         FT_TRY(fill<uint32_t>(ss, deg, cp.P, 0u));
         if (cp.F > 0)
             hipLaunchKernelGGL(k_p2t_count, dim3(grid1d(cp.F)), dim3(kBS), 0, ss, c->tris.as<int4>(), sc, deg);
+        // deg: the degrees, then (cleared by the scan) the fill's cursors
         FT_TRY(scan<uint32_t, uint32_t>(c, ss, deg, c->p2t_off.as<uint32_t>(), cp.P,
-                                        c->p2t_off.as<uint32_t>() + cp.P, LoadSame{}, &c->scan_side));
-        FT_TRY(fill<uint32_t>(ss, deg, cp.P, 0u));
+                                        c->p2t_off.as<uint32_t>() + cp.P, LoadClear{}, &c->scan_side));
         if (cp.F > 0)
             hipLaunchKernelGGL(k_p2t_fill, dim3(grid1d(cp.F)), dim3(kBS), 0, ss, c->tris.as<int4>(), sc,
                                c->p2t_off.as<uint32_t>(), deg, c->p2t.as<int32_t>());
@@ -4674,10 +4778,15 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
     uint32_t* lbin = c->leaf_bin.as<uint32_t>();
     uint32_t* first = c->nfirst.as<uint32_t>();
     uint32_t* code = c->pcode.as<uint32_t>();
-    FT_TRY(fill<uint64_t>(s, bits, W, 0ull));
-    FT_TRY(fill<uint32_t>(s, lcnt, lp.cap[0], 0u));
-    FT_TRY(fill<uint32_t>(s, c->roots.as<uint32_t>(), nf, ~0u));
-    FT_TRY(fill<uint64_t>(s, sc + S_BINS, 1, 0ull));      // the bitmap scan writes the low 32 bits
+    uint64_t* clamped = nf == 1 ? sc + S_CLAMP : c->fclamp.as<uint64_t>();
+    WordRanges clr;
+    clr.add(bits, 2 * W, 0u);
+    clr.add(lcnt, lp.cap[0], 0u);
+    clr.add(c->roots.p, nf, ~0u);
+    clr.add(sc + S_BINS, 2, 0u);                       // the bitmap scan writes the low 32 bits
+    clr.add(clamped, 2 * nf, 0u);
+    if (sp.work_queue) clr.add(sc + S_Q, 9, 0u);
+    FT_TRY(set_words(s, clr));
     if (n_cap > 0) {
         hipLaunchKernelGGL(k_prim_bin, dim3(grid1d(n_cap)), dim3(kBS), 0, s, mode, sc, ifp, tris,
                            nf > 1 ? c->ifp2e.as<int32_t>() : nullptr, ig, code, (unsigned long long*)bits);
@@ -4685,13 +4794,18 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
                                         reinterpret_cast<uint32_t*>(sc + S_BINS), LoadPopc{}));
         hipLaunchKernelGGL(k_prim_rank, dim3(grid1d(n_cap)), dim3(kBS), 0, s, mode, sc, bits,
                            c->bprefix.as<uint32_t>(), code, c->place.as<uint32_t>(), lcnt, lbin);
-        const int64_t nb = scan_blocks(lp.cap[0]);
-        ftd::Lv* bs = c->scan_bsum.as<ftd::Lv>();
-        hipLaunchKernelGGL(k_level_reduce, dim3((unsigned)nb), dim3(kBS), 0, s, sc, lcnt, lbin, ig, bs);
-        hipLaunchKernelGGL(k_scan_top<ftd::Lv>, dim3(1), dim3(1024), 0, s, bs, nb,
-                           reinterpret_cast<ftd::Lv*>(sc + S_LV));
-        hipLaunchKernelGGL(k_level_down, dim3((unsigned)nb), dim3(kBS), 0, s, sc, lcnt, lbin, ig, bs, lp.lo, first,
-                           c->roots.as<uint32_t>());
+        if (lp.cap[0] <= kLevelOne) {
+            hipLaunchKernelGGL(k_level_one, dim3(1), dim3(1024), 0, s, sc, lcnt, lbin, ig, lp.lo, first,
+                               c->roots.as<uint32_t>());
+        } else {
+            const int64_t nb = scan_blocks(lp.cap[0]);
+            ftd::Lv* bs = c->scan_bsum.as<ftd::Lv>();
+            hipLaunchKernelGGL(k_level_reduce, dim3((unsigned)nb), dim3(kBS), 0, s, sc, lcnt, lbin, ig, bs);
+            hipLaunchKernelGGL(k_scan_top<ftd::Lv>, dim3(1), dim3(1024), 0, s, bs, nb,
+                               reinterpret_cast<ftd::Lv*>(sc + S_LV));
+            hipLaunchKernelGGL(k_level_down, dim3((unsigned)nb), dim3(kBS), 0, s, sc, lcnt, lbin, ig, bs, lp.lo, first,
+                               c->roots.as<uint32_t>());
+        }
         hipLaunchKernelGGL(k_prim_scatter, dim3(grid1d(n_cap)), dim3(kBS), 0, s, mode, sc, ifp, tris, code,
                            c->place.as<uint32_t>(), first, lbin, ig, c->prec.as<float4>(), c->titem.as<Item>(),
                            c->trec.as<TriRec>(), c->pidx.as<int32_t>());
@@ -4705,7 +4819,6 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
     FT_TRY(check_launch());
 
     // ---- distance query with the fused epilogue --------------------------------
-    FT_TRY(fill<uint64_t>(s, c->fclamp.as<uint64_t>(), nf, 0ull));
     QueryArgs q{};
     q.n_slots = c->n_slots;
     q.sx = c->sx.as<float>(); q.sy = c->sy.as<float>(); q.sz = c->sz.as<float>();
@@ -4730,7 +4843,7 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
     q.epi = sp.epi;
     q.w_phi = sp.w_phi;
     q.w_ifn = sp.w_ifn;
-    q.n_clamped = c->fclamp.as<unsigned long long>();
+    q.n_clamped = reinterpret_cast<unsigned long long*>(clamped);
     static const bool want_stats = getenv("FT_QUERY_STATS") != nullptr;
     q.h_est = c->h_est;
     if (want_stats && eager) {
@@ -4767,7 +4880,6 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
             const int64_t waves = (int64_t)c->cu_count * 4 * wps;
             g = dim3((unsigned)std::max<int64_t>(kXcds, waves / (qb / 64)));
             q.queue = reinterpret_cast<uint32_t*>(sc + S_Q);
-            FT_TRY(fill<uint32_t>(s, q.queue, 9, 0u));
         }
         FT_TRY(launch_query(mode, qb, wps, g, b, s, q));
         if (q.split_out) {
@@ -4801,11 +4913,13 @@ int collect(ft_ctx* c, hipStream_t s, bool want_nearest, ft_counts* cnt)
     FT_HIP(hipMemcpyAsync(c->h_scalars, c->scalars.p, sizeof(uint64_t) * S_N, hipMemcpyDeviceToHost, s));
     std::vector<uint64_t> clamp(nf);
     std::vector<int64_t> fc(nf > 1 ? 3 * nf : 0);
-    FT_HIP(hipMemcpyAsync(clamp.data(), c->fclamp.p, 8 * nf, hipMemcpyDeviceToHost, s));
-    if (nf > 1)
+    if (nf > 1) {
+        FT_HIP(hipMemcpyAsync(clamp.data(), c->fclamp.p, 8 * nf, hipMemcpyDeviceToHost, s));
         FT_HIP(hipMemcpyAsync(fc.data(), c->fcounts.p, sizeof(int64_t) * 3 * nf, hipMemcpyDeviceToHost, s));
+    }
     FT_HIP(hipStreamSynchronize(s));
     const uint64_t* hs = c->h_scalars;
+    if (nf == 1) clamp[0] = hs[S_CLAMP];
     *cnt = ft_counts{};
     cnt->n_if_elems = (int64_t)(hs[S_BLK] >> 32);
     cnt->n_tri = (int64_t)(hs[S_BLK] & 0xffffffffull);
@@ -5730,8 +5844,7 @@ int surface_tension(ft_ctx* h, float st, int32_t rho, double* fx, double* fy, do
     const int2* edges = h->edges.as<int2>();
     FT_TRY(fill<uint32_t>(s, cnt, N, 0u));
     hipLaunchKernelGGL(k_st_count, dim3(grid1d(P)), dim3(kBS), 0, s, ifp2e, P, edges, cnt);
-    FT_TRY(scan<uint32_t, uint64_t>(h, s, cnt, off, N, off + N, LoadSame{}));
-    FT_TRY(fill<uint32_t>(s, cnt, N, 0u));
+    FT_TRY(scan<uint32_t, uint64_t>(h, s, cnt, off, N, off + N, LoadClear{}));   // cnt: then the fill's cursors
     hipLaunchKernelGGL(k_st_fill, dim3(grid1d(P)), dim3(kBS), 0, s, ifp2e, P, edges, off, cnt, ids);
     hipLaunchKernelGGL(k_n2t_sort, dim3(grid1d(N)), dim3(kBS), 0, s, off, N, ids);
     hipLaunchKernelGGL(k_st_apply, dim3(grid1d(N)), dim3(kBS), 0, s, off, ids, N, ifp2e, edges,
@@ -6046,10 +6159,13 @@ int ft_reset_phi_points(ft_handle h, const float* ifp, int64_t n_ifp, double* ph
     uint64_t* sc = h->scalars.as<uint64_t>();
     FT_TRY(index_setup(h, s, 0.0f, sp.mode));
     FT_TRY(ensure_stage(h, 0, cp, 0, true));
-    FT_TRY(fill<uint64_t>(s, sc + S_BLK, 1, 0ull));
-    FT_TRY(fill<uint64_t>(s, sc + S_EDGES, 1, (uint64_t)n_ifp));
-    FT_TRY(fill<uint64_t>(s, sc + S_ERR, 1, ~0ull));
-    FT_TRY(fill<uint64_t>(s, sc + S_CAP, 1, 0ull));
+    WordRanges set;
+    set.add(sc + S_BLK, 2, 0u);
+    set.add(sc + S_EDGES, 1, (uint32_t)n_ifp);
+    set.add(reinterpret_cast<uint32_t*>(sc + S_EDGES) + 1, 1, 0u);
+    set.add(sc + S_ERR, 2, ~0u);
+    set.add(sc + S_CAP, 2, 0u);
+    FT_TRY(set_words(s, set));
     SideJoin join{h, s};
     FT_TRY(enqueue_search(h, s, sp, cp, true, false));
     ft_counts cnt{};

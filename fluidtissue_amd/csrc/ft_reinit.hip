@@ -4231,27 +4231,30 @@ int sort_nodes(ft_ctx* c, bool blocks = true)
     if (c->N == 0) return FT_OK;
     hipStream_t s = c->stream;
     unsigned long long* misfit = c->scalars.as<unsigned long long>() + S_P2T;
-    FT_TRY(fill<unsigned long long>(s, misfit, 1, 0ull));
-    FT_TRY(fill<int32_t>(s, c->perm.as<int32_t>(), c->n_slots, -1));
+    WordRanges clr;
+    clr.add(misfit, 2, 0u);
+    clr.add(c->perm.p, c->n_slots, ~0u);
     for (int k = 0; k < nf; k++) {
         const int64_t n = c->node_off[k + 1] - c->node_off[k];
         if (n == 0) continue;
         const Grid& g = grids[k];
         const int64_t G = (int64_t)1 << (3 * lgs[k]);
         FT_TRY(ensure(c->bin_count, sizeof(uint32_t) * G));
-        FT_TRY(ensure(c->bin_prefix, sizeof(uint64_t) * G));
+        const int64_t nb = cpb[k] ? G / cpb[k] : 0;   // blocks
+        FT_TRY(ensure(c->bin_prefix, sizeof(uint32_t) * (G + nb)));
         FT_TRY(ensure(c->pcode, sizeof(uint32_t) * n));
         uint32_t* cnt = c->bin_count.as<uint32_t>();
         uint32_t* off = c->bin_prefix.as<uint32_t>();
-        uint32_t* btile = off + G;                     // per block (at most G of them)
+        uint32_t* btile = off + G;                     // per block
         uint32_t* total = reinterpret_cast<uint32_t*>(c->scalars.as<uint64_t>() + S_BINS);
         const float* xk = c->xyz.as<float>() + 3 * c->node_off[k];
         const int64_t sb = c->slot_off[k];
-        FT_TRY(fill<uint32_t>(s, cnt, G, 0u));
+        clr.add(cnt, G, 0u);
+        FT_TRY(set_words(s, clr));
+        clr = WordRanges{};
         hipLaunchKernelGGL(k_node_bin, dim3(grid1d(n)), dim3(kBS), 0, s, xk, n, g, c->pcode.as<uint32_t>(), cnt);
         FT_TRY(scan<uint32_t, uint32_t>(c, s, cnt, off, G, total, LoadSame{}));
         if (cpb[k]) {
-            const int64_t nb = G / cpb[k];
             hipLaunchKernelGGL(k_block_tiles, dim3(grid1d(nb)), dim3(kBS), 0, s, off, n, G, cpb[k], btile);
             FT_TRY(scan<uint32_t, uint32_t>(c, s, btile, btile, nb, total, LoadSame{}));
         }

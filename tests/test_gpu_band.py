@@ -1,0 +1,37 @@
+"""GPU: what a narrow band's search leaves out -- the nodes clamped per field,
+counted over runs of 1024 tiles that hold one field or several."""
+import numpy as np
+import pytest
+
+import fluidtissue_amd as fa
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("mode", ["points", "triangles"])
+@pytest.mark.parametrize("sizes", [[44], [45, 9, 3], [6, 44, 20, 45, 4]])
+def test_clamped_nodes_are_those_without_a_nearest(mode, sizes):
+    h = 1.0 / (max(sizes) - 1)
+    meshes = [fa.kuhn_mesh(n, spacing=h, jitter=0.1, seed=2) for n in sizes]
+    phis = [np.linalg.norm(m.xyz.astype(np.float64) - 0.4 * h * n, axis=1) - 0.2 * h * n for n, m in zip(sizes, meshes)]
+    r = fa.Reinit(0)
+    if len(sizes) == 1:
+        r.set_mesh(meshes[0])
+        off = np.array([0, meshes[0].n_nodes])
+    else:
+        r.set_batch(meshes)
+        off, _, _ = r.batch_info()
+    band = 2.5 * h
+    _, ifn, cnt = r.reset_phi(np.concatenate(phis), mode=mode, band=band, want_nearest=True)
+    none = r.nearest() == -1
+    per_field = [int(none[off[k]:off[k + 1]].sum()) for k in range(len(sizes))]
+    got = [c.n_clamped for c in r.field_counts()] if len(sizes) > 1 else [cnt.n_clamped]
+    assert got == per_field and cnt.n_clamped == sum(per_field) > 0
+    assert np.array_equal(np.abs(ifn[none]), np.full(none.sum(), np.float64(np.float32(band))))
+    # every node the full search finds inside the band keeps its distance
+    _, full, _ = r.reset_phi(np.concatenate(phis), mode=mode)
+    sure = np.abs(np.abs(full) / band - 1) > 1e-5          # (rounding decides at the band's edge)
+    inside = (np.abs(full) < band) & sure
+    assert np.array_equal(inside[sure], ~none[sure])
+    assert np.array_equal(ifn[inside].view(np.uint64), full[inside].view(np.uint64))
+    r.close()

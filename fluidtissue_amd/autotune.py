@@ -8,9 +8,8 @@ Tunes, on the caller's own resident batch and level set:
                   footprint and how workgroups spread over the XCDs);
   waves_per_simd  the query's launch bound, 5..8 waves per SIMD (registers
                   against occupancy; triangles mode only);
-  schedule        one tile per wave in a fixed deep-first order ("static"),
-                  or persistent waves taking tiles from per-XCD counters
-                  ("queue").
+  schedule        the deepest tiles split over several waves ("static"), or
+                  every tile whole ("queue").
 Each candidate runs the full reinit; the fastest median wins.  The search
 is staged: bin_scale x query_block at 8 waves, static; then waves_per_simd
 at the best of those; then the schedule.  Results are cached per (mode,

@@ -83,12 +83,16 @@ inline unsigned grid1d(int64_t n, int bs = kBS) { return (unsigned)((n + bs - 1)
 //   S_DEEP   query tiles scheduled first (low 32 bits), of which the very deep
 //            ones, split over several waves (high 32 bits)
 //   S_CAP    a stage total exceeded the capacity its buffers were sized for
-//   S_Q      the query's work-queue counters (9 x u32: deep tiles, then one
-//            per XCD), zeroed per launch
 //   S_LV     3 slots: primitives and tree nodes per level (ftd::Lv)
 //   S_CLAMP  nodes clamped to the band, of a single field
+// (S_TOP of them are read back), and after them
+//   S_Q      the query's counters (9 x u32: deep tiles, then one per XCD),
+//            zeroed per launch, each in a line of its own: in one line their
+//            atomics wait for each other (crossing points at 256^3 3.55 ms against
+//            3.15, a 256^3 band 3.59 against 1.90)
 enum Slot { S_BLK = 0, S_EDGES = 1, S_ERR = 2, S_P2T = 3, S_BINS = 4, S_DEEP = 5, S_CAP = 6,
-            S_Q = 7, S_LV = 12, S_CLAMP = 15, S_N = 16 };
+            S_LV = 7, S_CLAMP = 10, S_TOP = 16, S_Q = S_TOP, S_N = S_Q + 9 * 16 };
+constexpr int kQueueLine = 32;           // words between the query's counters
 
 // Stage totals of the running reinit as the kernels see them.  Kernels after
 // a scan read the total from the device, so a launch sized for a capacity
@@ -1452,34 +1456,35 @@ struct QueryArgs {
     float h_est;                     // node spacing (statistics only)
     int probe;                       // a first candidate from the search for the tile's centre
     const uint64_t* sc;              // stage totals and halt flags
-    unsigned xcd_chunk;              // tiles per XCD chunk (0: dispatch order)
-    uint32_t* queue;                 // work-queue schedule: deep counter, then one per XCD (null: static)
+    uint32_t* queue;                 // counters, kQueueLine apart: deep tiles, then one per XCD
     ulonglong2* split_out;           // best and second key per lane of each part of a split tile (null: none split)
 };
 
-// The dispatcher hands workgroup b to XCD b % 8, each XCD with its own L2.
-// Remapped, XCD x processes runs of `chunk` consecutive tiles (in Morton
-// order, a compact region whose triangle and tree records its L2 keeps)
-// instead of every 8th tile; the runs are dealt to the XCDs in turn, so costly
-// regions still spread over all of them (one contiguous run per XCD was
-// slower: the XCD holding the costliest region finished last).  A bijection
-// on [0, nb).
+// The dispatcher hands workgroup b to XCD b % 8, each XCD with its own L2, so
+// the tiles after the deep ones are dealt to the XCDs in runs of `chunk`
+// consecutive ones (in Morton order, a compact region whose triangle and tree
+// records its L2 keeps): the runs x, x + 8, x + 16, ... to XCD x.  At least 8
+// runs each, that costly regions spread over all of them (one run each was
+// slower), and up to 1024 tiles long (256^3; 512 is 1 % slower, 2048 0.5 %).
 constexpr unsigned kXcds = 8;
-// Workgroups per run, measured at 256^3 (triangles, deep tiles first): with
-// 256-thread workgroups 512 (2048 tiles; 1024 is 4% slower), with 64-thread
-// workgroups 1024 (1024 tiles; 512 is 1.3% slower, 2048 0.5%).
-constexpr unsigned kXcdChunk = 512;
-constexpr unsigned kXcdChunk64 = 1024;
-__device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned nb, unsigned chunk)
-{
-    if (chunk == 0) return b;
-    // chunks of `chunk` consecutive tiles, dealt to the XCDs in turn
-    const unsigned span = kXcds * chunk;
-    const unsigned full = nb - nb % span;          // blocks in whole spans
-    if (b >= full) return b;                       // the ragged tail keeps its order
-    const unsigned x = b % kXcds, i = b / kXcds;
-    return (i / chunk) * span + x * chunk + i % chunk;
-}
+struct XcdShare {
+    uint32_t n, chunk, span;         // tiles in all, per run, per run of every XCD
+    __device__ explicit XcdShare(uint32_t tiles) : n(tiles)
+    {
+        const uint32_t c = tiles / (kXcds * 8);
+        chunk = c < 1u ? 1u : c > 1024u ? 1024u : c;
+        span = kXcds * chunk;
+    }
+    __device__ uint32_t tiles(uint32_t x) const       // of XCD x
+    {
+        const uint32_t whole = n / span, rest = n - whole * span, at = x * chunk;
+        return whole * chunk + (rest <= at ? 0u : rest - at < chunk ? rest - at : chunk);
+    }
+    __device__ uint32_t tile(uint32_t x, uint32_t k) const   // the k-th of XCD x
+    {
+        return k / chunk * span + x * chunk + k % chunk;
+    }
+};
 
 // Margin of the box prune: a box is skipped only if its lower bound exceeds
 // the best distance by more than the float rounding of both (relative) plus
@@ -1576,9 +1581,8 @@ __device__ __forceinline__ void finish_node(const QueryArgs& a, const Found& S, 
 // spheres: 3.3 ms at phi_old = -29 h where the mean tile takes 0.14 ms), so
 // such tiles, started late or in a small field, set the kernel's end.  A tile
 // is deep when one of its nodes has phi_old <= -kDeepTile split_h h of its
-// field: the deep tiles are listed first and take the lowest workgroups, which
-// the dispatcher starts first and deals over all XCDs; the rest keep their
-// slot (Morton) order.  A tile is very deep from -split_h h: it is searched by
+// field: the deep tiles are listed first and are what the waves start with; the
+// rest keep their slot (Morton) order.  A tile is very deep from -split_h h: it is searched by
 // kSplitParts waves, each with all 64 nodes but testing only the leaves l with
 // l % kSplitParts equal to its part, and k_split_merge combines the parts.
 // Each part repeats the walk above the leaves, so splitting costs work, and
@@ -2198,16 +2202,19 @@ __device__ __forceinline__ void search_tile(const QueryArgs& a, int64_t base, Wa
     finish_node<MODE>(a, F, node);
 }
 
-// Query schedule of a launch: deep tiles first (k_tile_deep), the rest in
-// XCD-chunked Morton order (xcd_block).  Static: one tile per wave, the
-// deep tiles on the first workgroups (which the dispatcher deals over all
-// XCDs; a very deep tile on kSplitParts of them, a.split_out), the others
-// after them.  Work queue (a.queue; every tile whole): a persistent grid
-// whose waves take tiles from counters -- the deep tiles from one shared
-// counter, then the rest from the counter of their XCD (workgroup b runs on
-// XCD b % 8), each XCD's share being its chunks of the static order; a wave
-// whose XCD has none left takes from the other XCDs' counters in turn.
-// Every wave leaves once all nine counters are past their ends.
+// Query schedule of a launch: a persistent grid (as many waves as the device
+// holds, or as there are tiles).  The deep tiles (k_tile_deep) come first, a
+// very deep one (a.split_out) as kSplitParts parts, and wave w starts with
+// the w-th of them; the waves left over start with the first tiles of their
+// XCD (XcdShare).  After its first tile a wave takes the deep tiles that no
+// wave started with from one counter, then its XCD's from that XCD's, then
+// those of the XCDs that have any left, and leaves when none has: the
+// counters only grow, so every wave does.  Against one wave per tile in a fixed
+// order, which the dispatcher starts as places get free but on a fixed XCD:
+// triangles at 256^3 6.55 -> 6.2 ms, 160 x 144 x 131 1.61 -> 1.55, a 256^3
+// band 2.01 -> 1.86; crossing points at 256^3 3.33 -> 3.16; 128^3 and below the
+// same.  (Looking at every XCD's counter before each tile cost more than the
+// tiles: 8 ms, 5.3 in the band.)
 // Launch bound: WPS waves per SIMD.  Six (80 VGPRs, 52 B of spills around
 // the FP64 settle) beat five (no spills) and seven at 256^3: triangles 6.79 /
 // 6.10 / 6.33 ms at 5 / 6 / 7, points 3.57 / 3.20 / 3.31; the wave's LDS allows
@@ -2216,74 +2223,70 @@ __device__ __forceinline__ void search_tile(const QueryArgs& a, int64_t base, Wa
 template <int MODE, int BS, int WPS, bool STATS = false>
 __global__ __launch_bounds__(BS, WPS) void k_query_wave(QueryArgs a)
 {
-    __shared__ WaveLds<MODE> wlds[BS / 64];
+    constexpr uint32_t wpb = BS / 64;
+    __shared__ WaveLds<MODE> wlds[wpb];
     if (halted(a.sc)) return;                         // an earlier stage failed: phi untouched
-    const int w = threadIdx.x >> 6;
-    const int64_t n_tiles = a.n_slots / 64;
-    const uint64_t nd = a.tile_list ? ftd::cload(a.n_deep, 0) : 0ull;
-    const uint32_t K = (uint32_t)nd;                  // deep tiles (none in a narrow band: slot order)
-    unsigned src = 0;                                 // work queue: 0 the deep counter, 1..8 the XCDs'
-    for (;;) {
-        int64_t r;                                    // place in the launch order
-        int split = -1;
-        if (a.queue) {
-            const uint32_t nn = (uint32_t)(n_tiles - K);
-            const uint32_t chunk = a.xcd_chunk;
-            const unsigned xcd = blockIdx.x % kXcds;
-            uint32_t got = 0;
-            if (ftd::lane_id() == 0) got = atomicAdd(&a.queue[src == 0 ? 0 : 1 + (xcd + src - 1) % kXcds], 1u);
-            got = (uint32_t)__builtin_amdgcn_readfirstlane((int)got);
-            r = -1;
-            if (src == 0) {
-                if (got < K) r = got;
+    const uint32_t w = threadIdx.x >> 6, xcd = blockIdx.x % kXcds;
+    bool more_deep = true;                            // some that no wave started with
+    uint32_t from = 0;                                // the XCD after this one by `from` has some left
+    for (bool first = true;; first = false) {
+        const uint32_t n_tiles = (uint32_t)(a.n_slots / 64);
+        const uint64_t nd = a.tile_list ? ftd::cload(a.n_deep, 0) : 0ull;
+        const uint32_t K = (uint32_t)nd, cap = (uint32_t)split_tiles_cap(n_tiles);
+        const uint32_t K2 = !a.split_out ? 0u : (uint32_t)(nd >> 32) < cap ? (uint32_t)(nd >> 32) : cap;
+        const uint32_t D = K2 * kSplitParts + (K - K2);               // deep parts and tiles
+        const uint32_t Db = (D + wpb - 1) / wpb;                      // workgroups that start with them
+        const XcdShare share(n_tiles - K);
+        // tiles of XCD x that its waves start with
+        auto started = [&](uint32_t x) {
+            const uint32_t b0 = Db + ((x - Db) & (kXcds - 1));        // its first workgroup after those
+            return b0 < gridDim.x ? ((gridDim.x - b0 + kXcds - 1) / kXcds) * wpb : 0u;
+        };
+        uint32_t deep = ~0u, x = xcd, k = ~0u;                        // the deep-th, or XCD x's k-th
+        if (first) {
+            if (blockIdx.x < Db) {
+                deep = blockIdx.x * wpb + w;
+                if (deep >= D) continue;
             } else {
-                // the got-th tile of XCD x: its chunks are x, x + 8, x + 16, ...
-                // (increasing in got, so once past nn it stays past)
-                const unsigned x = (xcd + src - 1) % kXcds;
-                const uint64_t t = (uint64_t)(got / chunk) * kXcds * chunk + (uint64_t)x * chunk + got % chunk;
-                if (t < nn) r = (int64_t)K + (int64_t)t;
-            }
-            if (r < 0) {
-                if (++src > kXcds) return;            // every counter exhausted
-                continue;
-            }
-        } else if (a.tile_list) {
-            // deep tiles on the first Kb workgroups (Kb a multiple of the 8 XCDs):
-            // first kSplitParts waves for each split tile, then one per other deep
-            // tile; the rest on the workgroups after them in XCD-chunked order
-            constexpr unsigned wpb = BS / 64;
-            // (explicit compares: min() of two 64-bit integers resolves to a
-            // floating-point overload here and rounds them)
-            const uint64_t cap = (uint64_t)split_tiles_cap(n_tiles);
-            const unsigned K2 = a.split_out ? (unsigned)((nd >> 32) < cap ? (nd >> 32) : cap) : 0u;
-            const unsigned D = K2 * kSplitParts + (K - K2);          // deep waves
-            const unsigned Kb = ((D + wpb - 1) / wpb + 7u) & ~7u;
-            const unsigned b = blockIdx.x;
-            if (b < Kb) {
-                const unsigned rr = b * wpb + w;
-                if (rr >= D) return;                   // whole wave: padding of the deep workgroups
-                if (rr < K2 * kSplitParts) {
-                    split = (int)rr;
-                    r = rr / kSplitParts;
-                } else {
-                    r = (int64_t)K2 + (rr - K2 * kSplitParts);
-                }
-            } else {
-                const int64_t nn = n_tiles - K;
-                const unsigned nbn = (unsigned)((nn + wpb - 1) / wpb);
-                if (b - Kb >= nbn) return;             // whole wave: past the last tile
-                r = (int64_t)xcd_block(b - Kb, nbn, a.xcd_chunk) * wpb + w;
-                if (r >= nn) return;
-                r += K;
+                k = (blockIdx.x - (Db + ((xcd - Db) & (kXcds - 1)))) / kXcds * wpb + w;
+                if (k >= share.tiles(xcd)) continue;
             }
         } else {
-            r = (int64_t)xcd_block(blockIdx.x, gridDim.x, a.xcd_chunk) * (BS / 64) + w;
-            if (r >= n_tiles) return;                  // whole wave out of range
+            more_deep = more_deep && gridDim.x * wpb < D;
+            if (more_deep) {
+                uint32_t got = 0;
+                if (ftd::lane_id() == 0) got = atomicAdd(a.queue, 1u);
+                deep = gridDim.x * wpb + (uint32_t)__builtin_amdgcn_readfirstlane((int)got);
+                more_deep = deep < D;
+            }
+            if (!more_deep) {
+                deep = ~0u;
+                for (; from < kXcds; from++) {
+                    x = (xcd + from) % kXcds;
+                    const uint32_t nx = share.tiles(x), sx = started(x);
+                    if (sx >= nx) continue;
+                    uint32_t got = 0;
+                    if (ftd::lane_id() == 0) got = atomicAdd(a.queue + kQueueLine * (1 + x), 1u);
+                    k = sx + (uint32_t)__builtin_amdgcn_readfirstlane((int)got);
+                    if (k < nx) break;
+                }
+                if (from == kXcds) return;
+            }
+        }
+        int split = -1;
+        uint32_t r;                                                   // place in the launch order
+        if (deep != ~0u) {
+            r = K2 + (deep - K2 * kSplitParts);
+            if (deep < K2 * kSplitParts) {
+                split = (int)deep;
+                r = deep / kSplitParts;
+            }
+        } else {
+            r = K + share.tile(x, k);
         }
         // the wave's tile as uniform values
         const int64_t tile = __builtin_amdgcn_readfirstlane(a.tile_list ? a.tile_list[r] : (int)r);
         search_tile<MODE, STATS>(a, tile * 64, wlds[w], __builtin_amdgcn_readfirstlane(split));
-        if (!a.queue) return;
     }
 }
 
@@ -4322,7 +4325,7 @@ int sort_nodes(ft_ctx* c, bool blocks = true)
                        c->d_slot_off.as<int64_t>(), c->perm.as<int32_t>(), c->sx.as<float>(),
                        c->sy.as<float>(), c->sz.as<float>(), c->tile_field.as<int32_t>(), misfit);
     FT_TRY(check_launch());
-    FT_TRY(read_scalars(c, s, S_N));
+    FT_TRY(read_scalars(c, s, S_TOP));
     if (c->h_scalars[S_P2T]) {
         if (!blocks) return ft::set_error(FT_ERR_INTERNAL, "node sort: more nodes than slots");
         return sort_nodes(c, false);
@@ -4545,7 +4548,7 @@ struct SearchSpec {
     bool int_ifn = false;            // phi_ifn into the handle's buffer (normals need it)
     int query_block = 0;
     int waves_per_simd = 6;          // launch bound of the query (triangles: 5..8)
-    bool work_queue = false;         // persistent query over tile counters
+    bool whole_tiles = false;        // no tile is split over waves
 };
 
 // Copies of the resident meshes ms into the handle's concatenated arrays,
@@ -4694,7 +4697,7 @@ int enqueue_marching(ft_ctx* c, hipStream_t s, double* phi, int mode, bool want_
     FT_TRY(scan<uint64_t, uint64_t>(c, s, c->blk.as<uint64_t>(), c->blk.as<uint64_t>(), nblk,
                                     sc + S_BLK, LoadSame{}));
     if (eager) {
-        FT_TRY(read_scalars(c, s, S_N));
+        FT_TRY(read_scalars(c, s, S_TOP));
         cp.X = (int64_t)(c->h_scalars[S_BLK] >> 32);
         cp.F = (int64_t)(c->h_scalars[S_BLK] & 0xffffffffull);
         cnt->n_if_elems = cp.X;
@@ -4712,7 +4715,7 @@ int enqueue_marching(ft_ctx* c, hipStream_t s, double* phi, int mode, bool want_
     FT_TRY(scan<uint64_t, uint32_t>(c, s, c->ebits.as<uint64_t>(), c->eprefix.as<uint32_t>(),
                                     nw_edges, reinterpret_cast<uint32_t*>(sc + S_EDGES), LoadPopc{}));
     if (eager) {
-        FT_TRY(read_scalars(c, s, S_N));
+        FT_TRY(read_scalars(c, s, S_TOP));
         cp.P = (int64_t)(c->h_scalars[S_EDGES] & 0xffffffffull);
         cnt->n_ifp = cp.P;
         FT_TRY(stage_error(c->h_scalars[S_ERR], cnt));
@@ -4843,7 +4846,7 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
     clr.add(c->roots.p, nf, ~0u);
     clr.add(sc + S_BINS, 2, 0u);                       // the bitmap scan writes the low 32 bits
     clr.add(clamped, 2 * nf, 0u);
-    if (sp.work_queue) clr.add(sc + S_Q, 9, 0u);
+    clr.add(sc + S_Q, 9 * kQueueLine, 0u);
     FT_TRY(set_words(s, clr));
     if (n_cap > 0) {
         hipLaunchKernelGGL(k_prim_bin, dim3(grid1d(n_cap)), dim3(kBS), 0, s, mode, sc, ifp, tris,
@@ -4915,7 +4918,6 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
     // query 0.597 -> 0.511 ms)
     q.probe = !(getenv("FT_PROBE") && !strcmp(getenv("FT_PROBE"), "0"));
     q.sc = sc;
-    q.xcd_chunk = kXcdChunk;
     if (timed) (void)hipEventRecord(c->ev[2], s);
     FT_TRY(side_join(c, s));                          // the schedule and the point lists
     if (tile_list) {
@@ -4924,22 +4926,14 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
     }
     if (c->n_slots > 0) {
         const int qb = q.stats || sp.query_block == 0 ? 64 : sp.query_block;
-        q.xcd_chunk = qb == 64 ? kXcdChunk64 : kXcdChunk;
         const int wps = mode == 0 ? 6 : sp.waves_per_simd;
-        // with a tile list: up to 7 padding workgroups after the deep ones,
-        // one more for the split of the remainder, and the extra waves of
-        // the split tiles (static schedule)
-        if (q.tile_list && !sp.work_queue) q.split_out = c->deep_part.as<ulonglong2>();
-        const int64_t split_waves = q.split_out ? split_tiles_cap(n_tiles) * (kSplitParts - 1) : 0;
-        dim3 g(grid1d(c->n_slots, qb) + (q.tile_list ? 8u : 0u) + (unsigned)((split_waves + qb / 64 - 1) / (qb / 64))),
-            b(qb);
-        if (sp.work_queue) {
-            // persistent: as many waves as the device holds at this launch
-            // bound (4 SIMDs per CU), whole workgroups, at least one per XCD
-            const int64_t waves = (int64_t)c->cu_count * 4 * wps;
-            g = dim3((unsigned)std::max<int64_t>(kXcds, waves / (qb / 64)));
-            q.queue = reinterpret_cast<uint32_t*>(sc + S_Q);
-        }
+        if (q.tile_list && !sp.whole_tiles) q.split_out = c->deep_part.as<ulonglong2>();
+        // as many waves as the device holds at this launch bound (4 SIMDs per
+        // CU), or as there may be tiles and parts; whole workgroups
+        const int64_t items = n_tiles + (q.split_out ? split_tiles_cap(n_tiles) * (kSplitParts - 1) : 0);
+        const int64_t waves = std::min<int64_t>((int64_t)c->cu_count * 4 * wps, items);
+        const dim3 g(grid1d(waves, qb / 64)), b(qb);
+        q.queue = reinterpret_cast<uint32_t*>(sc + S_Q);
         FT_TRY(launch_query(mode, qb, wps, g, b, s, q));
         if (sp.band > 0.0f) {
             hipLaunchKernelGGL(k_clamp_sum, dim3(grid1d((n_tiles + kClampRun - 1) / kClampRun * 64)), dim3(kBS), 0, s,
@@ -4974,7 +4968,7 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
 int collect(ft_ctx* c, hipStream_t s, bool want_nearest, ft_counts* cnt)
 {
     const int nf = c->nf;
-    FT_HIP(hipMemcpyAsync(c->h_scalars, c->scalars.p, sizeof(uint64_t) * S_N, hipMemcpyDeviceToHost, s));
+    FT_HIP(hipMemcpyAsync(c->h_scalars, c->scalars.p, sizeof(uint64_t) * S_TOP, hipMemcpyDeviceToHost, s));
     std::vector<uint64_t> clamp(nf);
     std::vector<int64_t> fc(nf > 1 ? 3 * nf : 0);
     if (nf > 1) {
@@ -5049,7 +5043,7 @@ SearchSpec reinit_search_spec(double* phi, double* phi_ifn, const ft_opts* o)
     sp.int_ifn = sp.want_normals && !phi_ifn;
     sp.query_block = o->query_block;
     sp.waves_per_simd = o->waves_per_simd > 0 ? o->waves_per_simd : 6;
-    sp.work_queue = o->schedule == FT_SCHED_QUEUE;
+    sp.whole_tiles = o->schedule == FT_SCHED_QUEUE;
     return sp;
 }
 
@@ -5427,7 +5421,7 @@ int ft_create(int32_t device, ft_handle* out)
         return ft::set_error(FT_ERR_HIP, "side stream set-up failed");
     }
     if (ensure(c->scalars, 8 * S_N) != FT_OK ||
-        hipHostMalloc((void**)&c->h_scalars, 8 * S_N, hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc((void**)&c->h_scalars, 8 * S_TOP, hipHostMallocDefault) != hipSuccess) {
         (void)hipStreamDestroy(c->stream);
         (void)hipStreamDestroy(c->side);
         (void)hipEventDestroy(c->side_fork_ev);

@@ -83,9 +83,9 @@ typedef struct ft_opts {
     int32_t waves_per_simd; /* launch bound of the triangle-mode query: 5..8
                             waves per SIMD (register budget against
                             occupancy); 0 = 6                                  */
-    int32_t schedule;    /* FT_SCHED_STATIC: one tile per wave, deep tiles on
-                            the first workgroups; FT_SCHED_QUEUE: persistent
-                            waves taking tiles from per-XCD counters;
+    int32_t schedule;    /* FT_SCHED_STATIC: the deepest tiles split over
+                            several waves; FT_SCHED_QUEUE: every tile whole
+                            (persistent waves take the tiles in either);
                             FT_SCHED_BINS (narrow band, triangles only): as
                             FT_SCHED_STATIC (a search of the band's bins
                             without the tree was slower than the tree walk) */

@@ -81,7 +81,8 @@ inline unsigned grid1d(int64_t n, int bs = kBS) { return (unsigned)((n + bs - 1)
 //   S_ERR    ~0, or (code << 40) | first failing tet
 //   S_BINS   leaves of the index (low 32 bits)
 //   S_DEEP   query tiles scheduled first (low 32 bits), of which the very deep
-//            ones, split over several waves (high 32 bits)
+//            ones, split over several waves (high 32 bits); in a narrow band
+//            the tiles to search (k_tile_near)
 //   S_CAP    a stage total exceeded the capacity its buffers were sized for
 //   S_LV     3 slots: primitives and tree nodes per level (ftd::Lv)
 //   S_CLAMP  nodes clamped to the band, of a single field
@@ -1887,6 +1888,37 @@ struct TileSearch {
         return __ballot(keep != 0u);
     }
 
+    // The points that reach any of the boxes [c0, c0 + cnt), cnt <= 64, which
+    // then admit nothing more.
+    __device__ __forceinline__ uint64_t reached(uint32_t c0, uint32_t cnt)
+    {
+        const int lane = fresh_lane();
+        uint64_t all[4] = {0, 0, 0, 0};
+        v4h av;
+        float4 e;
+        load4(a.items + c0, lane, av, e);
+        for (uint32_t i = 0; i < cnt; i += 4) {
+            v4h av1 = av;
+            float4 e1 = e;
+            if (i + 4 < cnt) load4(a.items + c0 + i + 4, lane, av1, e1);
+            uint64_t m[4];
+            cull4(av, e, cnt - i, m);
+#pragma unroll
+            for (int cb = 0; cb < 4; cb++) all[cb] |= m[cb];
+            av = av1;
+            e = e1;
+        }
+        uint64_t hit = 0;
+#pragma unroll
+        for (int cb = 0; cb < 4; cb++) {
+            uint64_t v = all[cb] | (all[cb] >> 32);
+            v = (v | (v >> 16)) & 0xffffull;
+            hit |= v << (16 * cb);
+            if ((v >> (lane & 15)) & 1ull) thr[cb] = -1.0f;
+        }
+        return hit;
+    }
+
     // Range of element b of list d.
     __device__ __forceinline__ void range_of(int d, uint32_t b, uint32_t& s0, uint32_t& s1) const
     {
@@ -2109,6 +2141,14 @@ struct TileSearch {
     }
 };
 
+// The key of a node without a candidate.
+template <int MODE>
+__device__ __forceinline__ uint64_t no_key(const QueryArgs& a)
+{
+    return MODE == 0 ? cand_key(a.band > 0.0f ? a.band : FLT_MAX, -1)
+                     : cand_key(a.band > 0.0f ? a.band * a.band : INFINITY, -1);
+}
+
 // A wave's tile: 64 consecutive slots of one field in Morton order.
 // split >= 0: part split % kSplitParts of split tile split / kSplitParts,
 // whose best and second keys go to a.split_out instead of the epilogue.
@@ -2126,8 +2166,7 @@ __device__ __forceinline__ void search_tile(const QueryArgs& a, int64_t base, Wa
     F.x = a.sx[slot]; F.y = a.sy[slot]; F.z = a.sz[slot];
     const int field = __builtin_amdgcn_readfirstlane(a.tile_field[base >> 6]);
     const uint32_t root = (uint32_t)__builtin_amdgcn_readfirstlane((int)ftd::cload(a.roots, field));
-    const uint64_t none = MODE == 0 ? cand_key(a.band > 0.0f ? a.band : FLT_MAX, -1)
-                                    : cand_key(a.band > 0.0f ? a.band * a.band : INFINITY, -1);
+    const uint64_t none = no_key<MODE>(a);
     F.bkey = F.skey = none;
     if (root != ~0u) {                                 // the field has primitives
         const Grid* g = a.grids + field;
@@ -2202,6 +2241,139 @@ __device__ __forceinline__ void search_tile(const QueryArgs& a, int64_t base, Wa
     finish_node<MODE>(a, F, node);
 }
 
+// Narrow band: the tiles any primitive can reach, 64 tiles per wave: cls 1 and
+// a place in the list, from its front those inside the surface (where the
+// longest ones are: they start first), from its end the others, counted in
+// `count` (inside << 32 | others).
+// A tile counts as its box's ball, and is left out only if the boxes of all
+// nodes above the leaves (indices below `last`: those, and the leaves of a field
+// that has no such nodes) are farther from the centre than the band and the
+// radius, both raised well past the rounding of the boxes and of the distances:
+// a tile left out would find nothing.  The walk is the search's, with tiles for
+// nodes; a tile leaves it at the first box that it reaches.  Latency is all
+// its time, so it does not go down to the leaves, which would leave out few
+// more (128^3: 123 us, and 37 down to the nodes above them).
+// Searching every tile, 95 % of which end at the root's children, took 1.86 ms
+// at 256^3 in a 6 h band; this 0.10 ms, their epilogue (k_far_tiles) 0.13 beside
+// the search of the rest, 1.06.  At 128^3 0.32, now 0.04 and 0.22.
+__global__ __launch_bounds__(64) void k_tile_near(QueryArgs a, uint32_t last, uint32_t* cls, int32_t* list,
+                                                  unsigned long long* count)
+{
+    __shared__ WaveLds<1> lds;
+    if (halted(a.sc)) return;
+    int lane = ftd::lane_id();
+    asm volatile("" : "+v"(lane));
+    const int64_t n_tiles = a.n_slots / 64;
+    const int64_t tile = (int64_t)blockIdx.x * 64 + lane;
+    const int64_t mine = tile < n_tiles ? tile : n_tiles - 1;
+    float lo[3], hi[3], odd = 0.0f;
+    const float* axes[3] = {a.sx, a.sy, a.sz};
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        lo[k] = INFINITY;
+        hi[k] = -INFINITY;
+        const float4* v = reinterpret_cast<const float4*>(axes[k] + 64 * mine);
+#pragma unroll 4
+        for (int q = 0; q < 16; q++) {
+            const float4 u = v[q];
+            lo[k] = fminf(lo[k], fminf(fminf(u.x, u.y), fminf(u.z, u.w)));
+            hi[k] = fmaxf(hi[k], fmaxf(fmaxf(u.x, u.y), fmaxf(u.z, u.w)));
+            odd += 0.0f * ((u.x + u.y) + (u.z + u.w));         // NaN if a coordinate is not finite
+        }
+    }
+    float c[3], ext2 = 0.0f;
+    for (int k = 0; k < 3; k++) {
+        c[k] = 0.5f * lo[k] + 0.5f * hi[k];
+        const float e = 0.5f * (hi[k] - lo[k]);
+        ext2 += e * e;
+    }
+    const bool ok = odd == 0.0f && ext2 < INFINITY;
+    const int field = a.tile_field[mine];
+    TileSearch<1, false> S(a, lds, lane);
+    uint64_t near = __ballot(!ok);
+    // one field of the wave's tiles at a time
+    for (uint64_t todo = __ballot(ok && tile < n_tiles); todo;) {
+        const int f = __builtin_amdgcn_readlane(field, __ffsll((unsigned long long)todo) - 1);
+        const uint64_t here = __ballot(field == f) & todo;
+        todo &= ~here;
+        const uint32_t root = (uint32_t)__builtin_amdgcn_readfirstlane((int)ftd::cload(a.roots, f));
+        if (root == ~0u) continue;                     // the field has no primitives
+        const Grid* g = a.grids + f;
+        const float ox = ftd::cload(&g->org[0], 0), oy = ftd::cload(&g->org[1], 0), oz = ftd::cload(&g->org[2], 0);
+        const float inv_s = ftd::cload(&g->inv_s, 0);
+        const bool in = __builtin_amdgcn_inverse_ballot_w64(here);
+        const float lim = (a.band + sqrtf(ext2)) * inv_s * (1.0f + 0x1.0p-12f) + 0x1.0p-16f;
+        wave_lds_sync();
+        lds.px[lane] = in ? (c[0] - ox) * inv_s : 0.0f;
+        lds.py[lane] = in ? (c[1] - oy) * inv_s : 0.0f;
+        lds.pz[lane] = in ? (c[2] - oz) * inv_s : 0.0f;
+        lds.thr[lane] = in ? lim * lim : -1.0f;
+        wave_lds_sync();
+#pragma unroll
+        for (int cb = 0; cb < 4; cb++) {
+            const int j = 16 * cb + (lane & 15);
+            const Row r = make_row(lds.px[j], lds.py[j], lds.pz[j], 1.0f);
+            S.B[cb] = ((lane >> 4) & 1) ? r.lo : r.hi;
+            S.thr[cb] = lds.thr[j];
+        }
+        uint32_t c0 = ftd::cload(a.first, root), c1 = ftd::cload(a.first, root + 1);
+        int sp = 0;                                    // list sp: the children of a node
+        for (;;) {
+            uint32_t f0 = c0;
+            uint64_t mask;
+            if (f0 < last) {
+                near |= S.reached(c0, c1 - c0);
+                if (!(here & ~near)) break;
+                mask = 0;
+            } else {
+                mask = S.admitted(c0, c1 - c0, sp);
+            }
+            while (!mask && sp > 0) {                  // back to a list with something left
+                sp--;
+                const uint4 t = lds.stack[sp];
+                f0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)t.x);
+                mask = (uint32_t)__builtin_amdgcn_readfirstlane((int)t.y) |
+                       ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)t.z) << 32);
+            }
+            if (!mask) break;
+            const uint32_t b = (uint32_t)(__ffsll((unsigned long long)mask) - 1);
+            mask &= mask - 1;
+            S.range_of(sp, b, c0, c1);
+            if (lane == 0) lds.stack[sp] = make_uint4(f0, (uint32_t)mask, (uint32_t)(mask >> 32), 0u);
+            sp++;
+        }
+    }
+    const bool reach = tile < n_tiles && ((near >> lane) & 1ull);
+    const bool inside = reach && a.phi_old[a.perm[64 * mine]] < 0.0;   // (a tile's first slot is a node)
+    if (tile < n_tiles) cls[tile] = reach;
+    const uint64_t m2 = __ballot(inside), m1 = __ballot(reach && !inside), below = (1ull << lane) - 1ull;
+    if (!(m1 | m2)) return;
+    uint64_t at = 0;
+    if (lane == 0) at = atomicAdd(count, ((unsigned long long)__popcll(m2) << 32) | (unsigned long long)__popcll(m1));
+    const uint32_t a2 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)), a1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+    if (inside) list[a2 + (uint32_t)__popcll(m2 & below)] = (int32_t)tile;
+    else if (reach) list[n_tiles - 1 - (int64_t)(a1 + (uint32_t)__popcll(m1 & below))] = (int32_t)tile;
+}
+
+// Narrow band: the epilogue of the tiles that no primitive reaches (cls 0), one
+// per wave.
+template <int MODE>
+__global__ __launch_bounds__(kBS) void k_far_tiles(QueryArgs a, const uint32_t* cls)
+{
+    if (halted(a.sc)) return;
+    const int64_t tile = ((int64_t)blockIdx.x * kBS + threadIdx.x) >> 6;
+    if (tile >= a.n_slots / 64 || cls[tile]) return;   // whole wave
+    const int lane = threadIdx.x & 63;
+    const int32_t node = a.perm[tile * 64 + lane];
+    const uint64_t m = __ballot(node >= 0);
+    if (lane == 0) a.clamped[tile] = (uint32_t)__popcll(m);
+    if (node < 0) return;
+    Found F;
+    F.x = F.y = F.z = 0.0f;                            // (of no use without a candidate)
+    F.bkey = F.skey = no_key<MODE>(a);
+    finish_node<MODE>(a, F, node);
+}
+
 // Query schedule of a launch: a persistent grid (as many waves as the device
 // holds, or as there are tiles).  The deep tiles (k_tile_deep) come first, a
 // very deep one (a.split_out) as kSplitParts parts, and wave w starts with
@@ -2230,8 +2402,11 @@ __global__ __launch_bounds__(BS, WPS) void k_query_wave(QueryArgs a)
     bool more_deep = true;                            // some that no wave started with
     uint32_t from = 0;                                // the XCD after this one by `from` has some left
     for (bool first = true;; first = false) {
-        const uint32_t n_tiles = (uint32_t)(a.n_slots / 64);
-        const uint64_t nd = a.tile_list ? ftd::cload(a.n_deep, 0) : 0ull;
+        // in a narrow band only the tiles that a primitive can reach, as they come
+        const uint64_t listed = a.tile_list ? ftd::cload(a.n_deep, 0) : 0ull;
+        const uint32_t inside = (uint32_t)(listed >> 32);
+        const uint32_t n_tiles = a.band > 0.0f ? inside + (uint32_t)listed : (uint32_t)(a.n_slots / 64);
+        const uint64_t nd = a.band > 0.0f ? 0ull : listed;
         const uint32_t K = (uint32_t)nd, cap = (uint32_t)split_tiles_cap(n_tiles);
         const uint32_t K2 = !a.split_out ? 0u : (uint32_t)(nd >> 32) < cap ? (uint32_t)(nd >> 32) : cap;
         const uint32_t D = K2 * kSplitParts + (K - K2);               // deep parts and tiles
@@ -2283,6 +2458,7 @@ __global__ __launch_bounds__(BS, WPS) void k_query_wave(QueryArgs a)
             }
         } else {
             r = K + share.tile(x, k);
+            if (a.band > 0.0f && r >= inside) r = (uint32_t)(a.n_slots / 64) - 1u - (r - inside);   // (k_tile_near)
         }
         // the wave's tile as uniform values
         const int64_t tile = __builtin_amdgcn_readfirstlane(a.tile_list ? a.tile_list[r] : (int)r);
@@ -4812,18 +4988,18 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
     if (c->idx_layout != c->layout_gen)
         return ft::set_error(FT_ERR_STATE, "index grids not set up for this field layout");
     FT_TRY(ensure_stage(c, 3, cp, mode, sp.want_nearest));
-    // Deep tiles first, in a full-domain search (in a narrow band they end
-    // early, clamped).  The schedule reads only phi and the slots: it is
-    // built on the side stream while the index is built here.
+    // Deep tiles first, in a full-domain search.  That schedule reads only phi
+    // and the slots: it is built on the side stream while the index is built
+    // here.  (A narrow band's follows the index, below.)
     const int64_t n_tiles = c->n_slots / 64;
     int32_t* tile_list = nullptr;
+    // tile_sched: classes (u32), the launch order (i32), the scan (u64)
+    uint32_t* cls = c->tile_sched.as<uint32_t>();
+    uint64_t* ex = reinterpret_cast<uint64_t*>(cls + 2 * n_tiles);
+    if (n_tiles > 0) tile_list = reinterpret_cast<int32_t*>(cls + n_tiles);
     if (sp.band <= 0.0f && n_tiles > 0) {
         FT_TRY(side_fork(c, s));
         hipStream_t ss = c->side;
-        // tile_sched: classes (u32), the launch order (i32), the scan (u64)
-        uint32_t* cls = c->tile_sched.as<uint32_t>();
-        tile_list = reinterpret_cast<int32_t*>(cls + n_tiles);
-        uint64_t* ex = reinterpret_cast<uint64_t*>(cls + 2 * n_tiles);
         hipLaunchKernelGGL(k_tile_deep, dim3(grid1d(64 * n_tiles)), dim3(kBS), 0, ss, n_tiles,
                            c->perm.as<int32_t>(), sp.phi_old, c->tile_field.as<int32_t>(),
                            c->d_grids.as<Grid>(), kDeepTile * split_tile_h(n_tiles), split_tile_h(n_tiles), cls, sc);
@@ -4847,6 +5023,7 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
     clr.add(sc + S_BINS, 2, 0u);                       // the bitmap scan writes the low 32 bits
     clr.add(clamped, 2 * nf, 0u);
     clr.add(sc + S_Q, 9 * kQueueLine, 0u);
+    if (sp.band > 0.0f) clr.add(sc + S_DEEP, 2, 0u);
     FT_TRY(set_words(s, clr));
     if (n_cap > 0) {
         hipLaunchKernelGGL(k_prim_bin, dim3(grid1d(n_cap)), dim3(kBS), 0, s, mode, sc, ifp, tris,
@@ -4905,7 +5082,7 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
     q.w_phi = sp.w_phi;
     q.w_ifn = sp.w_ifn;
     // (the schedule's scan, which nothing reads any more)
-    q.clamped = c->tile_sched.as<uint32_t>() + 2 * n_tiles;
+    q.clamped = reinterpret_cast<uint32_t*>(ex);
     static const bool want_stats = getenv("FT_QUERY_STATS") != nullptr;
     q.h_est = c->h_est;
     if (want_stats && eager) {
@@ -4924,10 +5101,19 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
         q.tile_list = tile_list;
         q.n_deep = sc + S_DEEP;
     }
+    if (c->n_slots > 0 && sp.band > 0.0f) {
+        hipLaunchKernelGGL(k_tile_near, dim3(grid1d(n_tiles, 64)), dim3(64), 0, s, q, lp.lo.off[2], cls, tile_list,
+                           (unsigned long long*)(sc + S_DEEP));
+        // the others beside the search of those
+        FT_TRY(side_fork(c, s));
+        hipLaunchKernelGGL(mode == 0 ? k_far_tiles<0> : k_far_tiles<1>, dim3(grid1d(64 * n_tiles)), dim3(kBS), 0,
+                           c->side, q, cls);
+        FT_TRY(check_launch());
+    }
     if (c->n_slots > 0) {
         const int qb = q.stats || sp.query_block == 0 ? 64 : sp.query_block;
         const int wps = mode == 0 ? 6 : sp.waves_per_simd;
-        if (q.tile_list && !sp.whole_tiles) q.split_out = c->deep_part.as<ulonglong2>();
+        if (sp.band <= 0.0f && !sp.whole_tiles) q.split_out = c->deep_part.as<ulonglong2>();
         // as many waves as the device holds at this launch bound (4 SIMDs per
         // CU), or as there may be tiles and parts; whole workgroups
         const int64_t items = n_tiles + (q.split_out ? split_tiles_cap(n_tiles) * (kSplitParts - 1) : 0);
@@ -4936,6 +5122,7 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
         q.queue = reinterpret_cast<uint32_t*>(sc + S_Q);
         FT_TRY(launch_query(mode, qb, wps, g, b, s, q));
         if (sp.band > 0.0f) {
+            FT_TRY(side_join(c, s));
             hipLaunchKernelGGL(k_clamp_sum, dim3(grid1d((n_tiles + kClampRun - 1) / kClampRun * 64)), dim3(kBS), 0, s,
                                n_tiles, q.clamped, q.tile_field, reinterpret_cast<unsigned long long*>(clamped), sc);
             FT_TRY(check_launch());

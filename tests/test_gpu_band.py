@@ -35,3 +35,29 @@ def test_clamped_nodes_are_those_without_a_nearest(mode, sizes):
     assert np.array_equal(inside[sure], ~none[sure])
     assert np.array_equal(ifn[inside].view(np.uint64), full[inside].view(np.uint64))
     r.close()
+
+
+@pytest.mark.parametrize("mode", ["points", "triangles"])
+@pytest.mark.parametrize("n,bin_scale,band_h", [(5, 1e6, 1.0), (9, 0.0, 0.2), (33, 0.0, 0.7), (33, 0.0, 100.0), (68, 0.5, 4.0),
+                                                (68, 0.0, 9.0), ((130, 7, 5), 0.0, 3.0)])
+def test_tiles_left_out_have_no_primitive_in_the_band(mode, n, bin_scale, band_h):
+    """Tiles are left out whole, by boxes above the leaves: from one-leaf trees to
+    three levels, bands below a spacing to the whole field."""
+    dims = (n, n, n) if np.isscalar(n) else n
+    h = 1.0 / (max(dims) - 1)
+    m = fa.kuhn_mesh(dims, spacing=h, jitter=0.2, seed=3)
+    mid = 0.5 * h * (np.array(dims) - 1)
+    phi = np.linalg.norm((m.xyz - mid) / (mid + h), axis=1) - 0.55
+    band = band_h * h
+    with fa.Reinit(0) as r:
+        r.set_mesh(m)
+        _, full, _ = r.reset_phi(phi, mode=mode, bin_scale=bin_scale)
+        out, ifn, cnt = r.reset_phi(phi, mode=mode, bin_scale=bin_scale, band=band, want_nearest=True)
+        none = r.nearest() == -1
+        again, _, _ = r.reset_phi(phi, mode=mode, bin_scale=bin_scale, band=band, schedule="queue", query_block=256)
+    assert np.array_equal(out.view(np.uint64), again.view(np.uint64))
+    sure = np.abs(np.abs(full) / band - 1) > 1e-5          # (rounding decides at the band's edge)
+    inside = (np.abs(full) < band) & sure
+    assert np.array_equal(inside[sure], ~none[sure]) and cnt.n_clamped == none.sum()
+    assert np.array_equal(ifn[inside].view(np.uint64), full[inside].view(np.uint64))
+    assert np.array_equal(np.abs(ifn[none]), np.full(none.sum(), np.float64(np.float32(band))))

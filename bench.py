@@ -133,9 +133,9 @@ def run_advect(args):
     nnz = int(row_off[-1])
     log(f"advect {n}^3: {ms:.3f} ms per step, {np.mean(its):.1f} BiCGSTAB iterations, "
         f"error {info.error:.3g}, nnz {nnz}")
-    # per iteration: two SpMVs (8 B value + 4 B column per entry) and the
-    # vector passes (p 32, v 32, t 32, x/r 72 bytes per row)
-    it_bytes = 24 * nnz + 168 * N
+    # per iteration: two SpMVs (8 B value per entry; columns as diagonals and a
+    # mask, 6 B per row) and the vector passes (p 32, v 32, t 32, x/r 72 bytes per row)
+    it_bytes = 16 * nnz + 180 * N
     cpu = None
     if not args.no_cpu:
         import oracle
@@ -731,12 +731,12 @@ def _read_counters(dirpath):
     return rows
 
 
-def live_counters(args, N, q_ms, out_root):
+def live_counters(args, N, E, q_ms, out_root):
     """rocprofv3 counter passes of one reinit of this workload (a child run of
     this script per pass, `--profile-child`): FETCH_SIZE, WRITE_SIZE and the
     instruction counts of the query kernel, scaled by what the same counters
     read for k_node_signs, whose traffic is known (it reads 8 B of phi per
-    node and writes 1 bit per node)."""
+    node, writes 2 bits per node and clears 1 bit per edge)."""
     import shutil
     import subprocess
     prof = shutil.which("rocprofv3")
@@ -780,11 +780,11 @@ def live_counters(args, N, q_ms, out_root):
     if None in (fetch_raw, write_raw, sig_f, sig_w):
         return {"status": "counters missing from the rocprofv3 output", "commands": cmds}
     f_scale = 8.0 * N / (sig_f * 1024.0)
-    w_scale = (N / 8.0) / (sig_w * 1024.0)
+    w_scale = (N / 4.0 + E / 8.0) / (sig_w * 1024.0)
     traffic = fetch_raw * 1024.0 * f_scale + write_raw * 1024.0 * w_scale
     res = {"status": "ok", "traffic_bytes": traffic, "fetch_kib_raw": fetch_raw, "write_kib_raw": write_raw,
            "fetch_scale": f_scale, "write_scale": w_scale,
-           "calibration": "k_node_signs: reads 8 B/node of phi, writes 1 bit/node", "commands": cmds}
+           "calibration": "k_node_signs: reads 8 B/node of phi, writes 2 bits/node and 1 bit/edge", "commands": cmds}
     waves = last(got["sq"], qk, "SQ_WAVES")
     valu = last(got["sq"], qk, "SQ_INSTS_VALU")
     if waves and valu:
@@ -1018,7 +1018,7 @@ def main():
         # folder (the JSON line carries what they say)
         import tempfile
         out_root = os.environ.get("FT_BENCH_PROFILE_DIR") or tempfile.mkdtemp(prefix="ft_bench_counters_")
-        counters = live_counters(args, N, ph[2], out_root)
+        counters = live_counters(args, N, len(m.edges), ph[2], out_root)
         log(f"counters: { {k: v for k, v in counters.items() if k != 'commands'} }")
 
     # The CPU leg: the oracle on the host, as the reference CPU path's timed

@@ -1783,8 +1783,8 @@ __device__ __forceinline__ void wave_lds_sync()
 // its rounding: scaled coordinates are good to 2^-20 along each axis, so the
 // bound is (sqrt(best) + 2^-19)^2; results are the exact search's.
 //
-// What bounds it: vector issue (79% of its rate at 256^3: 11.1k vector
-// instructions per tile, 205k matrix ones in all).  256^3, 64 spheres, full
+// What bounds it: vector issue (76-80% of its rate at 256^3: 12.0k vector
+// instructions per tile).  256^3, 64 spheres, full
 // domain: 6.1 ms, against 9.1-9.5 ms for a wave-wide walk of a binary tree that
 // tested every box and triangle on all 64 lanes (19.9k instructions per tile);
 // crossing points 3.2 against 3.9 ms.

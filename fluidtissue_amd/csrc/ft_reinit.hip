@@ -2109,8 +2109,11 @@ struct TileSearch {
         }
         wave_lds_sync();
         if (s0 == s1) return;
-        float t = INFINITY;
+        // a lane past the leaf loses to any of its primitives, also to one whose
+        // distance is not a number (its bits are above infinity's)
+        uint32_t key = ~0u;
         if (s0 + lane < s1) {
+            float t;
             if (MODE == 1) {
                 t = box_of(a.titem[s0 + lane], x, y, z);
             } else {
@@ -2118,8 +2121,10 @@ struct TileSearch {
                 const float dx = (r.x - cen[0]) * inv_s, dy = (r.y - cen[1]) * inv_s, dz = (r.z - cen[2]) * inv_s;
                 t = __fmaf_rn(dx, dx, __fmaf_rn(dy, dy, dz * dz));
             }
+            const uint32_t inf = 0x7f800000u, u = __float_as_uint(t);
+            key = ((u < inf ? u : inf) & ~63u) | (uint32_t)lane;
         }
-        slot = s0 + (wave_min_u32((__float_as_uint(t) & ~63u) | (uint32_t)lane) & 63u);
+        slot = s0 + (wave_min_u32(key) & 63u);
     }
 
     // The leaves of node g; part of parts: only leaves l % parts == part.

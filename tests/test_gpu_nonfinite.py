@@ -1,0 +1,60 @@
+"""GPU: crossing points that are not finite are nobody's nearest, and what is
+not finite changes nothing for the rest."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import fluidtissue_amd as fa
+from fluidtissue_amd._lib import check, lib
+
+pytestmark = pytest.mark.gpu
+
+FLT_MAX = float(np.finfo(np.float32).max)
+
+
+@pytest.mark.parametrize("n_bad", [1, 3, 17, 63, 64, 65, 200])
+def test_only_nan_points_after_a_larger_call(n_bad):
+    """A leaf of NaN points alone, where the call before left its points."""
+    m = fa.kuhn_mesh(16, jitter=0.1, seed=3)
+    rng = np.random.default_rng(6)
+    phi = rng.standard_normal(m.n_nodes)
+    with fa.EuclideanDistance(0) as d:
+        d.init(m.xyz)
+        good = rng.random((300, 3)).astype(np.float32)
+        d.reset_phi(good, len(good), phi.copy())
+        got = phi.copy()
+        d.reset_phi(np.full((n_bad, 3), np.nan, np.float32), n_bad, got)
+        near = np.empty(m.n_nodes, np.int32)
+        check(lib.ft_get_nearest(d._h, near.ctypes.data_as(C.c_void_p)))
+    assert np.array_equal(got, np.where(phi < 0, -FLT_MAX, FLT_MAX))
+    assert np.all(near == -1)
+
+
+@pytest.mark.parametrize("mode", ["points", "triangles"])
+def test_field_with_only_nan_points_in_a_batch(mode):
+    """phi infinite on both sides of every crossing edge: the field's points are
+    NaN, and the next field's are not its own."""
+    small, big = fa.kuhn_mesh(2), fa.kuhn_mesh(12, jitter=0.1, seed=4)
+    bad = np.full(small.n_nodes, np.inf)
+    bad[0] = -np.inf
+    fine = fa.phi_field("ellipsoids", big.xyz, seed=2)
+    with fa.Reinit(0) as r:
+        r.set_mesh(big)
+        alone, _, _ = r.reset_phi(fine, mode=mode, want_nearest=True)
+        near_alone = r.nearest()
+    for first in (True, False):
+        meshes, phis = ([small, big], [bad, fine]) if first else ([big, small], [fine, bad])
+        with fa.Reinit(0) as r:
+            r.set_batch(meshes)
+            off, _, _ = r.batch_info()
+            out, _, _ = r.reset_phi(np.concatenate(phis), mode=mode, want_nearest=True)
+            near = r.nearest()
+            cnt = r.field_counts()
+        k = 0 if first else 1
+        b, f = slice(off[k], off[k + 1]), slice(off[1 - k], off[2 - k])
+        assert cnt[k].n_ifp > 0
+        assert np.array_equal(out[b], np.where(bad < 0, -FLT_MAX, FLT_MAX)) and np.all(near[b] == -1)
+        assert np.array_equal(out[f].view(np.uint64), alone.view(np.uint64))
+        before = cnt[k].n_ifp if mode == "points" else cnt[k].n_tri
+        assert np.array_equal(near[f], near_alone + (before if first else 0))

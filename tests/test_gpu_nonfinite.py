@@ -1,11 +1,12 @@
-"""GPU: crossing points that are not finite are nobody's nearest, and what is
-not finite changes nothing for the rest."""
+"""GPU: crossing points and nodes that are not finite: such points are nobody's
+nearest, such nodes have none, and neither changes anything for the rest."""
 import ctypes as C
 
 import numpy as np
 import pytest
 
 import fluidtissue_amd as fa
+import oracle
 from fluidtissue_amd._lib import check, lib
 
 pytestmark = pytest.mark.gpu
@@ -58,3 +59,45 @@ def test_field_with_only_nan_points_in_a_batch(mode):
         assert np.array_equal(out[f].view(np.uint64), alone.view(np.uint64))
         before = cnt[k].n_ifp if mode == "points" else cnt[k].n_tri
         assert np.array_equal(near[f], near_alone + (before if first else 0))
+
+
+@pytest.mark.parametrize("share", [0.002, 0.3, 0.97])
+def test_nan_nodes_beside_others(share):
+    """Nodes with a NaN coordinate share tiles with finite ones, as their first,
+    last or most nodes."""
+    m = fa.kuhn_mesh(17, jitter=0.1, seed=5)
+    rng = np.random.default_rng(8)
+    xyz = m.xyz.copy()
+    bad = rng.random(len(xyz)) < share
+    bad[:8] = True                                    # among the first nodes of the first tiles
+    xyz[bad, rng.integers(0, 3, bad.sum())] = np.nan
+    ifp = rng.random((700, 3)).astype(np.float32)
+    phi = rng.standard_normal(len(xyz))
+    ref = oracle.reset_phi_points(xyz, ifp, phi.copy())
+    ref = ref[0] if isinstance(ref, tuple) else ref
+    with fa.EuclideanDistance(0) as d:
+        d.init(xyz)
+        got = phi.copy()
+        d.reset_phi(ifp, len(ifp), got)
+    assert np.array_equal(got.view(np.uint64), ref.view(np.uint64))
+    assert np.all(np.abs(got[bad]) == FLT_MAX) and np.all(np.abs(got[~bad]) < 2)
+
+
+@pytest.mark.parametrize("mode", ["points", "triangles"])
+@pytest.mark.parametrize("band", [0.0, 0.2])
+def test_nan_nodes_away_from_the_interface(mode, band):
+    m = fa.kuhn_mesh(18, jitter=0.1, seed=6)
+    phi = np.linalg.norm(m.xyz.astype(np.float64) - 0.5, axis=1) - 0.2
+    bad = np.zeros(m.n_nodes, bool)
+    bad[[0, 3, 17, 40, 324, m.n_nodes - 1]] = True    # of tets that do not cross
+    hurt = fa.Mesh(xyz=np.where(bad[:, None], np.float32(np.nan), m.xyz), tets=m.tets, edges=m.edges, t2e=m.t2e)
+    res = []
+    for mesh in (m, hurt):
+        with fa.Reinit(0) as r:
+            r.set_mesh(mesh)
+            out, ifn, _ = r.reset_phi(phi, mode=mode, blend="update", band=band, want_nearest=True)
+            res.append((out, ifn, r.nearest()))
+    (o1, i1, n1), (o2, i2, n2) = res
+    assert np.array_equal(o1[~bad].view(np.uint64), o2[~bad].view(np.uint64))
+    assert np.array_equal(i1[~bad].view(np.uint64), i2[~bad].view(np.uint64))
+    assert np.array_equal(n1[~bad], n2[~bad]) and np.all(n2[bad] == -1)

@@ -4199,11 +4199,15 @@ Grid make_grid(const FieldHost& f, float edge, int max_lg, int* lg_out)
     g.h = f.h;
     // scaled coordinates: about the box's middle, in units of a power of two
     // of at least twice its longest side (scaling rounds nothing; the field
-    // and what lies within half a side of it stay within one unit)
+    // and what lies within half a side of it stay within one unit).  A box
+    // without a finite size (a node that is not finite, or sides beyond
+    // FLT_MAX): about 0, in the largest unit, in which every finite coordinate
+    // stays below 4; the units' reciprocal is a normal number.
+    const bool sized = ext_max <= FLT_MAX;
     int ex = 0;
-    (void)std::frexp(std::min(std::max(ext_max, 1e-30f), 1e30f), &ex);   // ext_max < 2^ex
-    for (int k = 0; k < 3; k++) g.org[k] = f.lo[k] + 0.5f * (f.hi[k] - f.lo[k]);
-    g.inv_s = std::ldexp(1.0f, -(ex + 1));
+    (void)std::frexp(sized ? std::max(ext_max, 1e-30f) : FLT_MAX, &ex);   // ext_max < 2^ex
+    for (int k = 0; k < 3; k++) g.org[k] = sized ? f.lo[k] + 0.5f * (f.hi[k] - f.lo[k]) : 0.0f;
+    g.inv_s = std::ldexp(1.0f, -std::min(ex + 1, 126));
     g.root_lv = std::max(1, (lg + 1) / 2);
     *lg_out = lg;
     return g;

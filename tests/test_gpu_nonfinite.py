@@ -101,3 +101,24 @@ def test_nan_nodes_away_from_the_interface(mode, band):
     assert np.array_equal(o1[~bad].view(np.uint64), o2[~bad].view(np.uint64))
     assert np.array_equal(i1[~bad].view(np.uint64), i2[~bad].view(np.uint64))
     assert np.array_equal(n1[~bad], n2[~bad]) and np.all(n2[bad] == -1)
+
+
+@pytest.mark.parametrize("mode", ["points", "triangles"])
+@pytest.mark.parametrize("band", [0.0, 0.2])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, 3e38])
+def test_box_without_a_size(mode, band, value):
+    """A node at infinity, or two so far apart that their difference is: the
+    others' results are those of the mesh without."""
+    m = fa.kuhn_mesh(14, jitter=0.1, seed=7)
+    phi = np.linalg.norm(m.xyz.astype(np.float64) - 0.5, axis=1) - 0.2
+    far = np.array([m.n_nodes - 1, 0] if np.isfinite(value) else [m.n_nodes - 1])   # of tets that do not cross
+    xyz = m.xyz.copy()
+    xyz[far, 1] = value * np.array([1, -1])[:len(far)]
+    res = []
+    for mesh in (m, fa.Mesh(xyz=xyz, tets=m.tets, edges=m.edges, t2e=m.t2e)):
+        with fa.Reinit(0) as r:
+            r.set_mesh(mesh)
+            out, ifn, _ = r.reset_phi(phi, mode=mode, band=band, want_nearest=True)
+            res.append((np.delete(ifn, far), np.delete(r.nearest(), far)))
+    assert np.array_equal(res[0][0].view(np.uint64), res[1][0].view(np.uint64))
+    assert np.array_equal(res[0][1], res[1][1])

@@ -1176,6 +1176,7 @@ __global__ __launch_bounds__(kBS) void k_prim_scatter(int mode, const uint64_t* 
                       lbc > 0.0 ? (float)(1.0 / lbc) : 0.0f,
                       __int_as_float((int32_t)j | (interior ? 0 : INT32_MIN)));
     trec[slot] = r;
+    if (!titem) return;
     // The rectangle [0, L0] x [0, Cy] of the frame holds the triangle: ab is
     // the longest edge, so C projects inside [0, L0], and Cy >= 0.
     const Grid& g = ig.grids[bin_field(ig, leaf_bin[l])];
@@ -1473,8 +1474,8 @@ struct QueryArgs {
     const Item* items;               // boxes of the same
     uint32_t leaf_end;               // indices below are leaves
     const float4* prec;              // point records (mode 0): coordinates, id
-    const Item* titem;               // triangles' frames and rectangles (mode 1)
-    const TriRec* trec;              // their other constants
+    const Item* titem;               // triangles' frames and rectangles (mode 1; null: from the records)
+    const TriRec* trec;              // their records
     float band;                      // > 0: narrow band
     const float* ifp;
     const int4* tris;
@@ -1779,6 +1780,9 @@ __device__ __forceinline__ void wave_lds_sync()
 //    before the walk, and with bounds that good the order of the walk is
 //    worth 4% (in a model of the traversal at 256^3; without that first
 //    search the walk takes twice the boxes and triangles).
+//  - RECORDS: the triangles' rectangles are formed from their records where
+//    they are read, instead of from items of their own (64 bytes a triangle):
+//    for an allocation-free call whose scratch cannot take both.
 // Every cut is a lower bound compared with the node's best so far raised by
 // its rounding: scaled coordinates are good to 2^-20 along each axis, so the
 // bound is (sqrt(best) + 2^-19)^2; results are the exact search's.
@@ -1788,7 +1792,7 @@ __device__ __forceinline__ void wave_lds_sync()
 // domain: 6.1 ms, against 9.1-9.5 ms for a wave-wide walk of a binary tree that
 // tested every box and triangle on all 64 lanes (19.9k instructions per tile);
 // crossing points 3.2 against 3.9 ms.
-template <int MODE, bool STATS>
+template <int MODE, bool STATS, bool RECORDS = false>
 struct TileSearch {
     const QueryArgs& a;
     WaveLds<MODE>& lds;
@@ -1799,6 +1803,7 @@ struct TileSearch {
     float inv_s;
     float cen[3], pp = 0.0f;                  // tile centre; points: |p - cen|^2 of the lane's node, lowered
     float rel[MODE == 0 ? 4 : 1];             // points: operand about the centre
+    float org[RECORDS ? 3 : 1];               // origin of the scaled coordinates
     TileStats st;
 
     __device__ __forceinline__ TileSearch(const QueryArgs& q, WaveLds<MODE>& l, int ln) : a(q), lds(l), lane(ln) {}
@@ -1887,6 +1892,31 @@ struct TileSearch {
         const v4h* f = reinterpret_cast<const v4h*>(it);       // 8 per item: a row's hi and lo in turn
         av = f[(uint32_t)(((lane & 15) >> 2) * 8 + (lane & 3) * 2 + (lane >> 5))];
         e = *reinterpret_cast<const E*>(f + (uint32_t)((lane >> 4) * 8 + 6));
+    }
+
+    // The same of the triangles in slots s to s + 3, of which `left` are the
+    // leaf's (the rest as its last).  A rectangle's offsets formed in FP32 are
+    // good to 2^-22 of a scaled unit, beside the product's 2^-22.8, of the 2^-20
+    // that the bounds allow.
+    __device__ __forceinline__ void load_tris(uint32_t s, uint32_t left, int lane, v4h& av, float2& e) const
+    {
+        if (!RECORDS) {
+            load4(a.titem + s, lane, av, e);
+            return;
+        }
+        const float4* r = reinterpret_cast<const float4*>(a.trec + s);          // 5 per record: a, u, v, n, i
+        auto record = [&](int k) { return r + 5u * ((uint32_t)k < left ? (uint32_t)k : left - 1u); };
+        const float4* t = record((lane & 15) >> 2);
+        const int j = lane & 3;                                // row u, v or n (the fourth is a spare one)
+        const float4 o = t[0], x = t[j < 2 ? 1 + j : 3];
+        const float half = j == 0 ? 0.5f * x.w : j == 1 ? 0.5f * t[3].w : 0.0f;
+        const float dx = o.x - org[0], dy = o.y - org[1], dz = o.z - org[2];
+        const float w = -(__fmaf_rn(dz, x.z, __fmaf_rn(dy, x.y, dx * x.x)) + half) * inv_s;
+        const Row row = make_row(x.x, x.y, x.z, w);
+        av = lane < 32 ? row.hi : row.lo;
+        const float4* b = record(lane >> 4);
+        const float up = 0.5f * inv_s * (1.0f + 0x1.0p-20f);
+        e = make_float2(b[1].w * up, b[3].w * up);
     }
 
     // Which of the children [c0, c0 + cnt), cnt <= 64, some node admits; their
@@ -1984,13 +2014,13 @@ struct TileSearch {
         if (MODE == 1) {
             v4h av;
             float2 e;
-            load4(a.titem + s, lane, av, e);
+            load_tris(s, s1 - s, lane, av, e);
             for (;;) {
                 uint32_t ns = s + 4, ns1 = s1;
                 const bool more = ns < s1 || next_leaf(mask, d, ns, ns1);
                 v4h av1 = av;
                 float2 e1 = e;
-                if (more) load4(a.titem + ns, lane, av1, e1);
+                if (more) load_tris(ns, ns1 - ns, lane, av1, e1);
                 uint64_t m[4];
                 cull4(av, e, s1 - s, m);
                 if ((m[0] | m[1]) | (m[2] | m[3])) {
@@ -2114,7 +2144,9 @@ struct TileSearch {
         uint32_t key = ~0u;
         if (s0 + lane < s1) {
             float t;
-            if (MODE == 1) {
+            if (RECORDS) {
+                t = ftd::tri_dist2(cen[0], cen[1], cen[2], a.trec[s0 + lane]);
+            } else if (MODE == 1) {
                 t = box_of(a.titem[s0 + lane], x, y, z);
             } else {
                 const float4 r = a.prec[s0 + lane];
@@ -2190,14 +2222,14 @@ __device__ __forceinline__ uint64_t no_key(const QueryArgs& a)
 // A wave's tile: 64 consecutive slots of one field in Morton order.
 // split >= 0: part split % kSplitParts of split tile split / kSplitParts,
 // whose best and second keys go to a.split_out instead of the epilogue.
-template <int MODE, bool STATS>
+template <int MODE, bool STATS, bool RECORDS>
 __device__ __forceinline__ void search_tile(const QueryArgs& a, int64_t base, WaveLds<MODE>& lds, int split = -1)
 {
     // opaque to the compiler, which would else hoist everything that depends on
     // the lane alone out of the work queue's loop, and spill it
     int lane = ftd::lane_id();
     asm volatile("" : "+v"(lane));
-    TileSearch<MODE, STATS> S(a, lds, lane);
+    TileSearch<MODE, STATS, RECORDS> S(a, lds, lane);
     const int64_t slot = base + lane;
     const int32_t node = a.perm[slot];                 // -1: padding lane
     Found F;
@@ -2210,6 +2242,11 @@ __device__ __forceinline__ void search_tile(const QueryArgs& a, int64_t base, Wa
         const Grid* g = a.grids + field;
         const float ox = ftd::cload(&g->org[0], 0), oy = ftd::cload(&g->org[1], 0), oz = ftd::cload(&g->org[2], 0);
         S.inv_s = ftd::cload(&g->inv_s, 0);
+        if (RECORDS) {
+            S.org[0] = ox;
+            S.org[1] = oy;
+            S.org[2] = oz;
+        }
         wave_lds_sync();                               // the wave's last tile is done with its LDS
         lds.px[lane] = F.x;
         lds.py[lane] = F.y;
@@ -2440,7 +2477,7 @@ __global__ __launch_bounds__(kBS) void k_far_tiles(QueryArgs a, const uint32_t* 
 // 6.10 / 6.33 ms at 5 / 6 / 7, points 3.57 / 3.20 / 3.31; the wave's LDS allows
 // seven.  One wave per workgroup: with four, a workgroup's place is held by its
 // slowest wave (256^3: 8.8 ms).
-template <int MODE, int BS, int WPS, bool STATS = false>
+template <int MODE, int BS, int WPS, bool STATS = false, bool RECORDS = false>
 __global__ __launch_bounds__(BS, WPS) void k_query_wave(QueryArgs a)
 {
     constexpr uint32_t wpb = BS / 64;
@@ -2510,7 +2547,7 @@ __global__ __launch_bounds__(BS, WPS) void k_query_wave(QueryArgs a)
         }
         // the wave's tile as uniform values
         const int64_t tile = __builtin_amdgcn_readfirstlane(a.tile_list ? a.tile_list[r] : (int)r);
-        search_tile<MODE, STATS>(a, tile * 64, wlds[w], __builtin_amdgcn_readfirstlane(split));
+        search_tile<MODE, STATS, RECORDS>(a, tile * 64, wlds[w], __builtin_amdgcn_readfirstlane(split));
     }
 }
 
@@ -4133,6 +4170,12 @@ int ensure(DevBuf& b, size_t bytes)
     return FT_OK;
 }
 
+// Whether ensure(b, bytes) would have the memory.
+bool has_room(const DevBuf& b, size_t bytes)
+{
+    return !t_arena || bytes <= b.cap || t_arena->used + ((bytes + 255) & ~(size_t)255) <= t_arena->size;
+}
+
 void release(DevBuf& b)
 {
     if (b.p && !t_arena) (void)hipFree(b.p);
@@ -4639,6 +4682,20 @@ LevelPlan level_plan(const ft_ctx* c, int64_t n)
     return p;
 }
 
+// The primitives' bins (later leaves) and places while the index is built: in
+// the crossing tets' edges, which nothing reads once the triangles are made,
+// where those are large enough (two entries a primitive; a tet has 16 bytes
+// and at most two triangles).
+struct PrimWork {
+    uint32_t *code, *place;
+};
+bool prim_work_in_xedges(const ft_ctx* c, int64_t n) { return 2 * sizeof(uint32_t) * (size_t)n <= c->xedges.cap; }
+PrimWork prim_work(const ft_ctx* c, int64_t n)
+{
+    if (!prim_work_in_xedges(c, n)) return {c->pcode.as<uint32_t>(), c->place.as<uint32_t>()};
+    return {c->xedges.as<uint32_t>(), c->xedges.as<uint32_t>() + n};
+}
+
 // Device buffers of the stages of one reinit.  Stage 0: sized by the mesh;
 // 1: by crossing tets and triangles; 2: by crossing points; 3: the index over
 // n primitives (leaves <= min(bins, n)).
@@ -4694,15 +4751,13 @@ int ensure_stage(ft_ctx* c, int stage, const Caps& cp, int mode, bool want_neare
                                  t_arena->size);
         FT_TRY(ensure(c->bbits, 8 * at_least1(W)));
         FT_TRY(ensure(c->bprefix, 4 * at_least1(W)));
-        FT_TRY(ensure(c->pcode, sizeof(uint32_t) * at_least1(n)));
-        FT_TRY(ensure(c->place, sizeof(uint32_t) * at_least1(n)));
-        FT_TRY(ensure(c->pidx, sizeof(int32_t) * at_least1(n)));
-        if (mode == 0) {
-            FT_TRY(ensure(c->prec, sizeof(float4) * at_least1(n)));
-        } else {
-            FT_TRY(ensure(c->titem, sizeof(Item) * (n + 4)));        // the search reads items by fours
-            FT_TRY(ensure(c->trec, sizeof(TriRec) * at_least1(n)));
+        if (!prim_work_in_xedges(c, n)) {
+            FT_TRY(ensure(c->pcode, sizeof(uint32_t) * at_least1(n)));
+            FT_TRY(ensure(c->place, sizeof(uint32_t) * at_least1(n)));
         }
+        FT_TRY(ensure(c->pidx, sizeof(int32_t) * at_least1(n)));
+        if (mode == 0) FT_TRY(ensure(c->prec, sizeof(float4) * at_least1(n)));
+        else FT_TRY(ensure(c->trec, sizeof(TriRec) * at_least1(n)));
         FT_TRY(ensure(c->leaf_cnt, sizeof(uint32_t) * at_least1(lp.cap[0])));
         FT_TRY(ensure(c->leaf_bin, sizeof(uint32_t) * at_least1(lp.cap[0])));
         FT_TRY(ensure(c->nfirst, sizeof(uint32_t) * (lp.total + 64)));   // (read a wave at a time)
@@ -4713,6 +4768,12 @@ int ensure_stage(ft_ctx* c, int stage, const Caps& cp, int mode, bool want_neare
                                      3 * scan_blocks(lp.cap[0])});
         FT_TRY(ensure(c->scan_bsum, sizeof(uint64_t) * nb));
         FT_TRY(ensure(c->deep_part, sizeof(ulonglong2) * 64 * kSplitParts * at_least1(split_tiles_cap(c->n_slots / 64))));
+        // last, as the search does without them when the scratch has no room
+        // (a dense interface in large bins: 128^3 at 4 bin edges and 0.6M
+        // triangles take 152 MiB with them and 117 without)
+        const size_t titems = sizeof(Item) * (size_t)(n + 4);        // the search reads items by fours
+        if (mode == 1 && !has_room(c->titem, titems)) c->titem = DevBuf{};
+        else if (mode == 1) FT_TRY(ensure(c->titem, titems));
     }
     return FT_OK;
 }
@@ -5009,6 +5070,10 @@ int launch_query_bs(int wps, dim3 g, dim3 b, hipStream_t s, const QueryArgs& q)
 
 int launch_query(int mode, int qb, int wps, dim3 g, dim3 b, hipStream_t s, const QueryArgs& q)
 {
+    if (mode == 1 && !q.titem) {                      // (qb is 64)
+        hipLaunchKernelGGL((k_query_wave<1, 64, 6, false, true>), g, b, 0, s, q);
+        return check_launch();
+    }
     if (q.stats) {                                    // counting build (qb is 64)
         if (mode == 0) hipLaunchKernelGGL((k_query_wave<0, 64, 5, true>), g, b, 0, s, q);
         else hipLaunchKernelGGL((k_query_wave<1, 64, 5, true>), g, b, 0, s, q);
@@ -5066,7 +5131,7 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
     uint32_t* lcnt = c->leaf_cnt.as<uint32_t>();
     uint32_t* lbin = c->leaf_bin.as<uint32_t>();
     uint32_t* first = c->nfirst.as<uint32_t>();
-    uint32_t* code = c->pcode.as<uint32_t>();
+    const PrimWork work = prim_work(c, n_cap);
     uint64_t* clamped = nf == 1 ? sc + S_CLAMP : c->fclamp.as<uint64_t>();
     WordRanges clr;
     clr.add(bits, 2 * W, 0u);
@@ -5079,11 +5144,11 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
     FT_TRY(set_words(s, clr));
     if (n_cap > 0) {
         hipLaunchKernelGGL(k_prim_bin, dim3(grid1d(n_cap)), dim3(kBS), 0, s, mode, sc, ifp, tris,
-                           nf > 1 ? c->ifp2e.as<int32_t>() : nullptr, ig, code, (unsigned long long*)bits);
+                           nf > 1 ? c->ifp2e.as<int32_t>() : nullptr, ig, work.code, (unsigned long long*)bits);
         FT_TRY(scan<uint64_t, uint32_t>(c, s, bits, c->bprefix.as<uint32_t>(), W,
                                         reinterpret_cast<uint32_t*>(sc + S_BINS), LoadPopc{}));
         hipLaunchKernelGGL(k_prim_rank, dim3(grid1d(n_cap)), dim3(kBS), 0, s, mode, sc, bits,
-                           c->bprefix.as<uint32_t>(), code, c->place.as<uint32_t>(), lcnt, lbin);
+                           c->bprefix.as<uint32_t>(), work.code, work.place, lcnt, lbin);
         if (lp.cap[0] <= kLevelOne) {
             hipLaunchKernelGGL(k_level_one, dim3(1), dim3(1024), 0, s, sc, lcnt, lbin, ig, lp.lo, first,
                                c->roots.as<uint32_t>());
@@ -5096,8 +5161,8 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
             hipLaunchKernelGGL(k_level_down, dim3((unsigned)nb), dim3(kBS), 0, s, sc, lcnt, lbin, ig, bs, lp.lo, first,
                                c->roots.as<uint32_t>());
         }
-        hipLaunchKernelGGL(k_prim_scatter, dim3(grid1d(n_cap)), dim3(kBS), 0, s, mode, sc, ifp, tris, code,
-                           c->place.as<uint32_t>(), first, lbin, ig, c->prec.as<float4>(), c->titem.as<Item>(),
+        hipLaunchKernelGGL(k_prim_scatter, dim3(grid1d(n_cap)), dim3(kBS), 0, s, mode, sc, ifp, tris, work.code,
+                           work.place, first, lbin, ig, c->prec.as<float4>(), c->titem.as<Item>(),
                            c->trec.as<TriRec>(), c->pidx.as<int32_t>());
         hipLaunchKernelGGL(mode == 0 ? k_leaf_items<0> : k_leaf_items<1>, dim3(grid1d(kLeafLanes * lp.cap[0])),
                            dim3(kBS), 0, s, sc, first, lbin, ig, c->pidx.as<int32_t>(), ifp, tris,
@@ -5163,8 +5228,9 @@ int enqueue_search(ft_ctx* c, hipStream_t s, const SearchSpec& sp, const Caps& c
         FT_TRY(check_launch());
     }
     if (c->n_slots > 0) {
-        const int qb = q.stats || sp.query_block == 0 ? 64 : sp.query_block;
-        const int wps = mode == 0 ? 6 : sp.waves_per_simd;
+        const bool records = mode == 1 && !q.titem;
+        const int qb = q.stats || records || sp.query_block == 0 ? 64 : sp.query_block;
+        const int wps = mode == 0 || records ? 6 : sp.waves_per_simd;
         if (sp.band <= 0.0f && !sp.whole_tiles) q.split_out = c->deep_part.as<ulonglong2>();
         // as many waves as the device holds at this launch bound (4 SIMDs per
         // CU), or as there may be tiles and parts; whole workgroups

@@ -102,3 +102,34 @@ def test_noalloc_rejects_outputs_it_cannot_keep():
     rc = lib.ft_reinit_device_noalloc(r._h, C.c_void_p(d.data_ptr()), None, C.byref(o), C.byref(cnt), None)
     assert rc == _lib.FT_ERR_ARG
     r.close()
+
+
+@pytest.mark.parametrize("n,period,noise,bin_scale", [(56, 0.14, 0.02, 2.0), (56, 0.2, 0.03, 4.0), (64, 0.2, 0.02, 4.0),
+                                                        (64, 0.0, 0.01, 2.0)])
+@pytest.mark.parametrize("band", [0.0, 0.03])
+def test_noalloc_takes_dense_interfaces(n, period, noise, bin_scale, band):
+    """Interfaces of 0.7M triangles and more in large bins: their 105 to 122 MiB
+    are within the scratch only without the triangles' boxes (64 bytes each),
+    which the search then forms from their records.  The last field is dense
+    in two fifths of the domain and deep inside in the rest."""
+    import torch
+    m = fa.kuhn_mesh(n, jitter=0.2, seed=1)
+    x = m.xyz.astype(np.float64)
+    rough = noise * np.random.default_rng(1).standard_normal(len(x))
+    phi = (np.sin(2 * np.pi * x / period).sum(1) * period / 6 + rough if period else
+           np.where(x[:, 0] < 0.4, rough, 0.39 - x[:, 0]))
+    res = []
+    with fa.Reinit(0) as r:
+        r.set_mesh(m)
+        for fn in (r.reset_phi_device_noalloc, r.reset_phi_device):
+            d = torch.from_numpy(phi).cuda()
+            di = torch.empty_like(d)
+            torch.cuda.synchronize()
+            c = fn(d.data_ptr(), di.data_ptr(), mode="triangles", blend="update", bin_scale=bin_scale, band=band)
+            torch.cuda.synchronize()
+            res.append((d.cpu().numpy(), di.cpu().numpy(), (c.n_ifp, c.n_tri, c.n_if_elems, c.n_clamped)))
+    (o1, i1, c1), (o2, i2, c2) = res
+    print(f"{n}^3: counts {c1}", flush=True)
+    assert c1 == c2 and c1[1] > 690000
+    assert np.array_equal(o1.view(np.uint64), o2.view(np.uint64))
+    assert np.array_equal(i1.view(np.uint64), i2.view(np.uint64))

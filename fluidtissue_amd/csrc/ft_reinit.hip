@@ -4743,12 +4743,6 @@ int ensure_stage(ft_ctx* c, int stage, const Caps& cp, int mode, bool want_neare
         const LevelPlan lp = level_plan(c, n);
         if (lp.total > (int64_t)UINT32_MAX)
             return ft::set_error(FT_ERR_ARG, "index: too many leaves (%lld)", (long long)lp.total);
-        // the limit of ft_reinit_device_noalloc on the index's bins (about
-        // 128^3 nodes) is part of its contract: 12 bytes a bin
-        if (t_arena && t_arena->used + 12 * (size_t)c->idx_G > t_arena->size)
-            return ft::set_error(FT_ERR_BUDGET, "%lld index bins are more than the %zu-byte scratch of "
-                                 "ft_reinit_device_noalloc takes; use ft_reinit_device", (long long)c->idx_G,
-                                 t_arena->size);
         FT_TRY(ensure(c->bbits, 8 * at_least1(W)));
         FT_TRY(ensure(c->bprefix, 4 * at_least1(W)));
         if (!prim_work_in_xedges(c, n)) {
@@ -4769,8 +4763,8 @@ int ensure_stage(ft_ctx* c, int stage, const Caps& cp, int mode, bool want_neare
         FT_TRY(ensure(c->scan_bsum, sizeof(uint64_t) * nb));
         FT_TRY(ensure(c->deep_part, sizeof(ulonglong2) * 64 * kSplitParts * at_least1(split_tiles_cap(c->n_slots / 64))));
         // last, as the search does without them when the scratch has no room
-        // (a dense interface in large bins: 128^3 at 4 bin edges and 0.6M
-        // triangles take 152 MiB with them and 117 without)
+        // (a dense interface in large bins: 56^3 with 0.74M triangles in bins of
+        // two spacings takes 159 MiB with them, 114 without)
         const size_t titems = sizeof(Item) * (size_t)(n + 4);        // the search reads items by fours
         if (mode == 1 && !has_room(c->titem, titems)) c->titem = DevBuf{};
         else if (mode == 1) FT_TRY(ensure(c->titem, titems));

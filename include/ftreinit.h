@@ -322,7 +322,9 @@ int ft_reinit_device(ft_handle h, double* d_phi, double* d_phi_ifn,
  * the end of the process; the handle's resident mesh is set up beforehand as
  * usual.  Results are those of ft_reinit_device, bit for bit.  A reinit whose
  * workspace exceeds the scratch fails with FT_ERR_BUDGET before phi is
- * written (up to about 128^3 nodes fits, depending on the interface).
+ * written.  It grows with the mesh (4 to 5 bytes a node) and the interface: at
+ * the default bins 128^3 nodes fit with up to about 0.49M triangles (0.64M
+ * crossing points in points mode), 256^3 with 0.18M (0.24M).
  * want_nearest and want_normals must be 0, and ft_get_interface has nothing
  * after this call: those outputs would live in the scratch.  Calls that
  * overlap on one GPU (from several threads or streams) share that scratch and

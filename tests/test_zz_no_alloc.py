@@ -133,3 +133,39 @@ def test_noalloc_takes_dense_interfaces(n, period, noise, bin_scale, band):
     assert c1 == c2 and c1[1] > 690000
     assert np.array_equal(o1.view(np.uint64), o2.view(np.uint64))
     assert np.array_equal(i1.view(np.uint64), i2.view(np.uint64))
+
+
+@pytest.mark.parametrize("mode", ["triangles", "points"])
+def test_noalloc_refuses_by_what_it_takes(mode):
+    """A 200^3 field with a small interface (35 MiB, of which the bitmap of its
+    2^24 bins is 2 and its prefix 1) is taken; a 64^3 one with 1.9M
+    triangles (1.25 a tet, 290 MiB) is not, and phi stays as it was."""
+    import torch
+    n = 200
+    mid = C.c_int32()
+    check(lib.ft_mesh_create_kuhn(0, n, n, n, 0.0, 0, C.byref(mid)))
+    phi = np.linalg.norm(_grid_xyz(n).astype(np.float64) - 0.5, axis=1) - 0.1
+    outs = []
+    with fa.Reinit(0) as r:
+        r.set_batch_meshes([mid.value])
+        for fn in (r.reset_phi_device_noalloc, r.reset_phi_device):
+            d = torch.from_numpy(phi).cuda()
+            torch.cuda.synchronize()
+            fn(d.data_ptr(), None, mode=mode)
+            torch.cuda.synchronize()
+            outs.append(d.cpu().numpy())
+    check(lib.ft_mesh_release(mid.value))
+    assert np.array_equal(outs[0].view(np.uint64), outs[1].view(np.uint64))
+    m = fa.kuhn_mesh(64)
+    phi = np.random.default_rng(2).standard_normal(m.n_nodes)
+    with fa.Reinit(0) as r:
+        r.set_mesh(m)
+        d = torch.from_numpy(phi).cuda()
+        if mode == "triangles":
+            with pytest.raises(_lib.FtError) as e:
+                r.reset_phi_device_noalloc(d.data_ptr(), None, mode=mode)
+            assert e.value.code == _lib.FT_ERR_BUDGET and "scratch" in str(e.value)
+            torch.cuda.synchronize()
+            assert np.array_equal(d.cpu().numpy().view(np.uint64), phi.view(np.uint64))
+        c = r.reset_phi_device(d.data_ptr(), None, mode=mode)
+        assert abs(c.n_tri - 1.25 * len(m.tets)) < 0.01 * len(m.tets)

@@ -4072,8 +4072,8 @@ struct ft_ctx {
     DevBuf bbits, bprefix, pcode, place, prec, titem, trec, pidx;
     DevBuf leaf_cnt, leaf_bin, nfirst, nitem, naxis, stats;
     DevBuf d_grids, d_cnt_off, roots;
-    uint64_t idx_layout = ~0ull;     // layout and bin scale the grids were made for
-    float idx_bin_scale = 0.0f;
+    uint64_t idx_layout = ~0ull;     // layout, bin scale and reach the grids were made for
+    float idx_bin_scale = 0.0f, idx_reach = 0.0f;
     int64_t idx_G = 0;               // bins over all fields (a multiple of 64)
     int64_t idx_words[5] = {0, 0, 0, 0, 0};   // blocks of 64^k bins over all fields
     int idx_top = 1;                 // highest level that holds a field's root
@@ -4223,7 +4223,8 @@ int scan(ft_ctx* c, hipStream_t s, const TI* in, TO* out, int64_t n, TO* d_total
 
 // Uniform cubic grid over a field's box with edge >= `edge` and at most
 // 2^max_lg bins per axis; *lg receives log2 of the Morton side.
-Grid make_grid(const FieldHost& f, float edge, int max_lg, int* lg_out)
+// reach: a power of two (far_reach); the unit of the scaled coordinates is at least this.
+Grid make_grid(const FieldHost& f, float edge, int max_lg, int* lg_out, float reach = 0.0f)
 {
     Grid g{};
     float ext_max = 0.0f;
@@ -4248,7 +4249,7 @@ Grid make_grid(const FieldHost& f, float edge, int max_lg, int* lg_out)
     // stays below 4; the units' reciprocal is a normal number.
     const bool sized = ext_max <= FLT_MAX;
     int ex = 0;
-    (void)std::frexp(sized ? std::max(ext_max, 1e-30f) : FLT_MAX, &ex);   // ext_max < 2^ex
+    (void)std::frexp(sized ? std::max(std::max(ext_max, 0.25f * reach), 1e-30f) : FLT_MAX, &ex);   // ext_max < 2^ex
     for (int k = 0; k < 3; k++) g.org[k] = sized ? f.lo[k] + 0.5f * (f.hi[k] - f.lo[k]) : 0.0f;
     g.inv_s = std::ldexp(1.0f, -std::min(ex + 1, 126));
     g.root_lv = std::max(1, (lg + 1) / 2);
@@ -4619,12 +4620,42 @@ int sort_nodes(ft_ctx* c, bool blocks = true)
 // 1.25.
 constexpr float kDefaultBinScale[2] = {2.0f, 1.25f};
 
-// Per-field bin grids of the index for one bin_scale (0: the mode's default),
-// on the device; cached per field layout.
-int index_setup(ft_ctx* c, hipStream_t s, float bin_scale, int mode)
+// For given points that may lie far outside the mesh: a bound on the distance
+// of every node of the field to its nearest point, as a power of two, if that
+// is more than a unit of make_grid; else 0 (the first point inside the box, or
+// near it, says so).  The search cuts distances along an axis at one unit: with
+// all points beyond it every box would be admitted (48^3 nodes, 6000 points on a
+// sphere 7.5 sides off: 846 us, and 280 with units of that size).
+float far_reach(const FieldHost& f, const float* p, int64_t n)
+{
+    double c[3], ext_max = 0.0, half2 = 0.0, near2 = INFINITY;
+    for (int k = 0; k < 3; k++) {
+        const double e = (double)f.hi[k] - f.lo[k];
+        c[k] = 0.5 * ((double)f.lo[k] + f.hi[k]);
+        ext_max = std::max(ext_max, e);
+        half2 += 0.25 * e * e;
+    }
+    const double near_enough = 2.0 * ext_max - std::sqrt(half2);
+    if (!(near_enough < FLT_MAX)) return 0.0f;
+    for (int64_t j = 0; j < n; j++) {
+        double d2 = 0.0;
+        for (int k = 0; k < 3; k++) d2 += (p[3 * j + k] - c[k]) * (p[3 * j + k] - c[k]);
+        near2 = d2 < near2 ? d2 : near2;                             // (not for a NaN)
+        if (near2 <= near_enough * near_enough) return 0.0f;
+    }
+    const double reach = std::sqrt(near2) + std::sqrt(half2);
+    if (!(reach < 0.25 * FLT_MAX)) return 0.0f;
+    int e = 0;
+    (void)std::frexp((float)reach * (1.0f + 0x1.0p-20f), &e);
+    return std::ldexp(1.0f, e);
+}
+
+// Per-field bin grids of the index for one bin_scale (0: the mode's default)
+// and reach, on the device; cached per field layout.
+int index_setup(ft_ctx* c, hipStream_t s, float bin_scale, int mode, float reach = 0.0f)
 {
     const float bs = bin_scale > 0.0f ? bin_scale : kDefaultBinScale[mode];
-    if (c->idx_layout == c->layout_gen && c->idx_bin_scale == bs) return FT_OK;
+    if (c->idx_layout == c->layout_gen && c->idx_bin_scale == bs && c->idx_reach == reach) return FT_OK;
     const int nf = c->nf;
     const int fb = field_bits(nf);
     // bins of all fields together stay near 2^30
@@ -4635,7 +4666,7 @@ int index_setup(ft_ctx* c, hipStream_t s, float bin_scale, int mode)
     int top = 1;
     for (int k = 0; k < nf; k++) {
         int lg = 0;
-        grids[k] = make_grid(c->fh[k], bs * c->fh[k].h, max_lg, &lg);
+        grids[k] = make_grid(c->fh[k], bs * c->fh[k].h, max_lg, &lg, reach);
         top = std::max(top, grids[k].root_lv);
         const int64_t bins = (int64_t)1 << (3 * lg);
         cnt_off[k + 1] = cnt_off[k] + std::max<int64_t>(64, bins);   // whole bitmap words
@@ -4655,6 +4686,7 @@ int index_setup(ft_ctx* c, hipStream_t s, float bin_scale, int mode)
     c->idx_top = top;
     c->idx_layout = c->layout_gen;
     c->idx_bin_scale = bs;
+    c->idx_reach = reach;
     return FT_OK;
 }
 
@@ -5615,7 +5647,7 @@ int reinit_noalloc(ft_ctx* c, double* d_phi, double* d_phi_ifn, const ft_opts* o
     if (bufs.size() > 64) return ft::set_error(FT_ERR_STATE, "too many call buffers");
     for (size_t i = 0; i < bufs.size(); i++) { saved[i] = *bufs[i]; *bufs[i] = DevBuf{}; }
     const uint64_t idx_layout = c->idx_layout;
-    const float idx_bs = c->idx_bin_scale;
+    const float idx_bs = c->idx_bin_scale, idx_reach = c->idx_reach;
     const int64_t idx_G = c->idx_G;
     int64_t idx_words[kLevels];
     std::copy(c->idx_words, c->idx_words + kLevels, idx_words);
@@ -5633,6 +5665,7 @@ int reinit_noalloc(ft_ctx* c, double* d_phi, double* d_phi_ifn, const ft_opts* o
     for (size_t i = 0; i < bufs.size(); i++) *bufs[i] = saved[i];
     c->idx_layout = idx_layout;
     c->idx_bin_scale = idx_bs;
+    c->idx_reach = idx_reach;
     c->idx_G = idx_G;
     std::copy(idx_words, idx_words + kLevels, c->idx_words);
     c->idx_top = idx_top;
@@ -6536,7 +6569,7 @@ int ft_reset_phi_points(ft_handle h, const float* ifp, int64_t n_ifp, double* ph
     sp.epi = EPI_RAW;
     sp.want_nearest = true;
     uint64_t* sc = h->scalars.as<uint64_t>();
-    FT_TRY(index_setup(h, s, 0.0f, sp.mode));
+    FT_TRY(index_setup(h, s, 0.0f, sp.mode, far_reach(h->fh[0], ifp, n_ifp)));
     FT_TRY(ensure_stage(h, 0, cp, 0, true));
     WordRanges set;
     set.add(sc + S_BLK, 2, 0u);

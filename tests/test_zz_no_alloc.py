@@ -137,7 +137,7 @@ def test_noalloc_takes_dense_interfaces(n, period, noise, bin_scale, band):
 
 @pytest.mark.parametrize("mode", ["triangles", "points"])
 def test_noalloc_refuses_by_what_it_takes(mode):
-    """A 200^3 field with a small interface (35 MiB, of which the bitmap of its
+    """A 200^3 field with a small interface (under 50 MiB, of which the bitmap of its
     2^24 bins is 2 and its prefix 1) is taken; a 64^3 one with 1.9M
     triangles (1.25 a tet, 290 MiB) is not, and phi stays as it was."""
     import torch

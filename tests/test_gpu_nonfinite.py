@@ -122,3 +122,42 @@ def test_box_without_a_size(mode, band, value):
             res.append((np.delete(ifn, far), np.delete(r.nearest(), far)))
     assert np.array_equal(res[0][0].view(np.uint64), res[1][0].view(np.uint64))
     assert np.array_equal(res[0][1], res[1][1])
+
+
+@pytest.mark.parametrize("value", [1e15, 1e20, 1e25, 1e37])
+def test_huge_nodes_beside_others(value):
+    """Nodes whose squares overflow (beyond 1.8e19) or dwarf the rest."""
+    m = fa.kuhn_mesh(15, jitter=0.1, seed=5)
+    rng = np.random.default_rng(8)
+    xyz = m.xyz.copy()
+    bad = rng.random(len(xyz)) < 0.05
+    bad[:8] = True
+    xyz[bad, rng.integers(0, 3, bad.sum())] = value * rng.choice([-1, 1], bad.sum())
+    ifp = rng.random((500, 3)).astype(np.float32)
+    phi = rng.standard_normal(len(xyz))
+    ref = oracle.reset_phi_points(xyz, ifp, phi.copy())
+    ref = ref[0] if isinstance(ref, tuple) else ref
+    with fa.EuclideanDistance(0) as d:
+        d.init(xyz)
+        got = phi.copy()
+        d.reset_phi(ifp, len(ifp), got)
+    assert np.array_equal(got.view(np.uint64), ref.view(np.uint64))
+
+
+@pytest.mark.parametrize("mode", ["points", "triangles"])
+@pytest.mark.parametrize("band", [0.0, 0.2])
+@pytest.mark.parametrize("value", [1e6, 1e22, 1e33, 3e38])
+def test_one_node_far_off(mode, band, value):
+    """A box whose size is one far node's: the others' results stay."""
+    m = fa.kuhn_mesh(14, jitter=0.1, seed=7)
+    phi = np.linalg.norm(m.xyz.astype(np.float64) - 0.5, axis=1) - 0.2
+    xyz = m.xyz.copy()
+    xyz[-1, 2] = value                                  # of tets that do not cross
+    res = []
+    for mesh in (m, fa.Mesh(xyz=xyz, tets=m.tets, edges=m.edges, t2e=m.t2e)):
+        with fa.Reinit(0) as r:
+            r.set_mesh(mesh)
+            _, ifn, _ = r.reset_phi(phi, mode=mode, band=band, want_nearest=True)
+            res.append((ifn[:-1], r.nearest()[:-1]))
+    assert np.array_equal(res[0][0].view(np.uint64), res[1][0].view(np.uint64))
+    assert np.array_equal(res[0][1], res[1][1])

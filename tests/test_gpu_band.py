@@ -114,3 +114,30 @@ def test_bins_schedule_is_for_a_band_to_the_triangles():
             with pytest.raises(fa._lib.FtError) as e:
                 r.reset_phi(phi, mode=mode, band=band, schedule="bins")
             assert e.value.code == fa._lib.FT_ERR_ARG
+
+
+@pytest.mark.parametrize("mode", ["points", "triangles"])
+@pytest.mark.parametrize("sizes", [[26], [24, 9, 31]])
+def test_captured_band_replays(mode, sizes):
+    """A band's two streams inside a captured graph: every replay, on other
+    level sets and with eager work in between, equals the eager call."""
+    import torch
+    meshes = [fa.kuhn_mesh(n, jitter=0.1, seed=n) for n in sizes]
+    xyz = np.concatenate([m.xyz for m in meshes]).astype(np.float64)
+    band = 0.15
+    with fa.Reinit(0) as r, fa.Reinit(0) as e:
+        for h in (r, e):
+            h.set_batch(meshes)
+        d = torch.empty(len(xyz), dtype=torch.float64, device="cuda")
+        di = torch.empty_like(d)
+        for k in range(5):
+            phi = np.linalg.norm(xyz - 0.5, axis=1) - (0.3, 0.31, 0.2, 0.42, 0.3)[k]
+            want, ifn, cnt = e.reset_phi(phi, mode=mode, band=band)
+            d.copy_(torch.from_numpy(phi))
+            torch.cuda.synchronize()
+            per = r.reset_phi_graph_device(d.data_ptr(), di.data_ptr(), mode=mode, band=band)
+            torch.cuda.synchronize()
+            assert np.array_equal(d.cpu().numpy().view(np.uint64), want.view(np.uint64))
+            assert np.array_equal(di.cpu().numpy().view(np.uint64), ifn.view(np.uint64))
+            clamped = [c.n_clamped for c in e.field_counts()]
+            assert [c.n_clamped for c in per] == clamped and sum(clamped) == cnt.n_clamped > 0

@@ -911,8 +911,10 @@ __device__ __forceinline__ void lane_run(uint32_t v, int& first, int& end)
 // Bin of each primitive, marked in the bitmap.  Neighbouring primitives often
 // share their bin: the first lane of a run marks it, and needs no atomic where
 // the word already holds the bit.  The atomics bound it and k_prim_rank: at
-// 256^3 (1.2M triangles) 111 and 58 us with every lane on its own, now 53 and
-// 20; 0.6M points 79 and 34, now 36 and below 20.
+// 256^3 (1.2M triangles) 111 and 58 us with every lane on its own, now 55 and
+// 20; 0.6M points 79 and 34, now 36 and 12.  (That is without the point lists
+// beside them: while k_p2t_count and k_p2t_fill run on the side stream both
+// take 80 to 105 us in some calls.)
 __global__ __launch_bounds__(kBS) void k_prim_bin(int mode, const uint64_t* sc, const float* ifp,
                                                   const int4* tris, const int32_t* ifp2e,
                                                   IndexGeom ig, uint32_t* code, unsigned long long* bits)
@@ -1773,13 +1775,14 @@ __device__ __forceinline__ void wave_lds_sync()
 //
 // Pruning is separated from the exact distances:
 //  - four boxes (the children of a node, or the rectangles of a leaf's
-//    triangles) are taken against the 64 nodes by four 16 x 16 x 4 matrix
-//    instructions: the coordinates of 16 nodes along the 12 box axes at once.
+//    triangles) are taken against the 64 nodes by four 16 x 16 x 16 matrix
+//    instructions on halves (Item): the coordinates of 16 nodes along the 12 box
+//    axes at once.
 //    In the product lane l holds box l / 16 and node l % 16 of the 16, its
 //    three coordinates in three registers, so the distance to the box is 6 or
 //    7 instructions for 64 (node, box) pairs and a compare against the node's
-//    bound.  Crossing points take 16 per instruction: |q|^2 - 2 p.q about the
-//    tile's centre against the bound less |p|^2.
+//    bound.  Crossing points take 16 per FP32 instruction (16 x 16 x 4):
+//    |q|^2 - 2 p.q about the tile's centre against the bound less |p|^2.
 //  - the pairs that pass go to a queue in LDS, and every 64 of them are
 //    evaluated together, one pair per lane, whichever nodes and primitives
 //    they are: a primitive that concerns 9 nodes costs 9 lanes and not 64.
@@ -1798,7 +1801,7 @@ __device__ __forceinline__ void wave_lds_sync()
 //
 // What bounds it: vector issue (76-80% of its rate at 256^3: 12.0k vector
 // instructions per tile).  256^3, 64 spheres, full
-// domain: 6.1 ms, against 9.1-9.5 ms for a wave-wide walk of a binary tree that
+// domain: 5.9-6.3 ms, against 9.1-9.5 ms for a wave-wide walk of a binary tree that
 // tested every box and triangle on all 64 lanes (19.9k instructions per tile);
 // crossing points 3.2 against 3.9 ms.
 template <int MODE, bool STATS, bool RECORDS = false>
@@ -1998,8 +2001,8 @@ struct TileSearch {
         s1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds.range[d][b + 1]);
     }
 
-    // The next leaf of a list: element b of mask, taken out of it; of a split
-    // tile's leaves only those of its part.  False when there is none.
+    // The next leaf of a list: the first element of mask, taken out of it.
+    // False when there is none.
     __device__ __forceinline__ bool next_leaf(uint64_t& mask, int d, uint32_t& s0, uint32_t& s1)
     {
         if (!mask) return false;
@@ -2349,8 +2352,10 @@ __device__ __forceinline__ void search_tile(const QueryArgs& a, int64_t base, Wa
 // its time, so it does not go down to the leaves, which would leave out few
 // more (128^3: 123 us, and 37 down to the nodes above them).
 // Searching every tile, 95 % of which end at the root's children, took 1.86 ms
-// at 256^3 in a 6 h band; this 0.10 ms, their epilogue (k_far_tiles) 0.13 beside
-// the search of the rest, 1.06.  At 128^3 0.32, now 0.04 and 0.22.
+// at 256^3 in a 6 h band; this 0.10 ms, and the search of the rest 1.03 to 1.2,
+// with the others' epilogue (k_far_tiles) beside it: 0.16 ms of its own, or 0.97
+// from its first block to its last where those wait for the search's persistent
+// waves to leave.  At 128^3 0.32, now 0.04 and 0.23.
 __global__ __launch_bounds__(64) void k_tile_near(QueryArgs a, uint32_t last, uint32_t* cls, int32_t* list,
                                                   unsigned long long* count)
 {
@@ -2585,10 +2590,12 @@ __global__ __launch_bounds__(kBS) void k_clamp_sum(int64_t n_tiles, const uint32
 
 // The parts of each split tile combined, one wave per tile: per lane the
 // least key and the least key other than it over the parts' best and second
-// keys (a part's two differ, and a triangle is tested by one part only, the
-// one owning its leaf), then the node's epilogue.  Every triangle that can be
-// the best or a second within the FP64 settle's margin is tested by its part:
-// a part prunes with its own best, which is no better than the tile's.
+// keys, then the node's epilogue.  A part's two differ.  A triangle is tested by
+// one part only, the one owning its leaf, but for the seed, which every part
+// starts with: the same key from several parts counts once (k1, k2 are keys
+// other than the least).  Every triangle that can be the best or a second within
+// the FP64 settle's margin is tested by its part: a part prunes with its own
+// best, which is no better than the tile's.
 template <int MODE>
 __global__ __launch_bounds__(kBS) void k_split_merge(QueryArgs a)
 {
@@ -4483,6 +4490,11 @@ void boxes_from_host(ft_ctx* c, const float* xyz)
 // blocks would be emptier than kBlockFill keep the packed order (*cpb = 0),
 // as does any other field, on a grid of about one node per bin.  The order
 // only affects speed: each node's result is the same in any slot.
+// Blocks against packed slots, a reinit to the triangles: 33^3 (0.77 full) 272
+// and 342 us, 65^3 (0.89) 380 and 467, 129 x 33 x 9 (0.67) 356 and 537; 17^3
+// (0.61) and 25^3 (0.72) the same within 2 %, as are 9^3, 13^3, 129 x 129 x 5 and
+// 900 x 9 x 9 (0.42 to 0.60), where blocks would only take more slots.  37^3
+// (0.79) loses 2 %, to the points 9 %.
 constexpr double kBlockFill = 0.6;
 Grid node_sort_grid(const FieldHost& f, int64_t n, int max_lg, int* lg_out, int* cpb, int64_t* tiles)
 {
@@ -4632,8 +4644,10 @@ int sort_nodes(ft_ctx* c, bool blocks = true)
 // Default bin edge, in node spacings, per distance mode (0 points, 1
 // triangles).  A bin's primitives form one leaf.  Points are cheap to test and
 // their least-squares-plane box tightens with more points, so their
-// optimum is larger: measured on 32^3..256^3 fields, points 2.0-2.5, triangles
-// 1.25.
+// optimum is larger.  A whole reinit (64 spheres), triangles at 1.0 / 1.25 / 1.5 /
+// 2.0 / 2.5: 256^3 7.33 / 7.41 / 7.48 / 7.41 / 8.26 ms, 128^3 1.33 / 1.37 / 1.25 /
+// 1.29 / 1.39, 64^3 0.49 / 0.49 / 0.50 / 0.51 / 0.52; points at 1.5 / 2.0 / 2.5 / 3.0:
+// 256^3 4.59 / 4.14 / 4.14 / 4.31, 128^3 0.86 / 0.82 / 0.82 / 0.83.
 constexpr float kDefaultBinScale[2] = {2.0f, 1.25f};
 
 // For given points that may lie far outside the mesh: a bound on the distance

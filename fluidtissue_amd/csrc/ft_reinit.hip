@@ -2651,7 +2651,9 @@ __device__ __forceinline__ int n2t_slot(int32_t* key, int32_t v)
     return -1;
 }
 
-__global__ __launch_bounds__(kBS) void k_n2t_count(const int4* tets, int64_t T, uint32_t* cnt)
+// twice: raised when a tet names a node twice.
+__global__ __launch_bounds__(kBS) void k_n2t_count(const int4* tets, int64_t T, uint32_t* cnt,
+                                                   unsigned long long* twice)
 {
     static_assert(kN2tHash == 1 << 10, "the slot hash takes 10 bits");
     __shared__ int32_t key[kN2tHash];
@@ -2665,6 +2667,7 @@ __global__ __launch_bounds__(kBS) void k_n2t_count(const int4* tets, int64_t T, 
     if (t < T) {
         const int4 q = tets[t];
         const int32_t v[4] = {q.x, q.y, q.z, q.w};
+        if (q.x == q.y || q.x == q.z || q.x == q.w || q.y == q.z || q.y == q.w || q.z == q.w) *twice = 1ull;
         for (int j = 0; j < 4; j++) {
             const int sl = n2t_slot(key, v[j]);
             if (sl >= 0) atomicAdd(&num[sl], 1u);
@@ -3036,6 +3039,7 @@ struct FemEll {
     const int32_t* ndiag;              // per slice: its diagonals, 0 if they are more than kFemDiags
     const int32_t* diag;               // their offsets col - row, ascending, kFemDiags a slice
     const uint32_t* dmask;             // per row: which of its slice's diagonals it has
+    int twice;                         // a tet of the mesh names a node twice
 };
 __device__ __forceinline__ int64_t ell_at(const FemEll& e, int64_t i, int k)
 {
@@ -3433,14 +3437,23 @@ __device__ void fem_rows(const uint64_t* __restrict__ n2t_off, const uint32_t* _
                 for (int j = 0; j < 4; j++) add[j] = (s02[j] + s13[j]) * detB;
             }
         }
-        // a tet's four nodes are four distinct columns: each of the row's lanes
-        // adds one of them; tets stay in order (the lanes are of one wave, whose
-        // LDS operations are done in order)
+        // a tet's four nodes are four distinct columns, unless a tet of the mesh
+        // names one twice: each of the row's lanes adds one of them (in turn, then);
+        // tets stay in order (the lanes are of one wave, whose LDS operations are
+        // done in order)
         quad_transpose(add, lane);
         const uint32_t pos[4] = {quad_lane<0>(mp), quad_lane<1>(mp), quad_lane<2>(mp), quad_lane<3>(mp)};
-        for (int t = 0; t < 4; t++) {
-            if (r0 + t < na) acc[(pos[t] >> (8 * lane)) & 0xffu] += add[t];
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (!e.twice) {
+            for (int t = 0; t < 4; t++) {
+                if (r0 + t < na) acc[(pos[t] >> (8 * lane)) & 0xffu] += add[t];
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            }
+        } else {
+            for (int t = 0; t < 4; t++)
+                for (int l = 0; l < kFemLanes; l++) {
+                    if (r0 + t < na && lane == l) acc[(pos[t] >> (8 * lane)) & 0xffu] += add[t];
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                }
         }
     }
 }
@@ -4083,6 +4096,7 @@ struct ft_ctx {
     hipEvent_t bcg_ev[kBcgAhead] = {};
     const double* last_phi = nullptr;   // device phi of the last reinit (blended)
     uint64_t n2t_layout = ~0ull;
+    bool tets_twice = false;         // a tet names a node twice (found with the node -> tets lists)
     bool have_normals = false;
     // index
     DevBuf bin_count, bin_prefix;    // the node sort's bins (mesh set-up)
@@ -4865,8 +4879,11 @@ int build_node_tets(ft_ctx* c, hipStream_t s)
     FT_TRY(ensure(c->pcode, sizeof(uint32_t) * at_least1(N)));          // counters
     uint32_t* cnt = c->pcode.as<uint32_t>();
     uint64_t* off = c->n2t_off.as<uint64_t>();
+    // raised in the pinned mirror, read after the wait below
+    unsigned long long* twice = reinterpret_cast<unsigned long long*>(c->h_scalars) + S_P2T;
+    *twice = 0ull;
     FT_TRY(fill<uint32_t>(s, cnt, N, 0u));
-    if (T > 0) hipLaunchKernelGGL(k_n2t_count, dim3(grid1d(T)), dim3(kBS), 0, s, c->tets.as<int4>(), T, cnt);
+    if (T > 0) hipLaunchKernelGGL(k_n2t_count, dim3(grid1d(T)), dim3(kBS), 0, s, c->tets.as<int4>(), T, cnt, twice);
     FT_TRY(scan<uint32_t, uint64_t>(c, s, cnt, off, N, off + N, LoadClear{}));   // cnt: then the fill's cursors
     if (T > 0)
         hipLaunchKernelGGL(k_n2t_fill, dim3(grid1d(T)), dim3(kBS), 0, s, c->tets.as<int4>(), T, off, cnt,
@@ -4874,6 +4891,7 @@ int build_node_tets(ft_ctx* c, hipStream_t s)
     if (N > 0) hipLaunchKernelGGL(k_n2t_sort, dim3(grid1d(N)), dim3(kBS), 0, s, off, N, c->n2t_ids.as<int32_t>());
     FT_TRY(check_launch());
     FT_HIP(hipStreamSynchronize(s));
+    c->tets_twice = *(volatile unsigned long long*)twice != 0ull;
     c->n2t_layout = c->layout_gen;
     return FT_OK;
 }
@@ -6325,7 +6343,7 @@ unsigned fem_grid(int64_t N) { return (unsigned)((N + kFemRowsPerWave - 1) / kFe
 FemEll fem_ell(ft_ctx* h)
 {
     return FemEll{h->fem_len.as<int32_t>(), h->fem_soff.as<uint64_t>(), h->fem_cols.as<int32_t>(),
-                  h->fem_nd.as<int32_t>(), h->fem_diag.as<int32_t>(), h->fem_dmask.as<uint32_t>()};
+                  h->fem_nd.as<int32_t>(), h->fem_diag.as<int32_t>(), h->fem_dmask.as<uint32_t>(), h->tets_twice};
 }
 
 // The sliced-ELL pattern and the mass matrix (LevelSet::init,

@@ -44,3 +44,25 @@ def test_products_match_the_oracle(n, shuffled):
     ro, co, L, b = oracle.advect_system(m.xyz, m.tets, phi, flow, dt)
     res = b - oracle.spmv(ro, co, L, got)
     assert np.linalg.norm(res) <= 1.01 * tol * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("pair", [(0, 1), (1, 2), (2, 3), (0, 3)])
+def test_tets_that_name_a_node_twice(pair):
+    """Their determinant is rarely computed as exactly 0 on a jittered mesh, and
+    then both of the node's terms go into one entry, one after the other."""
+    m = fa.kuhn_mesh(9, jitter=0.2, seed=3)
+    N = len(m.xyz)
+    rng = np.random.default_rng(1)
+    tets = m.tets.copy()
+    k = rng.choice(len(tets), 200, replace=False)
+    tets[k, pair[1]] = tets[k, pair[0]]
+    tets[k[:20], :] = tets[k[:20], :1]                     # one node four times
+    vel = rng.standard_normal(3 * N)
+    ro, co = oracle.fem_pattern(N, tets)
+    with fa.Reinit(0) as r:
+        r.set_mesh(fa.Mesh(xyz=m.xyz, tets=tets, edges=m.edges, t2e=m.t2e))
+        for form, args in ((0, ()), (1, (vel,))):
+            off, cols, got = r.fem_matrix(form, *args)
+            want, _ = oracle.fem_assemble(form, m.xyz, tets, ro, co, *args)
+            assert np.array_equal(off, ro) and np.array_equal(cols, co)
+            assert np.array_equal(got.view(np.uint64), want.view(np.uint64))

@@ -4599,8 +4599,11 @@ int sort_nodes(ft_ctx* c, bool blocks = true)
         max_n = std::max(max_n, n);
     }
     FT_TRY(set_slots(c, slots));
-    if (c->N == 0) return FT_OK;
     hipStream_t s = c->stream;
+    if (c->N == 0) {
+        FT_HIP(hipStreamSynchronize(s));
+        return FT_OK;
+    }
     FT_TRY(ensure(c->bin_count, sizeof(uint32_t) * max_bins));
     FT_TRY(ensure(c->bin_prefix, sizeof(uint32_t) * (max_bins + max_blocks)));
     FT_TRY(ensure(c->pcode, sizeof(uint32_t) * max_n));

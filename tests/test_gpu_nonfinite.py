@@ -61,7 +61,7 @@ def test_field_with_only_nan_points_in_a_batch(mode):
         assert np.array_equal(near[f], near_alone + (before if first else 0))
 
 
-@pytest.mark.parametrize("share", [0.002, 0.3, 0.97])
+@pytest.mark.parametrize("share", [0.002, 0.3, 0.97, 1.0])
 def test_nan_nodes_beside_others(share):
     """Nodes with a NaN coordinate share tiles with finite ones, as their first,
     last or most nodes."""

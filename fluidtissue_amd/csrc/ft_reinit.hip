@@ -1136,6 +1136,14 @@ __global__ __launch_bounds__(kBS) void k_prim_scatter(int mode, const uint64_t* 
     }
     float v3[3][3];
     tri_vertices(tris, ifp, (int32_t)j, v3[0], v3[1], v3[2]);
+    // A triangle with a vertex that is not finite is nobody's nearest, not by its
+    // other vertices' edge either: all its distances are NaN.
+    bool finite = true;
+    for (int q = 0; q < 3; q++)
+        for (int k = 0; k < 3; k++) finite = finite && fabsf(v3[q][k]) < INFINITY;
+    if (!finite)
+        for (int q = 0; q < 3; q++)
+            for (int k = 0; k < 3; k++) v3[q][k] = NAN;
     // Rotate (orientation kept) so that ab is the longest edge, then build the
     // frame in FP64: u along ab, n the unit normal, v = n x u.  Collinear or
     // coincident vertices get a frame along ab and no interior: the distance

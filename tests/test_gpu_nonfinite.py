@@ -161,3 +161,45 @@ def test_one_node_far_off(mode, band, value):
             res.append((ifn[:-1], r.nearest()[:-1]))
     assert np.array_equal(res[0][0].view(np.uint64), res[1][0].view(np.uint64))
     assert np.array_equal(res[0][1], res[1][1])
+
+
+@pytest.mark.parametrize("mode", ["points", "triangles"])
+@pytest.mark.parametrize("band", [0.0, 0.12])
+@pytest.mark.parametrize("share", [0.01, 0.4])
+def test_level_sets_with_nan_and_infinity(mode, band, share):
+    """Crossing points and triangles that are not finite among others: the
+    finite ones' distances are the oracle's."""
+    m = fa.kuhn_mesh(15, jitter=0.1, seed=2)
+    rng = np.random.default_rng(3)
+    phi = fa.phi_field("ellipsoids", m.xyz, seed=5)
+    bad = rng.random(m.n_nodes) < share
+    phi[bad] = rng.choice([np.nan, -np.nan, np.inf, -np.inf], bad.sum())
+    with np.errstate(all="ignore"):
+        ifp, ifp2e = oracle.find_interface_nodes(m.edges, m.xyz, phi)
+        tris, _, _ = oracle.reconstruct_interface(m.tets, m.t2e, m.edges, m.xyz, phi, ifp, ifp2e)
+    with fa.Reinit(0) as r:
+        r.set_mesh(m)
+        _, ifn, cnt = r.reset_phi(phi, mode=mode, band=band, want_nearest=True)
+        near, itf = r.nearest(), r.interface()
+    assert np.array_equal(itf.ifp, ifp, equal_nan=True) and cnt.n_tri == len(tris)
+    assert not np.isfinite(ifp).all()
+    h, nodes = 1.0 / 14, np.arange(m.n_nodes)
+    limit = float(np.float32(band)) if band else FLT_MAX
+    if mode == "points":
+        d, j = oracle.point_distance(m.xyz, ifp, nodes)
+        d = d.astype(np.float64)
+        tol = 0.0
+    else:
+        ok = np.isfinite(ifp[tris[:, :3]]).all((1, 2))
+        assert ok.any() and not ok.all()
+        d, j = oracle.triangle_distance(m.xyz, ifp, np.ascontiguousarray(tris[ok]), nodes)
+        d = np.where(np.isfinite(d), d, FLT_MAX)
+        tol = 1e-5 * h
+    none = near == -1
+    if band:
+        assert none[d > limit + 1e-5 * h].all() and not none[d < limit - 1e-5 * h].any()
+    else:
+        assert not none.any()
+    assert np.all(np.abs(ifn[none]) == limit)
+    assert np.max(np.abs(np.abs(ifn[~none]) - d[~none])) <= tol
+    assert np.array_equal(np.signbit(ifn), phi < 0)
